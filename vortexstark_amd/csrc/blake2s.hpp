@@ -3,8 +3,28 @@
 //
 // All state lives in VGPRs. Rotations lower to v_alignbit_b32 and the
 // three-input adds to v_add3_u32, so one G costs 12 VALU ops; the feed-forward
-// is one v_bitop3_b32 per word: a compression is 960 + 8 VALU ops. The round schedule is written out with compile-time message
-// indices so no message word is ever addressed dynamically.
+// is one v_bitop3_b32 per word: a compression is 960 + 8 VALU ops. The round
+// schedule is written out with compile-time message indices so no message word
+// is ever addressed dynamically.
+//
+// Issue order. A gfx950 SIMD issues a second VALU instruction of another wave
+// beside the one of its first-chosen wave when that second instruction is a
+// plain two-operand add, subtract, logic op, right shift or move (measured:
+// streams of v_add_u32 / v_xor_b32 / v_bitop3_b32 run at 62-66 T lane-ops/s,
+// of v_add3_u32, v_alignbit_b32, v_min_u32 or v_mad_u64_u32 at 30-38 T). The
+// first choice goes to the wave of highest priority, then the oldest, so left
+// alone the younger waves all come to wait at a rotation or a three-input add
+// while the oldest wave owns the SIMD, and nothing pairs: 38 T. The rounds
+// below therefore run row-wise over the four G functions (and over K
+// independent compressions), with the wave's priority raised for the rows only
+// the first slot takes (add3, rotate) and dropped for the rows either slot
+// takes (xor, add): a wave at a rotation goes first and another wave's xors
+// and adds fill the second slot. Measured on one MI355X, node hashes in a
+// loop: 40.1 G/s as single G functions at any occupancy; row-wise with
+// priorities 55.8 / 58.0 / 66.1 / 69.9 G/s at 2 / 3 / 4 / 8 waves a SIMD, and
+// with two compressions interleaved 59.7 / 60.1 / 68.9 / 69.6 G/s. A lone wave
+// a SIMD has nothing to pair with and pays for the s_setprio instructions
+// (about 10 %).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -34,41 +54,115 @@ struct Digest {
         c = c + d;                  \
         b = VX_ROTR(b ^ c, 7);      \
     } while (0)
-#define VX_ROUND(m, s0, s1, s2, s3, s4, s5, s6, s7, s8, s9, s10, s11, s12, s13, s14, s15) \
-    do {                                                                                     \
-        VX_G(v0, v4, v8, v12, m[s0], m[s1]);                                                 \
-        VX_G(v1, v5, v9, v13, m[s2], m[s3]);                                                 \
-        VX_G(v2, v6, v10, v14, m[s4], m[s5]);                                                \
-        VX_G(v3, v7, v11, v15, m[s6], m[s7]);                                                \
-        VX_G(v0, v5, v10, v15, m[s8], m[s9]);                                                \
-        VX_G(v1, v6, v11, v12, m[s10], m[s11]);                                              \
-        VX_G(v2, v7, v8, v13, m[s12], m[s13]);                                               \
-        VX_G(v3, v4, v9, v14, m[s14], m[s15]);                                               \
+
+// Message schedule of round r (RFC 7693, section 2.7).
+constexpr uint8_t B2S_SIGMA[10][16] = {
+    {0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15}, {14, 10, 4, 8, 9, 15, 13, 6, 1, 12, 0, 2, 11, 7, 5, 3},
+    {11, 8, 12, 0, 5, 2, 15, 13, 10, 14, 3, 6, 7, 1, 9, 4}, {7, 9, 3, 1, 13, 12, 11, 14, 2, 6, 5, 10, 4, 0, 15, 8},
+    {9, 0, 5, 7, 2, 4, 10, 15, 14, 1, 11, 12, 6, 8, 3, 13}, {2, 12, 6, 10, 0, 11, 8, 3, 4, 13, 7, 5, 15, 14, 1, 9},
+    {12, 5, 1, 15, 14, 13, 4, 10, 0, 7, 6, 3, 9, 2, 8, 11}, {13, 11, 7, 14, 12, 1, 3, 9, 5, 0, 15, 4, 8, 6, 2, 10},
+    {6, 15, 14, 9, 11, 3, 0, 8, 12, 2, 13, 7, 1, 4, 10, 5}, {10, 2, 8, 4, 7, 6, 1, 5, 15, 11, 9, 14, 3, 12, 13, 0},
+};
+
+// Wave priority p from here on; the barriers keep the rows on their side of it.
+#define VX_PRIO(p)                            \
+    do {                                      \
+        __builtin_amdgcn_sched_barrier(0);    \
+        __builtin_amdgcn_s_setprio(p);        \
+        __builtin_amdgcn_sched_barrier(0);    \
     } while (0)
 
-// h <- compress(h, m, t, f). m must be indexable with constants only.
+// Whether a row of additions takes a message word that is not known to be zero
+// (words NZ .. 15 are): if not, its adds are two-operand ones.
+template <int NZ>
+constexpr bool b2s_row_has_word(int r, int j) {
+    return B2S_SIGMA[r][j] < NZ || B2S_SIGMA[r][j + 2] < NZ || B2S_SIGMA[r][j + 4] < NZ || B2S_SIGMA[r][j + 6] < NZ;
+}
+
+// Half of the G functions of one step of round R, row by row: message words
+// sigma[R][J + 2i], rotations R1 and R2; column i of the state takes b, c, d
+// rotated by SH, 2 SH, 3 SH columns (SH = 0: columns, 1: diagonals). On entry
+// and exit the wave is at priority 1.
+template <int K, int NZ, int R, int J, int SH, int R1, int R2>
+__device__ __forceinline__ void b2s_half(uint32_t v[K][16], const uint32_t m[K][16]) {
+    constexpr bool WORDS = b2s_row_has_word<NZ>(R, J);
+    if (!WORDS) VX_PRIO(0);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int k = 0; k < K; k++) v[k][i] = v[k][i] + v[k][4 + ((i + SH) & 3)] + m[k][B2S_SIGMA[R][J + 2 * i]];
+    if (WORDS) VX_PRIO(0);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int k = 0; k < K; k++) v[k][12 + ((i + 3 * SH) & 3)] ^= v[k][i];
+    VX_PRIO(1);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int k = 0; k < K; k++) v[k][12 + i] = VX_ROTR(v[k][12 + i], R1);
+    VX_PRIO(0);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int k = 0; k < K; k++) v[k][8 + ((i + 2 * SH) & 3)] += v[k][12 + ((i + 3 * SH) & 3)];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int k = 0; k < K; k++) v[k][4 + ((i + SH) & 3)] ^= v[k][8 + ((i + 2 * SH) & 3)];
+    VX_PRIO(1);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int k = 0; k < K; k++) v[k][4 + i] = VX_ROTR(v[k][4 + i], R2);
+}
+template <int K, int NZ, int R>
+__device__ __forceinline__ void b2s_rounds(uint32_t v[K][16], const uint32_t m[K][16]) {
+    if constexpr (R < 10) {
+        b2s_half<K, NZ, R, 0, 0, 16, 12>(v, m);
+        b2s_half<K, NZ, R, 1, 0, 8, 7>(v, m);
+        b2s_half<K, NZ, R, 8, 1, 16, 12>(v, m);
+        b2s_half<K, NZ, R, 9, 1, 8, 7>(v, m);
+        b2s_rounds<K, NZ, R + 1>(v, m);
+    }
+}
+
+// h[k] <- compress(h[k], m[k], t, f) for K independent blocks. Words NZ .. 15
+// of every block are zero. m must be indexable with constants only.
+template <int K, int NZ>
+__device__ __forceinline__ void b2s_compress_n(uint32_t h[K][8], const uint32_t m[K][16], uint32_t t, uint32_t f) {
+    uint32_t v[K][16];
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[k][i] = h[k][i];
+        v[k][8] = B2S_IV0;
+        v[k][9] = B2S_IV1;
+        v[k][10] = B2S_IV2;
+        v[k][11] = B2S_IV3;
+        v[k][12] = B2S_IV4 ^ t;
+        v[k][13] = B2S_IV5;
+        v[k][14] = B2S_IV6 ^ f;
+        v[k][15] = B2S_IV7;
+    }
+    VX_PRIO(1);
+    b2s_rounds<K, NZ, 0>(v, m);
+    VX_PRIO(0);
+#pragma unroll
+    for (int k = 0; k < K; k++)
+#pragma unroll
+        for (int i = 0; i < 8; i++) h[k][i] = VX_XOR3(h[k][i], v[k][i], v[k][8 + i]);
+}
+template <int NZ = 16>
 __device__ __forceinline__ void b2s_compress(uint32_t h[8], const uint32_t m[16], uint32_t t, uint32_t f) {
-    uint32_t v0 = h[0], v1 = h[1], v2 = h[2], v3 = h[3], v4 = h[4], v5 = h[5], v6 = h[6], v7 = h[7];
-    uint32_t v8 = B2S_IV0, v9 = B2S_IV1, v10 = B2S_IV2, v11 = B2S_IV3;
-    uint32_t v12 = B2S_IV4 ^ t, v13 = B2S_IV5, v14 = B2S_IV6 ^ f, v15 = B2S_IV7;
-    VX_ROUND(m, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
-    VX_ROUND(m, 14, 10, 4, 8, 9, 15, 13, 6, 1, 12, 0, 2, 11, 7, 5, 3);
-    VX_ROUND(m, 11, 8, 12, 0, 5, 2, 15, 13, 10, 14, 3, 6, 7, 1, 9, 4);
-    VX_ROUND(m, 7, 9, 3, 1, 13, 12, 11, 14, 2, 6, 5, 10, 4, 0, 15, 8);
-    VX_ROUND(m, 9, 0, 5, 7, 2, 4, 10, 15, 14, 1, 11, 12, 6, 8, 3, 13);
-    VX_ROUND(m, 2, 12, 6, 10, 0, 11, 8, 3, 4, 13, 7, 5, 15, 14, 1, 9);
-    VX_ROUND(m, 12, 5, 1, 15, 14, 13, 4, 10, 0, 7, 6, 3, 9, 2, 8, 11);
-    VX_ROUND(m, 13, 11, 7, 14, 12, 1, 3, 9, 5, 0, 15, 4, 8, 6, 2, 10);
-    VX_ROUND(m, 6, 15, 14, 9, 11, 3, 0, 8, 12, 2, 13, 7, 1, 4, 10, 5);
-    VX_ROUND(m, 10, 2, 8, 4, 7, 6, 1, 5, 15, 11, 9, 14, 3, 12, 13, 0);
-    h[0] = VX_XOR3(h[0], v0, v8);
-    h[1] = VX_XOR3(h[1], v1, v9);
-    h[2] = VX_XOR3(h[2], v2, v10);
-    h[3] = VX_XOR3(h[3], v3, v11);
-    h[4] = VX_XOR3(h[4], v4, v12);
-    h[5] = VX_XOR3(h[5], v5, v13);
-    h[6] = VX_XOR3(h[6], v6, v14);
-    h[7] = VX_XOR3(h[7], v7, v15);
+    uint32_t hk[1][8], mk[1][16];
+#pragma unroll
+    for (int i = 0; i < 8; i++) hk[0][i] = h[i];
+#pragma unroll
+    for (int i = 0; i < 16; i++) mk[0][i] = m[i];
+    b2s_compress_n<1, NZ>(hk, mk, t, f);
+#pragma unroll
+    for (int i = 0; i < 8; i++) h[i] = hk[0][i];
 }
 
 __device__ __forceinline__ void b2s_init(uint32_t h[8]) {
@@ -101,18 +195,45 @@ __device__ __forceinline__ void b2s_node(const uint32_t l[8], const uint32_t r[8
     b2s_compress(out, m, 64u, 0xFFFFFFFFu);
 }
 
+// Leaves of N words each (N <= 4), K at once: K = 1, or both leaves of a pair
+// with their rounds interleaved (two compressions' rows side by side keep more
+// instructions between dependent ones; see the figures above).
+template <int K, int N>
+__device__ __forceinline__ void b2s_leaves(const uint32_t w[K][N], uint32_t out[K][8]) {
+    uint32_t m[K][16];
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) m[k][i] = i < N ? w[k][i < N ? i : 0] : 0u;
+        b2s_init(out[k]);
+    }
+    b2s_compress_n<K, N>(out, m, 4u * N, 0xFFFFFFFFu);
+}
+
 // Leaf of one M31 word (single-column trace tree, t = 4).
 __device__ __forceinline__ void b2s_leaf1(uint32_t v, uint32_t out[8]) {
-    uint32_t m[16] = {v, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    b2s_init(out);
-    b2s_compress(out, m, 4u, 0xFFFFFFFFu);
+    const uint32_t w[1][1] = {{v}};
+    uint32_t h[1][8];
+    b2s_leaves<1, 1>(w, h);
+#pragma unroll
+    for (int i = 0; i < 8; i++) out[i] = h[0][i];
 }
 
 // Leaf of one QM31 (SoA4 trees, t = 16).
 __device__ __forceinline__ void b2s_leaf4(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t out[8]) {
-    uint32_t m[16] = {a, b, c, d, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    b2s_init(out);
-    b2s_compress(out, m, 16u, 0xFFFFFFFFu);
+    const uint32_t w[1][4] = {{a, b, c, d}};
+    uint32_t h[1][8];
+    b2s_leaves<1, 4>(w, h);
+#pragma unroll
+    for (int i = 0; i < 8; i++) out[i] = h[0][i];
+}
+
+// Parent of two leaves of N words.
+template <int N>
+__device__ __forceinline__ void b2s_leaf_pair(const uint32_t w[2][N], uint32_t out[8]) {
+    uint32_t h[2][8];
+    b2s_leaves<2, N>(w, h);
+    b2s_node(h[0], h[1], out);
 }
 
 // ---------------------------------------------------------------- quad-cooperative form
@@ -124,15 +245,6 @@ __device__ __forceinline__ void b2s_leaf4(uint32_t a, uint32_t b, uint32_t c, ui
 // its latency. The message lives in LDS (16 words per quad); every lane of the
 // quad holds all 16 words in registers and selects the ones its two G
 // functions of each round use.
-
-// Message schedule of round r (RFC 7693, section 2.7).
-constexpr uint8_t B2S_SIGMA[10][16] = {
-    {0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15}, {14, 10, 4, 8, 9, 15, 13, 6, 1, 12, 0, 2, 11, 7, 5, 3},
-    {11, 8, 12, 0, 5, 2, 15, 13, 10, 14, 3, 6, 7, 1, 9, 4}, {7, 9, 3, 1, 13, 12, 11, 14, 2, 6, 5, 10, 4, 0, 15, 8},
-    {9, 0, 5, 7, 2, 4, 10, 15, 14, 1, 11, 12, 6, 8, 3, 13}, {2, 12, 6, 10, 0, 11, 8, 3, 4, 13, 7, 5, 15, 14, 1, 9},
-    {12, 5, 1, 15, 14, 13, 4, 10, 0, 7, 6, 3, 9, 2, 8, 11}, {13, 11, 7, 14, 12, 1, 3, 9, 5, 0, 15, 4, 8, 6, 2, 10},
-    {6, 15, 14, 9, 11, 3, 0, 8, 12, 2, 13, 7, 1, 4, 10, 5}, {10, 2, 8, 4, 7, 6, 1, 5, 15, 11, 9, 14, 3, 12, 13, 0},
-};
 
 // value from lane (l + k) % 4 of the same quad. A quad permute reads only lanes
 // of its own quad, so no lane ever reads an invalid source and bound_ctrl

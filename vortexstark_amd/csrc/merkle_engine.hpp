@@ -81,6 +81,12 @@ __device__ __forceinline__ void load8(const uint32_t* src, uint32_t h[8]) {
     h[7] = b.w;
 }
 
+// Parent of the SoA4 leaves of two QM31 values.
+__device__ __forceinline__ void b2s_leaf_pair4(const QM31& x, const QM31& y, uint32_t h[8]) {
+    const uint32_t w[2][4] = {{x.v[0], x.v[1], x.v[2], x.v[3]}, {y.v[0], y.v[1], y.v[2], y.v[3]}};
+    b2s_leaf_pair<4>(w, h);
+}
+
 // ---------------------------------------------------------------- sources
 // pair(i, h): i even; h = parent of items i and i+1.
 // leaf(i, h) / values(i, v): used by decommitment (leaf sources only).
@@ -108,10 +114,8 @@ struct SrcCol1 {
     __device__ __forceinline__ void leaf(uint64_t i, uint32_t h[8]) const { b2s_leaf1(col[i], h); }
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         uint2 v = *(const uint2*)(col + i);
-        uint32_t l[8], r[8];
-        b2s_leaf1(v.x, l);
-        b2s_leaf1(v.y, r);
-        b2s_node(l, r, h);
+        const uint32_t w[2][1] = {{v.x}, {v.y}};
+        b2s_leaf_pair<1>(w, h);
     }
 };
 
@@ -135,10 +139,8 @@ struct SrcSoa4 {
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         uint2 a = *(const uint2*)(c0 + i), b = *(const uint2*)(c1 + i);
         uint2 c = *(const uint2*)(c2 + i), d = *(const uint2*)(c3 + i);
-        uint32_t l[8], r[8];
-        b2s_leaf4(a.x, b.x, c.x, d.x, l);
-        b2s_leaf4(a.y, b.y, c.y, d.y, r);
-        b2s_node(l, r, h);
+        const uint32_t w[2][4] = {{a.x, b.x, c.x, d.x}, {a.y, b.y, c.y, d.y}};
+        b2s_leaf_pair<4>(w, h);
     }
 };
 
@@ -172,10 +174,7 @@ struct SrcQuotient {
         uint2 b = *(const uint2*)(t + ((i + 2) & mask));
         QM31 q0 = quotient_at(a.x, a.y, b.x, al);
         QM31 q1 = quotient_at(a.y, b.x, b.y, al);
-        uint32_t l[8], r[8];
-        b2s_leaf4(q0.v[0], q0.v[1], q0.v[2], q0.v[3], l);
-        b2s_leaf4(q1.v[0], q1.v[1], q1.v[2], q1.v[3], r);
-        b2s_node(l, r, h);
+        b2s_leaf_pair4(q0, q1, h);
     }
 };
 
@@ -220,10 +219,7 @@ struct SrcCircleFold {
         *(uint2*)(o1 + i) = make_uint2(f0.v[1], f1.v[1]);
         *(uint2*)(o2 + i) = make_uint2(f0.v[2], f1.v[2]);
         *(uint2*)(o3 + i) = make_uint2(f0.v[3], f1.v[3]);
-        uint32_t l[8], r[8];
-        b2s_leaf4(f0.v[0], f0.v[1], f0.v[2], f0.v[3], l);
-        b2s_leaf4(f1.v[0], f1.v[1], f1.v[2], f1.v[3], r);
-        b2s_node(l, r, h);
+        b2s_leaf_pair4(f0, f1, h);
     }
 };
 
@@ -254,10 +250,7 @@ struct SrcLineFold {
         *(uint2*)(o1 + i) = make_uint2(f0.v[1], f1.v[1]);
         *(uint2*)(o2 + i) = make_uint2(f0.v[2], f1.v[2]);
         *(uint2*)(o3 + i) = make_uint2(f0.v[3], f1.v[3]);
-        uint32_t l[8], r[8];
-        b2s_leaf4(f0.v[0], f0.v[1], f0.v[2], f0.v[3], l);
-        b2s_leaf4(f1.v[0], f1.v[1], f1.v[2], f1.v[3], r);
-        b2s_node(l, r, h);
+        b2s_leaf_pair4(f0, f1, h);
     }
 };
 
@@ -443,10 +436,7 @@ struct SrcWideFold {
         *(uint2*)(o1 + i) = make_uint2(g0.v[1], g1.v[1]);
         *(uint2*)(o2 + i) = make_uint2(g0.v[2], g1.v[2]);
         *(uint2*)(o3 + i) = make_uint2(g0.v[3], g1.v[3]);
-        uint32_t l[8], r[8];
-        b2s_leaf4(g0.v[0], g0.v[1], g0.v[2], g0.v[3], l);
-        b2s_leaf4(g1.v[0], g1.v[1], g1.v[2], g1.v[3], r);
-        b2s_node(l, r, h);
+        b2s_leaf_pair4(g0, g1, h);
     }
 };
 

@@ -41,7 +41,7 @@ __device__ __forceinline__ void ch_squeeze(const uint32_t st[8], uint32_t n_draw
 #pragma unroll
     for (int i = 9; i < 16; i++) m[i] = 0;
     b2s_init(out);
-    b2s_compress(out, m, 37u, 0xFFFFFFFFu);
+    b2s_compress<9>(out, m, 37u, 0xFFFFFFFFu);
 }
 
 // draw_felt with rejection until all 8 words < 2p (channel.rs:67-86). The
