@@ -29,28 +29,26 @@ void commit_tree(const Src& src, uint64_t n_leaves, LevelStore st, TailOut out, 
         mark("tail");
         return;
     }
-    uint32_t logc = pick_logc(n_leaves, StageLogcMax<Src>::value, batch, stage_uses_plan<Src>());
-    uint64_t waves = n_leaves >> (7 + logc);
-    // deep leaf stages hand on MERKLE_STAGE_KEEP nodes a wave (at most n / 128
-    // in all, the scratch bound of the shallowest stage); the others one
-    const uint32_t keep = logc >= MERKLE_KEEP_LOGC ? MERKLE_STAGE_KEEP : 1u;
-    merkle_stage_kernel<Src><<<dim3(ceil_div(waves, MERKLE_STAGE_WAVES), batch), 64 * MERKLE_STAGE_WAVES, 0, s>>>(
-        src, 0, n_leaves, logc, sc.a, st, bs, keep);
+    auto grid = [&](uint64_t waves) { return dim3(ceil_div(waves, MERKLE_STAGE_WAVES), batch); };
+    StageShape sh = pick_stage(n_leaves, StageLogcMax<Src>::value, batch, stage_uses_plan<Src>(), false);
+    uint64_t waves = n_leaves >> (7 + sh.logc);
+    merkle_stage_kernel<Src><<<grid(waves), 64 * MERKLE_STAGE_WAVES, stage_lds_bytes(sh.logc), s>>>(
+        src, 0, n_leaves, sh.logc, sc.a, st, bs, sh.keep);
     check_launch("merkle_stage_kernel");
     mark("stage_leaf");
-    uint64_t n = waves * keep;
-    uint32_t lvl = 7 + logc - (keep == 1 ? 0u : 4u);  // 16 = 64 >> 2 nodes: two of the six levels done
+    uint64_t n = waves * sh.keep;
+    uint32_t lvl = 7 + sh.logc - floor_log2(sh.keep);
     uint32_t* cur = sc.a;
     uint32_t* nxt = sc.b;
     while (n > PROVER_TAIL_ITEMS) {
-        logc = pick_logc(n, MERKLE_LOGC_MAX, batch);
-        waves = n >> (7 + logc);
-        merkle_stage_kernel<SrcNodes><<<dim3(ceil_div(waves, MERKLE_STAGE_WAVES), batch), 64 * MERKLE_STAGE_WAVES,
-                                        0, s>>>(SrcNodes{cur}, lvl, n, logc, nxt, st, bs, 1u);
+        sh = pick_stage(n, MERKLE_LOGC_MAX, batch, true, true);
+        waves = n >> (7 + sh.logc);
+        merkle_stage_kernel<SrcNodes><<<grid(waves), 64 * MERKLE_STAGE_WAVES, stage_lds_bytes(sh.logc), s>>>(
+            SrcNodes{cur}, lvl, n, sh.logc, nxt, st, bs, sh.keep);
         check_launch("merkle_stage_kernel<nodes>");
         mark("stage_node");
         n = waves;
-        lvl += 7 + logc;
+        lvl += 7 + sh.logc;
         uint32_t* tmp = cur;
         cur = nxt;
         nxt = tmp;
@@ -99,8 +97,13 @@ void commit_line_fold_quad(const SrcLineFold& src, uint64_t n, LevelStore st, Ta
     mark("tail");
 }
 
-// Largest stage output of a tree of n_leaves items (per proof), for sizing
-// the stage scratch buffers.
-inline uint64_t max_stage_nodes(uint64_t n_leaves) { return max_stage_nodes(n_leaves, PROVER_TAIL_ITEMS); }
+// Nodes per proof of the two stage scratch buffers of a tree of n_leaves items:
+// a takes the leaf stage's output and every other node stage's, b the rest.
+inline uint64_t scratch_nodes_a(uint64_t n_leaves) {
+    return std::max<uint64_t>(1, max_leaf_stage_nodes(n_leaves, PROVER_TAIL_ITEMS));
+}
+inline uint64_t scratch_nodes_b(uint64_t n_leaves) {
+    return std::max<uint64_t>(1, max_stage_nodes(scratch_nodes_a(n_leaves), 0));
+}
 
 }  // namespace vx

@@ -42,8 +42,6 @@ namespace vx {
 
 constexpr uint32_t MERKLE_TAIL_MAX = 2048;  // most items one tail-kernel block reduces
 constexpr uint32_t MERKLE_STAGE_WAVES = 4;  // waves per stage workgroup
-constexpr uint32_t MERKLE_STAGE_KEEP = 16;  // nodes a wave of a deep leaf stage hands on
-constexpr uint32_t MERKLE_KEEP_LOGC = 4;    // chunk depth from which leaf stages do so
 
 // Nodes of levels [from, depth] of a tree with 2^depth leaves, level-major.
 struct LevelStore {
@@ -276,7 +274,7 @@ typedef const __attribute__((address_space(1))) u32x4 GlobalV4;
 __device__ __forceinline__ ConstLiftCol* const_table(const LiftCol* t) { return (ConstLiftCol*)t; }
 
 struct SrcLifted {
-    static constexpr uint32_t STAGE_LOGC_MAX = 4;
+    static constexpr uint32_t STAGE_LOGC_MAX = 2;  // 2^22 leaves: depth 1 312 us, 2 306, 3 323, 4 374
     const LiftCol* cols;  // device, hashing order
     uint32_t n_cols;
     __device__ __forceinline__ SrcLifted at(uint64_t) const { return *this; }
@@ -295,31 +293,31 @@ struct SrcLifted {
             }
         }
     }
+    // One block's loads at a time: holding the next block's 32 words as well
+    // (to have them in flight while this one is hashed) costs 146 VGPRs, three
+    // waves a SIMD; without them seven waves share it and cover each other's
+    // loads, and the hashing itself pairs better (34 columns, 2^22 leaves:
+    // 368 -> 306 us).
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         ConstLiftCol* tab = const_table(cols);
         uint32_t ha[8], hb[8];
         b2s_init(ha);
         b2s_init(hb);
-        uint2 cur[16];
-        load_block(tab, 0, i, cur);
         for (uint32_t c0 = 0;; c0 += 16) {
-            // the next block's loads are in flight while this block is hashed
             const bool last = c0 + 16 >= n_cols;
-            uint2 nxt[16];
-            if (!last) load_block(tab, c0 + 16, i, nxt);
+            uint2 v[16];
+            load_block(tab, c0, i, v);
             uint32_t ma[16], mb[16];
 #pragma unroll
             for (uint32_t k = 0; k < 16; k++) {
-                ma[k] = cur[k].x;
-                mb[k] = cur[k].y;
+                ma[k] = v[k].x;
+                mb[k] = v[k].y;
             }
             const uint32_t nw = n_cols - c0 < 16 ? n_cols - c0 : 16;
             const uint32_t t = 4 * (c0 + nw), f = last ? 0xFFFFFFFFu : 0u;
             b2s_compress(ha, ma, t, f);
             b2s_compress(hb, mb, t, f);
             if (last) break;
-#pragma unroll
-            for (uint32_t k = 0; k < 16; k++) cur[k] = nxt[k];
         }
         b2s_node(ha, hb, h);
     }
@@ -341,8 +339,8 @@ __device__ __forceinline__ uint32_t reduce64(uint64_t x) {
 // on the fly from the LDE columns, circle-folded pairwise (2j, 2j + 1) with
 // alpha and tw[j], stored to out and hashed as an SoA4 leaf.
 struct SrcWideFold {
-    static constexpr uint32_t STAGE_LOGC_MAX = 4;
-    const LiftCol* cols;
+    static constexpr uint32_t STAGE_LOGC_MAX = 2;  // 2^21 leaves: depth 1 170 us, 2 180, 3 213
+    const LiftCol* cols;  // ascending in size: the lifted columns come before the full-size ones
     uint32_t n_cols;
     const uint32_t* beta_pows;  // device, 4 words per column
     const uint32_t* alpha;
@@ -352,82 +350,79 @@ struct SrcWideFold {
     uint32_t* o2;
     uint32_t* o3;
     __device__ __forceinline__ SrcWideFold at(uint64_t) const { return *this; }
-    // Column c's values at f indices j .. j + 3 (j a multiple of 4): a full-size
-    // column gives four rows, a lifted one rows r, r + 1 (repeated for j + 2, j + 3).
-    __device__ __forceinline__ u32x4 load_col(ConstLiftCol* tab, uint32_t c, uint64_t j) const {
-        const uint32_t* p = tab[c].p;
-        const uint32_t sh = tab[c].sh;
-        if (sh == 0) return *(GlobalV4*)(p + j);
-        const u32x2 v = *(GlobalV2*)(p + ((j >> sh) << 1));
-        return u32x4{v.x, v.y, 0u, 0u};
-    }
+    // sum_c beta^c * v_c with 64-bit products accumulated unreduced: three
+    // products (< 2^62 each) fit on top of a folded (< 2^33) accumulator, so
+    // accumulators are folded after every group of three columns. A lifted
+    // column gives the four f indices two values (rows r, r + 1, repeated), so
+    // the lifted columns are summed first into two accumulators, which then
+    // start the four of the full-size columns: 32 fewer registers than keeping
+    // both sets, and no prefetched group, leave five waves a SIMD instead of
+    // three (34 columns, 2^21 leaves: 219 -> 180 us).
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         const uint64_t j = 2 * i;  // f index of the first of four inputs (a multiple of 4)
         ConstLiftCol* tab = const_table(cols);
         typedef const __attribute__((address_space(4))) uint32_t ConstU32;
         ConstU32* bp = (ConstU32*)beta_pows;
-        // sum_c beta^c * v_c with 64-bit products accumulated unreduced: three
-        // products (< 2^62 each) fit on top of a folded (< 2^33) accumulator,
-        // so accumulators are folded after every group of three columns.
-        // Full-size columns feed af (four points), lifted ones ag (two).
-        uint64_t af[4][4], ag[2][4];
-#pragma unroll
-        for (int m = 0; m < 4; m++) {
-            for (int k = 0; k < 4; k++) af[k][m] = 0;
-            ag[0][m] = ag[1][m] = 0;
-        }
         constexpr uint32_t G = 3;
-        u32x4 cur[G], nxt[G];
+        uint64_t ag[2][4] = {};
+        uint32_t c = 0;
+        while (c < n_cols && tab[c].sh != 0) {
+            u32x2 v[G];
+            uint32_t n = 0;  // lifted columns in this group
 #pragma unroll
-        for (uint32_t k = 0; k < G; k++)
-            if (k < n_cols) cur[k] = load_col(tab, k, j);
-        for (uint32_t c0 = 0; c0 < n_cols; c0 += G) {
-            // the next group's loads are in flight while this group accumulates
-#pragma unroll
-            for (uint32_t k = 0; k < G; k++)
-                if (c0 + G + k < n_cols) nxt[k] = load_col(tab, c0 + G + k, j);
-            bool tf = false, tl = false;
-#pragma unroll
-            for (uint32_t k = 0; k < G; k++) {
-                const uint32_t c = c0 + k;
-                if (c >= n_cols) break;
-                const uint32_t w[4] = {bp[4 * c], bp[4 * c + 1], bp[4 * c + 2], bp[4 * c + 3]};
-                const u32x4 v = cur[k];
-                if (tab[c].sh == 0) {
-                    tf = true;
-#pragma unroll
-                    for (int m = 0; m < 4; m++) {
-                        af[0][m] += (uint64_t)w[m] * v.x;
-                        af[1][m] += (uint64_t)w[m] * v.y;
-                        af[2][m] += (uint64_t)w[m] * v.z;
-                        af[3][m] += (uint64_t)w[m] * v.w;
-                    }
-                } else {
-                    tl = true;
-#pragma unroll
-                    for (int m = 0; m < 4; m++) {
-                        ag[0][m] += (uint64_t)w[m] * v.x;
-                        ag[1][m] += (uint64_t)w[m] * v.y;
-                    }
+            for (uint32_t g = 0; g < G; g++) {
+                v[g] = u32x2{0u, 0u};
+                if (c + g < n_cols && tab[c + g].sh != 0) {
+                    v[g] = *(GlobalV2*)(tab[c + g].p + ((j >> tab[c + g].sh) << 1));
+                    n = g + 1;
                 }
             }
-            if (tf)
 #pragma unroll
-                for (int m = 0; m < 4; m++)
-                    for (int k = 0; k < 4; k++) af[k][m] = fold62(af[k][m]);
-            if (tl)
+            for (uint32_t g = 0; g < G; g++) {
+                if (g >= n) break;
 #pragma unroll
                 for (int m = 0; m < 4; m++) {
-                    ag[0][m] = fold62(ag[0][m]);
-                    ag[1][m] = fold62(ag[1][m]);
+                    const uint64_t w = bp[4 * (c + g) + m];
+                    ag[0][m] += w * v[g].x;
+                    ag[1][m] += w * v[g].y;
                 }
+            }
 #pragma unroll
-            for (uint32_t k = 0; k < G; k++) cur[k] = nxt[k];
+            for (int m = 0; m < 4; m++) {
+                ag[0][m] = fold62(ag[0][m]);
+                ag[1][m] = fold62(ag[1][m]);
+            }
+            c += n;
+        }
+        uint64_t af[4][4];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            for (int m = 0; m < 4; m++) af[k][m] = ag[k & 1][m];
+        for (; c < n_cols; c += G) {
+            u32x4 v[G];
+#pragma unroll
+            for (uint32_t g = 0; g < G; g++)
+                if (c + g < n_cols) v[g] = *(GlobalV4*)(tab[c + g].p + j);
+#pragma unroll
+            for (uint32_t g = 0; g < G; g++) {
+                if (c + g >= n_cols) break;
+#pragma unroll
+                for (int m = 0; m < 4; m++) {
+                    const uint64_t w = bp[4 * (c + g) + m];
+                    af[0][m] += w * v[g].x;
+                    af[1][m] += w * v[g].y;
+                    af[2][m] += w * v[g].z;
+                    af[3][m] += w * v[g].w;
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < 4; m++)
+                for (int k = 0; k < 4; k++) af[k][m] = fold62(af[k][m]);
         }
         QM31 f[4];
 #pragma unroll
         for (int k = 0; k < 4; k++)
-            for (int m = 0; m < 4; m++) f[k].v[m] = reduce64(af[k][m] + ag[k & 1][m]);
+            for (int m = 0; m < 4; m++) f[k].v[m] = reduce64(af[k][m]);
         const QM31 al = load_alpha(alpha);
         const uint2 w = *(const uint2*)(tw + i);
         const QM31 g0 = fold_pair(f[0], f[1], al, w.x);
@@ -575,10 +570,8 @@ __device__ __forceinline__ void quad_transcript(DevChannel* ch, const uint32_t* 
 }
 
 // ---------------------------------------------------------------- stage kernel
-// LDS per wave: up to logc_max pending chunks + 1 exchange chunk, each 64
-// nodes stored word-major ([word][lane]) so chunk writes are conflict-free.
-// A source may cap logc_max (STAGE_LOGC_MAX) to trade tree depth per wave for
-// occupancy: memory-heavy leaf sources need more waves in flight.
+// A source may cap logc_max (STAGE_LOGC_MAX): leaves that take more work each
+// fill the device at a smaller depth.
 template <class S, class = void>
 struct StageLogcMax {
     static constexpr uint32_t value = MERKLE_LOGC_MAX;
@@ -587,38 +580,36 @@ template <class S>
 struct StageLogcMax<S, std::void_t<decltype(S::STAGE_LOGC_MAX)>> {
     static constexpr uint32_t value = S::STAGE_LOGC_MAX;
 };
-// The tuned depth table is timed on single-column leaves, whose stage is
-// compute-bound; a source that caps its depth is memory-heavy and keeps the
-// occupancy rule of pick_logc (a tuned depth of 4-5 leaves it one wave per
-// SIMD, with its leaf loads exposed).
+// The tuned depth table is timed on single-column leaves; a source that caps
+// its depth takes the default rule of pick_stage instead.
 template <class S>
 constexpr bool stage_uses_plan() {
     return StageLogcMax<S>::value == MERKLE_LOGC_MAX;
 }
-template <class S>
-constexpr uint32_t stage_wave_lds() {
-    return (StageLogcMax<S>::value + 1) * 8 * 64;
-}
+// LDS words of a stage wave: one slot of 64 nodes per pending level of its
+// binary counter, and room for the 64 -> keep reduction (64 nodes and the next
+// level's 32).
+__host__ __device__ inline uint32_t stage_wave_words(uint32_t logc) { return logc >= 2 ? logc * 512 : 768; }
+inline uint32_t stage_lds_bytes(uint32_t logc) { return 4 * MERKLE_STAGE_WAVES * stage_wave_words(logc); }
 
 // blockIdx.y selects the proof of a batch: every per-proof buffer (items,
 // out_nodes, level store) lies blockIdx.y * bs words past proof 0's.
-// A wave hands on `keep` (1 or MERKLE_STAGE_KEEP) nodes of its subtree: the
-// last levels of its 64 -> 1 reduction leave most of the wave's quads idle, and
-// the next stage computes those nodes one per lane instead.
+// A wave hands on `keep` (a power of two <= 32) nodes of its subtree: the last
+// levels of its 64 -> 1 reduction leave most of the wave's quads idle, and the
+// next stage computes those nodes one per lane instead. Dynamic LDS:
+// stage_lds_bytes(logc).
 template <class Src>
 __global__ __launch_bounds__(64 * MERKLE_STAGE_WAVES) void merkle_stage_kernel(Src src0, uint32_t item_level,
                                                                              uint64_t n_items, uint32_t logc,
                                                                              uint32_t* out_nodes, LevelStore st0,
                                                                              uint64_t bs, uint32_t keep) {
-    constexpr uint32_t WAVE_LDS = stage_wave_lds<Src>();
-    __shared__ uint32_t lds[MERKLE_STAGE_WAVES * WAVE_LDS];
+    extern __shared__ uint32_t stage_lds[];
     const uint64_t boff = (uint64_t)blockIdx.y * bs;
     const Src src = src0.at(boff);
     const LevelStore st = st0.shifted(boff);
     out_nodes += boff;
     const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    uint32_t* wl = lds + w * WAVE_LDS;
-    uint32_t* xchg = wl + StageLogcMax<Src>::value * 8 * 64;
+    uint32_t* wl = stage_lds + w * stage_wave_words(logc);
     const uint64_t wave_id = (uint64_t)blockIdx.x * MERKLE_STAGE_WAVES + w;
     const uint64_t base = wave_id << (7 + logc);
     if (base >= n_items) return;  // wave-uniform
@@ -630,17 +621,29 @@ __global__ __launch_bounds__(64 * MERKLE_STAGE_WAVES) void merkle_stage_kernel(S
         uint32_t lvl = item_level + 1, d = 0, k = c;
         if (st.want(lvl)) store8(st.at(lvl, i >> 1), h);
         while (k & 1) {
-            // left sibling chunk waits in slot d, right chunk is h
-#pragma unroll
-            for (int q = 0; q < 8; q++) xchg[q * 64 + lane] = h[q];
-            VX_WAVE_SYNC();
-            const uint32_t* srcc = lane < 32 ? wl + d * 8 * 64 : xchg;
+            // The left sibling chunk waits in slot d, the right chunk is h: lanes
+            // 0-31 take the left chunk's pairs, then h takes the slot and lanes
+            // 32-63 its pairs. Slots hold 64 nodes word-major ([word][lane]).
+            uint32_t* slot = wl + d * 512;
             const uint32_t li = (lane & 31) * 2;
             uint32_t l[8], r[8];
+            if (lane < 32) {
 #pragma unroll
-            for (int q = 0; q < 8; q++) {
-                l[q] = srcc[q * 64 + li];
-                r[q] = srcc[q * 64 + li + 1];
+                for (int q = 0; q < 8; q++) {
+                    l[q] = slot[q * 64 + li];
+                    r[q] = slot[q * 64 + li + 1];
+                }
+            }
+            VX_WAVE_SYNC();
+#pragma unroll
+            for (int q = 0; q < 8; q++) slot[q * 64 + lane] = h[q];
+            VX_WAVE_SYNC();
+            if (lane >= 32) {
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    l[q] = slot[q * 64 + li];
+                    r[q] = slot[q * 64 + li + 1];
+                }
             }
             VX_WAVE_SYNC();
             b2s_node(l, r, h);
@@ -654,7 +657,7 @@ __global__ __launch_bounds__(64 * MERKLE_STAGE_WAVES) void merkle_stage_kernel(S
         }
         if (c + 1 < n_chunks) {
 #pragma unroll
-            for (int q = 0; q < 8; q++) wl[d * 8 * 64 + q * 64 + lane] = h[q];
+            for (int q = 0; q < 8; q++) wl[d * 512 + q * 64 + lane] = h[q];
             VX_WAVE_SYNC();
         }
     }

@@ -537,9 +537,8 @@ void plan_arena(vx_prover* p) {
         const uint32_t d = depth_of(t);
         p->o_store.push_back(take(level_store_words(d, store_from(d))));
     }
-    const uint64_t mx = std::max(max_stage_nodes(p->E), max_line_quad_nodes(p->E));
-    p->o_scr_a = take(8 * (mx ? mx : 1));
-    p->o_scr_b = take(8 * (mx ? mx : 1));
+    p->o_scr_a = take(8 * std::max(scratch_nodes_a(p->E), max_line_quad_nodes(p->E)));
+    p->o_scr_b = take(8 * scratch_nodes_b(p->E));
     p->o_ch = take(sizeof(DevChannel) / 4);
     p->o_alpha = take(4ull * (1 + p->J));
     p->o_queries = take(p->n_q);
@@ -1076,13 +1075,13 @@ int32_t vx_merkle_autotune(uint32_t log_min, uint32_t log_max, float* best_ms) {
         set_error(-2, "vx_merkle_autotune: sizes must satisfy 12 <= log_min <= log_max <= 27");
         return -1;
     }
-    const uint64_t N = 1ull << log_max, mx = max_stage_nodes(N);
+    const uint64_t N = 1ull << log_max;
     hipStream_t st = nullptr;
     uint32_t *data = nullptr, *sa = nullptr, *sb = nullptr, *root = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     bool ok = check(hipStreamCreateWithFlags(&st, hipStreamNonBlocking), "hipStreamCreate") &&
-              check(hipMalloc((void**)&data, 4 * N), "hipMalloc") && check(hipMalloc((void**)&sa, 32 * mx), "hipMalloc") &&
-              check(hipMalloc((void**)&sb, 32 * mx), "hipMalloc") && check(hipMalloc((void**)&root, 32), "hipMalloc") &&
+              check(hipMalloc((void**)&data, 4 * N), "hipMalloc") && check(hipMalloc((void**)&sa, 32 * scratch_nodes_a(N)), "hipMalloc") &&
+              check(hipMalloc((void**)&sb, 32 * scratch_nodes_b(N)), "hipMalloc") && check(hipMalloc((void**)&root, 32), "hipMalloc") &&
               check(hipEventCreate(&e0), "hipEvent") && check(hipEventCreate(&e1), "hipEvent") &&
               check(hipMemsetAsync(data, 0x11, 4 * N, st), "hipMemsetAsync");  // canonical M31 words
     const LevelStore none = {nullptr, 0, 0};

@@ -376,9 +376,9 @@ vx_wide* vx_wide_create(uint32_t n_cols, const uint32_t* log_sizes, uint32_t log
     ok = ok && check(hipHostMalloc((void**)&w->h_src_ptrs, 8ull * n_cols), "hipHostMalloc");
     w->layer.assign(w->J, nullptr);
     for (uint32_t j = 0; ok && j < w->J; j++) ok = w->alloc((void**)&w->layer[j], 16 * w->layer_size(j));
-    const uint64_t mxn = std::max(max_stage_nodes(1ull << S), max_line_quad_nodes(1ull << (S + 1)));
-    ok = ok && w->alloc((void**)&w->scratch.a, 32 * (mxn ? mxn : 1)) &&
-         w->alloc((void**)&w->scratch.b, 32 * (mxn ? mxn : 1));
+    const uint64_t nodes_a = std::max(scratch_nodes_a(1ull << S), max_line_quad_nodes(1ull << (S + 1)));
+    ok = ok && w->alloc((void**)&w->scratch.a, 32 * nodes_a) &&
+         w->alloc((void**)&w->scratch.b, 32 * scratch_nodes_b(1ull << S));
     ok = ok && w->alloc((void**)&w->ch, sizeof(DevChannel)) && w->alloc((void**)&w->chal, 16ull * (w->J + 1)) &&
          w->alloc((void**)&w->beta_pows, 16ull * n_cols) && w->alloc((void**)&w->roots, 32ull * (w->J + 1));
     if (ok) {
