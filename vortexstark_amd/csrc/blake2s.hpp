@@ -24,7 +24,7 @@
 // priorities 55.8 / 58.0 / 66.1 / 69.9 G/s at 2 / 3 / 4 / 8 waves a SIMD, and
 // with two compressions interleaved 59.7 / 60.1 / 68.9 / 69.6 G/s. A lone wave
 // a SIMD has nothing to pair with and pays for the s_setprio instructions
-// (about 10 %).
+// (1.64 -> 2.15 us a compression): PRIO = false.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -83,25 +83,25 @@ constexpr bool b2s_row_has_word(int r, int j) {
 // sigma[R][J + 2i], rotations R1 and R2; column i of the state takes b, c, d
 // rotated by SH, 2 SH, 3 SH columns (SH = 0: columns, 1: diagonals). On entry
 // and exit the wave is at priority 1.
-template <int K, int NZ, int R, int J, int SH, int R1, int R2>
+template <int K, int NZ, bool PRIO, int R, int J, int SH, int R1, int R2>
 __device__ __forceinline__ void b2s_half(uint32_t v[K][16], const uint32_t m[K][16]) {
     constexpr bool WORDS = b2s_row_has_word<NZ>(R, J);
-    if (!WORDS) VX_PRIO(0);
+    if (PRIO && !WORDS) VX_PRIO(0);
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int k = 0; k < K; k++) v[k][i] = v[k][i] + v[k][4 + ((i + SH) & 3)] + m[k][B2S_SIGMA[R][J + 2 * i]];
-    if (WORDS) VX_PRIO(0);
+    if (PRIO && WORDS) VX_PRIO(0);
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int k = 0; k < K; k++) v[k][12 + ((i + 3 * SH) & 3)] ^= v[k][i];
-    VX_PRIO(1);
+    if (PRIO) VX_PRIO(1);
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int k = 0; k < K; k++) v[k][12 + i] = VX_ROTR(v[k][12 + i], R1);
-    VX_PRIO(0);
+    if (PRIO) VX_PRIO(0);
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -110,26 +110,27 @@ __device__ __forceinline__ void b2s_half(uint32_t v[K][16], const uint32_t m[K][
     for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int k = 0; k < K; k++) v[k][4 + ((i + SH) & 3)] ^= v[k][8 + ((i + 2 * SH) & 3)];
-    VX_PRIO(1);
+    if (PRIO) VX_PRIO(1);
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int k = 0; k < K; k++) v[k][4 + i] = VX_ROTR(v[k][4 + i], R2);
 }
-template <int K, int NZ, int R>
+template <int K, int NZ, bool PRIO, int R>
 __device__ __forceinline__ void b2s_rounds(uint32_t v[K][16], const uint32_t m[K][16]) {
     if constexpr (R < 10) {
-        b2s_half<K, NZ, R, 0, 0, 16, 12>(v, m);
-        b2s_half<K, NZ, R, 1, 0, 8, 7>(v, m);
-        b2s_half<K, NZ, R, 8, 1, 16, 12>(v, m);
-        b2s_half<K, NZ, R, 9, 1, 8, 7>(v, m);
-        b2s_rounds<K, NZ, R + 1>(v, m);
+        b2s_half<K, NZ, PRIO, R, 0, 0, 16, 12>(v, m);
+        b2s_half<K, NZ, PRIO, R, 1, 0, 8, 7>(v, m);
+        b2s_half<K, NZ, PRIO, R, 8, 1, 16, 12>(v, m);
+        b2s_half<K, NZ, PRIO, R, 9, 1, 8, 7>(v, m);
+        b2s_rounds<K, NZ, PRIO, R + 1>(v, m);
     }
 }
 
 // h[k] <- compress(h[k], m[k], t, f) for K independent blocks. Words NZ .. 15
-// of every block are zero. m must be indexable with constants only.
-template <int K, int NZ>
+// of every block are zero. m must be indexable with constants only. PRIO =
+// false leaves the priorities alone, for waves that have a SIMD to themselves.
+template <int K, int NZ, bool PRIO = true>
 __device__ __forceinline__ void b2s_compress_n(uint32_t h[K][8], const uint32_t m[K][16], uint32_t t, uint32_t f) {
     uint32_t v[K][16];
 #pragma unroll
@@ -145,22 +146,22 @@ __device__ __forceinline__ void b2s_compress_n(uint32_t h[K][8], const uint32_t 
         v[k][14] = B2S_IV6 ^ f;
         v[k][15] = B2S_IV7;
     }
-    VX_PRIO(1);
-    b2s_rounds<K, NZ, 0>(v, m);
-    VX_PRIO(0);
+    if (PRIO) VX_PRIO(1);
+    b2s_rounds<K, NZ, PRIO, 0>(v, m);
+    if (PRIO) VX_PRIO(0);
 #pragma unroll
     for (int k = 0; k < K; k++)
 #pragma unroll
         for (int i = 0; i < 8; i++) h[k][i] = VX_XOR3(h[k][i], v[k][i], v[k][8 + i]);
 }
-template <int NZ = 16>
+template <int NZ = 16, bool PRIO = true>
 __device__ __forceinline__ void b2s_compress(uint32_t h[8], const uint32_t m[16], uint32_t t, uint32_t f) {
     uint32_t hk[1][8], mk[1][16];
 #pragma unroll
     for (int i = 0; i < 8; i++) hk[0][i] = h[i];
 #pragma unroll
     for (int i = 0; i < 16; i++) mk[0][i] = m[i];
-    b2s_compress_n<1, NZ>(hk, mk, t, f);
+    b2s_compress_n<1, NZ, PRIO>(hk, mk, t, f);
 #pragma unroll
     for (int i = 0; i < 8; i++) h[i] = hk[0][i];
 }
@@ -184,6 +185,7 @@ __device__ __forceinline__ void b2s_leaf(const uint32_t m[16], uint32_t n_words,
 }
 
 // Merkle node: H(left || right), t = 64 (cuda/blake2s.cu:65-89).
+template <bool PRIO = true>
 __device__ __forceinline__ void b2s_node(const uint32_t l[8], const uint32_t r[8], uint32_t out[8]) {
     uint32_t m[16];
 #pragma unroll
@@ -192,7 +194,7 @@ __device__ __forceinline__ void b2s_node(const uint32_t l[8], const uint32_t r[8
         m[8 + i] = r[i];
     }
     b2s_init(out);
-    b2s_compress(out, m, 64u, 0xFFFFFFFFu);
+    b2s_compress<16, PRIO>(out, m, 64u, 0xFFFFFFFFu);
 }
 
 // Leaves of N words each (N <= 4), K at once: K = 1, or both leaves of a pair
@@ -238,19 +240,21 @@ __device__ __forceinline__ void b2s_leaf_pair(const uint32_t w[2][N], uint32_t o
 
 // ---------------------------------------------------------------- quad-cooperative form
 // Four lanes (a quad: lanes 4q..4q+3 of a wave) compute one compression; lane
-// l holds column l of the 4x4 state (v[l], v[4+l], v[8+l], v[12+l]). The
-// diagonal step rotates rows 1..3 by 1..3 lanes with DPP quad permutes and
-// rotates them back afterwards, so a compression is ~400 instructions per lane
-// instead of ~980: used where a tree level is too narrow to fill a wave, cutting
-// its latency. The message lives in LDS (16 words per quad); every lane of the
-// quad holds all 16 words in registers and selects the ones its two G
-// functions of each round use.
+// l holds column l of the 4x4 state (v[l], v[4+l], v[8+l], v[12+l]). Used where
+// a tree level is too narrow to fill a wave: such a level's time is one lone
+// wave's instruction count (about 4 cycles each), which this form cuts from
+// about 980 to about 300.
+//
+// The diagonal step keeps row 1 in place (its rotation ends every half step, so
+// it is the one row the next half waits for) and brings rows 0, 2 and 3 over
+// from lanes l - 1, l + 1, l + 2; the quad permutes fold into the adds and xors
+// that consume the rows (DPP operands), back again in the next column step.
+// Lane l then works on diagonal l - 1, so it takes that diagonal's words.
 
 // value from lane (l + k) % 4 of the same quad. A quad permute reads only lanes
 // of its own quad, so no lane ever reads an invalid source and bound_ctrl
 // changes nothing in the result; set, it lets the compiler fold the move into
-// the add or xor that consumes it (a DPP operand), saving about 40 of the ~450
-// instructions of a compression.
+// the add or xor that consumes it.
 __device__ __forceinline__ uint32_t quad_rot1(uint32_t x) {
     return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x39, 0xF, 0xF, true);
 }
@@ -261,39 +265,78 @@ __device__ __forceinline__ uint32_t quad_rot3(uint32_t x) {
     return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x93, 0xF, 0xF, true);
 }
 
-// mask ? a : b for a mask of all ones or all zeros: one v_bfi_b32
+// mask ? a : b for a mask of all ones or all zeros: one v_bitop3_b32
 __device__ __forceinline__ uint32_t b2s_pick(uint32_t mask, uint32_t a, uint32_t b) {
     return __builtin_amdgcn_bitop3_b32(mask, a, b, 0xCA);
 }
 
-// Message word sigma[R][2l + J] of quad lane l, chosen among the four
-// candidates of the quad with the lane's bit masks (m0: bit 0 of l set, m1:
-// bit 1): three selects on registers, independent of the round's state.
-template <int R, int J>
-__device__ __forceinline__ uint32_t b2s_quad_word(const uint32_t m[16], uint32_t m0, uint32_t m1) {
-    constexpr int w0 = B2S_SIGMA[R][J], w1 = B2S_SIGMA[R][2 + J], w2 = B2S_SIGMA[R][4 + J], w3 = B2S_SIGMA[R][6 + J];
-    return b2s_pick(m1, b2s_pick(m0, m[w3], m[w2]), b2s_pick(m0, m[w1], m[w0]));
+// Word of sigma[r] that lane l takes as its K-th (0, 1: column step; 2, 3: diagonal step).
+__host__ __device__ constexpr int b2s_lane_word(int r, int l, int k) {
+    return k < 2 ? B2S_SIGMA[r][2 * l + k] : B2S_SIGMA[r][8 + 2 * ((l + 3) & 3) + (k - 2)];
 }
 
+// One round on the lane's words x[0..3]. First half of a step: rows 0, 2, 3
+// come from the lanes of the previous step's alignment.
+template <bool FIRST>
+__device__ __forceinline__ void b2s_quad_round(const uint32_t x[4], uint32_t& a, uint32_t& b, uint32_t& c,
+                                               uint32_t& d) {
+    if (FIRST) {
+        a = a + b + x[0];
+        d ^= a;
+    } else {
+        a = quad_rot1(a) + x[0] + b;
+        d = quad_rot2(d) ^ a;
+    }
+    d = VX_ROTR(d, 16);
+    c = (FIRST ? c : quad_rot3(c)) + d;
+    b = VX_ROTR(b ^ c, 12);
+    a = a + b + x[1];
+    d = VX_ROTR(d ^ a, 8);
+    c += d;
+    b = VX_ROTR(b ^ c, 7);
+    a = quad_rot3(a) + x[2] + b;
+    d = VX_ROTR(quad_rot2(d) ^ a, 16);
+    c = quad_rot1(c) + d;
+    b = VX_ROTR(b ^ c, 12);
+    a = a + b + x[3];
+    d = VX_ROTR(d ^ a, 8);
+    c += d;
+    b = VX_ROTR(b ^ c, 7);
+}
+__device__ __forceinline__ void b2s_quad_start(uint32_t t, uint32_t f, uint32_t& c, uint32_t& d) {
+    const uint32_t l = threadIdx.x & 3;
+    const uint32_t m0 = 0u - (l & 1u), m1 = 0u - ((l >> 1) & 1u);
+    c = b2s_pick(m1, b2s_pick(m0, B2S_IV3, B2S_IV2), b2s_pick(m0, B2S_IV1, B2S_IV0));
+    d = b2s_pick(m1, b2s_pick(m0, B2S_IV7, B2S_IV6 ^ f), b2s_pick(m0, B2S_IV5, B2S_IV4 ^ t));
+}
+// Feed-forward; rows 0, 2, 3 leave the last diagonal step's alignment.
+__device__ __forceinline__ void b2s_quad_finish(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t& hl,
+                                                uint32_t& hh) {
+    hl = VX_XOR3(hl, quad_rot1(a), quad_rot3(c));
+    hh = VX_XOR3(hh, b, quad_rot2(d));
+}
+
+// Message word b2s_lane_word(R, l, K) of quad lane l, chosen among the four
+// candidates with the lane's bit masks (m0: bit 0 of l set, m1: bit 1).
+template <int R, int K>
+__device__ __forceinline__ uint32_t b2s_quad_word(const uint32_t m[16], uint32_t m0, uint32_t m1) {
+    constexpr int w0 = b2s_lane_word(R, 0, K), w1 = b2s_lane_word(R, 1, K), w2 = b2s_lane_word(R, 2, K),
+                  w3 = b2s_lane_word(R, 3, K);
+    return b2s_pick(m1, b2s_pick(m0, m[w3], m[w2]), b2s_pick(m0, m[w1], m[w0]));
+}
 template <int R>
-__device__ __forceinline__ void b2s_quad_round(const uint32_t m[16], uint32_t m0, uint32_t m1, uint32_t& a,
-                                               uint32_t& b, uint32_t& c, uint32_t& d) {
+__device__ __forceinline__ void b2s_quad_rounds(const uint32_t m[16], uint32_t m0, uint32_t m1, uint32_t& a,
+                                                uint32_t& b, uint32_t& c, uint32_t& d) {
     if constexpr (R < 10) {
-        // column step: lane l runs G on column l; diagonal step: on diagonal l
-        VX_G(a, b, c, d, (b2s_quad_word<R, 0>(m, m0, m1)), (b2s_quad_word<R, 1>(m, m0, m1)));
-        b = quad_rot1(b);
-        c = quad_rot2(c);
-        d = quad_rot3(d);
-        VX_G(a, b, c, d, (b2s_quad_word<R, 8>(m, m0, m1)), (b2s_quad_word<R, 9>(m, m0, m1)));
-        b = quad_rot3(b);
-        c = quad_rot2(c);
-        d = quad_rot1(d);
-        b2s_quad_round<R + 1>(m, m0, m1, a, b, c, d);
+        const uint32_t x[4] = {b2s_quad_word<R, 0>(m, m0, m1), b2s_quad_word<R, 1>(m, m0, m1),
+                               b2s_quad_word<R, 2>(m, m0, m1), b2s_quad_word<R, 3>(m, m0, m1)};
+        b2s_quad_round<R == 0>(x, a, b, c, d);
+        b2s_quad_rounds<R + 1>(m, m0, m1, a, b, c, d);
     }
 }
 
 // Lane l: in hl = h[l], hh = h[4+l]; out the same words of the new chaining value.
-// msg: the quad's 16 message words (LDS). All four lanes of the quad must be active.
+// msg: the quad's 16 message words. All four lanes of the quad must be active.
 // Every lane reads the whole message into registers before the first round and
 // picks the words of its G functions by selects, so no LDS access waits inside
 // the dependent chain of the rounds.
@@ -303,13 +346,11 @@ __device__ __forceinline__ void b2s_compress_quad(const uint32_t* msg, uint32_t 
     const uint32_t m0 = 0u - (l & 1u), m1 = 0u - ((l >> 1) & 1u);
     uint32_t m[16];
 #pragma unroll
-    for (int i = 0; i < 16; i++) m[i] = msg[i];
-    uint32_t a = hl, b = hh;
-    uint32_t c = b2s_pick(m1, b2s_pick(m0, B2S_IV3, B2S_IV2), b2s_pick(m0, B2S_IV1, B2S_IV0));
-    uint32_t d = b2s_pick(m1, b2s_pick(m0, B2S_IV7, B2S_IV6 ^ f), b2s_pick(m0, B2S_IV5, B2S_IV4 ^ t));
-    b2s_quad_round<0>(m, m0, m1, a, b, c, d);
-    hl = VX_XOR3(hl, a, c);
-    hh = VX_XOR3(hh, b, d);
+    for (int i = 0; i < 16; i++) m[i] = msg[i];  // two words a read: 16-byte reads deliver later
+    uint32_t a = hl, b = hh, c, d;
+    b2s_quad_start(t, f, c, d);
+    b2s_quad_rounds<0>(m, m0, m1, a, b, c, d);
+    b2s_quad_finish(a, b, c, d, hl, hh);
 }
 
 // Initial chaining words of lane l (IV with the parameter block folded in).
@@ -317,6 +358,45 @@ __device__ __forceinline__ void b2s_quad_init(uint32_t& hl, uint32_t& hh) {
     const uint32_t l = threadIdx.x & 3;
     hl = l == 0 ? B2S_H0 : l == 1 ? B2S_IV1 : l == 2 ? B2S_IV2 : B2S_IV3;
     hh = l == 0 ? B2S_IV4 : l == 1 ? B2S_IV5 : l == 2 ? B2S_IV6 : B2S_IV7;
+}
+
+// Leaf of N words (N <= 4, t = 4 N), quad-cooperatively; every lane of the quad
+// holds all of w. Words N .. 15 are zero, so of a round's sixteen words few
+// are not: each word is kept masked per lane, and a lane's word of a round is
+// the or of the (mostly one or no) masked words that can land there.
+template <int N, int R, int K>
+__device__ __forceinline__ uint32_t b2s_leaf_word(const uint32_t mk[N][4]) {
+    uint32_t x = 0;
+#pragma unroll
+    for (int l = 0; l < 4; l++) {
+        const int w = b2s_lane_word(R, l, K);
+        if (w < N) x |= mk[w < N ? w : 0][l];
+    }
+    return x;
+}
+template <int N, int R>
+__device__ __forceinline__ void b2s_leaf_quad_rounds(const uint32_t mk[N][4], uint32_t& a, uint32_t& b, uint32_t& c,
+                                                     uint32_t& d) {
+    if constexpr (R < 10) {
+        const uint32_t x[4] = {b2s_leaf_word<N, R, 0>(mk), b2s_leaf_word<N, R, 1>(mk), b2s_leaf_word<N, R, 2>(mk),
+                               b2s_leaf_word<N, R, 3>(mk)};
+        b2s_quad_round<R == 0>(x, a, b, c, d);
+        b2s_leaf_quad_rounds<N, R + 1>(mk, a, b, c, d);
+    }
+}
+template <int N>
+__device__ __forceinline__ void b2s_leaf_quad(const uint32_t w[N], uint32_t& hl, uint32_t& hh) {
+    const uint32_t l = threadIdx.x & 3;
+    uint32_t mk[N][4];
+#pragma unroll
+    for (int i = 0; i < N; i++)
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) mk[i][k] = l == k ? w[i] : 0u;
+    b2s_quad_init(hl, hh);
+    uint32_t a = hl, b = hh, c, d;
+    b2s_quad_start(4u * N, 0xFFFFFFFFu, c, d);
+    b2s_leaf_quad_rounds<N, 0>(mk, a, b, c, d);
+    b2s_quad_finish(a, b, c, d, hl, hh);
 }
 
 }  // namespace vx

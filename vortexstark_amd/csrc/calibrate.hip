@@ -50,7 +50,7 @@ template <bool QUAD>
 __global__ __launch_bounds__(64) void hash_latency_kernel(uint32_t n, uint32_t* out) {
     const uint32_t lane = threadIdx.x;
     if constexpr (QUAD) {
-        __shared__ uint32_t msg[16 * 16];
+        __shared__ __align__(16) uint32_t msg[16 * 16];
         uint32_t* qm = msg + 16 * (lane >> 2);
         const uint32_t l = lane & 3;
         uint32_t hl, hh;
@@ -77,7 +77,7 @@ __global__ __launch_bounds__(64) void hash_latency_kernel(uint32_t n, uint32_t* 
         for (int k = 0; k < 8; k++) h[k] = lane * 8 + k;
         for (uint32_t i = 0; i < n; i++) {
             uint32_t o[8];
-            b2s_node(h, h, o);
+            b2s_node<false>(h, h, o);
 #pragma unroll
             for (int k = 0; k < 8; k++) h[k] = o[k];
         }

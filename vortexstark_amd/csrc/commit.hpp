@@ -2,6 +2,8 @@
 // kernel over the leaves, stage kernels over node layers while more than
 // PROVER_TAIL_ITEMS nodes remain, and the tail kernel (root + transcript).
 #pragma once
+#include <algorithm>
+
 #include "common.hpp"
 #include "merkle_engine.hpp"
 
@@ -11,6 +13,10 @@ namespace vx {
 // ones are reduced by stage kernels until this many nodes remain (one more
 // tail level is cheaper than one more stage launch).
 constexpr uint32_t PROVER_TAIL_ITEMS = MERKLE_TAIL_MAX;
+
+// Leaf trees of at most this many leaves are one tail launch; larger ones spread
+// their leaves over many CUs first.
+constexpr uint32_t QUAD_DIRECT_MAX = 1024;
 
 struct Scratch {
     uint32_t* a;
@@ -58,49 +64,56 @@ void commit_tree(const Src& src, uint64_t n_leaves, LevelStore st, TailOut out, 
     mark("tail");
 }
 
-// Line-fold layers of at most LINE_QUAD_MAX values (and more than the FRI tail
-// kernel takes) of a single proof commit through line_fold_quad_stage_kernel:
-// 16 leaves a wave up to 2^13 values, 32 at 2^14, so the tail starts from at
-// most 512 nodes. Such a layer's chain is latency-bound for one proof; a batch
-// of proofs fills the device with its waves, where the lane-per-pair stage
-// does the same hashing in fewer instructions (about 980 a compression
-// against 4 x 410), so batches keep it.
-constexpr uint64_t LINE_QUAD_MAX = 1ull << 14;
-inline uint32_t line_quad_leaves(uint64_t n) { return n <= (1ull << 13) ? 16u : 32u; }
-// Stage output (nodes per proof) of the quad line-fold stages of the layers
-// E/4, E/8, ... that take it: 0 if none does.
-inline uint64_t max_line_quad_nodes(uint64_t e) {
-    uint64_t mx = 0;
-    for (uint64_t n = e / 4; n >= 2; n /= 2)
-        if (n <= LINE_QUAD_MAX && n >= 2048) mx = std::max<uint64_t>(mx, n / line_quad_leaves(n));
-    return mx;
-}
+// Trees of at most LEAF_QUAD_MAX leaves (and more than a tail kernel should
+// hash by itself) of a single proof commit through leaf_quad_stage_kernel, 16
+// leaves a wave up to 2^13 leaves, 32 at 2^14, 64 at 2^15, so the tail starts
+// from at most 512 nodes. Such a tree's chain is latency-bound for one proof;
+// a batch of proofs fills the device with its waves, where the lane-per-pair
+// stage does the same hashing in fewer instructions (about 980 a compression
+// against 4 x 390), so batches keep it.
+constexpr uint64_t LEAF_QUAD_MAX = 1ull << 15;
+inline uint32_t quad_stage_leaves(uint64_t n) { return n <= (1ull << 13) ? 16u : n <= (1ull << 14) ? 32u : 64u; }
 
-// Commits a line-fold layer of n values (2048 <= n <= LINE_QUAD_MAX, a power
-// of two) with the quad leaf stage and the tail kernel.
-template <class Mark>
-void commit_line_fold_quad(const SrcLineFold& src, uint64_t n, LevelStore st, TailOut out, Scratch sc, hipStream_t s,
-                           Mark&& mark, uint32_t batch = 1, uint64_t bs = 0) {
-    const uint32_t lpw = line_quad_leaves(n);
+// Commits a tree of n leaves (1024 <= n <= LEAF_QUAD_MAX, a power of two) with
+// the quad leaf stage and the tail kernel. Its stage hands on n / 16 nodes at
+// most, inside the scratch of any tree of n leaves (n / 32 from 2^14 leaves
+// on; scratch_nodes_a covers the smaller ones).
+template <class Src, class Mark>
+void commit_tree_quad(const Src& src, uint64_t n, LevelStore st, TailOut out, Scratch sc, hipStream_t s, Mark&& mark,
+                      uint32_t batch = 1, uint64_t bs = 0) {
+    const uint32_t lpw = quad_stage_leaves(n);
     const uint64_t waves = n / lpw;
-    const dim3 grid((uint32_t)ceil_div(waves, LINE_QUAD_WAVES), batch);
+    const dim3 grid((uint32_t)ceil_div(waves, LEAF_QUAD_WAVES), batch);
     if (lpw == 16)
-        line_fold_quad_stage_kernel<1><<<grid, 64 * LINE_QUAD_WAVES, 0, s>>>(src, n, sc.a, st, bs);
+        leaf_quad_stage_kernel<Src, 1><<<grid, 64 * LEAF_QUAD_WAVES, 0, s>>>(src, n, sc.a, st, bs);
+    else if (lpw == 32)
+        leaf_quad_stage_kernel<Src, 2><<<grid, 64 * LEAF_QUAD_WAVES, 0, s>>>(src, n, sc.a, st, bs);
     else
-        line_fold_quad_stage_kernel<2><<<grid, 64 * LINE_QUAD_WAVES, 0, s>>>(src, n, sc.a, st, bs);
-    check_launch("line_fold_quad_stage_kernel");
+        leaf_quad_stage_kernel<Src, 4><<<grid, 64 * LEAF_QUAD_WAVES, 0, s>>>(src, n, sc.a, st, bs);
+    check_launch("leaf_quad_stage_kernel");
     mark("stage_leaf");
-    const uint32_t lvl = lpw == 16 ? 4u : 5u;
-    merkle_tail_kernel<SrcNodes><<<dim3(1, batch), TAIL_THREADS, 0, s>>>(SrcNodes{sc.a}, lvl, (uint32_t)waves, st, out,
-                                                                         bs);
+    merkle_tail_kernel<SrcNodes><<<dim3(1, batch), TAIL_THREADS, 0, s>>>(SrcNodes{sc.a}, floor_log2(lpw),
+                                                                         (uint32_t)waves, st, out, bs);
     check_launch("merkle_tail_kernel<nodes>");
     mark("tail");
+}
+
+// A tree of a prover: by quads for a single proof's small trees, by commit_tree
+// otherwise; trees of at most direct_max leaves are one tail launch.
+template <class Src, class Mark>
+void commit_leaves(const Src& src, uint64_t n, LevelStore st, TailOut out, Scratch sc, hipStream_t s, Mark&& mark,
+                   uint32_t batch, uint64_t bs) {
+    if (batch == 1 && n > QUAD_DIRECT_MAX && n <= LEAF_QUAD_MAX)
+        commit_tree_quad(src, n, st, out, sc, s, mark, batch, bs);
+    else
+        commit_tree(src, n, st, out, sc, s, mark, batch, bs, QUAD_DIRECT_MAX);
 }
 
 // Nodes per proof of the two stage scratch buffers of a tree of n_leaves items:
 // a takes the leaf stage's output and every other node stage's, b the rest.
 inline uint64_t scratch_nodes_a(uint64_t n_leaves) {
-    return std::max<uint64_t>(1, max_leaf_stage_nodes(n_leaves, PROVER_TAIL_ITEMS));
+    const uint64_t quad = n_leaves <= QUAD_DIRECT_MAX ? 0 : std::min<uint64_t>(n_leaves, LEAF_QUAD_MAX) / 16;
+    return std::max<uint64_t>({1, max_leaf_stage_nodes(n_leaves, QUAD_DIRECT_MAX), quad});
 }
 inline uint64_t scratch_nodes_b(uint64_t n_leaves) {
     return std::max<uint64_t>(1, max_stage_nodes(scratch_nodes_a(n_leaves), 0));

@@ -5,13 +5,16 @@
 // itself. fri_tail_kernel runs every remaining line fold of a proof in one
 // workgroup of 1024 threads: fold (cuda/fri.cu:10-39) into the next layer,
 // hash it as an SoA4 tree (level-store nodes written as by the stage/tail
-// kernels; one leaf per thread; levels wider than the block's 256 quads with
-// one compression per thread, the rest quad-cooperatively across the whole
-// block), reduce to the root, mix the root into the transcript and draw the
-// next challenge, which stays in LDS for the next layer (and is also written
-// to device memory). A 2048-value layer is left to a stage launch and a tree
-// tail: its 4095 compressions in one workgroup are bound by one CU's issue
-// rate (about 34 us, against about 20 us for a stage over 16 CUs and a tail).
+// kernels), reduce to the root, mix the root into the transcript and draw the
+// next challenge. A layer is a chain of about log2(n) + 3 dependent
+// compressions, so what counts is the latency between them: a layer's values
+// stay in LDS for the next fold, the next twiddles are fetched while a layer
+// is hashed, and the transcript's state stays in the registers of one wave
+// (device memory gets all of them, but nothing is read back from it). Leaves
+// of layers of at most 128 values are hashed a quad each (0.68 us for up to
+// 64), larger ones a lane each (1.7 us at one wave a SIMD). A 2048-value layer
+// is left to a stage launch and a tree tail: its 4095 compressions in one
+// workgroup are bound by one CU's issue rate.
 // blockIdx.y selects the proof of a batch (buffers bs words apart).
 #pragma once
 #include "merkle_engine.hpp"
@@ -39,78 +42,102 @@ struct FriTailArgs {
     DevChannel* channel;
 };
 
+constexpr uint32_t FRI_TAIL_QUAD_LEAVES = 128;  // largest layer whose leaves are hashed by quads
+
 static __global__ __launch_bounds__(FRI_TAIL_THREADS) void fri_tail_kernel(FriTailArgs args, uint64_t bs) {
-    constexpr uint32_t QUADS = FRI_TAIL_THREADS / 4;
-    __shared__ uint4 bufa[2 * FRI_TAIL_MAX_ITEMS];  // node-major: node j in bufa[2j], bufa[2j + 1]
-    __shared__ uint4 bufb[FRI_TAIL_MAX_ITEMS];      // half of that
-    __shared__ uint32_t msg[16];
+    constexpr uint32_t W = FRI_TAIL_MAX_ITEMS;
+    __shared__ uint32_t nodes[8 * W];  // wide levels, word-major
+    __shared__ __align__(16) uint32_t qa[8 * TAIL_QUAD_NODES], qb[4 * TAIL_QUAD_NODES];
+    __shared__ __align__(8) uint32_t val[4][W];  // the layer's values
+    __shared__ __align__(16) uint32_t msg[16];
     __shared__ uint32_t al[4];
     const uint32_t tid = threadIdx.x;
     const uint64_t boff = (uint64_t)blockIdx.y * bs;
     DevChannel* ch = (DevChannel*)((uint32_t*)args.channel + boff);
-    if (tid < 4) al[tid] = args.alpha0[boff + tid];
-    __syncthreads();
+    QuadTranscript tr = {};
+    if (tid < 64) {
+        tr.load(ch, false);
+        tr.put_state(msg);
+        if (tid < 4) al[tid] = args.alpha0[boff + tid];
+    }
+    // value index of this thread in a layer of n values: a quad per value in the
+    // layers whose leaves quads hash
+    auto slot = [&](uint32_t n) { return n <= FRI_TAIL_QUAD_LEAVES ? tid >> 2 : tid; };
+    uint32_t n = args.L[0].n;
+    uint32_t k = slot(n);
+    uint2 in[4];
+    uint32_t tw = 0;
+    if (k < n) {
+        tw = args.L[0].tw[k];
+#pragma unroll
+        for (int c = 0; c < 4; c++) in[c] = *(const uint2*)(args.L[0].in[c] + boff + 2 * k);
+    }
+    lds_barrier();
     for (uint32_t li = 0; li < args.n_layers; li++) {
         const FriTailLayer& L = args.L[li];
         const LevelStore st = L.st.shifted(boff);
-        const QM31 alpha = {{al[0], al[1], al[2], al[3]}};
-        const uint32_t* i0 = L.in[0] + boff;
-        const uint32_t* i1 = L.in[1] + boff;
-        const uint32_t* i2 = L.in[2] + boff;
-        const uint32_t* i3 = L.in[3] + boff;
-        uint32_t* cur = (uint32_t*)bufa;
-        uint32_t* nxt = (uint32_t*)bufb;
-        // one leaf per thread, each a fold of two values; their parents are the
-        // first of the parallel levels below (a thread hashing two leaves and
-        // their parent in turn would leave most lanes idle)
-        const uint32_t k = tid;
-        if (k < L.n) {
-            const uint32_t x = 2 * k;
-            const uint2 a = *(const uint2*)(i0 + x), b = *(const uint2*)(i1 + x);
-            const uint2 c = *(const uint2*)(i2 + x), d = *(const uint2*)(i3 + x);
-            const QM31 f = fold_pair({{a.x, b.x, c.x, d.x}}, {{a.y, b.y, c.y, d.y}}, alpha, L.tw[k]);
-            L.out[0][boff + k] = f.v[0];
-            L.out[1][boff + k] = f.v[1];
-            L.out[2][boff + k] = f.v[2];
-            L.out[3][boff + k] = f.v[3];
-            uint32_t h[8];
-            b2s_leaf4(f.v[0], f.v[1], f.v[2], f.v[3], h);
-            bufa[2 * k] = make_uint4(h[0], h[1], h[2], h[3]);
-            bufa[2 * k + 1] = make_uint4(h[4], h[5], h[6], h[7]);
-        }
-        uint32_t m = L.n, lvl = 0;
-        __syncthreads();
-        // wide levels (more compressions than quads): one per thread, all lanes busy
-        while (m > 2 * QUADS) {
-            const uint32_t hm = m / 2;
-            for (uint32_t j = tid; j < hm; j += FRI_TAIL_THREADS) {
-                const uint4* c4 = (const uint4*)cur + 4 * j;
-                const uint4 p0 = c4[0], p1 = c4[1], p2 = c4[2], p3 = c4[3];
-                const uint32_t lh[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
-                const uint32_t rh[8] = {p2.x, p2.y, p2.z, p2.w, p3.x, p3.y, p3.z, p3.w};
+        const bool quads = n <= FRI_TAIL_QUAD_LEAVES;
+        const bool more = li + 1 < args.n_layers;
+        const uint32_t k1 = slot(n / 2);
+        uint32_t tw1 = 0;
+        if (more && k1 < n / 2) tw1 = args.L[li + 1].tw[k1];  // in flight while this layer is hashed
+        uint32_t m = n, lvl = 0;
+        if (k < n) {
+            const QM31 alpha = {{al[0], al[1], al[2], al[3]}};
+            const QM31 f = fold_pair({{in[0].x, in[1].x, in[2].x, in[3].x}}, {{in[0].y, in[1].y, in[2].y, in[3].y}},
+                                     alpha, tw);
+            if (quads) {
+                const uint32_t l = tid & 3;
+                const uint32_t fl = l == 0 ? f.v[0] : l == 1 ? f.v[1] : l == 2 ? f.v[2] : f.v[3];
+                val[l][k] = fl;
+                uint32_t* o = l == 0 ? L.out[0] : l == 1 ? L.out[1] : l == 2 ? L.out[2] : L.out[3];
+                o[boff + k] = fl;
+                uint32_t hl, hh;
+                b2s_leaf_quad<4>(f.v, hl, hh);
+                qa[8 * k + l] = hl;
+                qa[8 * k + 4 + l] = hh;
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    val[c][k] = f.v[c];
+                    L.out[c][boff + k] = f.v[c];
+                }
                 uint32_t h[8];
-                b2s_node(lh, rh, h);
-                if (st.want(lvl + 1)) store8(st.at(lvl + 1, j), h);
-                uint4* n4 = (uint4*)nxt + 2 * j;
-                n4[0] = make_uint4(h[0], h[1], h[2], h[3]);
-                n4[1] = make_uint4(h[4], h[5], h[6], h[7]);
+                b2s_leaf4(f.v[0], f.v[1], f.v[2], f.v[3], h);
+                if (n > TAIL_QUAD_NODES) {
+#pragma unroll
+                    for (int q = 0; q < 8; q++) nodes[q * W + k] = h[q];
+                } else {
+                    store8(qa + 8 * k, h);
+                }
             }
-            __syncthreads();
-            uint32_t* t = cur;
-            cur = nxt;
-            nxt = t;
-            m = hm;
-            lvl++;
         }
-        const uint32_t* root = block_quad_reduce<FRI_TAIL_THREADS>(cur, nxt, m, lvl, 0, st);
-        if (tid < 64) {  // one wave: root and transcript
+        lds_barrier();
+        block_lane_levels<W>(nodes, qa, m, lvl, 0, st);
+        uint64_t idx0 = 0;
+        uint32_t *cur = qa, *nxt = qb;
+        block_quad_reduce(cur, nxt, m, lvl, idx0, st);
+        // the next layer's inputs, before its values overwrite them
+        n /= 2;
+        k = k1;
+        tw = tw1;
+        if (more && k < n) {
+#pragma unroll
+            for (int c = 0; c < 4; c++) in[c] = *(const uint2*)(&val[c][2 * k]);
+        }
+        if (tid < 64) {  // one wave: narrow levels and transcript
+            const uint32_t* root = narrow_reduce(cur, nxt, m, lvl, idx0, st, 1u, msg + 8);
             if (tid < 8) L.root_dst[boff + tid] = root[tid];
-            uint32_t* adst = L.alpha_dst ? L.alpha_dst + boff : nullptr;
-            quad_transcript(ch, root, msg, false, adst);
-            if (adst && tid < 4) al[tid] = adst[tid];  // written by this wave
+            tr.mix(msg);
+            uint32_t w = 0;
+            if (L.alpha_dst && tr.draw(msg, w) && tid < 4) {
+                al[tid] = w;
+                L.alpha_dst[boff + tid] = w;
+            }
         }
-        __syncthreads();
+        lds_barrier();
     }
+    if (tid < 64) tr.store(ch);
 }
 
 // Launches fri_tail_kernel over layers [j0, J) (in chunks of FRI_TAIL_MAX_LAYERS);

@@ -40,6 +40,15 @@ namespace vx {
         __builtin_amdgcn_wave_barrier();                      \
     } while (0)
 
+// Workgroup barrier that orders LDS accesses only. __syncthreads also waits
+// for the block's outstanding device-memory stores, which a chain of levels
+// that never reads them back would wait for once a level.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 constexpr uint32_t MERKLE_TAIL_MAX = 2048;  // most items one tail-kernel block reduces
 constexpr uint32_t MERKLE_STAGE_WAVES = 4;  // waves per stage workgroup
 
@@ -92,6 +101,9 @@ __device__ __forceinline__ void b2s_leaf_pair4(const QM31& x, const QM31& y, uin
 // `off` words further (batched provers give every proof an equal-size arena;
 // shared tables such as twiddles do not move).
 
+// words(i, l, v): the WIDTH words of leaf i, for a quad whose four lanes all call
+// it; a source that stores what it forms stores coordinate l.
+
 struct SrcNodes {
     const uint32_t* nodes;
     __device__ __forceinline__ SrcNodes at(uint64_t off) const { return {nodes + off}; }
@@ -109,6 +121,7 @@ struct SrcCol1 {
     static constexpr uint32_t WIDTH = 1;
     __device__ __forceinline__ SrcCol1 at(uint64_t off) const { return {col + off}; }
     __device__ __forceinline__ void values(uint64_t i, uint32_t v[4]) const { v[0] = col[i]; }
+    __device__ __forceinline__ void words(uint64_t i, uint32_t, uint32_t v[1]) const { v[0] = col[i]; }
     __device__ __forceinline__ void leaf(uint64_t i, uint32_t h[8]) const { b2s_leaf1(col[i], h); }
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         uint2 v = *(const uint2*)(col + i);
@@ -162,6 +175,7 @@ struct SrcQuotient {
         QM31 r = q(i, load_alpha(alpha));
         for (int k = 0; k < 4; k++) v[k] = r.v[k];
     }
+    __device__ __forceinline__ void words(uint64_t i, uint32_t, uint32_t v[4]) const { values(i, v); }
     __device__ __forceinline__ void leaf(uint64_t i, uint32_t h[8]) const {
         QM31 r = q(i, load_alpha(alpha));
         b2s_leaf4(r.v[0], r.v[1], r.v[2], r.v[3], h);
@@ -202,6 +216,20 @@ struct SrcCircleFold {
         for (int k = 0; k < 4; k++) r.v[k] = madd(mmul(aq.v[k], s), mmul(g.v[k], u));
         return r;
     }
+    static constexpr uint32_t WIDTH = 4;
+    __device__ __forceinline__ void words(uint64_t i, uint32_t l, uint32_t v[4]) const {
+        const QM31 aq = load_alpha(alpha_q), g = qmul(load_alpha(alpha_f), aq);
+        const uint64_t j = 2 * i;
+        const uint2 a = *(const uint2*)(t + j);
+        const uint2 b = *(const uint2*)(t + ((j + 2) & mask));
+        const QM31 f = fold_d(msub(b.x, madd(a.y, a.x)), msub(b.y, madd(b.x, a.y)), aq, g, tw[i]);
+        for (int k = 0; k < 4; k++) v[k] = f.v[k];
+        store_coord(i, l, f);
+    }
+    __device__ __forceinline__ void store_coord(uint64_t i, uint32_t l, const QM31& f) const {
+        uint32_t* o = l == 0 ? o0 : l == 1 ? o1 : l == 2 ? o2 : o3;
+        o[i] = l == 0 ? f.v[0] : l == 1 ? f.v[1] : l == 2 ? f.v[2] : f.v[3];
+    }
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         const QM31 aq = load_alpha(alpha_q), g = qmul(load_alpha(alpha_f), aq);
         uint64_t j = 2 * i;  // quotient index of the first of four inputs
@@ -235,6 +263,15 @@ struct SrcLineFold {
     uint32_t* o3;
     __device__ __forceinline__ SrcLineFold at(uint64_t off) const {
         return {i0 + off, i1 + off, i2 + off, i3 + off, alpha + off, tw, o0 + off, o1 + off, o2 + off, o3 + off};
+    }
+    static constexpr uint32_t WIDTH = 4;
+    __device__ __forceinline__ void words(uint64_t i, uint32_t l, uint32_t v[4]) const {
+        const uint2 a = *(const uint2*)(i0 + 2 * i), b = *(const uint2*)(i1 + 2 * i);
+        const uint2 c = *(const uint2*)(i2 + 2 * i), d = *(const uint2*)(i3 + 2 * i);
+        const QM31 f = fold_pair({{a.x, b.x, c.x, d.x}}, {{a.y, b.y, c.y, d.y}}, load_alpha(alpha), tw[i]);
+        for (int k = 0; k < 4; k++) v[k] = f.v[k];
+        uint32_t* o = l == 0 ? o0 : l == 1 ? o1 : l == 2 ? o2 : o3;
+        o[i] = l == 0 ? f.v[0] : l == 1 ? f.v[1] : l == 2 ? f.v[2] : f.v[3];
     }
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         QM31 al = load_alpha(alpha);
@@ -438,114 +475,125 @@ struct SrcWideFold {
 // ---------------------------------------------------------------- narrow levels
 // Reduces n (a power of two <= 64) nodes stored node-major ([node][8 words]) in
 // the LDS buffer `a` to `stop` nodes (a power of two, default one) with the
-// quads of the calling wave, ping-ponging with `b`. The nodes are at tree level
-// `lvl`, node 0 having index idx0 there. Every lane of the wave must call this;
-// returns the buffer holding the remaining nodes.
+// quads of the calling wave, ping-ponging with `b`; a single last node goes to
+// `root` instead when that is given. The buffers are 16-byte aligned. The nodes
+// are at tree level `lvl`, node 0 having index idx0 there. Every lane of the
+// wave must call this; returns the buffer holding the remaining nodes.
+// A level is a lone wave's instruction count, so what does not change from
+// level to level (and the level store's addresses) stays out of it.
 __device__ __forceinline__ uint32_t* narrow_reduce(uint32_t* a, uint32_t* b, uint32_t n, uint32_t lvl, uint64_t idx0,
-                                                   const LevelStore& st, uint32_t stop = 1) {
+                                                   const LevelStore& st, uint32_t stop = 1, uint32_t* root = nullptr) {
     const uint32_t lane = threadIdx.x & 63, quad = lane >> 2, l = lane & 3;
+    if (root && n == 1) {
+        if (lane < 8) root[lane] = a[lane];
+        VX_WAVE_SYNC();
+        return root;
+    }
+    n = __builtin_amdgcn_readfirstlane(n);
+    lvl = __builtin_amdgcn_readfirstlane(lvl);
+    uint32_t h0, h1;
+    b2s_quad_init(h0, h1);
+    // this quad's place in the level store
+    const bool store = st.base != nullptr;
+    uint32_t* dst = store ? st.at(lvl + 1, idx0 >> 1) + 8 * quad + l : nullptr;
     while (n > stop) {
         const uint32_t half = n / 2;
+        uint32_t* out = root && half == 1 ? root : b;
+        const bool want = store && lvl + 1 >= st.from && lvl + 1 <= st.depth;
         for (uint32_t q0 = 0; q0 < half; q0 += 16) {
             const uint32_t q = q0 + quad;
-            const uint32_t qq = q < half ? q : half - 1;  // whole quads stay active for the DPP permutes
-            uint32_t hl, hh;
-            b2s_quad_init(hl, hh);
+            const uint32_t qq = min(q, half - 1);  // whole quads stay active for the DPP permutes
+            uint32_t hl = h0, hh = h1;
             b2s_compress_quad(a + 16 * qq, 64u, 0xFFFFFFFFu, hl, hh);
             if (q < half) {
-                b[8 * q + l] = hl;
-                b[8 * q + 4 + l] = hh;
-                if (st.want(lvl + 1)) {
-                    uint32_t* dst = st.at(lvl + 1, (idx0 >> 1) + q);
-                    dst[l] = hl;
-                    dst[4 + l] = hh;
+                out[8 * q + l] = hl;
+                out[8 * q + 4 + l] = hh;
+                if (want) {
+                    dst[8 * q0] = hl;
+                    dst[8 * q0 + 4] = hh;
                 }
             }
         }
         VX_WAVE_SYNC();
-        uint32_t* t = a;
-        a = b;
-        b = t;
-        n = half;
         lvl++;
         idx0 >>= 1;
+        if (store) dst = st.at(lvl + 1, idx0 >> 1) + 8 * quad + l;
+        b = a;
+        a = out;
+        n = half;
     }
     return a;
 }
 
-// Block-wide form of narrow_reduce: n (a power of two) nodes stored node-major
-// in LDS buffer a are reduced to one, every quad of the block taking one
-// compression per level (ping-ponging with b), so a level of up to
-// THREADS / 4 compressions costs one quad-cooperative compression of latency.
-// The nodes are at tree level lvl, node 0 having index idx0 there; it stops at
-// `stop` nodes (a power of two >= 1). All threads of the block must call it;
-// returns the buffer holding the remaining nodes.
-template <uint32_t THREADS>
-__device__ __forceinline__ uint32_t* block_quad_reduce(uint32_t* a, uint32_t* b, uint32_t& n, uint32_t& lvl,
-                                                       uint64_t& idx0, const LevelStore& st, uint32_t stop) {
-    constexpr uint32_t QUADS = THREADS / 4;
+// One level of a block: the half = n / 2 parents (at most THREADS / 4, and a
+// multiple of 16) of the nodes at `in` go to `out`, a quad per parent; the
+// parents' level is lvl + 1, their first index idx0 >> 1.
+__device__ __forceinline__ void block_quad_level(const uint32_t* in, uint32_t* out, uint32_t half, uint32_t lvl,
+                                                 uint64_t idx0, const LevelStore& st) {
     const uint32_t quad = threadIdx.x >> 2, l = threadIdx.x & 3;
-    const uint32_t wave_q0 = (threadIdx.x >> 6) * 16;  // first quad of this wave
-    while (n > stop) {
-        const uint32_t half = n / 2;
-        for (uint32_t q0 = 0; q0 < half; q0 += QUADS) {
-            if (q0 + wave_q0 >= half) continue;  // wave-uniform: no quad of this wave has a node
-            const uint32_t q = q0 + quad;
-            const uint32_t qq = q < half ? q : half - 1;  // whole quads stay active for the DPP permutes
-            uint32_t hl, hh;
-            b2s_quad_init(hl, hh);
-            b2s_compress_quad(a + 16 * qq, 64u, 0xFFFFFFFFu, hl, hh);
-            if (q < half) {
-                b[8 * q + l] = hl;
-                b[8 * q + 4 + l] = hh;
-                if (st.want(lvl + 1)) {
-                    uint32_t* dst = st.at(lvl + 1, (idx0 >> 1) + q);
-                    dst[l] = hl;
-                    dst[4 + l] = hh;
-                }
-            }
+    if ((threadIdx.x >> 6) * 16 < half) {  // wave-uniform
+        uint32_t hl, hh;
+        b2s_quad_init(hl, hh);
+        b2s_compress_quad(in + 16 * quad, 64u, 0xFFFFFFFFu, hl, hh);
+        out[8 * quad + l] = hl;
+        out[8 * quad + 4 + l] = hh;
+        if (st.want(lvl + 1)) {
+            uint32_t* dst = st.at(lvl + 1, (idx0 >> 1) + quad);
+            dst[l] = hl;
+            dst[4 + l] = hh;
         }
-        __syncthreads();
+    }
+}
+// n nodes (a power of two) node-major in the LDS buffer a down to at most 32,
+// ping-ponging with b: a level costs one quad compression of latency while its
+// waves have a SIMD each. All threads of the block must call it, the buffer
+// complete; afterwards a holds the remaining nodes.
+__device__ __forceinline__ void block_quad_reduce(uint32_t*& a, uint32_t*& b, uint32_t& n, uint32_t& lvl,
+                                                  uint64_t& idx0, const LevelStore& st) {
+    while (n > 32) {
+        block_quad_level(a, b, n / 2, lvl, idx0, st);
+        lds_barrier();
         uint32_t* t = a;
         a = b;
         b = t;
-        n = half;
+        n /= 2;
         lvl++;
         idx0 >>= 1;
     }
-    return a;
-}
-template <uint32_t THREADS>
-__device__ __forceinline__ uint32_t* block_quad_reduce(uint32_t* a, uint32_t* b, uint32_t n, uint32_t lvl,
-                                                       uint64_t idx0, const LevelStore& st) {
-    return block_quad_reduce<THREADS>(a, b, n, lvl, idx0, st, 1u);
 }
 
-// Fiat-Shamir step after a commitment, by one whole wave (quad 0 is the one whose
-// results are kept): optional reset, mix_digest(root) and n_felts draw_felt
-// calls into alpha_dst[4k..4k+4) (channel.rs:30-39, 67-86). root and msg are
-// LDS (8 and 16 words).
-__device__ __forceinline__ void quad_transcript(DevChannel* ch, const uint32_t* root, uint32_t* msg, bool init,
-                                                uint32_t* alpha_dst, uint32_t n_felts = 1) {
-    const uint32_t lane = threadIdx.x & 63, l = lane & 3;
-    if (init && lane == 0) ch->failed = 0;
-    if (lane < 8) msg[lane] = init ? 0u : ch->state[lane];
-    if (lane >= 8 && lane < 16) msg[lane] = root[lane - 8];
-    VX_WAVE_SYNC();
-    uint32_t hl, hh;
-    b2s_quad_init(hl, hh);
-    b2s_compress_quad(msg, 64u, 0xFFFFFFFFu, hl, hh);
-    VX_WAVE_SYNC();
-    // new state words l and 4 + l live in every quad; publish quad 0's
-    if (lane < 4) {
-        msg[l] = hl;
-        msg[4 + l] = hh;
+// The transcript while a wave holds it: lane l of every quad has state words l
+// and 4 + l (channel.rs:15-25). msg (16 LDS words) is the hash input: its first
+// half holds the state, its second takes the root to mix.
+struct QuadTranscript {
+    uint32_t sl, sh, n_draws, failed;
+    __device__ __forceinline__ void load(const DevChannel* ch, bool init) {
+        const uint32_t l = threadIdx.x & 3;
+        sl = init ? 0u : ch->state[l];
+        sh = init ? 0u : ch->state[4 + l];
+        failed = init ? 0u : ch->failed;
+        n_draws = 0;
     }
-    VX_WAVE_SYNC();
-    if (lane < 8) ch->state[lane] = msg[lane];
-    uint32_t n_draws = 0;
-    for (uint32_t k = 0; alpha_dst && k < n_felts; k++) {
-        bool got = false;
+    __device__ __forceinline__ void put_state(uint32_t* msg) const {
+        const uint32_t lane = threadIdx.x & 63, l = lane & 3;
+        if (lane < 4) {
+            msg[l] = sl;
+            msg[4 + l] = sh;
+        }
+    }
+    // mix_digest (channel.rs:30-39): msg holds state || root
+    __device__ __forceinline__ void mix(uint32_t* msg) {
+        VX_WAVE_SYNC();
+        b2s_quad_init(sl, sh);
+        b2s_compress_quad(msg, 64u, 0xFFFFFFFFu, sl, sh);
+        VX_WAVE_SYNC();
+        put_state(msg);
+        n_draws = 0;
+    }
+    // draw_felt (channel.rs:67-86); lane l of every quad gets word l. msg holds
+    // the state. False when the retry budget is exhausted.
+    __device__ __forceinline__ bool draw(uint32_t* msg, uint32_t& w) {
+        const uint32_t lane = threadIdx.x & 63;
         for (int tries = 0; tries < 64; tries++) {
             if (lane < 8) msg[8 + lane] = lane == 0 ? n_draws : 0u;
             VX_WAVE_SYNC();
@@ -556,18 +604,25 @@ __device__ __forceinline__ void quad_transcript(DevChannel* ch, const uint32_t* 
             const uint64_t ok = __ballot(wl < 2u * P && wh < 2u * P);
             VX_WAVE_SYNC();
             if ((ok & 0xFull) == 0xFull) {
-                if (lane < 4) alpha_dst[4 * k + l] = canon(wl);
-                got = true;
-                break;
+                w = canon(wl);
+                return true;
             }
         }
-        if (!got) {
-            if (lane == 0) ch->failed = 1;
-            break;
+        failed = 1;
+        return false;
+    }
+    __device__ __forceinline__ void store(DevChannel* ch) const {
+        const uint32_t lane = threadIdx.x & 63, l = lane & 3;
+        if (lane < 4) {
+            ch->state[l] = sl;
+            ch->state[4 + l] = sh;
+        }
+        if (lane == 0) {
+            ch->n_draws = n_draws;
+            ch->failed = failed;
         }
     }
-    if (lane == 0) ch->n_draws = n_draws;
-}
+};
 
 // ---------------------------------------------------------------- stage kernel
 // A source may cap logc_max (STAGE_LOGC_MAX): leaves that take more work each
@@ -603,7 +658,7 @@ __global__ __launch_bounds__(64 * MERKLE_STAGE_WAVES) void merkle_stage_kernel(S
                                                                              uint64_t n_items, uint32_t logc,
                                                                              uint32_t* out_nodes, LevelStore st0,
                                                                              uint64_t bs, uint32_t keep) {
-    extern __shared__ uint32_t stage_lds[];
+    extern __shared__ __align__(16) uint32_t stage_lds[];
     const uint64_t boff = (uint64_t)blockIdx.y * bs;
     const Src src = src0.at(boff);
     const LevelStore st = st0.shifted(boff);
@@ -669,54 +724,39 @@ __global__ __launch_bounds__(64 * MERKLE_STAGE_WAVES) void merkle_stage_kernel(S
     for (uint32_t k = lane; k < 8 * keep; k += 64) out_nodes[8 * keep * wave_id + k] = top[k];
 }
 
-// ---------------------------------------------------------------- small line folds
-// Leaf stage of a small line-fold layer (fri.cu:10-39 and the SoA4 leaf rule):
-// one leaf per quad, hashed quad-cooperatively, 16 * R leaves a wave reduced to
-// one node. On the few waves such a layer has (one per SIMD), a wave's chain is
-// then one quad compression for the leaves and log2(16 R) node levels, where
-// the lane-per-pair form (128 leaves a wave) takes three lane compressions and
-// seven quad rounds. Value i of the layer: every lane of its quad folds it,
-// lane l stores and hashes coordinate l.
-constexpr uint32_t LINE_QUAD_WAVES = 4;  // waves per workgroup
-template <uint32_t R>
-__global__ __launch_bounds__(64 * LINE_QUAD_WAVES) void line_fold_quad_stage_kernel(SrcLineFold src0, uint64_t n_items,
-                                                                                  uint32_t* out_nodes, LevelStore st0,
-                                                                                  uint64_t bs) {
+// ---------------------------------------------------------------- small leaf stages
+// Leaf stage of a small tree: one leaf per quad, hashed quad-cooperatively,
+// 16 * R leaves a wave reduced to one node. On the few waves such a tree has
+// (at most one per SIMD), a wave's chain is then R quad compressions for the
+// leaves and log2(16 R) node levels, where the lane-per-pair form (128 leaves
+// a wave) takes three lane compressions and seven quad rounds. Every lane of a
+// quad forms its leaf's words.
+constexpr uint32_t LEAF_QUAD_WAVES = 4;  // waves per workgroup
+template <class Src, uint32_t R>
+__global__ __launch_bounds__(64 * LEAF_QUAD_WAVES) void leaf_quad_stage_kernel(Src src0, uint64_t n_items,
+                                                                             uint32_t* out_nodes, LevelStore st0,
+                                                                             uint64_t bs) {
     constexpr uint32_t LPW = 16 * R;  // leaves a wave
-    __shared__ uint32_t lds[LINE_QUAD_WAVES][2 * 8 * LPW + 16 * 16];
+    __shared__ __align__(16) uint32_t lds[LEAF_QUAD_WAVES][8 * LPW + 4 * LPW];
     const uint64_t boff = (uint64_t)blockIdx.y * bs;
-    const SrcLineFold src = src0.at(boff);
+    const Src src = src0.at(boff);
     const LevelStore st = st0.shifted(boff);
     out_nodes += boff;
     const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6, quad = lane >> 2, l = lane & 3;
-    const uint64_t wave_id = (uint64_t)blockIdx.x * LINE_QUAD_WAVES + w;
+    const uint64_t wave_id = (uint64_t)blockIdx.x * LEAF_QUAD_WAVES + w;
     const uint64_t base = wave_id * LPW;
     if (base >= n_items) return;  // wave-uniform
-    uint32_t* na = lds[w];                         // LPW nodes, node-major
-    uint32_t* nb = na + 8 * LPW;                   // the next level
-    uint32_t* msg = nb + 8 * LPW + 16 * quad;      // the quad's leaf message
-    const QM31 al = load_alpha(src.alpha);
-    uint32_t* out = l == 0 ? src.o0 : l == 1 ? src.o1 : l == 2 ? src.o2 : src.o3;
+    uint32_t* na = lds[w];        // LPW nodes, node-major
+    uint32_t* nb = na + 8 * LPW;  // the next level
     for (uint32_t r = 0; r < R; r++) {
-        const uint64_t i = base + 16 * r + quad;
-        const uint2 a = *(const uint2*)(src.i0 + 2 * i), b = *(const uint2*)(src.i1 + 2 * i);
-        const uint2 c = *(const uint2*)(src.i2 + 2 * i), d = *(const uint2*)(src.i3 + 2 * i);
-        const QM31 f = fold_pair({{a.x, b.x, c.x, d.x}}, {{a.y, b.y, c.y, d.y}}, al, src.tw[i]);
-        const uint32_t fl = l == 0 ? f.v[0] : l == 1 ? f.v[1] : l == 2 ? f.v[2] : f.v[3];
-        out[i] = fl;
-        msg[l] = fl;
-        msg[4 + l] = 0;
-        msg[8 + l] = 0;
-        msg[12 + l] = 0;
-        VX_WAVE_SYNC();
-        uint32_t hl, hh;
-        b2s_quad_init(hl, hh);
-        b2s_compress_quad(msg, 16u, 0xFFFFFFFFu, hl, hh);
         const uint32_t k = 16 * r + quad;
+        uint32_t v[Src::WIDTH], hl, hh;
+        src.words(base + k, l, v);
+        b2s_leaf_quad<Src::WIDTH>(v, hl, hh);
         na[8 * k + l] = hl;
         na[8 * k + 4 + l] = hh;
-        VX_WAVE_SYNC();  // the message is rewritten next round; the leaves are read below
     }
+    VX_WAVE_SYNC();
     const uint32_t* top = narrow_reduce(na, nb, LPW, 0, base, st);
     if (lane < 8) out_nodes[8 * wave_id + lane] = top[lane];
 }
@@ -731,45 +771,25 @@ struct TailOut {
 };
 
 constexpr uint32_t TAIL_THREADS = 1024;
+// Most nodes of a level whose parents are hashed by quads: 128 parents are eight
+// waves, two a SIMD (measured against one parent a lane at the same width, the
+// quads of 128 parents are faster, of 256 slower).
+constexpr uint32_t TAIL_QUAD_NODES = 256;
 
-// Block b reduces items [b * n_items, (b + 1) * n_items) to one root (the
-// tiled form used by the reference-ABI entry points runs many blocks; the
-// prover runs one). n_items is a power of two in [2, MERKLE_TAIL_MAX].
-// blockIdx.y selects the proof of a batch as in merkle_stage_kernel; the root,
-// transcript and challenge destinations move with it.
-template <class Src>
-__global__ __launch_bounds__(TAIL_THREADS) void merkle_tail_kernel(Src src0, uint32_t item_level, uint32_t n_items,
-                                                                  LevelStore st0, TailOut out, uint64_t bs) {
-    constexpr uint32_t W = MERKLE_TAIL_MAX / 2;
-    constexpr uint32_t QUADS = TAIL_THREADS / 4;
-    const uint64_t boff = (uint64_t)blockIdx.y * bs;
-    const Src src = src0.at(boff);
-    const LevelStore st = st0.shifted(boff);
-    if (boff) {
-        if (out.root_dst) out.root_dst += boff;
-        if (out.channel) out.channel = (DevChannel*)((uint32_t*)out.channel + boff);
-        if (out.alpha_dst) out.alpha_dst += boff;
-    }
-    __shared__ uint32_t nodes[8 * W];  // wide levels, word-major: word q of node j at q * W + j
-    __shared__ uint4 qa[4 * QUADS];    // quad levels, node-major: up to 2 * QUADS nodes
-    __shared__ uint4 qb[2 * QUADS];
-    __shared__ uint32_t na[8 * 64], nb[8 * 64];
-    __shared__ uint32_t msg[16];
+template <class S>
+struct IsNodes : std::false_type {};
+template <>
+struct IsNodes<SrcNodes> : std::true_type {};
+
+// Lane-per-parent levels of a block: m nodes word-major in `nodes` (word q of
+// node j at q * W + j) down to TAIL_QUAD_NODES nodes, which end node-major in
+// out; the caller synchronises before. The nodes are at level lvl.
+template <uint32_t W>
+__device__ __forceinline__ void block_lane_levels(uint32_t* nodes, uint32_t* out, uint32_t& m, uint32_t& lvl,
+                                                  uint64_t idx0, const LevelStore& st) {
     const uint32_t tid = threadIdx.x;
-    const uint64_t item_base = (uint64_t)blockIdx.x * n_items;
-    uint32_t n = n_items / 2;
-    uint32_t lvl = item_level + 1;
-    for (uint32_t j = tid; j < n; j += TAIL_THREADS) {
-        uint32_t h[8];
-        src.pair(item_base + 2ull * j, h);
-        if (st.want(lvl)) store8(st.at(lvl, (item_base >> 1) + j), h);
-#pragma unroll
-        for (int q = 0; q < 8; q++) nodes[q * W + j] = h[q];
-    }
-    __syncthreads();
-    // wide levels (more compressions than the block has quads): one per thread
-    while (n > 2 * QUADS) {
-        const uint32_t half = n / 2;
+    while (m > TAIL_QUAD_NODES) {
+        const uint32_t half = m / 2;
         uint32_t l[8], r[8];
         if (tid < half) {
 #pragma unroll
@@ -778,42 +798,92 @@ __global__ __launch_bounds__(TAIL_THREADS) void merkle_tail_kernel(Src src0, uin
                 r[q] = nodes[q * W + 2 * tid + 1];
             }
         }
-        __syncthreads();
+        lds_barrier();
         lvl++;
+        idx0 >>= 1;
         if (tid < half) {
             uint32_t h[8];
-            b2s_node(l, r, h);
+            if (half > TAIL_QUAD_NODES) {
+                b2s_node(l, r, h);
 #pragma unroll
-            for (int q = 0; q < 8; q++) nodes[q * W + tid] = h[q];
-            if (st.want(lvl)) store8(st.at(lvl, (item_base >> (lvl - item_level)) + tid), h);
+                for (int q = 0; q < 8; q++) nodes[q * W + tid] = h[q];
+            } else {
+                b2s_node<false>(l, r, h);  // one wave a SIMD
+                store8(out + 8 * tid, h);
+            }
+            if (st.want(lvl)) store8(st.at(lvl, idx0 + tid), h);
         }
-        __syncthreads();
-        n = half;
+        lds_barrier();
+        m = half;
     }
-    // levels of 32 to 256 compressions: quad-cooperative across the whole block
-    uint64_t idx0 = item_base >> (lvl - item_level);
-    uint32_t* cur = na;
-    if (n > 64) {
-        uint32_t* qaw = (uint32_t*)qa;
-        for (uint32_t j = tid; j < n; j += TAIL_THREADS)
-#pragma unroll
-            for (int q = 0; q < 8; q++) qaw[8 * j + q] = nodes[q * W + j];
-        __syncthreads();
-        cur = block_quad_reduce<TAIL_THREADS>(qaw, (uint32_t*)qb, n, lvl, idx0, st, 64u);
+}
+
+// Block b reduces items [b * n_items, (b + 1) * n_items) to one root (the
+// tiled form used by the reference-ABI entry points runs many blocks; the
+// prover runs one). n_items is a power of two in [2, MERKLE_TAIL_MAX].
+// blockIdx.y selects the proof of a batch as in merkle_stage_kernel; the root,
+// transcript and challenge destinations move with it.
+//
+// A chain of dependent levels: one lane compression (about 1.7 us) a level
+// while it has more than 128 parents, one quad compression (0.68 us) below,
+// then the transcript's two. The transcript's state is fetched before the first
+// level, and the last level writes the root where the transcript hashes it.
+template <class Src>
+__global__ __launch_bounds__(TAIL_THREADS) void merkle_tail_kernel(Src src0, uint32_t item_level, uint32_t n_items,
+                                                                  LevelStore st0, TailOut out, uint64_t bs) {
+    constexpr uint32_t W = MERKLE_TAIL_MAX / 2;
+    const uint64_t boff = (uint64_t)blockIdx.y * bs;
+    const Src src = src0.at(boff);
+    const LevelStore st = st0.shifted(boff);
+    if (boff) {
+        if (out.root_dst) out.root_dst += boff;
+        if (out.channel) out.channel = (DevChannel*)((uint32_t*)out.channel + boff);
+        if (out.alpha_dst) out.alpha_dst += boff;
+    }
+    __shared__ uint32_t nodes[8 * W];
+    __shared__ __align__(16) uint32_t qa[8 * TAIL_QUAD_NODES], qb[4 * TAIL_QUAD_NODES];
+    __shared__ __align__(16) uint32_t msg[16];
+    const uint32_t tid = threadIdx.x;
+    const uint64_t item_base = (uint64_t)blockIdx.x * n_items;
+    QuadTranscript tr = {};
+    if (out.channel && tid < 64) tr.load(out.channel, out.init_channel != 0);
+    uint32_t n = n_items / 2, lvl = item_level + 1;
+    bool narrow = false;
+    if constexpr (IsNodes<Src>::value) narrow = n_items <= TAIL_QUAD_NODES && n_items > 16;
+    if (narrow) {
+        // the first level's quads read the nodes in place
+        if constexpr (IsNodes<Src>::value) block_quad_level(src.nodes + 8 * item_base, qa, n, item_level, item_base, st);
+        lds_barrier();
     } else {
-        for (uint32_t j = tid; j < n; j += TAIL_THREADS)
+        for (uint32_t j = tid; j < n; j += TAIL_THREADS) {
+            uint32_t h[8];
+            src.pair(item_base + 2ull * j, h);
+            if (st.want(lvl)) store8(st.at(lvl, (item_base >> 1) + j), h);
+            if (n > TAIL_QUAD_NODES) {
 #pragma unroll
-            for (int q = 0; q < 8; q++) na[8 * j + q] = nodes[q * W + j];
-        __syncthreads();
+                for (int q = 0; q < 8; q++) nodes[q * W + j] = h[q];
+            } else {
+                store8(qa + 8 * j, h);
+            }
+        }
+        lds_barrier();
+        block_lane_levels<W>(nodes, qa, n, lvl, item_base >> (lvl - item_level), st);
     }
+    uint64_t idx0 = item_base >> (lvl - item_level);
+    uint32_t *cur = qa, *nxt = qb;
+    block_quad_reduce(cur, nxt, n, lvl, idx0, st);
     if (tid >= 64) return;  // one wave finishes: narrow levels and transcript
-    if (cur != na) {
-        for (uint32_t k = tid; k < 8 * n; k += 64) na[k] = cur[k];
-        VX_WAVE_SYNC();
-    }
-    uint32_t* root = narrow_reduce(na, nb, n, lvl, idx0, st);
+    if (out.channel) tr.put_state(msg);
+    const uint32_t* root = narrow_reduce(cur, nxt, n, lvl, idx0, st, 1u, msg + 8);
     if (out.root_dst && tid < 8) out.root_dst[8ull * blockIdx.x + tid] = root[tid];
-    if (out.channel) quad_transcript(out.channel, root, msg, out.init_channel != 0, out.alpha_dst, out.n_felts);
+    if (!out.channel) return;
+    tr.mix(msg);
+    for (uint32_t k = 0; out.alpha_dst && k < out.n_felts; k++) {
+        uint32_t w = 0;
+        if (!tr.draw(msg, w)) break;
+        if (tid < 4) out.alpha_dst[4 * k + tid] = w;
+    }
+    tr.store(out.channel);
 }
 
 }  // namespace vx

@@ -81,7 +81,7 @@ __global__ __launch_bounds__(256) void queries_kernel(DevChannel* ch0, const uin
                                                      const uint32_t* ab, uint64_t bs) {
     __shared__ uint32_t words[MAX_LAST_WORDS];
     __shared__ uint32_t st[8];
-    __shared__ uint32_t msg[16];
+    __shared__ __align__(16) uint32_t msg[16];
     const uint32_t tid = threadIdx.x;
     const uint64_t off = (uint64_t)blockIdx.x * bs;
     DevChannel* ch = (DevChannel*)((uint32_t*)ch0 + off);
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(256) void queries_kernel(DevChannel* ch0, const uin
             proof[last_off + 4 * i + c] = v[c];
         }
     }
-    __syncthreads();
+    lds_barrier();
     if (tid < 64) {
         // mix_felts (channel.rs:48-61: Blake2s over state || felts in 64-byte
         // blocks) by wave 0 quad-cooperatively: every quad hashes the same
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256) void queries_kernel(DevChannel* ch0, const uin
             proof[4] = ab[2 * blockIdx.x + 1];
         }
     }
-    __syncthreads();
+    lds_barrier();
     uint32_t s[8];
     for (int c = 0; c < 8; c++) s[c] = st[c];
     for (uint32_t i = tid; i < n_q; i += blockDim.x) {
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(DECOMMIT_THREADS) void decommit_kernel(const TreeDe
             proof[t.sib_off + (uint64_t)q * width + k] = sv[k];
         }
     }
-    __syncthreads();
+    lds_barrier();
     {
         const uint32_t g = tid >> lam, k = tid & lmask;
         if (g < nq) {
@@ -237,7 +237,7 @@ __global__ __launch_bounds__(DECOMMIT_THREADS) void decommit_kernel(const TreeDe
             for (int w = 0; w < 8; w++) lv[w * NW + g * S + k] = h[w];
         }
     }
-    __syncthreads();
+    lds_barrier();
     if (tid < 8 * nq) {
         const uint32_t g = tid >> 3, w = tid & 7;
         leaf_self[g][w] = lv[w * NW + g * S + ((uint32_t)li_s[g] & lmask)];
@@ -260,14 +260,14 @@ __global__ __launch_bounds__(DECOMMIT_THREADS) void decommit_kernel(const TreeDe
                 r[w] = lv[w * NW + g * S + 2 * k + 1];
             }
         }
-        __syncthreads();
+        lds_barrier();
         if (act) {
             uint32_t h[8];
             b2s_node(l, r, h);
 #pragma unroll
             for (int w = 0; w < 8; w++) lv[w * NW + g * S + k] = h[w];
         }
-        __syncthreads();
+        lds_barrier();
     }
     const LevelStore st = LevelStore{t.store, D, lam}.shifted(off);
     const uint32_t up = D - lam;
@@ -275,7 +275,7 @@ __global__ __launch_bounds__(DECOMMIT_THREADS) void decommit_kernel(const TreeDe
         const uint32_t w = idx & 7, L = lam + (idx >> 3) % up, g = (idx >> 3) / up;
         path[g][L * 8 + w] = st.at(L, (li_s[g] >> L) ^ 1)[w];
     }
-    __syncthreads();
+    lds_barrier();
     const uint64_t rec = 1 + 8ull * D;
     for (uint32_t idx = tid; idx < nq * (1 + 8 * D); idx += DECOMMIT_THREADS) {
         const uint32_t g = idx / (1 + 8 * D), k = idx % (1 + 8 * D);
@@ -537,7 +537,7 @@ void plan_arena(vx_prover* p) {
         const uint32_t d = depth_of(t);
         p->o_store.push_back(take(level_store_words(d, store_from(d))));
     }
-    p->o_scr_a = take(8 * std::max(scratch_nodes_a(p->E), max_line_quad_nodes(p->E)));
+    p->o_scr_a = take(8 * scratch_nodes_a(p->E));
     p->o_scr_b = take(8 * scratch_nodes_b(p->E));
     p->o_ch = take(sizeof(DevChannel) / 4);
     p->o_alpha = take(4ull * (1 + p->J));
@@ -563,16 +563,16 @@ void enqueue_heavy(vx_prover* p, uint32_t count) {
     uint32_t* pr = p->proof();
     uint32_t* ev = p->at(p->o_eval);
     phase = "trace_commit";
-    commit_tree(SrcCol1{ev}, E, p->stores[0], TailOut{pr + 5, p->ch(), p->alpha_q(), 1}, sc, s, mk, count, R);
+    commit_leaves(SrcCol1{ev}, E, p->stores[0], TailOut{pr + 5, p->ch(), p->alpha_q(), 1}, sc, s, mk, count, R);
     phase = "quotient_commit";
-    commit_tree(SrcQuotient{ev, E - 1, p->alpha_q()}, E, p->stores[1], TailOut{pr + 13, p->ch(), p->alpha_f(0), 0},
+    commit_leaves(SrcQuotient{ev, E - 1, p->alpha_q()}, E, p->stores[1], TailOut{pr + 13, p->ch(), p->alpha_f(0), 0},
                 sc, s, mk, count, R);
     {
         phase = "fri0_circle_fold_commit";
         SrcCircleFold src = {ev,           E - 1,        p->alpha_q(), p->alpha_f(0), p->fri_tw[0],
                              p->col(0, 0), p->col(0, 1), p->col(0, 2), p->col(0, 3)};
         uint32_t* nxt = p->J > 1 ? p->alpha_f(1) : nullptr;
-        commit_tree(src, E / 2, p->stores[2], TailOut{pr + p->off_fri_roots, p->ch(), nxt, 0}, sc, s, mk, count, R);
+        commit_leaves(src, E / 2, p->stores[2], TailOut{pr + p->off_fri_roots, p->ch(), nxt, 0}, sc, s, mk, count, R);
     }
 }
 
@@ -585,9 +585,7 @@ void enqueue_light(vx_prover* p, uint32_t count) {
     auto mk = [&](const char* what) { p->mark(phase + ":" + what); };
     Scratch sc = {p->at(p->o_scr_a), p->at(p->o_scr_b)};
     uint32_t* pr = p->proof();
-    // layers of at most FRI_TAIL_MAX_ITEMS values all go to one fri_tail_kernel
-    // launch; the larger ones take a stage launch even where the tree would fit
-    // one tail block (direct_max), so that their leaves spread over many CUs
+    // layers of at most FRI_TAIL_MAX_ITEMS values all go to one fri_tail_kernel launch
     uint32_t js = 1;
     while (js < p->J && (E >> (js + 1)) > FRI_TAIL_MAX_ITEMS) js++;
     for (uint32_t j = 1; j < js; j++) {
@@ -595,11 +593,8 @@ void enqueue_light(vx_prover* p, uint32_t count) {
         SrcLineFold src = {p->col(j - 1, 0), p->col(j - 1, 1), p->col(j - 1, 2), p->col(j - 1, 3), p->alpha_f(j),
                            p->fri_tw[j],     p->col(j, 0),     p->col(j, 1),     p->col(j, 2),     p->col(j, 3)};
         uint32_t* nxt = j + 1 < p->J ? p->alpha_f(j + 1) : nullptr;
-        const TailOut to{pr + p->off_fri_roots + 8ull * j, p->ch(), nxt, 0};
-        if (count == 1 && (E >> (j + 1)) <= LINE_QUAD_MAX)
-            commit_line_fold_quad(src, E >> (j + 1), p->stores[2 + j], to, sc, s, mk, count, R);
-        else
-            commit_tree(src, E >> (j + 1), p->stores[2 + j], to, sc, s, mk, count, R, FRI_TAIL_MAX_ITEMS);
+        commit_leaves(src, E >> (j + 1), p->stores[2 + j], TailOut{pr + p->off_fri_roots + 8ull * j, p->ch(), nxt, 0},
+                      sc, s, mk, count, R);
     }
     if (js < p->J) {
         auto layer = [&](uint32_t j) {
