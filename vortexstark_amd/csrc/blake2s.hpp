@@ -29,6 +29,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "field.hpp"
+
 namespace vx {
 
 constexpr uint32_t B2S_IV0 = 0x6A09E667u, B2S_IV1 = 0xBB67AE85u, B2S_IV2 = 0x3C6EF372u, B2S_IV3 = 0xA54FF53Au;
@@ -63,14 +65,6 @@ constexpr uint8_t B2S_SIGMA[10][16] = {
     {12, 5, 1, 15, 14, 13, 4, 10, 0, 7, 6, 3, 9, 2, 8, 11}, {13, 11, 7, 14, 12, 1, 3, 9, 5, 0, 15, 4, 8, 6, 2, 10},
     {6, 15, 14, 9, 11, 3, 0, 8, 12, 2, 13, 7, 1, 4, 10, 5}, {10, 2, 8, 4, 7, 6, 1, 5, 15, 11, 9, 14, 3, 12, 13, 0},
 };
-
-// Wave priority p from here on; the barriers keep the rows on their side of it.
-#define VX_PRIO(p)                            \
-    do {                                      \
-        __builtin_amdgcn_sched_barrier(0);    \
-        __builtin_amdgcn_s_setprio(p);        \
-        __builtin_amdgcn_sched_barrier(0);    \
-    } while (0)
 
 // Whether a row of additions takes a message word that is not known to be zero
 // (words NZ .. 15 are): if not, its adds are two-operand ones.

@@ -40,15 +40,6 @@ namespace vx {
         __builtin_amdgcn_wave_barrier();                      \
     } while (0)
 
-// Workgroup barrier that orders LDS accesses only. __syncthreads also waits
-// for the block's outstanding device-memory stores, which a chain of levels
-// that never reads them back would wait for once a level.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 constexpr uint32_t MERKLE_TAIL_MAX = 2048;  // most items one tail-kernel block reduces
 constexpr uint32_t MERKLE_STAGE_WAVES = 4;  // waves per stage workgroup
 
@@ -304,10 +295,8 @@ struct LiftCol {
 // use scalar loads, and the column data through the global one plain vector
 // loads (a generic pointer would make them flat loads).
 typedef const __attribute__((address_space(4))) LiftCol ConstLiftCol;
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef const __attribute__((address_space(1))) u32x2 GlobalV2;
-typedef const __attribute__((address_space(1))) u32x4 GlobalV4;
+typedef const gu32x2 GlobalV2;
+typedef const gu32x4 GlobalV4;
 __device__ __forceinline__ ConstLiftCol* const_table(const LiftCol* t) { return (ConstLiftCol*)t; }
 
 struct SrcLifted {

@@ -108,11 +108,13 @@ __device__ __forceinline__ uint2 ldw2(const uint32_t* T, uint32_t h) {
     return *(const uint2*)((const char*)T + (h << 3));
 }
 
-// Threads of a pass over 2^M x 2^C tiles: one radix-8 group per thread, 64 to 256.
+// Threads of a pass over 2^M x 2^C tiles: two radix-8 groups a thread (16 words)
+// from 2^12 words on, so that every tile size keeps eight waves a SIMD within
+// the CU's LDS (8 workgroups of 2^12 words, 2 of 2^14).
 template <int M, int C>
 constexpr uint32_t ntt_threads() {
-    constexpr uint32_t groups = 1u << (M + C > 3 ? M + C - 3 : 0);
-    return groups >= 256 ? 256 : (groups < 64 ? 64 : groups);
+    constexpr uint32_t words = 1u << (M + C);
+    return words >= (1u << 14) ? 1024 : words >= (1u << 13) ? 512 : words >= (1u << 11) ? 256 : words >= (1u << 9) ? words >> 3 : 64;
 }
 
 // Twiddle h of a layer whose table is T; circle0: the layer is stride bit 0.
@@ -129,6 +131,90 @@ __device__ __forceinline__ uint32_t ntt_twiddle(const uint32_t* T, bool circle0,
     }
 }
 
+// The 2^(R-1) butterflies of layer t on a group's values, row by row: the
+// products, reductions and sums of all butterflies side by side, at priority 1
+// the rows of v_mad_u64_u32, v_alignbit_b32 and v_min_u32, at priority 0 the
+// adds and ands, which then issue beside another wave's products (see VX_PRIO).
+// w[k] is the twiddle of the butterflies with d >> (t + 1) = k; with NEG
+// (stwo's circle layer) t = 0 and butterflies 1 and 2 take -w: forward that
+// swaps the outputs, inverse it negates the difference. Leaves the wave at
+// priority 1. Contiguous 12-layer pass of 2^26 points: 177 us as one butterfly
+// after another.
+template <bool FWD, int R, bool CIRCLE>
+__device__ __forceinline__ void butterflies(uint32_t v[1 << R], const uint32_t* w, const int t) {
+    constexpr int NB = 1 << (R - 1);
+    uint32_t lo[NB], hi[NB], m[NB], r[NB];
+    auto i0 = [&](int b) { return ((b >> t) << (t + 1)) | (b & ((1 << t) - 1)); };
+    auto i1 = [&](int b) { return i0(b) | (1 << t); };
+    auto neg = [&](int b) { return CIRCLE && t == 0 && (b == 1 || b == 2); };
+    auto wd = [&](int b) { return CIRCLE && t == 0 ? w[b] : w[b >> t]; };
+    auto product = [&](const uint32_t* x) {  // priority 1: m = x * w, reduced to [0, 2p)
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            const uint64_t p = (uint64_t)x[b] * wd(b);
+            lo[b] = (uint32_t)p;
+            hi[b] = (uint32_t)(p >> 32);
+        }
+#pragma unroll
+        for (int b = 0; b < NB; b++) hi[b] = __builtin_amdgcn_alignbit(hi[b], lo[b], 31);
+        VX_PRIO(0);
+#pragma unroll
+        for (int b = 0; b < NB; b++) m[b] = (lo[b] & P) + hi[b];
+#pragma unroll
+        for (int b = 0; b < NB; b++) r[b] = m[b] - P;
+        VX_PRIO(1);
+    };
+    if (FWD) {
+        uint32_t x[NB], s[NB], s2[NB], a[NB], a2[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++) x[b] = v[i1(b)];
+        VX_PRIO(1);
+        product(x);
+#pragma unroll
+        for (int b = 0; b < NB; b++) m[b] = min(m[b], r[b]);
+        VX_PRIO(0);
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            s[b] = v[i0(b)] - m[b];
+            a[b] = v[i0(b)] + m[b];
+        }
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            s2[b] = s[b] + P;
+            a2[b] = a[b] - P;
+        }
+        VX_PRIO(1);
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            const uint32_t lo_ = min(s[b], s2[b]), hi_ = min(a[b], a2[b]);
+            v[i1(b)] = neg(b) ? hi_ : lo_;
+            v[i0(b)] = neg(b) ? lo_ : hi_;
+        }
+    } else {
+        uint32_t s[NB], s2[NB], a[NB], a2[NB];
+        VX_PRIO(0);
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            s[b] = neg(b) ? v[i1(b)] - v[i0(b)] : v[i0(b)] - v[i1(b)];
+            a[b] = v[i0(b)] + v[i1(b)];
+        }
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            s2[b] = s[b] + P;
+            a2[b] = a[b] - P;
+        }
+        VX_PRIO(1);
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            s[b] = min(s[b], s2[b]);
+            v[i0(b)] = min(a[b], a2[b]);
+        }
+        product(s);
+#pragma unroll
+        for (int b = 0; b < NB; b++) v[i1(b)] = min(m[b], r[b]);
+    }
+}
+
 // One radix-2^R round over row bits [J, J + R) of an LDS tile of 2^M rows x
 // 2^C columns. Each group of 2^R values (fixed column and other row bits) is
 // loaded into registers, transformed through R layers, and written back.
@@ -140,42 +226,90 @@ __device__ __forceinline__ uint32_t ntt_twiddle(const uint32_t* T, bool circle0,
 // are zero on entry, so the top two layers only copy: (x, 0) -> (x, x). Those
 // rounds load two values and replicate them instead of running 8 butterflies.
 // ALT: the layers' twiddle tables are a.tw2 (the LDE bridge's inverse layers)
+//
+// Thread t takes groups g = t + it * NT; a group is (row_hi, row_lo, q) =
+// (g >> (C+J), the J bits above C, the C low bits) and starts at tile index
+// ((row_hi << (J+R) | row_lo) << C) + q. With NT a multiple of 2^(C+J) the
+// next group of a thread has the same column and low row bits and row_hi
+// larger by NT >> (C+J); otherwise (NT < 2^(C+J), t < 2^(C+J)) group it has
+// row_hi = it / P and its low bits t + (it % P) * NT, P = 2^(C+J) / NT.
+// Either way a thread's groups sit at constant distances from its first in
+// the tile and in each layer's twiddle table, which the unrolled loops fold
+// into instruction offsets.
+template <int M, int C, int R, int J>
+struct RoundShape {
+    static constexpr uint32_t GROUPS = 1u << (M + C - R);
+    static constexpr uint32_t STEP = 1u << (J + C);  // tile index distance between rows d and d + 1
+    static constexpr uint32_t NT = ntt_threads<M, C>();
+    static constexpr uint32_t ITER = (GROUPS + NT - 1) / NT;
+    static constexpr uint32_t CJ = 1u << (C + J);
+    static constexpr bool WIDE = NT >= CJ;
+    static constexpr uint32_t PER = WIDE ? 1u : CJ / NT;
+    __device__ __forceinline__ static bool live(uint32_t tid, uint32_t it) {
+        return GROUPS % NT == 0 || tid + it * NT < GROUPS;  // fewer groups than threads
+    }
+    __device__ __forceinline__ static uint32_t row_hi(uint32_t tid, uint32_t it) {
+        return WIDE ? ((tid >> C) >> J) + it * (NT / CJ) : it / PER;
+    }
+    __device__ __forceinline__ static uint32_t first(uint32_t tid, uint32_t it) {
+        const uint32_t rest = tid >> C, row_lo = rest & ((1u << J) - 1);
+        const uint32_t e00 = ((((rest >> J) << (J + R)) | row_lo) << C) + (tid & ((1u << C) - 1));
+        return WIDE ? e00 + it * (NT << R) : e00 + (it % PER) * NT + ((it / PER) << (J + R + C));
+    }
+};
+
+// The twiddles of a thread's groups in one round: w[it][t][k] of layer t.
+template <int M, int C, int R, int J>
+struct RoundTwiddles {
+    uint32_t w[RoundShape<M, C, R, J>::ITER][R][1 << (R - 1)];
+};
 template <bool FWD, int M, int C, int R, int J, bool STWO, bool ALT = false>
-__device__ __forceinline__ void ntt_round(uint32_t* tile, const NttPassArgs& a, uint64_t hi, uint32_t tid,
-                                          bool zero_top = false) {
-    constexpr uint32_t GROUPS = 1u << (M + C - R);
-    constexpr uint32_t STEP = 1u << (J + C);  // tile index distance between rows d and d + 1
-    constexpr uint32_t NT = ntt_threads<M, C>();
-    constexpr uint32_t ITER = (GROUPS + NT - 1) / NT;
-    // Thread t takes groups g = t + it * NT; a group is (row_hi, row_lo, q) =
-    // (g >> (C+J), the J bits above C, the C low bits) and starts at tile index
-    // ((row_hi << (J+R) | row_lo) << C) + q. With NT a multiple of 2^(C+J) the
-    // next group of a thread has the same column and low row bits and row_hi
-    // larger by NT >> (C+J); otherwise (NT < 2^(C+J), t < 2^(C+J)) group it has
-    // row_hi = it / P and its low bits t + (it % P) * NT, P = 2^(C+J) / NT.
-    // Either way a thread's groups sit at constant distances from its first in
-    // the tile and in each layer's twiddle table, which the unrolled loop folds
-    // into instruction offsets.
-    constexpr uint32_t CJ = 1u << (C + J);
-    constexpr bool WIDE = NT >= CJ;
-    constexpr uint32_t P = WIDE ? 1u : CJ / NT;
-    const uint32_t g0 = tid;
-    const uint32_t q = g0 & ((1u << C) - 1);
-    const uint32_t rest = g0 >> C;
-    const uint32_t row_lo = rest & ((1u << J) - 1);
-    const uint32_t row_hi0 = rest >> J;  // 0 unless WIDE
-    const uint32_t e00 = ((((row_hi0 << (J + R)) | row_lo)) << C) + q;
+__device__ __forceinline__ void load_twiddles(RoundTwiddles<M, C, R, J>& tw, const NttPassArgs& a, uint64_t hi,
+                                              uint32_t tid, bool zero_top = false) {
+    using S = RoundShape<M, C, R, J>;
 #pragma unroll
-    for (uint32_t it = 0; it < ITER; it++) {
-        if (GROUPS % NT != 0 && g0 + it * NT >= GROUPS) break;  // fewer groups than threads
-        const uint32_t e0 = WIDE ? e00 + it * (NT << R) : e00 + (it % P) * NT + ((it / P) << (J + R + C));
-        const uint32_t row_hi = WIDE ? row_hi0 + it * (NT / CJ) : it / P;
+    for (uint32_t it = 0; it < S::ITER; it++) {
+        if (!S::live(tid, it)) break;
+        const uint32_t row_hi = S::row_hi(tid, it);
+#pragma unroll
+        for (int t = 0; t < R; t++) {
+            if (FWD && R == 3 && t >= 1 && zero_top) continue;
+            const uint32_t rb = J + t;  // row bit of the layer
+            const uint32_t* T = ALT ? a.tw2[rb] : a.tw[rb];
+            // h(d) = (hi << (M - rb - 1)) + (row >> (rb + 1)) = hb + (d >> (t + 1))
+            const uint32_t hb = (uint32_t)(hi << (M - rb - 1)) + (row_hi << (R - t - 1));
+            // only the contiguous pass (stride bits from 0) has a stwo variant,
+            // so the circle layer is row bit 0, known at compile time
+            if (STWO && R == 3 && J == 0 && t == 0) {
+                // its four butterflies take h = hb .. hb + 3 with hb a multiple of
+                // 4, i.e. [y, -y, -x, x] of the pair at hb / 2; the negated ones
+                // swap the butterfly's outputs instead (butterflies)
+                const uint2 xy = ldw2(T, hb >> 2);
+                tw.w[it][t][0] = tw.w[it][t][1] = xy.y;
+                tw.w[it][t][2] = tw.w[it][t][3] = xy.x;
+            } else {
+#pragma unroll
+                for (int k = 0; k < (1 << (R - 1 - t)); k++)
+                    tw.w[it][t][k] = ntt_twiddle<STWO>(T, STWO && rb == 0, hb + k);
+            }
+        }
+    }
+}
+
+template <bool FWD, int M, int C, int R, int J, bool STWO>
+__device__ __forceinline__ void ntt_round(uint32_t* tile, const RoundTwiddles<M, C, R, J>& tw, uint32_t tid,
+                                          bool zero_top = false) {
+    using S = RoundShape<M, C, R, J>;
+#pragma unroll
+    for (uint32_t it = 0; it < S::ITER; it++) {
+        if (!S::live(tid, it)) break;
+        const uint32_t e0 = S::first(tid, it);
         uint32_t v[1 << R];
         uint32_t addr[1 << R];
 #pragma unroll
         for (int d = 0; d < (1 << R); d++) {
             // lpad is linear in d once the row step is a multiple of 8 words
-            addr[d] = (J + C >= 3) ? lpad(e0) + (uint32_t)d * (STEP + STEP / 8) : lpad(e0 + (uint32_t)d * STEP);
+            addr[d] = (J + C >= 3) ? lpad(e0) + (uint32_t)d * (S::STEP + S::STEP / 8) : lpad(e0 + (uint32_t)d * S::STEP);
         }
         if (FWD && R == 3 && zero_top) {
             v[0] = tile[addr[0]];
@@ -190,82 +324,69 @@ __device__ __forceinline__ void ntt_round(uint32_t* tile, const NttPassArgs& a, 
         for (int tt = 0; tt < R; tt++) {
             const int t = FWD ? (R - 1 - tt) : tt;  // layer inside the group
             if (FWD && R == 3 && t >= 1 && zero_top) continue;
-            const uint32_t rb = J + t;                 // row bit of the layer
-            const uint32_t* T = ALT ? a.tw2[rb] : a.tw[rb];
-            // only the contiguous pass (stride bits from 0) has a stwo variant,
-            // so the circle layer is row bit 0, known at compile time
-            const bool circle0 = STWO && rb == 0;
-            // h(d) = (hi << (M - rb - 1)) + (row >> (rb + 1)) = hb + (d >> (t + 1))
-            const uint32_t hb = (uint32_t)(hi << (M - rb - 1)) + (row_hi << (R - t - 1));
-            if (STWO && R == 3 && J == 0 && t == 0) {
-                // the circle layer in a radix-8 round: its four butterflies
-                // (d = 0, 2, 4, 6) take h = hb .. hb + 3 with hb a multiple of
-                // 4, i.e. [y, -y, -x, x] of the pair at hb / 2; a negated
-                // twiddle swaps the two outputs (forward) or negates the
-                // difference (inverse), so no negation is computed
-                const uint2 xy = ldw2(T, hb >> 2);
-#pragma unroll
-                for (int d = 0; d < 8; d += 2) {
-                    const uint32_t w = d < 4 ? xy.y : xy.x;
-                    const bool neg = d == 2 || d == 4;
-                    uint32_t& x0 = v[d];
-                    uint32_t& x1 = v[d + 1];
-                    if (FWD) {
-                        const uint32_t m = mmul(x1, w);
-                        const uint32_t s0 = madd(x0, m), s1 = msub(x0, m);
-                        x0 = neg ? s1 : s0;
-                        x1 = neg ? s0 : s1;
-                    } else {
-                        const uint32_t s0 = madd(x0, x1);
-                        x1 = mmul(neg ? msub(x1, x0) : msub(x0, x1), w);
-                        x0 = s0;
-                    }
-                }
-                continue;
-            }
-#pragma unroll
-            for (int d = 0; d < (1 << R); d++) {
-                if (d & (1 << t)) continue;
-                const uint32_t w = ntt_twiddle<STWO>(T, circle0, hb + ((uint32_t)d >> (t + 1)));
-                uint32_t& x0 = v[d];
-                uint32_t& x1 = v[d | (1 << t)];
-                if (FWD) {
-                    uint32_t m = mmul(x1, w);
-                    x1 = msub(x0, m);
-                    x0 = madd(x0, m);
-                } else {
-                    uint32_t s0 = madd(x0, x1);
-                    x1 = mmul(msub(x0, x1), w);
-                    x0 = s0;
-                }
-            }
+            butterflies<FWD, R, STWO && R == 3 && J == 0>(v, tw.w[it][t], t);
         }
+        VX_PRIO(0);
 #pragma unroll
         for (int d = 0; d < (1 << R); d++) tile[addr[d]] = v[d];
     }
 }
 
 // Radix-8 rounds over the M layers of a tile, top down (forward) or bottom up
-// (inverse), unrolled at compile time.
+// (inverse), unrolled at compile time. A round's twiddles are loaded before the
+// round in front of it runs (the first round's by the caller, before it waits
+// for its tile), so that no round begins by waiting for device memory: with few
+// tiles on the device those waits are most of a pass.
 // tid is the thread's index in the block (see the replicating pass for why it
 // is a parameter).
-template <bool FWD, int M, int C, bool STWO, int TOP>
-__device__ __forceinline__ void fwd_rounds(uint32_t* tile, const NttPassArgs& a, uint64_t hi, uint32_t tid) {
-    if constexpr (TOP > 0) {
-        constexpr int R = TOP >= 3 ? 3 : TOP;
-        // only the pass's first round (its top three row bits) may skip its top two layers
-        ntt_round<FWD, M, C, R, TOP - R, STWO>(tile, a, hi, tid, TOP == M && a.zero_top2 != 0);
-        __syncthreads();
-        fwd_rounds<FWD, M, C, STWO, TOP - R>(tile, a, hi, tid);
+template <int M, int TOP>
+constexpr int fwd_radix() {
+    return TOP >= 3 ? 3 : TOP;
+}
+template <int M, int C, int TOP>
+using FwdTwiddles = RoundTwiddles<M, C, fwd_radix<M, TOP>(), TOP - fwd_radix<M, TOP>()>;
+template <int M, int LO>
+constexpr int inv_radix() {
+    return M - LO >= 3 ? 3 : M - LO;
+}
+template <int M, int C, int LO>
+using InvTwiddles = RoundTwiddles<M, C, inv_radix<M, LO>(), LO>;
+
+template <int M, int C, bool STWO, int TOP>
+__device__ __forceinline__ void load_fwd(FwdTwiddles<M, C, TOP>& w, const NttPassArgs& a, uint64_t hi, uint32_t tid) {
+    constexpr int R = fwd_radix<M, TOP>();
+    // only the pass's first round (its top three row bits) may skip its top two layers
+    load_twiddles<true, M, C, R, TOP - R, STWO>(w, a, hi, tid, TOP == M && a.zero_top2 != 0);
+}
+template <int M, int C, bool STWO, int TOP>
+__device__ __forceinline__ void fwd_rounds(uint32_t* tile, const FwdTwiddles<M, C, TOP>& w, const NttPassArgs& a,
+                                           uint64_t hi, uint32_t tid) {
+    constexpr int R = fwd_radix<M, TOP>();
+    const bool zero_top = TOP == M && a.zero_top2 != 0;
+    if constexpr (TOP - R > 0) {
+        FwdTwiddles<M, C, TOP - R> next;
+        load_fwd<M, C, STWO, TOP - R>(next, a, hi, tid);
+        ntt_round<true, M, C, R, TOP - R, STWO>(tile, w, tid, zero_top);
+        lds_barrier();
+        fwd_rounds<M, C, STWO, TOP - R>(tile, next, a, hi, tid);
+    } else {
+        ntt_round<true, M, C, R, TOP - R, STWO>(tile, w, tid, zero_top);
+        lds_barrier();
     }
 }
-template <bool FWD, int M, int C, bool STWO, int LO, bool ALT = false>
-__device__ __forceinline__ void inv_rounds(uint32_t* tile, const NttPassArgs& a, uint64_t hi, uint32_t tid) {
-    if constexpr (LO < M) {
-        constexpr int R = M - LO >= 3 ? 3 : M - LO;
-        ntt_round<FWD, M, C, R, LO, STWO, ALT>(tile, a, hi, tid);
-        __syncthreads();
-        inv_rounds<FWD, M, C, STWO, LO + R, ALT>(tile, a, hi, tid);
+template <int M, int C, bool STWO, int LO, bool ALT = false>
+__device__ __forceinline__ void inv_rounds(uint32_t* tile, const InvTwiddles<M, C, LO>& w, const NttPassArgs& a,
+                                           uint64_t hi, uint32_t tid) {
+    constexpr int R = inv_radix<M, LO>();
+    if constexpr (LO + R < M) {
+        InvTwiddles<M, C, LO + R> next;
+        load_twiddles<false, M, C, inv_radix<M, LO + R>(), LO + R, STWO, ALT>(next, a, hi, tid);
+        ntt_round<false, M, C, R, LO, STWO>(tile, w, tid);
+        lds_barrier();
+        inv_rounds<M, C, STWO, LO + R, ALT>(tile, next, a, hi, tid);
+    } else {
+        ntt_round<false, M, C, R, LO, STWO>(tile, w, tid);
+        lds_barrier();
     }
 }
 
@@ -289,7 +410,7 @@ __device__ __forceinline__ uint32_t tile_word(uint32_t base, uint32_t s, uint32_
     return base + ((e >> C) << s) + (e & ((1u << C) - 1));
 }
 template <bool FWD, int M, int C>
-__device__ __forceinline__ void tile_load(uint32_t* tile, const uint32_t* src, uint32_t base, uint32_t s,
+__device__ __forceinline__ void tile_load(uint32_t* tile, const gu32* src, uint32_t base, uint32_t s,
                                           uint64_t src_n, bool vec, uint32_t tid) {
     constexpr uint32_t TILE = 1u << (M + C);
     constexpr uint32_t NT = ntt_threads<M, C>();
@@ -299,7 +420,7 @@ __device__ __forceinline__ void tile_load(uint32_t* tile, const uint32_t* src, u
             const uint32_t e = 4 * tid + it * 4 * NT;
             if (TILE % (4 * NT) != 0 && e >= TILE) break;
             const uint32_t g = tile_word<M, C>(base, s, e);
-            const uint4 x = g < src_n ? *(const uint4*)(src + g) : make_uint4(0, 0, 0, 0);
+            const u32x4 x = g < src_n ? *(const gu32x4*)(src + g) : u32x4{0, 0, 0, 0};
             const uint32_t p = lpad(e);  // e % 4 == 0: the four words stay within one padded group
             tile[p] = x.x;
             tile[p + 1] = x.y;
@@ -317,7 +438,7 @@ __device__ __forceinline__ void tile_load(uint32_t* tile, const uint32_t* src, u
     }
 }
 template <bool FWD, int M, int C>
-__device__ __forceinline__ void tile_store(const uint32_t* tile, uint32_t* dst, uint32_t base, uint32_t s,
+__device__ __forceinline__ void tile_store(const uint32_t* tile, gu32* dst, uint32_t base, uint32_t s,
                                            uint32_t scale, bool vec, uint32_t tid) {
     constexpr uint32_t TILE = 1u << (M + C);
     constexpr uint32_t NT = ntt_threads<M, C>();
@@ -328,9 +449,9 @@ __device__ __forceinline__ void tile_store(const uint32_t* tile, uint32_t* dst, 
             if (TILE % (4 * NT) != 0 && e >= TILE) break;
             const uint32_t g = tile_word<M, C>(base, s, e);
             const uint32_t p = lpad(e);
-            uint4 x = make_uint4(tile[p], tile[p + 1], tile[p + 2], tile[p + 3]);
-            if (scale) x = make_uint4(mmul(x.x, scale), mmul(x.y, scale), mmul(x.z, scale), mmul(x.w, scale));
-            *(uint4*)(dst + g) = x;
+            u32x4 x = {tile[p], tile[p + 1], tile[p + 2], tile[p + 3]};
+            if (scale) x = u32x4{mmul(x.x, scale), mmul(x.y, scale), mmul(x.z, scale), mmul(x.w, scale)};
+            *(gu32x4*)(dst + g) = x;
         }
     } else {
 #pragma unroll
@@ -345,12 +466,12 @@ __device__ __forceinline__ void tile_store(const uint32_t* tile, uint32_t* dst, 
 }
 
 template <bool FWD, int M, int C, bool STWO, bool REPL>
-__global__ __launch_bounds__(256) void ntt_pass_kernel(NttPassArgs a) {
+__global__ __launch_bounds__((ntt_threads<M, C>())) void ntt_pass_kernel(NttPassArgs a) {
     static_assert(!STWO || C == 0, "the stwo variant is the contiguous pass (stride bits from 0)");
     static_assert(!REPL || FWD, "only an evaluation replicates its input");
     __shared__ uint32_t tile[(1u << (M + C)) + (1u << (M + C)) / 8];
-    uint32_t* dst = a.cols ? a.cols[blockIdx.y] : a.dst;
-    const uint32_t* src = a.cols ? (a.srcs ? a.srcs[blockIdx.y] : a.cols[blockIdx.y]) : a.src;
+    gu32* dst = as_global(a.cols ? a.cols[blockIdx.y] : a.dst);
+    const gu32* src = as_global((const uint32_t*)(a.cols ? (a.srcs ? a.srcs[blockIdx.y] : a.cols[blockIdx.y]) : a.src));
     const uint32_t s = a.s;
     constexpr uint32_t TILE = 1u << (M + C);
     const uint32_t mid_bits = s - C;
@@ -368,7 +489,7 @@ __global__ __launch_bounds__(256) void ntt_pass_kernel(NttPassArgs a) {
         // word moves reload it.
         constexpr uint32_t NT = ntt_threads<M, C>();
         constexpr uint32_t KV = (TILE + 4 * NT - 1) / (4 * NT);
-        uint4 keep[KV];
+        u32x4 keep[KV];
         auto put = [&](uint32_t tid) {
 #pragma unroll
             for (uint32_t it = 0; it < KV; it++) {
@@ -387,13 +508,12 @@ __global__ __launch_bounds__(256) void ntt_pass_kernel(NttPassArgs a) {
                 const uint32_t e = 4 * threadIdx.x + it * 4 * NT;
                 if (TILE % (4 * NT) != 0 && e >= TILE) break;
                 const uint32_t g = tile_word<M, C>(base, s, e);
-                keep[it] = g < a.src_n ? *(const uint4*)(src + g) : make_uint4(0, 0, 0, 0);
+                keep[it] = g < a.src_n ? *(const gu32x4*)(src + g) : u32x4{0, 0, 0, 0};
             }
             put(threadIdx.x);
         } else {
             tile_load<FWD, M, C>(tile, src, base, s, a.src_n, false, threadIdx.x);
         }
-        __syncthreads();
 #pragma unroll 1
         for (int q = 3; q >= 0; q--) {
             // Addresses within the tile do not depend on the quarter: left to
@@ -402,24 +522,33 @@ __global__ __launch_bounds__(256) void ntt_pass_kernel(NttPassArgs a) {
             // thread index it cannot see through keeps them inside the loop.
             uint32_t tid = threadIdx.x;
             asm volatile("" : "+v"(tid));
+            FwdTwiddles<M, C, M> w;
+            load_fwd<M, C, STWO, M>(w, a, (uint64_t)q, tid);
             if (q != 3) {
                 if (vec)
                     put(tid);
                 else
                     tile_load<FWD, M, C>(tile, src, base, s, a.src_n, false, tid);
-                __syncthreads();
             }
-            fwd_rounds<FWD, M, C, STWO, M>(tile, a, (uint64_t)q, tid);
+            lds_barrier();
+            fwd_rounds<M, C, STWO, M>(tile, w, a, (uint64_t)q, tid);
             tile_store<FWD, M, C>(tile, dst, base + ((uint32_t)q << (s + M)), s, 0u, vec, tid);
-            __syncthreads();  // the next quarter overwrites the tile
+            lds_barrier();  // the next quarter overwrites the tile
         }
     } else {
-        tile_load<FWD, M, C>(tile, src, base, s, a.src_n, vec, threadIdx.x);
-        __syncthreads();
-        if constexpr (FWD)
-            fwd_rounds<FWD, M, C, STWO, M>(tile, a, hi, threadIdx.x);
-        else
-            inv_rounds<FWD, M, C, STWO, 0>(tile, a, hi, threadIdx.x);
+        if constexpr (FWD) {
+            FwdTwiddles<M, C, M> w;
+            load_fwd<M, C, STWO, M>(w, a, hi, threadIdx.x);
+            tile_load<FWD, M, C>(tile, src, base, s, a.src_n, vec, threadIdx.x);
+            lds_barrier();
+            fwd_rounds<M, C, STWO, M>(tile, w, a, hi, threadIdx.x);
+        } else {
+            InvTwiddles<M, C, 0> w;
+            load_twiddles<false, M, C, inv_radix<M, 0>(), 0, STWO>(w, a, hi, threadIdx.x);
+            tile_load<FWD, M, C>(tile, src, base, s, a.src_n, vec, threadIdx.x);
+            lds_barrier();
+            inv_rounds<M, C, STWO, 0>(tile, w, a, hi, threadIdx.x);
+        }
         tile_store<FWD, M, C>(tile, dst, base, s, a.scale, vec, threadIdx.x);
     }
 }
@@ -435,20 +564,24 @@ __global__ __launch_bounds__(256) void ntt_pass_kernel(NttPassArgs a) {
 // go to memory. Vector moves only (an LDE's column buffers are 16-byte
 // aligned); the driver uses the two passes otherwise.
 template <int M, int C, bool STWO>
-__global__ __launch_bounds__(256) void ntt_lde_bridge_kernel(NttPassArgs a) {
+__global__ __launch_bounds__((ntt_threads<M, C>())) void ntt_lde_bridge_kernel(NttPassArgs a) {
     static_assert(C >= 2 || C == 0, "vector moves need rows of at least 4 words");
     constexpr uint32_t TILE = 1u << (M + C);
     constexpr uint32_t NT = ntt_threads<M, C>();
     constexpr uint32_t KV = (TILE + 4 * NT - 1) / (4 * NT);
     __shared__ uint32_t tile[TILE + TILE / 8];
-    uint32_t* dst = a.cols ? a.cols[blockIdx.y] : a.dst;
-    const uint32_t* src = a.cols ? (a.srcs ? a.srcs[blockIdx.y] : a.cols[blockIdx.y]) : a.src;
+    gu32* dst = as_global(a.cols ? a.cols[blockIdx.y] : a.dst);
+    const gu32* src = as_global((const uint32_t*)(a.cols ? (a.srcs ? a.srcs[blockIdx.y] : a.cols[blockIdx.y]) : a.src));
     const uint32_t s = a.s;
     const uint32_t mid = blockIdx.x;  // the grid holds no row bits above the tile
     const uint32_t base = mid << C;
-    tile_load<false, M, C>(tile, src, base, s, a.src_n, true, threadIdx.x);
-    __syncthreads();
-    inv_rounds<false, M, C, STWO, 0, true>(tile, a, 0, threadIdx.x);
+    {
+        InvTwiddles<M, C, 0> w;
+        load_twiddles<false, M, C, inv_radix<M, 0>(), 0, STWO, true>(w, a, 0, threadIdx.x);
+        tile_load<false, M, C>(tile, src, base, s, a.src_n, true, threadIdx.x);
+        lds_barrier();
+        inv_rounds<M, C, STWO, 0, true>(tile, w, a, 0, threadIdx.x);
+    }
     uint4 keep[KV];
 #pragma unroll
     for (uint32_t it = 0; it < KV; it++) {
@@ -463,6 +596,8 @@ __global__ __launch_bounds__(256) void ntt_lde_bridge_kernel(NttPassArgs a) {
     for (int q = 3; q >= 0; q--) {
         uint32_t tid = threadIdx.x;  // hidden from the compiler, as in the replicating pass
         asm volatile("" : "+v"(tid));
+        FwdTwiddles<M, C, M> w;
+        load_fwd<M, C, STWO, M>(w, a, (uint64_t)q, tid);
 #pragma unroll
         for (uint32_t it = 0; it < KV; it++) {
             const uint32_t e = 4 * tid + it * 4 * NT;
@@ -473,10 +608,10 @@ __global__ __launch_bounds__(256) void ntt_lde_bridge_kernel(NttPassArgs a) {
             tile[p + 2] = keep[it].z;
             tile[p + 3] = keep[it].w;
         }
-        __syncthreads();
-        fwd_rounds<true, M, C, STWO, M>(tile, a, (uint64_t)q, tid);
+        lds_barrier();
+        fwd_rounds<M, C, STWO, M>(tile, w, a, (uint64_t)q, tid);
         tile_store<true, M, C>(tile, dst, base + ((uint32_t)q << (s + M)), s, 0u, true, tid);
-        __syncthreads();  // the next quarter overwrites the tile
+        lds_barrier();  // the next quarter overwrites the tile
     }
 }
 
