@@ -33,12 +33,6 @@ namespace {
 constexpr uint32_t DEEP_THREADS = 256;
 constexpr uint32_t COMBINE_ROWS = 8;  // rows per thread of quotients_combine
 
-// x < 2^64 -> x mod p (2^31 = 1 mod p: x = lo + mid 2^31 + hi 2^62 = lo + mid + hi).
-__device__ __forceinline__ uint32_t reduce64(uint64_t x) {
-    const uint64_t s = (x & P) + ((x >> 31) & P) + (x >> 62);  // < 2^32 + 2
-    return canon((uint32_t)(s & P) + (uint32_t)(s >> 31));
-}
-
 // ROWS rows per thread (row_of): 8 (uint4 loads and stores; n_rows % 512 == 0
 // and 16-byte aligned outputs, checked on the host; a column whose pointer is
 // not 16-byte aligned is read word by word, a wave-uniform branch) or 1.

@@ -103,6 +103,16 @@ __device__ __forceinline__ CM31 cmul(CM31 x, CM31 y) {
     return {msub(ac, bd), msub(msub(s, ac), bd)};
 }
 
+// x < 2^64 -> a value < 2^34 congruent to it mod p (2^32 = 2): one
+// v_mad_u64_u32. Four products of canonical values still fit on top of it:
+// 4 (p - 1)^2 + 2^34 = 2^64 - 2^35 + 16 + 2^34.
+__device__ __forceinline__ uint64_t fold64(uint64_t x) { return (uint64_t)(uint32_t)(x >> 32) * 2u + (uint32_t)x; }
+// x < 2^64 -> x mod p
+__device__ __forceinline__ uint32_t reduce64(uint64_t x) {
+    const uint64_t y = fold64(x);
+    return canon(((uint32_t)y & P) + __builtin_amdgcn_alignbit((uint32_t)(y >> 32), (uint32_t)y, 31));
+}
+
 // QM31 = a + b*u with u^2 = 2 + i; stored as {a.a, a.b, b.a, b.b}.
 struct QM31 {
     uint32_t v[4];
@@ -129,9 +139,37 @@ __device__ __forceinline__ QM31 qmul(QM31 x, QM31 y) {
     return {{ra.a, ra.b, rb.a, rb.b}};
 }
 
+// Multiplication by a QM31 constant as a 4 x 4 matrix over M31: row k of the
+// product alpha * d is sum_j m[k][j] d_j, four products and one reduction, where
+// the three-product form takes nine products and some forty additions.
+struct QMatrix {
+    uint32_t m[4][4];
+    __device__ __forceinline__ explicit QMatrix(QM31 a) {
+        const uint32_t a0 = a.v[0], a1 = a.v[1], a2 = a.v[2], a3 = a.v[3];
+        const uint32_t t = msub(mdbl(a2), a3), s = madd(mdbl(a3), a2);  // 2 a2 - a3, 2 a3 + a2
+        m[0][0] = a0, m[0][1] = mneg(a1), m[0][2] = t, m[0][3] = mneg(s);
+        m[1][0] = a1, m[1][1] = a0, m[1][2] = s, m[1][3] = t;
+        m[2][0] = a2, m[2][1] = mneg(a3), m[2][2] = a0, m[2][3] = mneg(a1);
+        m[3][0] = a3, m[3][1] = a2, m[3][2] = a1, m[3][3] = a0;
+    }
+    __device__ __forceinline__ uint64_t row(int k, const uint32_t d[4]) const {  // < 2^64
+        uint64_t x = (uint64_t)m[k][0] * d[0];
+        x += (uint64_t)m[k][1] * d[1];
+        x += (uint64_t)m[k][2] * d[2];
+        x += (uint64_t)m[k][3] * d[3];
+        return x;
+    }
+};
+
 // FRI fold of one pair: (f0 + f1) + alpha * ((f0 - f1) * tw)   (cuda/fri.cu:26-33)
-__device__ __forceinline__ QM31 fold_pair(QM31 f0, QM31 f1, QM31 alpha, uint32_t tw) {
-    return qadd(qadd(f0, f1), qmul(alpha, qmul_m31(qsub(f0, f1), tw)));
+__device__ __forceinline__ QM31 fold_pair(QM31 f0, QM31 f1, const QMatrix& alpha, uint32_t tw) {
+    uint32_t d[4];
+    QM31 r;
+#pragma unroll
+    for (int k = 0; k < 4; k++) d[k] = mmul(msub(f0.v[k], f1.v[k]), tw);
+#pragma unroll
+    for (int k = 0; k < 4; k++) r.v[k] = madd(madd(f0.v[k], f1.v[k]), reduce64(alpha.row(k, d)));
+    return r;
 }
 
 // Circle group (src/circle.rs:33-39)

@@ -7,63 +7,145 @@
 
 namespace vx {
 
-__global__ void fold_line_soa_kernel(const uint32_t* __restrict__ in0, const uint32_t* __restrict__ in1,
-                                     const uint32_t* __restrict__ in2, const uint32_t* __restrict__ in3,
-                                     const uint32_t* __restrict__ tw, uint32_t* __restrict__ out0,
-                                     uint32_t* __restrict__ out1, uint32_t* __restrict__ out2,
-                                     uint32_t* __restrict__ out3, QM31 alpha, uint32_t half_n) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+// All four kernels are bound by device memory (52 bytes a folded value, 20 a
+// quotient value), so a thread takes two folded values, or four quotient or
+// padded words, with 16-byte accesses (VEC: the pointers allow it); a ragged
+// end and unaligned pointers go word by word.
+struct SoaIn {
+    const uint32_t* c[4];
+};
+struct SoaOut {
+    uint32_t* c[4];
+};
+
+template <bool VEC>
+__global__ __launch_bounds__(256) void fold_line_soa_kernel(SoaIn in, const uint32_t* __restrict__ tw, SoaOut out,
+                                                          QM31 alpha, uint32_t half_n) {
+    const uint32_t i = (blockIdx.x * 256 + threadIdx.x) * (VEC ? 2 : 1);
     if (i >= half_n) return;
-    QM31 f0 = {{in0[2 * i], in1[2 * i], in2[2 * i], in3[2 * i]}};
-    QM31 f1 = {{in0[2 * i + 1], in1[2 * i + 1], in2[2 * i + 1], in3[2 * i + 1]}};
-    QM31 r = fold_pair(f0, f1, alpha, tw[i]);
-    out0[i] = r.v[0];
-    out1[i] = r.v[1];
-    out2[i] = r.v[2];
-    out3[i] = r.v[3];
+    const QMatrix al(alpha);
+    if (VEC && i + 1 < half_n) {
+        QM31 f[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const uint4 x = *(const uint4*)(in.c[c] + 2ull * i);
+            f[0].v[c] = x.x;
+            f[1].v[c] = x.y;
+            f[2].v[c] = x.z;
+            f[3].v[c] = x.w;
+        }
+        const uint2 w = *(const uint2*)(tw + i);
+        const QM31 r0 = fold_pair(f[0], f[1], al, w.x), r1 = fold_pair(f[2], f[3], al, w.y);
+#pragma unroll
+        for (int c = 0; c < 4; c++) *(uint2*)(out.c[c] + i) = make_uint2(r0.v[c], r1.v[c]);
+        return;
+    }
+    QM31 f0, f1;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        f0.v[c] = in.c[c][2ull * i];
+        f1.v[c] = in.c[c][2ull * i + 1];
+    }
+    const QM31 r = fold_pair(f0, f1, al, tw[i]);
+#pragma unroll
+    for (int c = 0; c < 4; c++) out.c[c][i] = r.v[c];
 }
 
-__global__ void fold_circle_soa_kernel(uint32_t* __restrict__ d0, uint32_t* __restrict__ d1,
-                                       uint32_t* __restrict__ d2, uint32_t* __restrict__ d3,
-                                       const uint32_t* __restrict__ s0, const uint32_t* __restrict__ s1,
-                                       const uint32_t* __restrict__ s2, const uint32_t* __restrict__ s3,
-                                       const uint32_t* __restrict__ tw, QM31 alpha, QM31 alpha_sq,
-                                       uint32_t half_n) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+// dst = dst * alpha_sq + fold; the product and the fold's share one reduction.
+__device__ __forceinline__ QM31 fold_onto(QM31 prev, QM31 f0, QM31 f1, const QMatrix& al, const QMatrix& sq,
+                                          uint32_t tw) {
+    uint32_t d[4];
+    QM31 r;
+#pragma unroll
+    for (int k = 0; k < 4; k++) d[k] = mmul(msub(f0.v[k], f1.v[k]), tw);
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        r.v[k] = madd(madd(f0.v[k], f1.v[k]), reduce64(fold64(al.row(k, d)) + fold64(sq.row(k, prev.v))));
+    return r;
+}
+
+template <bool VEC>
+__global__ __launch_bounds__(256) void fold_circle_soa_kernel(SoaOut dst, SoaIn src, const uint32_t* __restrict__ tw,
+                                                            QM31 alpha, QM31 alpha_sq, uint32_t half_n) {
+    const uint32_t i = (blockIdx.x * 256 + threadIdx.x) * (VEC ? 2 : 1);
     if (i >= half_n) return;
-    QM31 f0 = {{s0[2 * i], s1[2 * i], s2[2 * i], s3[2 * i]}};
-    QM31 f1 = {{s0[2 * i + 1], s1[2 * i + 1], s2[2 * i + 1], s3[2 * i + 1]}};
-    QM31 fp = fold_pair(f0, f1, alpha, tw[i]);
-    QM31 prev = {{d0[i], d1[i], d2[i], d3[i]}};
-    QM31 r = qadd(qmul(prev, alpha_sq), fp);
-    d0[i] = r.v[0];
-    d1[i] = r.v[1];
-    d2[i] = r.v[2];
-    d3[i] = r.v[3];
+    const QMatrix al(alpha), sq(alpha_sq);
+    if (VEC && i + 1 < half_n) {
+        QM31 f[4], p[2];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const uint4 x = *(const uint4*)(src.c[c] + 2ull * i);
+            const uint2 y = *(const uint2*)(dst.c[c] + i);
+            f[0].v[c] = x.x;
+            f[1].v[c] = x.y;
+            f[2].v[c] = x.z;
+            f[3].v[c] = x.w;
+            p[0].v[c] = y.x;
+            p[1].v[c] = y.y;
+        }
+        const uint2 w = *(const uint2*)(tw + i);
+        const QM31 r0 = fold_onto(p[0], f[0], f[1], al, sq, w.x), r1 = fold_onto(p[1], f[2], f[3], al, sq, w.y);
+#pragma unroll
+        for (int c = 0; c < 4; c++) *(uint2*)(dst.c[c] + i) = make_uint2(r0.v[c], r1.v[c]);
+        return;
+    }
+    QM31 f0, f1, prev;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        f0.v[c] = src.c[c][2ull * i];
+        f1.v[c] = src.c[c][2ull * i + 1];
+        prev.v[c] = dst.c[c][i];
+    }
+    const QM31 r = fold_onto(prev, f0, f1, al, sq, tw[i]);
+#pragma unroll
+    for (int c = 0; c < 4; c++) dst.c[c][i] = r.v[c];
 }
 
 // q[i] = alpha * (t[(i+2) mod n] - (t[(i+1) mod n] + t[i]))  (constraint.cu:10-36)
-__global__ void quotient_kernel(const uint32_t* __restrict__ t, uint32_t* __restrict__ o0,
-                                uint32_t* __restrict__ o1, uint32_t* __restrict__ o2, uint32_t* __restrict__ o3,
-                                QM31 alpha, uint32_t offset, uint32_t chunk_n, uint32_t n) {
-    uint32_t li = blockIdx.x * blockDim.x + threadIdx.x;
+// VEC: n >= 8, 16-byte aligned outputs and t + offset.
+template <bool VEC>
+__global__ __launch_bounds__(256) void quotient_kernel(const uint32_t* __restrict__ t, SoaOut out, QM31 alpha,
+                                                     uint32_t offset, uint32_t chunk_n, uint32_t n) {
+    const uint32_t li = (blockIdx.x * 256 + threadIdx.x) * (VEC ? 4 : 1);
     if (li >= chunk_n) return;
-    uint32_t i = offset + li;
-    // a full remainder, as the reference takes, so every n >= 1 wraps correctly
-    uint32_t i1 = (i + 1) % n;
-    uint32_t i2 = (i + 2) % n;
-    uint32_t c = msub(t[i2], madd(t[i1], t[i]));
-    QM31 r = qmul_m31(alpha, c);
-    o0[li] = r.v[0];
-    o1[li] = r.v[1];
-    o2[li] = r.v[2];
-    o3[li] = r.v[3];
+    if (VEC && chunk_n - li >= 4) {
+        const uint32_t i = offset + li;  // i + 3 < n
+        const uint4 a = *(const uint4*)(t + i);
+        const uint32_t e = i + 4 < n ? t[i + 4] : t[0];
+        const uint32_t f = n - i > 5 ? t[i + 5] : t[i + 5 - n];
+        const uint32_t d[4] = {msub(a.z, madd(a.y, a.x)), msub(a.w, madd(a.z, a.y)), msub(e, madd(a.w, a.z)),
+                               msub(f, madd(e, a.w))};
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+            *(uint4*)(out.c[c] + li) = make_uint4(mmul(alpha.v[c], d[0]), mmul(alpha.v[c], d[1]),
+                                                  mmul(alpha.v[c], d[2]), mmul(alpha.v[c], d[3]));
+        return;
+    }
+    for (uint32_t l = li; l < chunk_n && l < li + (VEC ? 4 : 1); l++) {
+        const uint32_t i = offset + l;
+        // one step at a time, so that every n >= 1 wraps as the reference's remainders do
+        const uint32_t i1 = i + 1 == n ? 0u : i + 1, i2 = i1 + 1 == n ? 0u : i1 + 1;
+        const uint32_t d = msub(t[i2], madd(t[i1], t[i]));
+#pragma unroll
+        for (int c = 0; c < 4; c++) out.c[c][l] = mmul(alpha.v[c], d);
+    }
 }
 
-__global__ void zero_pad_kernel(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst, uint32_t src_n,
-                                uint32_t dst_n) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < dst_n) dst[i] = i < src_n ? src[i] : 0u;
+template <bool VEC>
+__global__ __launch_bounds__(256) void zero_pad_kernel(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst,
+                                                     uint32_t src_n, uint32_t dst_n) {
+    const uint64_t i = (uint64_t)(blockIdx.x * 256ull + threadIdx.x) * (VEC ? 4 : 1);
+    if (i >= dst_n) return;
+    if (VEC && i + 4 <= dst_n && (i + 4 <= src_n || i >= src_n)) {
+        *(uint4*)(dst + i) = i < src_n ? *(const uint4*)(src + i) : make_uint4(0, 0, 0, 0);
+        return;
+    }
+    for (uint64_t k = i; k < dst_n && k < i + (VEC ? 4 : 1); k++) dst[k] = k < src_n ? src[k] : 0u;
+}
+
+template <class... T>
+static bool aligned(uintptr_t bytes, const T*... p) {
+    return (((uintptr_t)p | ...) & (bytes - 1)) == 0;
 }
 
 static QM31 q_from_host(const uint32_t* a) { return {{a[0], a[1], a[2], a[3]}}; }
@@ -78,8 +160,15 @@ void cuda_fold_line_soa(const uint32_t* in0, const uint32_t* in1, const uint32_t
                         const uint32_t* twiddles, uint32_t* out0, uint32_t* out1, uint32_t* out2, uint32_t* out3,
                         const uint32_t* alpha, uint32_t half_n) {
     if (!half_n) return;
-    fold_line_soa_kernel<<<ceil_div(half_n, 256), 256, 0, current_stream()>>>(
-        in0, in1, in2, in3, twiddles, out0, out1, out2, out3, q_from_host(alpha), half_n);
+    const SoaIn in = {{in0, in1, in2, in3}};
+    const SoaOut out = {{out0, out1, out2, out3}};
+    const bool vec = aligned(16, in0, in1, in2, in3) && aligned(8, twiddles, out0, out1, out2, out3);
+    if (vec)
+        fold_line_soa_kernel<true>
+            <<<ceil_div(half_n, 512), 256, 0, current_stream()>>>(in, twiddles, out, q_from_host(alpha), half_n);
+    else
+        fold_line_soa_kernel<false>
+            <<<ceil_div(half_n, 256), 256, 0, current_stream()>>>(in, twiddles, out, q_from_host(alpha), half_n);
     check_launch("cuda_fold_line_soa");
 }
 
@@ -88,8 +177,15 @@ void cuda_fold_circle_into_line_soa(uint32_t* dst0, uint32_t* dst1, uint32_t* ds
                                     const uint32_t* src3, const uint32_t* twiddles, const uint32_t* alpha,
                                     const uint32_t* alpha_sq, uint32_t half_n) {
     if (!half_n) return;
-    fold_circle_soa_kernel<<<ceil_div(half_n, 256), 256, 0, current_stream()>>>(
-        dst0, dst1, dst2, dst3, src0, src1, src2, src3, twiddles, q_from_host(alpha), q_from_host(alpha_sq), half_n);
+    const SoaIn src = {{src0, src1, src2, src3}};
+    const SoaOut dst = {{dst0, dst1, dst2, dst3}};
+    const bool vec = aligned(16, src0, src1, src2, src3) && aligned(8, twiddles, dst0, dst1, dst2, dst3);
+    if (vec)
+        fold_circle_soa_kernel<true><<<ceil_div(half_n, 512), 256, 0, current_stream()>>>(
+            dst, src, twiddles, q_from_host(alpha), q_from_host(alpha_sq), half_n);
+    else
+        fold_circle_soa_kernel<false><<<ceil_div(half_n, 256), 256, 0, current_stream()>>>(
+            dst, src, twiddles, q_from_host(alpha), q_from_host(alpha_sq), half_n);
     check_launch("cuda_fold_circle_into_line_soa");
 }
 
@@ -111,13 +207,21 @@ void cuda_fibonacci_quotient_chunk_stream(const uint32_t* trace, uint32_t* out0,
         set_error(-2, "cuda_fibonacci_quotient: need offset + chunk_n <= global_n");
         return;
     }
-    quotient_kernel<<<ceil_div(chunk_n, 256), 256, 0, (hipStream_t)stream>>>(
-        trace, out0, out1, out2, out3, q_from_host(alpha), offset, chunk_n, global_n);
+    const SoaOut out = {{out0, out1, out2, out3}};
+    if (global_n >= 8 && aligned(16, trace + offset, out0, out1, out2, out3))
+        quotient_kernel<true><<<ceil_div(chunk_n, 1024), 256, 0, (hipStream_t)stream>>>(
+            trace, out, q_from_host(alpha), offset, chunk_n, global_n);
+    else
+        quotient_kernel<false><<<ceil_div(chunk_n, 256), 256, 0, (hipStream_t)stream>>>(
+            trace, out, q_from_host(alpha), offset, chunk_n, global_n);
     check_launch("cuda_fibonacci_quotient");
 }
 void cuda_zero_pad(const uint32_t* src, uint32_t* dst, uint32_t src_n, uint32_t dst_n) {
     if (!dst_n) return;
-    zero_pad_kernel<<<ceil_div(dst_n, 256), 256, 0, current_stream()>>>(src, dst, src_n, dst_n);
+    if (aligned(16, src, dst))
+        zero_pad_kernel<true><<<ceil_div(dst_n, 1024), 256, 0, current_stream()>>>(src, dst, src_n, dst_n);
+    else
+        zero_pad_kernel<false><<<ceil_div(dst_n, 256), 256, 0, current_stream()>>>(src, dst, src_n, dst_n);
     check_launch("cuda_zero_pad");
 }
 

@@ -83,7 +83,7 @@ static __global__ __launch_bounds__(FRI_TAIL_THREADS) void fri_tail_kernel(FriTa
         if (more && k1 < n / 2) tw1 = args.L[li + 1].tw[k1];  // in flight while this layer is hashed
         uint32_t m = n, lvl = 0;
         if (k < n) {
-            const QM31 alpha = {{al[0], al[1], al[2], al[3]}};
+            const QMatrix alpha(QM31{{al[0], al[1], al[2], al[3]}});
             const QM31 f = fold_pair({{in[0].x, in[1].x, in[2].x, in[3].x}}, {{in[0].y, in[1].y, in[2].y, in[3].y}},
                                      alpha, tw);
             if (quads) {

@@ -151,7 +151,13 @@ struct SrcSoa4 {
 __device__ __forceinline__ QM31 quotient_at(uint32_t t0, uint32_t t1, uint32_t t2, QM31 alpha) {
     return qmul_m31(alpha, msub(t2, madd(t1, t0)));
 }
-__device__ __forceinline__ QM31 load_alpha(const uint32_t* a) { return {{a[0], a[1], a[2], a[3]}}; }
+// A challenge, written by an earlier launch: the same four words for every lane,
+// so they come by scalar loads.
+typedef const __attribute__((address_space(4))) uint32_t ConstU32;
+__device__ __forceinline__ QM31 load_alpha(const uint32_t* a) {
+    ConstU32* c = (ConstU32*)a;
+    return {{c[0], c[1], c[2], c[3]}};
+}
 
 struct SrcQuotient {
     const uint32_t* t;
@@ -199,12 +205,12 @@ struct SrcCircleFold {
     }
     // With q(i) = aq * d(i), d(i) = t[i+2] - t[i+1] - t[i] an M31 value, the fold
     // (q0 + q1) + af * ((q0 - q1) * tw) equals aq * (d0 + d1) + (af * aq) * ((d0 - d1) * tw):
-    // nine M31 products per output instead of twenty-one.
+    // nine M31 products and five reductions per output.
     __device__ __forceinline__ static QM31 fold_d(uint32_t d0, uint32_t d1, QM31 aq, QM31 g, uint32_t tw) {
         const uint32_t s = madd(d0, d1), u = mmul(msub(d0, d1), tw);
         QM31 r;
 #pragma unroll
-        for (int k = 0; k < 4; k++) r.v[k] = madd(mmul(aq.v[k], s), mmul(g.v[k], u));
+        for (int k = 0; k < 4; k++) r.v[k] = reduce64((uint64_t)aq.v[k] * s + (uint64_t)g.v[k] * u);
         return r;
     }
     static constexpr uint32_t WIDTH = 4;
@@ -227,9 +233,9 @@ struct SrcCircleFold {
         uint2 a = *(const uint2*)(t + j);
         uint2 b = *(const uint2*)(t + ((j + 2) & mask));
         uint2 c = *(const uint2*)(t + ((j + 4) & mask));
+        uint2 w = *(const uint2*)(tw + i);
         const uint32_t d0 = msub(b.x, madd(a.y, a.x)), d1 = msub(b.y, madd(b.x, a.y));
         const uint32_t d2 = msub(c.x, madd(b.y, b.x)), d3 = msub(c.y, madd(c.x, b.y));
-        uint2 w = *(const uint2*)(tw + i);
         QM31 f0 = fold_d(d0, d1, aq, g, w.x);
         QM31 f1 = fold_d(d2, d3, aq, g, w.y);
         *(uint2*)(o0 + i) = make_uint2(f0.v[0], f1.v[0]);
@@ -259,13 +265,13 @@ struct SrcLineFold {
     __device__ __forceinline__ void words(uint64_t i, uint32_t l, uint32_t v[4]) const {
         const uint2 a = *(const uint2*)(i0 + 2 * i), b = *(const uint2*)(i1 + 2 * i);
         const uint2 c = *(const uint2*)(i2 + 2 * i), d = *(const uint2*)(i3 + 2 * i);
-        const QM31 f = fold_pair({{a.x, b.x, c.x, d.x}}, {{a.y, b.y, c.y, d.y}}, load_alpha(alpha), tw[i]);
+        const QM31 f = fold_pair({{a.x, b.x, c.x, d.x}}, {{a.y, b.y, c.y, d.y}}, QMatrix(load_alpha(alpha)), tw[i]);
         for (int k = 0; k < 4; k++) v[k] = f.v[k];
         uint32_t* o = l == 0 ? o0 : l == 1 ? o1 : l == 2 ? o2 : o3;
         o[i] = l == 0 ? f.v[0] : l == 1 ? f.v[1] : l == 2 ? f.v[2] : f.v[3];
     }
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
-        QM31 al = load_alpha(alpha);
+        const QMatrix al(load_alpha(alpha));
         uint64_t j = 2 * i;
         uint4 a = *(const uint4*)(i0 + j), b = *(const uint4*)(i1 + j);
         uint4 c = *(const uint4*)(i2 + j), d = *(const uint4*)(i3 + j);
@@ -349,18 +355,6 @@ struct SrcLifted {
     }
 };
 
-// x < 2^64 -> a value < 2^33 congruent to it mod p: bits 0..30, plus bits
-// 31..62 (times 2^31 = 1), plus bit 63 (times 2^63 = 2 mod p).
-__device__ __forceinline__ uint64_t fold62(uint64_t x) {
-    const uint32_t lo = (uint32_t)x, hi = (uint32_t)(x >> 32);
-    return (uint64_t)(lo & P) + __builtin_amdgcn_alignbit(hi, lo, 31) + 2u * (hi >> 31);
-}
-// x < 2^64 -> x mod p
-__device__ __forceinline__ uint32_t reduce64(uint64_t x) {
-    x = fold62(fold62(x));  // < 2^31 + 4
-    return canon((uint32_t)x);
-}
-
 // First FRI layer of the wide commitment: f = sum_c beta^c * lifted_c is formed
 // on the fly from the LDE columns, circle-folded pairwise (2j, 2j + 1) with
 // alpha and tw[j], stored to out and hashed as an SoA4 leaf.
@@ -376,9 +370,9 @@ struct SrcWideFold {
     uint32_t* o2;
     uint32_t* o3;
     __device__ __forceinline__ SrcWideFold at(uint64_t) const { return *this; }
-    // sum_c beta^c * v_c with 64-bit products accumulated unreduced: three
-    // products (< 2^62 each) fit on top of a folded (< 2^33) accumulator, so
-    // accumulators are folded after every group of three columns. A lifted
+    // sum_c beta^c * v_c with 64-bit products accumulated unreduced: four
+    // products fit on top of a folded accumulator (fold64), so accumulators are
+    // folded after every group of four columns. A lifted
     // column gives the four f indices two values (rows r, r + 1, repeated), so
     // the lifted columns are summed first into two accumulators, which then
     // start the four of the full-size columns: 32 fewer registers than keeping
@@ -387,9 +381,8 @@ struct SrcWideFold {
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         const uint64_t j = 2 * i;  // f index of the first of four inputs (a multiple of 4)
         ConstLiftCol* tab = const_table(cols);
-        typedef const __attribute__((address_space(4))) uint32_t ConstU32;
         ConstU32* bp = (ConstU32*)beta_pows;
-        constexpr uint32_t G = 3;
+        constexpr uint32_t G = 4;
         uint64_t ag[2][4] = {};
         uint32_t c = 0;
         while (c < n_cols && tab[c].sh != 0) {
@@ -415,8 +408,8 @@ struct SrcWideFold {
             }
 #pragma unroll
             for (int m = 0; m < 4; m++) {
-                ag[0][m] = fold62(ag[0][m]);
-                ag[1][m] = fold62(ag[1][m]);
+                ag[0][m] = fold64(ag[0][m]);
+                ag[1][m] = fold64(ag[1][m]);
             }
             c += n;
         }
@@ -443,13 +436,13 @@ struct SrcWideFold {
             }
 #pragma unroll
             for (int m = 0; m < 4; m++)
-                for (int k = 0; k < 4; k++) af[k][m] = fold62(af[k][m]);
+                for (int k = 0; k < 4; k++) af[k][m] = fold64(af[k][m]);
         }
         QM31 f[4];
 #pragma unroll
         for (int k = 0; k < 4; k++)
             for (int m = 0; m < 4; m++) f[k].v[m] = reduce64(af[k][m]);
-        const QM31 al = load_alpha(alpha);
+        const QMatrix al(load_alpha(alpha));
         const uint2 w = *(const uint2*)(tw + i);
         const QM31 g0 = fold_pair(f[0], f[1], al, w.x);
         const QM31 g1 = fold_pair(f[2], f[3], al, w.y);
