@@ -69,7 +69,7 @@ def test_fold_sources(vx, log_n, n, use_y):
     got = out.to_host()
     assert got[n // 2] == 7
     half = n // 2
-    picks = range(half) if half <= 512 else sorted(set(rnd(5, 300) % half) | {0, 15, 16, 4095, half - 1})
+    picks = range(half) if half <= 512 else sorted(set(rnd(5, 300) % half) | {0, 15, 16, 1023, 1024, 4095, half - 1})
     for i in picks:
         e = brev((2 * int(i)) & ((1 << log_n) - 1), log_n)
         assert got[i] == mul(initial, power(step, e))[use_y], i

@@ -48,16 +48,6 @@ void lde_batch(uint32_t* const* cols, uint32_t n_cols, const NttTables& ti, cons
                const uint32_t* const* srcs, bool src_aligned,
                const std::function<void(const char*)>& mark = nullptr);
 
-// Builds the twiddles of coset (initial, step) of size 2^log_n directly on the
-// device: line (2^log_n - 1 words), circle (2^(log_n-1) words) and, when the
-// i* pointers are non-null, their inverses. offs receives the layer offsets.
-void build_ntt_tables(CPt initial, CPt step, uint32_t log_n, uint32_t* line, uint32_t* circle, uint32_t* iline,
-                      uint32_t* icircle, uint32_t offs[32], hipStream_t s);
-// FRI fold twiddles of a domain: out[i] = 1 / coord(initial * step^bitrev(2i)), i < 2^(log_n-1).
-void build_fold_twiddles(CPt initial, CPt step, uint32_t log_n, bool use_y, uint32_t* out, uint32_t* scratch,
-                         hipStream_t s);
-void batch_inverse(const uint32_t* in, uint32_t* out, uint64_t n, hipStream_t s);
-
 // Host-side circle arithmetic used to derive coset parameters.
 struct HostPt {
     uint32_t x, y;
@@ -67,5 +57,25 @@ HostPt host_repeated_double(HostPt p, uint32_t n);
 HostPt host_generator();
 // kind: 0 subgroup, 1 half_coset, 2 half_odds (src/circle.rs:98-143)
 void host_coset(int kind, uint32_t log_size, HostPt& initial, HostPt& step);
+
+// Builds the twiddles of coset (initial, step) of size 2^log_n directly on the
+// device, or (inverse) their inverses, no twiddle being zero: line (2^log_n - 1
+// words) and circle (2^(log_n-1) words). offs receives the layer offsets.
+void build_ntt_tables(HostPt initial, HostPt step, uint32_t log_n, uint32_t* line, uint32_t* circle, bool inverse,
+                      uint32_t offs[32], hipStream_t s);
+// FRI fold twiddles of a domain of 2^(log_len+1) points:
+// out[i] = 1 / coord(initial * step^bitrev(i)), i < 2^log_len (log_len <= 30).
+struct FoldDomain {
+    HostPt initial, step;
+    uint32_t log_len;
+    bool use_y;
+    uint32_t* out;
+};
+// of several domains, none of whose coordinates is zero; layers that follow one
+// another as FRI folds share a launch
+void build_fold_twiddles(const FoldDomain* d, uint32_t n, hipStream_t s);
+// of one domain with zero coordinates (scratch: as many words as out)
+void build_fold_twiddles_chunked(const FoldDomain& d, uint32_t* scratch, hipStream_t s);
+void batch_inverse(const uint32_t* in, uint32_t* out, uint64_t n, hipStream_t s);
 
 }  // namespace vx

@@ -60,15 +60,6 @@ void host_coset(int kind, uint32_t k, HostPt& initial, HostPt& step) {
     else
         initial = host_repeated_double(g, k >= 29 ? 0 : 29 - k);
 }
-static HostPt host_pow(HostPt p, uint64_t e) {
-    HostPt r = {1, 0};
-    while (e) {
-        if (e & 1) r = host_pmul(r, p);
-        p = host_pmul(p, p);
-        e >>= 1;
-    }
-    return r;
-}
 
 // ---------------------------------------------------------------- pass kernel
 struct NttPassArgs {
@@ -882,38 +873,102 @@ __global__ void coset_points_kernel(CPt initial, CPt step, uint32_t* ox, uint32_
     ox[i] = p.x;
     oy[i] = p.y;
 }
-// Points of a geometric progression: thread t of T visits i = t + k * T for
-// k < PROG_K (i < n), one point product per step after a single power.
-constexpr uint32_t PROG_K = 16;
-template <class F>
-__device__ __forceinline__ void progression(CPt initial, CPt step, uint64_t n, F&& f) {
-    const uint64_t T = (n + PROG_K - 1) / PROG_K;
-    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= T) return;
-    const CPt stride = cp_pow_mul(CPt{1, 0}, step, T);
-    CPt p = cp_pow_mul(initial, step, t);
-#pragma unroll 4
-    for (uint32_t k = 0; k < PROG_K; k++) {
-        const uint64_t i = t + (uint64_t)k * T;
-        if (i >= n) break;
-        f(i, p);
-        p = cpmul(p, stride);
+// Fold twiddles and their sources. Word i of a domain of 2^(L+1) points is a
+// coordinate of initial * step^bitrev_L(i), so bit b of i contributes the point
+// u[b] = step^(2^(L-1-b)) whatever the rest of i is, and a domain whose step is
+// the square of the one before it (each FRI layer's) has the same u: one launch
+// makes every layer. A thread makes a run of consecutive words from its first
+// point and the products of u[0], u[1], ..: two multiplications a word where a
+// power per word took 30, and none of the bits above a block costs a vector
+// instruction. The inverses of the thread's words then cost three more each and
+// one inversion, in registers, where they took two more passes. 2^19 sources: 18
+// -> 6 us; the 14 layers of a 2^18-point domain with their inverses: 6.6 us, where
+// each layer took two launches of 4 to 17.
+constexpr uint32_t TABLE_THREADS = 256;
+constexpr uint32_t TABLE_RUN_LOG = 4;   // with inverses, and in the NTT tables
+constexpr uint32_t SOURCE_RUN_LOG = 2;  // sources alone: a shorter chain
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(4)));  // any word address
+
+// w[r] -> 1 / w[r]; a zero stays zero
+template <uint32_t RUN>
+__device__ __forceinline__ void invert_run(uint32_t (&w)[RUN]) {
+    uint32_t pre[RUN], acc = 1;
+#pragma unroll
+    for (uint32_t r = 0; r < RUN; r++) {
+        pre[r] = acc;
+        acc = mmul(acc, w[r] ? w[r] : 1u);
+    }
+    uint32_t iv = minv(acc);
+#pragma unroll
+    for (int r = RUN - 1; r >= 0; r--) {
+        const uint32_t v = w[r];
+        w[r] = v ? mmul(iv, pre[r]) : 0u;
+        iv = mmul(iv, v ? v : 1u);
     }
 }
-inline uint32_t progression_blocks(uint64_t n, uint32_t threads) {
-    return (uint32_t)ceil_div((n + PROG_K - 1) / PROG_K, threads);
+// words i .. i + RUN - 1 of an array of len words
+template <uint32_t RUN>
+__device__ __forceinline__ void store_run(uint32_t* out, uint64_t i, uint64_t len, const uint32_t (&w)[RUN]) {
+    if (i + RUN <= len) {
+#pragma unroll
+        for (uint32_t r = 0; r < RUN; r += 4) {
+            const u32x4_any v = {w[r], w[r + 1], w[r + 2], w[r + 3]};
+            *(__attribute__((address_space(1))) u32x4_any*)(out + i + r) = v;
+        }
+    } else {
+#pragma unroll
+        for (uint32_t r = 0; r < RUN; r++)
+            if (i + r < len) out[i + r] = w[r];
+    }
+}
+// start * the points of the set bits of run number blk * TABLE_THREADS + tid,
+// bit b being pts[RUN_LOG + b]
+template <uint32_t RUN_LOG>
+__device__ __forceinline__ CPt run_start(CPt start, const CPt* pts, uint32_t blk) {
+    CPt p = start;
+    constexpr uint32_t TB = 8;
+    static_assert(TABLE_THREADS == 1u << TB);
+    for (uint32_t b = RUN_LOG + TB; blk; b++, blk >>= 1)
+        if (blk & 1) p = cpmul(p, pts[b]);
+#pragma unroll
+    for (uint32_t b = 0; b < TB; b++) {
+        const bool on = (threadIdx.x >> b) & 1;
+        const CPt q = pts[RUN_LOG + b];
+        p = cpmul(p, CPt{on ? q.x : 1u, on ? q.y : 0u});
+    }
+    return p;
+}
+struct FoldTables {
+    CPt u[32];                // the point of each bit of a word's index
+    CPt top[1u << TABLE_RUN_LOG];  // the products of u[0..3]
+    CPt initial[32];          // per layer
+    uint32_t* out[32];
+    uint32_t first_block[33];
+    uint32_t log_len[32];
+    uint32_t use_y;           // bit l: layer l takes y
+    uint32_t n_layers;
+};
+template <bool INV>
+__global__ __launch_bounds__(TABLE_THREADS) void fold_tables_kernel(FoldTables m) {
+    constexpr uint32_t LOG = INV ? TABLE_RUN_LOG : SOURCE_RUN_LOG, RUN = 1u << LOG;
+    uint32_t l = 0;
+    while (blockIdx.x >= m.first_block[l + 1]) l++;
+    const uint32_t blk = blockIdx.x - m.first_block[l];
+    const uint64_t len = 1ull << m.log_len[l], i = ((uint64_t)blk * TABLE_THREADS + threadIdx.x) * RUN;
+    if (i >= len) return;
+    const CPt p = run_start<LOG>(m.initial[l], m.u, blk);
+    const bool y = (m.use_y >> l) & 1;
+    uint32_t w[RUN];
+#pragma unroll
+    for (uint32_t r = 0; r < RUN; r++) {
+        const uint32_t c0 = y ? m.top[r].y : m.top[r].x, c1 = y ? m.top[r].x : P - m.top[r].y;
+        w[r] = reduce64((uint64_t)p.x * c0 + (uint64_t)p.y * c1);
+    }
+    if constexpr (INV) invert_run(w);
+    store_run(m.out[l], i, len, w);
 }
 
-// Fold-twiddle sources of a domain of n = 2^log_n points: out[i] = coordinate
-// of initial * step^(bitrev(2i)). The exponents bitrev(2i) are exactly the
-// j < n/2, so the points are made in natural order and stored to
-// i = bitrev(j) / 2.
-__global__ void fold_sources_pow2_kernel(CPt initial, CPt step, uint32_t* out, uint32_t half_n, uint32_t log_n,
-                                         int use_y) {
-    progression(initial, step, half_n, [&](uint64_t j, CPt p) {
-        out[brev_bits((uint32_t)j, log_n) >> 1] = use_y ? p.y : p.x;
-    });
-}
+// Sources of any n: out[i] = coordinate of initial * step^bitrev_(log_n)(2i).
 __global__ void fold_sources_kernel(CPt initial, CPt step, uint32_t* out, uint32_t half_n, uint32_t log_n,
                                     int use_y) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -933,103 +988,176 @@ __global__ void squash_kernel(const uint32_t* in, uint32_t* tw_out, uint32_t* sq
 // Closed form of the line twiddles: layer l, entry i equals
 // x(initial^(2^l) * step^(i * 2^(2l+1))), i.e. the x-coordinate that the
 // extract-and-squash chain of circle.rs:394-425 produces for that slot
-// (each squash doubles the point and keeps every second one).
-// Per-layer starting point, step and word offset of the line twiddles, passed
-// by value (at most 31 layers).
-struct LineTwiddleMeta {
-    CPt base[32];
-    CPt step[32];
+// (each squash doubles the point and keeps every second one); the circle
+// twiddles are y(initial * step^i). Bit b of i contributes step^(2^(b+shift)),
+// so all layers draw on one table of squares and one launch makes them all,
+// each thread 16 consecutive words of one, inverted in registers where
+// the transform wants the inverses.
+struct NttTableArgs {
+    CPt sq[64];               // step^(2^b)
+    CPt base[32];             // per line layer; the circle layer comes last
     uint32_t offs[32];
+    uint32_t first_block[33];
+    uint32_t* line;
+    uint32_t* circle;
+    uint32_t log_n, n_line;
 };
-__global__ void line_twiddles_kernel(LineTwiddleMeta m, uint32_t* line, uint64_t n) {
-    const uint32_t l = blockIdx.y;  // layer l holds n / 2^(l+1) words
-    const uint64_t len = n >> (l + 1);
-    uint32_t* dst = line + m.offs[l];
-    progression(m.base[l], m.step[l], len, [&](uint64_t i, CPt p) { dst[i] = p.x; });
-}
-__global__ void circle_twiddles_kernel(CPt initial, CPt step, uint32_t* circle, uint32_t half_n) {
-    progression(initial, step, half_n, [&](uint64_t i, CPt p) { circle[i] = p.y; });
+template <bool INV>
+__global__ __launch_bounds__(TABLE_THREADS) void ntt_tables_kernel(NttTableArgs m) {
+    constexpr uint32_t RUN = 1u << TABLE_RUN_LOG;
+    uint32_t l = 0;
+    while (blockIdx.x >= m.first_block[l + 1]) l++;
+    const uint32_t blk = blockIdx.x - m.first_block[l];
+    const bool circle = l == m.n_line;
+    const uint32_t shift = circle ? 0u : 2 * l + 1;
+    const uint64_t len = (1ull << m.log_n) >> (circle ? 1 : l + 1);
+    const uint64_t i = ((uint64_t)blk * TABLE_THREADS + threadIdx.x) * RUN;
+    // word n - 2 of the n - 1 word layout belongs to no layer; it is zero
+    if (circle && m.n_line && i == 0) m.line[(1ull << m.log_n) - 2] = 0;
+    if (i >= len) return;
+    CPt p = run_start<TABLE_RUN_LOG>(m.base[l], m.sq + shift, blk);
+    const CPt step = m.sq[shift];
+    uint32_t w[RUN];
+#pragma unroll
+    for (uint32_t r = 0; r < RUN; r++) {
+        w[r] = circle ? p.y : p.x;
+        if (r + 1 < RUN) p = cpmul(p, step);
+    }
+    if constexpr (INV) invert_run(w);
+    store_run(circle ? m.circle : m.line + m.offs[l], i, len, w);
 }
 
 // Montgomery batch inverse with the outputs of cuda/batch_inverse.cu:8-41.
 // That kernel runs one thread per 64-word chunk whose prefix products skip zero
 // words but start from the chunk's first word as it is: zeros map to zero,
 // other words to their inverses, and a chunk whose first word is zero maps
-// entirely to zero (its product is zero). Here thread t of T inverts the BI_K
+// entirely to zero (its product is zero). Here thread t of T inverts the K
 // words t + k * T, so each load and store of a wave is contiguous and the
 // prefix products stay in registers, and the chunk rule is applied per word.
-constexpr uint32_t BI_K = 32;
+// K = 8 costs eight multiplications a word and fills the chip from 2^20 words on
+// (2^24: 48.5 us at K = 32, 34.2 at 8, 34.6 at 16); below, K = 4 shortens the
+// chain of one thread, which is all the launch then is (2^19: 15 -> 4 us).
+constexpr uint64_t BI_WIDE_MIN = 1u << 20;
+template <uint32_t K>
 __global__ __launch_bounds__(128) void batch_inverse_kernel(const uint32_t* in, uint32_t* out, uint64_t n) {
-    const uint64_t T = (n + BI_K - 1) / BI_K;
+    const uint64_t T = (n + K - 1) / K;
     const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= T) return;
-    uint32_t v[BI_K], pre[BI_K];
+    uint32_t v[K], pre[K];
+    bool live[K];
     uint32_t acc = 1;
 #pragma unroll
-    for (uint32_t k = 0; k < BI_K; k++) {
+    for (uint32_t k = 0; k < K; k++) {
         const uint64_t i = t + (uint64_t)k * T;
         v[k] = i < n ? in[i] : 0;
+        live[k] = i < n && in[i & ~63ull];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < K; k++) {
         pre[k] = acc;  // product of the non-zero v[0 .. k-1]
         if (v[k]) acc = mmul(acc, v[k]);
     }
     uint32_t iv = minv(acc);  // 1 / product of all non-zero v
 #pragma unroll
-    for (int k = BI_K - 1; k >= 0; k--) {
+    for (int k = K - 1; k >= 0; k--) {
         const uint64_t i = t + (uint64_t)k * T;
-        if (i < n) out[i] = (v[k] && in[i & ~63ull]) ? mmul(iv, pre[k]) : 0;
+        if (i < n) out[i] = (v[k] && live[k]) ? mmul(iv, pre[k]) : 0;
         if (v[k]) iv = mmul(iv, v[k]);
     }
 }
 
 void batch_inverse(const uint32_t* in, uint32_t* out, uint64_t n, hipStream_t s) {
     if (!n) return;
-    batch_inverse_kernel<<<ceil_div((n + BI_K - 1) / BI_K, 128), 128, 0, s>>>(in, out, n);
+    if (n >= BI_WIDE_MIN)
+        batch_inverse_kernel<8><<<ceil_div((n + 7) / 8, 128), 128, 0, s>>>(in, out, n);
+    else
+        batch_inverse_kernel<4><<<ceil_div((n + 3) / 4, 128), 128, 0, s>>>(in, out, n);
     check_launch("batch_inverse_kernel");
 }
 
-void build_ntt_tables(CPt initial, CPt step, uint32_t log_n, uint32_t* line, uint32_t* circle, uint32_t* iline,
-                      uint32_t* icircle, uint32_t offs[32], hipStream_t s) {
-    uint64_t n = 1ull << log_n;
-    uint32_t n_line = log_n > 0 ? log_n - 1 : 0;
-    for (int i = 0; i < 32; i++) offs[i] = 0;
-    uint64_t off = 0, cur = n;
-    LineTwiddleMeta meta = {};
-    HostPt hi = {initial.x, initial.y}, hs = {step.x, step.y};
-    for (uint32_t l = 0; l < n_line; l++) {
-        offs[l] = (uint32_t)off;
-        meta.offs[l] = (uint32_t)off;
-        HostPt b = host_repeated_double(hi, l);                 // initial^(2^l)
-        HostPt st = host_pow(hs, 1ull << (2 * l + 1));          // step^(2^(2l+1))
-        meta.base[l] = {b.x, b.y};
-        meta.step[l] = {st.x, st.y};
-        off += cur / 2;
-        cur /= 2;
-    }
-    if (n_line) {
-        // n - 1 line words in total; the last entry of each layer is unused by
-        // the transform but is part of the reference layout.
-        line_twiddles_kernel<<<dim3(progression_blocks(n / 2, 256), n_line), 256, 0, s>>>(meta, line, n);
-        check_launch("line_twiddles_kernel");
-        // Word n-2 of the n-1 word layout belongs to no layer; keep it defined (zero)
-        // so the batch inverse below never reads an undefined value.
-        check(hipMemsetAsync(line + off, 0, 4 * (n - 1 - off), s), "hipMemsetAsync");
-    }
-    if (n >= 2) {
-        circle_twiddles_kernel<<<progression_blocks(n / 2, 256), 256, 0, s>>>(initial, step, circle, (uint32_t)(n / 2));
-        check_launch("circle_twiddles_kernel");
-    }
-    if (iline && n_line) batch_inverse(line, iline, n - 1, s);
-    if (icircle && n >= 2) batch_inverse(circle, icircle, n / 2, s);
+static CPt cpt(HostPt h) { return {h.x, h.y}; }
+static uint32_t table_blocks(uint64_t len, uint32_t run_log) {
+    return (uint32_t)ceil_div(((len - 1) >> run_log) + 1, TABLE_THREADS);
 }
 
-void build_fold_twiddles(CPt initial, CPt step, uint32_t log_n, bool use_y, uint32_t* out, uint32_t* scratch,
-                         hipStream_t s) {
-    uint32_t half = (uint32_t)((1ull << log_n) / 2);
-    if (!half) return;
-    fold_sources_pow2_kernel<<<progression_blocks(half, 256), 256, 0, s>>>(initial, step, scratch, half, log_n,
-                                                                           use_y ? 1 : 0);
-    check_launch("fold_sources_pow2_kernel");
-    batch_inverse(scratch, out, half, s);
+void build_ntt_tables(HostPt initial, HostPt step, uint32_t log_n, uint32_t* line, uint32_t* circle, bool inverse,
+                      uint32_t offs[32], hipStream_t s) {
+    const uint64_t n = 1ull << log_n;
+    NttTableArgs m = {};
+    m.line = line;
+    m.circle = circle;
+    m.log_n = log_n;
+    m.n_line = log_n > 0 ? log_n - 1 : 0;
+    uint64_t off = 0;
+    HostPt b = initial;
+    for (uint32_t l = 0; l < m.n_line; l++) {  // the last entry of each layer is unused, but part of the layout
+        m.offs[l] = (uint32_t)off;
+        m.base[l] = cpt(b);  // initial^(2^l)
+        m.first_block[l + 1] = m.first_block[l] + table_blocks(n >> (l + 1), TABLE_RUN_LOG);
+        b = host_pmul(b, b);
+        off += n >> (l + 1);
+    }
+    for (int i = 0; i < 32; i++) offs[i] = m.offs[i];
+    if (n < 2) return;
+    m.base[m.n_line] = cpt(initial);
+    m.first_block[m.n_line + 1] = m.first_block[m.n_line] + table_blocks(n / 2, TABLE_RUN_LOG);
+    for (uint32_t k = 0; k < 64; k++, step = host_pmul(step, step)) m.sq[k] = cpt(step);
+    if (inverse)
+        ntt_tables_kernel<true><<<m.first_block[m.n_line + 1], TABLE_THREADS, 0, s>>>(m);
+    else
+        ntt_tables_kernel<false><<<m.first_block[m.n_line + 1], TABLE_THREADS, 0, s>>>(m);
+    check_launch("ntt_tables_kernel");
+}
+
+// step^(2^(log_len-1-b)) for every bit b of a word's index
+static void index_points(HostPt step, uint32_t log_len, HostPt u[32]) {
+    for (uint32_t b = log_len; b-- > 0; step = host_pmul(step, step)) u[b] = step;
+}
+static void fold_tables(const FoldDomain* d, uint32_t n, bool inverse, hipStream_t s) {
+    while (n) {
+        FoldTables m = {};
+        HostPt u[32] = {}, v[32];
+        index_points(d[0].step, d[0].log_len, u);
+        for (uint32_t b = 0; b < d[0].log_len; b++) m.u[b] = cpt(u[b]);
+        for (uint32_t r = 0; r < 1u << TABLE_RUN_LOG; r++) {
+            HostPt q = {1, 0};
+            for (uint32_t b = 0; b < TABLE_RUN_LOG; b++)
+                if (((r >> b) & 1) && b < d[0].log_len) q = host_pmul(q, u[b]);
+            m.top[r] = cpt(q);
+        }
+        // the layers that follow with the same points of their (fewer) bits
+        uint32_t l = 0;
+        for (; l < n && l < 32 && d[l].log_len <= d[0].log_len; l++) {
+            index_points(d[l].step, d[l].log_len, v);
+            bool same = true;
+            for (uint32_t b = 0; b < d[l].log_len; b++) same &= u[b].x == v[b].x && u[b].y == v[b].y;
+            if (!same) break;
+            m.initial[l] = cpt(d[l].initial);
+            m.out[l] = d[l].out;
+            m.log_len[l] = d[l].log_len;
+            m.use_y |= (d[l].use_y ? 1u : 0u) << l;
+            m.first_block[l + 1] = m.first_block[l] + table_blocks(1ull << d[l].log_len, inverse ? TABLE_RUN_LOG : SOURCE_RUN_LOG);
+        }
+        m.n_layers = l;
+        if (inverse)
+            fold_tables_kernel<true><<<m.first_block[l], TABLE_THREADS, 0, s>>>(m);
+        else
+            fold_tables_kernel<false><<<m.first_block[l], TABLE_THREADS, 0, s>>>(m);
+        check_launch("fold_tables_kernel");
+        d += l;
+        n -= l;
+    }
+}
+void build_fold_twiddles(const FoldDomain* d, uint32_t n, hipStream_t s) { fold_tables(d, n, true, s); }
+
+// The whole group's fold twiddles (log_n = 31), by the two passes of the kernel
+// ABI: its points (1, 0) and (-1, 0) have y = 0, and the batch inverse makes the
+// 64-word chunk that begins with a zero all zero.
+void build_fold_twiddles_chunked(const FoldDomain& d, uint32_t* scratch, hipStream_t s) {
+    FoldDomain src = d;
+    src.out = scratch;
+    fold_tables(&src, 1, false, s);
+    batch_inverse(scratch, d.out, 1ull << d.log_len, s);
 }
 
 // ---------------------------------------------------------------- single layer / bit reverse
@@ -1230,7 +1358,7 @@ int32_t vx_ntt_autotune(uint32_t log_min, uint32_t log_max, float* best_ms) {
         t.line = line;
         t.circle = circle;
         t.log_n = k;
-        build_ntt_tables(CPt{hi.x, hi.y}, CPt{hs.x, hs.y}, k, line, circle, nullptr, nullptr, t.offs, st);
+        build_ntt_tables(hi, hs, k, line, circle, false, t.offs, st);
         const uint32_t n_cols = k >= LDE_LOG_WORDS ? 1u : std::min<uint32_t>(LDE_MAX_COLS, 1u << (LDE_LOG_WORDS - k));
         ok = check(hipMemsetAsync(data, 0x11, 4ull * n_cols << k, st), "hipMemsetAsync");  // canonical M31 words
         std::vector<uint32_t*> h_cols(n_cols);
@@ -1246,7 +1374,7 @@ int32_t vx_ntt_autotune(uint32_t log_min, uint32_t log_max, float* best_ms) {
             ti.line = line2;
             ti.circle = circle2;
             ti.log_n = k - 2;
-            build_ntt_tables(CPt{hi2.x, hi2.y}, CPt{hs2.x, hs2.y}, k - 2, line2, circle2, nullptr, nullptr, ti.offs, st);
+            build_ntt_tables(hi2, hs2, k - 2, line2, circle2, false, ti.offs, st);
         }
         // the general table on one full input, then the blowup-4 table on a batch
         // of LDEs (interpolation with the tuned plan of 2^(k-2), evaluation with
@@ -1310,6 +1438,11 @@ void cuda_compute_fold_twiddle_sources_stream(uint32_t ix, uint32_t iy, uint32_t
                                               uint32_t n, uint32_t log_n, int32_t extract_y, void* stream) {
     uint32_t half = n / 2;
     if (!half) return;
+    if (log_n <= 31 && n == 1u << log_n) {
+        const FoldDomain d = {{ix, iy}, {sx, sy}, log_n - 1, extract_y != 0, output};
+        fold_tables(&d, 1, false, (hipStream_t)stream);
+        return;
+    }
     fold_sources_kernel<<<ceil_div(half, 256), 256, 0, (hipStream_t)stream>>>(CPt{ix, iy}, CPt{sx, sy}, output,
                                                                               half, log_n, extract_y);
     check_launch("cuda_compute_fold_twiddle_sources");

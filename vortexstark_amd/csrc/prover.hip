@@ -516,8 +516,6 @@ uint64_t layout_words(const vx_prover* p) {
     return w;
 }
 
-CPt to_cpt(HostPt h) { return {h.x, h.y}; }
-
 // Word offsets of one arena (each region 256-byte aligned).
 void plan_arena(vx_prover* p) {
     uint64_t o = 0;
@@ -722,11 +720,11 @@ void set_sizes(vx_prover* p, uint32_t log_n, uint32_t n_queries, uint32_t log_la
 }
 
 // Device bytes vx_prover_create_batch allocates besides the arenas: NTT
-// twiddles of the trace and evaluation domains, fold twiddles and their
-// scratch, tree descriptors and per-proof call slots.
+// twiddles of the trace (inverse) and evaluation domains, fold twiddles (and,
+// for the whole group, their scratch), tree descriptors and per-proof call slots.
 uint64_t shared_bytes(const vx_prover* p) {
     const uint64_t N = p->N, E = p->E;
-    uint64_t b = 2 * 4 * (N - 1) + 2 * 4 * (N / 2) + 4 * (E - 1) + 4 * (E / 2) + 4 * (E / 2);
+    uint64_t b = 4 * (N - 1) + 4 * (N / 2) + 4 * (E - 1) + 4 * (E / 2) + (p->log_e == 31 ? 4 * (E / 2) : 0);
     for (uint32_t j = 0; j < p->J; j++) b += 4 * ((1ull << (p->log_e - j)) / 2);
     return b + sizeof(TreeDesc) * (2 + p->J) + (8 + 8 + 16) * (uint64_t)p->capacity;
 }
@@ -780,9 +778,8 @@ vx_prover* vx_prover_create_batch(uint32_t log_n, uint32_t n_queries, uint32_t l
     hipStream_t s = p->stream;
 
     // twiddle tables (ProverCache, prover.rs:159-176), shared by the batch
-    uint32_t *t_line, *t_circle, *t_iline, *t_icircle, *e_line, *e_circle;
-    ok = ok && p->alloc((void**)&t_line, 4 * (N - 1)) && p->alloc((void**)&t_circle, 4 * (N / 2)) &&
-         p->alloc((void**)&t_iline, 4 * (N - 1)) && p->alloc((void**)&t_icircle, 4 * (N / 2)) &&
+    uint32_t *t_iline, *t_icircle, *e_line, *e_circle;
+    ok = ok && p->alloc((void**)&t_iline, 4 * (N - 1)) && p->alloc((void**)&t_icircle, 4 * (N / 2)) &&
          p->alloc((void**)&e_line, 4 * (E - 1)) && p->alloc((void**)&e_circle, 4 * (E / 2));
     if (!ok) {
         delete p;
@@ -793,8 +790,8 @@ vx_prover* vx_prover_create_batch(uint32_t log_n, uint32_t n_queries, uint32_t l
     HostPt ti, ts, ei, es;
     host_coset(1, log_n, ti, ts);
     host_coset(p->log_e <= 30 ? 1 : 0, p->log_e, ei, es);
-    build_ntt_tables(to_cpt(ti), to_cpt(ts), log_n, t_line, t_circle, t_iline, t_icircle, p->trace_tab.offs, s);
-    build_ntt_tables(to_cpt(ei), to_cpt(es), p->log_e, e_line, e_circle, nullptr, nullptr, p->eval_tab.offs, s);
+    build_ntt_tables(ti, ts, log_n, t_iline, t_icircle, true, p->trace_tab.offs, s);
+    build_ntt_tables(ei, es, p->log_e, e_line, e_circle, false, p->eval_tab.offs, s);
     p->trace_tab.line = t_iline;
     p->trace_tab.circle = t_icircle;
     p->trace_tab.log_n = log_n;
@@ -806,17 +803,21 @@ vx_prover* vx_prover_create_batch(uint32_t log_n, uint32_t n_queries, uint32_t l
     // (subgroup(31) when log_e = 31, prover.rs:754-757: its points (1, 0) and
     // (-1, 0) have y = 0, whose inverse the batch inverse takes as 0);
     // [j] line on half_odds(log_e - j), x.
-    uint32_t* tw_scratch;
-    ok = p->alloc((void**)&tw_scratch, 4 * (E / 2));
+    const bool whole_group = p->log_e == 31;
+    uint32_t* tw_scratch = nullptr;
+    if (whole_group) ok = p->alloc((void**)&tw_scratch, 4 * (E / 2));
     p->fri_tw.assign(p->J, nullptr);
+    std::vector<FoldDomain> fd(p->J);
     for (uint32_t j = 0; ok && j < p->J; j++) {
-        uint32_t k = p->log_e - j;
+        const uint32_t k = p->log_e - j;
         ok = p->alloc((void**)&p->fri_tw[j], 4 * ((1ull << k) / 2));
-        if (!ok) break;
-        HostPt di, dstp;
-        host_coset(j == 0 ? (k <= 30 ? 1 : 0) : 2, k, di, dstp);
-        build_fold_twiddles(to_cpt(di), to_cpt(dstp), k, j == 0, p->fri_tw[j], tw_scratch, s);
+        host_coset(j == 0 ? (whole_group ? 0 : 1) : 2, k, fd[j].initial, fd[j].step);
+        fd[j].log_len = k - 1;
+        fd[j].use_y = j == 0;
+        fd[j].out = p->fri_tw[j];
     }
+    if (ok && whole_group) build_fold_twiddles_chunked(fd[0], tw_scratch, s);
+    if (ok) build_fold_twiddles(fd.data() + whole_group, p->J - whole_group, s);
 
     Layout L;
     build_layout(p, L);

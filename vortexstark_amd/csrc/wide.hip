@@ -51,14 +51,6 @@ __global__ void stwo_twiddles_kernel(uint32_t* out, uint64_t tc) {
     out[g] = cp_pow_mul(CPt{1, 0}, CPt{2u, 1268011823u}, e).x;
 }
 
-// coordinate of initial * step^bitrev_bits(i), i < n
-__global__ void brt_coord_kernel(CPt initial, CPt step, uint32_t* out, uint64_t n, uint32_t bits, int use_y) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const CPt p = cp_pow_mul(initial, step, brev_bits((uint32_t)i, bits));
-    out[i] = use_y ? p.y : p.x;
-}
-
 void build_stwo_twiddles(uint32_t log_n, uint32_t* fwd, uint32_t* inv, hipStream_t s) {
     const uint64_t tc = (1ull << log_n) / 2;
     if (!tc) return;
@@ -228,10 +220,6 @@ struct vx_wide {
     }
 };
 
-namespace {
-CPt cpt(HostPt h) { return {h.x, h.y}; }
-}  // namespace
-
 extern "C" {
 
 void cuda_stwo_ntt_evaluate(uint32_t* d_data, const uint32_t* d_twiddles, uint32_t n) {
@@ -344,26 +332,25 @@ vx_wide* vx_wide_create(uint32_t n_cols, const uint32_t* log_sizes, uint32_t log
     const uint64_t half = 1ull << (S - 1);
     ok = ok && w->alloc((void**)&w->tw_fwd, 4 * half) && w->alloc((void**)&w->tw_inv, 4 * half) &&
          w->alloc((void**)&w->tw_circle, 4 * half);
-    uint32_t* tw_scratch = nullptr;
-    ok = ok && w->alloc((void**)&tw_scratch, 4 * half);
     if (ok) {
         build_stwo_twiddles(S, w->tw_fwd, w->tw_inv, s);
-        // circle fold on the canonic domain: 1 / y(half_odds(S-1).at(bitrev_{S-1}(i)))
-        HostPt hi, hs;
-        host_coset(2, S - 1, hi, hs);
-        brt_coord_kernel<<<ceil_div(half, 256), 256, 0, s>>>(cpt(hi), cpt(hs), tw_scratch, half, S - 1, 1);
-        check_launch("brt_coord_kernel");
-        batch_inverse(tw_scratch, w->tw_circle, half, s);
+        // circle fold on the canonic domain: 1 / y(half_odds(S-1).at(bitrev_{S-1}(i)));
         // line fold j reads layer j-1 on half_odds(S - j) (fri.rs:143-160)
         w->tw_line.assign(w->J, nullptr);
+        std::vector<FoldDomain> fd(std::max(w->J, 1u));
+        host_coset(2, S - 1, fd[0].initial, fd[0].step);
+        fd[0].log_len = S - 1;
+        fd[0].use_y = true;
+        fd[0].out = w->tw_circle;
         for (uint32_t j = 1; ok && j < w->J; j++) {
             const uint32_t k = S - j;
             ok = w->alloc((void**)&w->tw_line[j], 4 * ((1ull << k) / 2));
-            if (!ok) break;
-            HostPt di, ds;
-            host_coset(2, k, di, ds);
-            build_fold_twiddles(cpt(di), cpt(ds), k, false, w->tw_line[j], tw_scratch, s);
+            host_coset(2, k, fd[j].initial, fd[j].step);
+            fd[j].log_len = k - 1;
+            fd[j].use_y = false;
+            fd[j].out = w->tw_line[j];
         }
+        if (ok) build_fold_twiddles(fd.data(), (uint32_t)fd.size(), s);
     }
     // LDE columns, contiguous, each 2^(log + blowup) words
     uint64_t total = 0;
