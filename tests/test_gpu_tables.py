@@ -1,5 +1,5 @@
 """Tile roots on both sides of the two switches of the work per tile, fold-twiddle
-sources at run and block edges, batch inverses of every words-per-thread count:
+sources and traces at run and block edges, batch inverses of every words-per-thread count:
 against the oracle. Runs on the MI355X."""
 
 import ctypes as C
@@ -88,4 +88,17 @@ def test_batch_inverse(vx, n):
     live = np.repeat(v[::64] != 0, 64)[:n] & (v != 0)
     assert (got[~live] == 0).all()
     assert (got[live] * v[live] % P == 1).all() and (got < P).all()
+    vx.check()
+
+
+@pytest.mark.parametrize("log_n", [1, 2, 3, 4, 5, 11, 12, 13, 20])
+@pytest.mark.parametrize("a,b", [(1, 1), (0, P - 1), (P - 1, 12345)])
+def test_fibonacci_trace(vx, log_n, a, b):
+    n = 1 << log_n
+    out = vx.DeviceBuffer.from_host(np.full(n + 2, 7, np.uint32))
+    vx.lib.vx_fibonacci_trace(a, b, log_n, C.c_void_p(out.addr + 4), None)
+    vx.synchronize()
+    got = out.to_host()
+    assert got[0] == 7 and got[n + 1] == 7
+    assert np.array_equal(got[1: n + 1], O.fibonacci_trace(a, b, log_n))
     vx.check()

@@ -194,4 +194,21 @@ __device__ __forceinline__ uint32_t brev_bits(uint32_t x, uint32_t bits) {
     return bits == 0 ? 0u : (__builtin_bitreverse32(x) >> (32 - bits));
 }
 
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(4)));  // any word address
+// words i .. i + RUN - 1 of an array of len words
+template <uint32_t RUN>
+__device__ __forceinline__ void store_run(uint32_t* out, uint64_t i, uint64_t len, const uint32_t (&w)[RUN]) {
+    if (i + RUN <= len) {
+#pragma unroll
+        for (uint32_t r = 0; r < RUN; r += 4) {
+            const u32x4_any v = {w[r], w[r + 1], w[r + 2], w[r + 3]};
+            *(__attribute__((address_space(1))) u32x4_any*)(out + i + r) = v;
+        }
+    } else {
+#pragma unroll
+        for (uint32_t r = 0; r < RUN; r++)
+            if (i + r < len) out[i + r] = w[r];
+    }
+}
+
 }  // namespace vx

@@ -887,7 +887,6 @@ __global__ void coset_points_kernel(CPt initial, CPt step, uint32_t* ox, uint32_
 constexpr uint32_t TABLE_THREADS = 256;
 constexpr uint32_t TABLE_RUN_LOG = 4;   // with inverses, and in the NTT tables
 constexpr uint32_t SOURCE_RUN_LOG = 2;  // sources alone: a shorter chain
-typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(4)));  // any word address
 
 // w[r] -> 1 / w[r]; a zero stays zero
 template <uint32_t RUN>
@@ -904,21 +903,6 @@ __device__ __forceinline__ void invert_run(uint32_t (&w)[RUN]) {
         const uint32_t v = w[r];
         w[r] = v ? mmul(iv, pre[r]) : 0u;
         iv = mmul(iv, v ? v : 1u);
-    }
-}
-// words i .. i + RUN - 1 of an array of len words
-template <uint32_t RUN>
-__device__ __forceinline__ void store_run(uint32_t* out, uint64_t i, uint64_t len, const uint32_t (&w)[RUN]) {
-    if (i + RUN <= len) {
-#pragma unroll
-        for (uint32_t r = 0; r < RUN; r += 4) {
-            const u32x4_any v = {w[r], w[r + 1], w[r + 2], w[r + 3]};
-            *(__attribute__((address_space(1))) u32x4_any*)(out + i + r) = v;
-        }
-    } else {
-#pragma unroll
-        for (uint32_t r = 0; r < RUN; r++)
-            if (i + r < len) out[i + r] = w[r];
     }
 }
 // start * the points of the set bits of run number blk * TABLE_THREADS + tid,

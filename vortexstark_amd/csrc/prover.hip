@@ -30,43 +30,63 @@
 namespace vx {
 
 // ---------------------------------------------------------------- trace generation
-// air.rs:85-131: (F(k), F(k+1)) from (a, b) by powers of [[1,1],[1,0]].
-__device__ void fib_at(uint32_t a, uint32_t b, uint64_t k, uint32_t& fk, uint32_t& fk1) {
-    uint32_t m00 = 1, m01 = 0, m10 = 0, m11 = 1;
-    uint32_t b00 = 1, b01 = 1, b10 = 1, b11 = 0;
-    while (k) {
-        if (k & 1) {
-            uint32_t t00 = madd(mmul(m00, b00), mmul(m01, b10)), t01 = madd(mmul(m00, b01), mmul(m01, b11));
-            uint32_t t10 = madd(mmul(m10, b00), mmul(m11, b10)), t11 = madd(mmul(m10, b01), mmul(m11, b11));
-            m00 = t00;
-            m01 = t01;
-            m10 = t10;
-            m11 = t11;
+// The trace f(0) = a, f(1) = b, f(i+2) = f(i) + f(i+1) (air.rs:85-131), one per
+// blockIdx.y: the pair (f(i), f(i+1)) moves k words on by
+// f(i+k) = F(k-1) f(i) + F(k) f(i+1), F the Fibonacci numbers, so a thread
+// reaches its run of FIB_RUN words by one such step for each set bit of the run's
+// number (a block's bits scalar) and then only adds. Latency-bound to 2^18 words:
+// 3-4 us, where a matrix power and 256 words a thread took 14 us at 2^10 and 38 at
+// 2^16; 2^24 words are bound by the stores.
+constexpr uint32_t FIB_RUN_LOG = 4, FIB_THREADS_LOG = 8;
+struct FibSteps {
+    uint32_t f[32][2] = {};  // (F(2^b - 1), F(2^b)) mod p
+    constexpr FibSteps() {
+        uint64_t x = 0, y = 1;
+        for (int b = 0; b < 32; b++) {
+            f[b][0] = (uint32_t)x;
+            f[b][1] = (uint32_t)y;
+            const uint64_t x2 = (x * x % P + y * y % P) % P, y2 = y * ((2 * x + y) % P) % P;
+            x = x2;
+            y = y2;
         }
-        uint32_t t00 = madd(mmul(b00, b00), mmul(b01, b10)), t01 = madd(mmul(b00, b01), mmul(b01, b11));
-        uint32_t t10 = madd(mmul(b10, b00), mmul(b11, b10)), t11 = madd(mmul(b10, b01), mmul(b11, b11));
-        b00 = t00;
-        b01 = t01;
-        b10 = t10;
-        b11 = t11;
-        k >>= 1;
     }
-    fk = madd(mmul(m10, b), mmul(m11, a));
-    fk1 = madd(mmul(m00, b), mmul(m01, a));
+};
+__device__ __forceinline__ void fib_step(uint32_t& f0, uint32_t& f1, uint32_t x, uint32_t y) {
+    const uint32_t z = madd(x, y);
+    const uint32_t g0 = reduce64((uint64_t)x * f0 + (uint64_t)y * f1);
+    f1 = reduce64((uint64_t)y * f0 + (uint64_t)z * f1);
+    f0 = g0;
 }
-__global__ void fib_trace_kernel(uint32_t a, uint32_t b, uint64_t n, uint32_t chunk, uint32_t* out) {
-    uint64_t start = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) * chunk;
-    if (start >= n) return;
-    uint32_t f0, f1;
-    fib_at(a, b, start, f0, f1);
-    uint64_t end = start + chunk < n ? start + chunk : n;
-    for (uint64_t i = start; i < end; i++) {
-        out[i] = f0;
-        uint32_t f2 = madd(f0, f1);
+__global__ __launch_bounds__(1 << FIB_THREADS_LOG) void fib_trace_kernel(const uint32_t* ab, uint32_t a, uint32_t b,
+                                                                        uint64_t n, uint32_t* out, uint64_t bs) {
+    static constexpr FibSteps steps;
+    constexpr uint32_t RUN = 1u << FIB_RUN_LOG;
+    const uint64_t i = (((uint64_t)blockIdx.x << FIB_THREADS_LOG) + threadIdx.x) << FIB_RUN_LOG;
+    if (i >= n) return;
+    if (ab) {
+        a = ab[2 * blockIdx.y];
+        b = ab[2 * blockIdx.y + 1];
+    }
+    uint32_t f0 = reduce64(a), f1 = reduce64(b);
+    uint32_t blk = blockIdx.x;
+    for (uint32_t k = FIB_RUN_LOG + FIB_THREADS_LOG; blk; k++, blk >>= 1)
+        if (blk & 1) fib_step(f0, f1, steps.f[k][0], steps.f[k][1]);
+#pragma unroll
+    for (uint32_t k = 0; k < FIB_THREADS_LOG; k++) {
+        const bool on = (threadIdx.x >> k) & 1;
+        fib_step(f0, f1, on ? steps.f[FIB_RUN_LOG + k][0] : 1u, on ? steps.f[FIB_RUN_LOG + k][1] : 0u);
+    }
+    uint32_t w[RUN];
+#pragma unroll
+    for (uint32_t r = 0; r < RUN; r++) {
+        w[r] = f0;
+        const uint32_t f2 = madd(f0, f1);
         f0 = f1;
         f1 = f2;
     }
+    store_run(out + blockIdx.y * bs, i, n, w);
 }
+inline uint32_t fib_blocks(uint64_t n) { return (uint32_t)ceil_div(((n - 1) >> FIB_RUN_LOG) + 1, 1u << FIB_THREADS_LOG); }
 
 // ---------------------------------------------------------------- queries
 // Last layer into the proof, mix_felts(last layer), then n_q draw_number(E)
@@ -293,21 +313,6 @@ __global__ __launch_bounds__(DECOMMIT_THREADS) void decommit_kernel(const TreeDe
 
 // Fibonacci traces of a batch: proof blockIdx.y gets (a, b) = ab[2y], ab[2y+1]
 // and writes its trace bs words past proof 0's.
-__global__ void fib_trace_batch_kernel(const uint32_t* ab, uint64_t n, uint32_t chunk, uint32_t* out0, uint64_t bs) {
-    const uint32_t y = blockIdx.y;
-    uint64_t start = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) * chunk;
-    if (start >= n) return;
-    uint32_t* out = out0 + (uint64_t)y * bs;
-    uint32_t f0, f1;
-    fib_at(ab[2 * y], ab[2 * y + 1], start, f0, f1);
-    uint64_t end = start + chunk < n ? start + chunk : n;
-    for (uint64_t i = start; i < end; i++) {
-        out[i] = f0;
-        uint32_t f2 = madd(f0, f1);
-        f0 = f1;
-        f1 = f2;
-    }
-}
 
 // Copies words of src to count - 1 places stride words apart (dst0 = src + stride).
 __global__ void replicate_kernel(const uint32_t* src, uint64_t words, uint64_t stride) {
@@ -1010,11 +1015,9 @@ int32_t vx_prove_fibonacci_batch(vx_prover* p, const uint32_t* h_ab, uint32_t co
     std::vector<const uint32_t*> slots(count);
     for (uint32_t i = 0; i < count; i++) slots[i] = p->arena + (uint64_t)i * p->R + p->o_trace;
     if (!upload_call(p, slots.data(), h_ab, count)) return -1;
-    const uint32_t chunk = 256;
-    const uint64_t threads = (p->N + chunk - 1) / chunk;
-    fib_trace_batch_kernel<<<dim3(ceil_div(threads, 256), count), 256, 0, p->stream>>>(
-        p->ab_dev(), p->N, chunk, p->arena + p->o_trace, p->R);
-    if (!check_launch("fib_trace_batch_kernel")) return -1;
+    fib_trace_kernel<<<dim3(fib_blocks(p->N), count), 1 << FIB_THREADS_LOG, 0, p->stream>>>(
+        p->ab_dev(), 0, 0, p->N, p->arena + p->o_trace, p->R);
+    if (!check_launch("fib_trace_kernel")) return -1;
     return run_batch(p, count);
 }
 
@@ -1166,9 +1169,7 @@ float vx_prover_timeline_ms(vx_prover* p, uint32_t i) { return p ? p->tl.ms(i) :
 
 int32_t vx_fibonacci_trace(uint32_t a, uint32_t b, uint32_t log_n, uint32_t* d_out, void* stream) {
     uint64_t n = 1ull << log_n;
-    const uint32_t chunk = 256;
-    uint64_t threads = (n + chunk - 1) / chunk;
-    fib_trace_kernel<<<ceil_div(threads, 256), 256, 0, (hipStream_t)stream>>>(a, b, n, chunk, d_out);
+    fib_trace_kernel<<<fib_blocks(n), 1 << FIB_THREADS_LOG, 0, (hipStream_t)stream>>>(nullptr, a, b, n, d_out, 0);
     return check_launch("vx_fibonacci_trace") ? 0 : -1;
 }
 
