@@ -78,4 +78,21 @@ void build_fold_twiddles(const FoldDomain* d, uint32_t n, hipStream_t s);
 void build_fold_twiddles_chunked(const FoldDomain& d, uint32_t* scratch, hipStream_t s);
 void batch_inverse(const uint32_t* in, uint32_t* out, uint64_t n, hipStream_t s);
 
+// Several device arrays packed one after another into pinned host memory by one
+// launch on s: results reach the host behind the last kernel without a hand-off
+// to the copy engines for each array, and one synchronisation then covers them.
+struct Fetch {
+    const uint32_t* src[5];
+    uint64_t words[5];
+    uint32_t n = 0;
+    uint64_t total = 0;
+    // index of the array's first word in the packed result
+    uint64_t add(const void* p, uint64_t n_words) {
+        src[n] = (const uint32_t*)p;
+        words[n++] = n_words;
+        return (total += n_words) - n_words;
+    }
+};
+bool fetch_to_host(const Fetch& f, uint32_t* pinned, hipStream_t s);
+
 }  // namespace vx

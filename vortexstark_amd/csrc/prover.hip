@@ -18,6 +18,7 @@
 #include <algorithm>
 #include <cstddef>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -342,6 +343,22 @@ __global__ void proofs_to_host_kernel(const uint32_t* src, uint64_t R, uint64_t 
     __threadfence_system();
 }
 
+// Bound by the link (a 100 KB proof: about 5 us) and its own launch, where a copy
+// into pageable memory took 40 us an array.
+__global__ void fetch_kernel(Fetch f, uint32_t* dst) {
+    const uint64_t nth = (uint64_t)gridDim.x * blockDim.x, tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (uint32_t k = 0; k < f.n; k++) {
+        for (uint64_t i = tid; i < f.words[k]; i += nth) dst[i] = f.src[k][i];
+        dst += f.words[k];
+    }
+    __threadfence_system();
+}
+bool fetch_to_host(const Fetch& f, uint32_t* pinned, hipStream_t s) {
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>(P2H_BLOCKS, f.total / 1024 + 1);
+    fetch_kernel<<<blocks, 256, 0, s>>>(f, pinned);
+    return check_launch("fetch_kernel");
+}
+
 __global__ void raise_flag_kernel(uint32_t* flag) { *flag = 1; }
 
 }  // namespace vx
@@ -376,7 +393,8 @@ struct vx_prover {
     // call parameters: trace pointers (capacity) then (a, b) per proof
     uint64_t* d_call = nullptr;
     uint64_t* h_call = nullptr;  // pinned staging
-    uint8_t* h_setup = nullptr;  // pinned staging of the set-up copies (kept until destroy)
+    uint8_t* h_setup = nullptr;  // pinned staging of the set-up copies, then of the proofs copied out
+    std::mutex fetch_mu;         // held while a proof passes through it
     hipEvent_t call_copied = nullptr;  // recorded after the last copy out of h_call
     std::vector<uint64_t> last_call;
     bool traces_aligned = false;  // every trace pointer of the current call is 16-byte aligned
@@ -1028,12 +1046,17 @@ uint64_t vx_prover_proof_copy_at(vx_prover* p, uint32_t index, void* host_out, u
         set_error(-2, "vx_prover_proof_copy: buffer too small");
         return 0;
     }
-    DevChannel ch;
     const DevChannel* dch = (const DevChannel*)((const uint32_t*)p->ch() + (uint64_t)index * p->R);
-    if (!check(hipMemcpyAsync(host_out, p->proof(index), bytes, hipMemcpyDeviceToHost, p->stream), "D2H")) return 0;
-    if (!check(hipMemcpyAsync(&ch, dch, sizeof(ch), hipMemcpyDeviceToHost, p->stream), "D2H")) return 0;
-    if (!check(hipStreamSynchronize(p->stream), "vx_prover_proof_copy")) return 0;
-    if (ch.failed) {
+    Fetch f;
+    f.add(p->proof(index), p->proof_words);
+    const uint64_t failed = f.add(&dch->failed, 1);
+    // the set-up copies out of the staging precede this on the stream
+    std::lock_guard<std::mutex> g(p->fetch_mu);
+    uint32_t* pinned = (uint32_t*)p->h_setup;
+    if (!fetch_to_host(f, pinned, p->stream) || !check(hipStreamSynchronize(p->stream), "vx_prover_proof_copy"))
+        return 0;
+    std::memcpy(host_out, pinned, bytes);
+    if (pinned[failed]) {
         set_error(-3, "transcript: draw_felt exhausted its retry budget");
         return 0;
     }

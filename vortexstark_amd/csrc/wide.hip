@@ -20,6 +20,7 @@
 // single stream of launches with no host round trip.
 #include <algorithm>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -198,6 +199,8 @@ struct vx_wide {
     uint32_t* chal = nullptr;       // [beta, alpha_0, alpha_1, ...], 4 words each
     uint32_t* beta_pows = nullptr;  // 4 words per column
     uint32_t* roots = nullptr;      // lifted root, then J FRI roots
+    uint32_t* h_results = nullptr;  // pinned: the results on their way to the caller
+    std::mutex fetch_mu;            // held while they pass through it
     Timeline tl;
     void mark(const std::string& l) { tl.mark(l, stream); }
 
@@ -216,6 +219,7 @@ struct vx_wide {
         if (fork) (void)hipEventDestroy(fork);
         for (void* p : allocs) (void)hipFree(p);
         if (h_src_ptrs) (void)hipHostFree((void*)h_src_ptrs);
+        if (h_results) (void)hipHostFree(h_results);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
@@ -360,7 +364,9 @@ vx_wide* vx_wide_create(uint32_t n_cols, const uint32_t* log_sizes, uint32_t log
     }
     ok = ok && w->alloc((void**)&w->lde, 4 * total) && w->alloc((void**)&w->d_lde_ptrs, 8ull * n_cols) &&
          w->alloc((void**)&w->d_src_ptrs, 8ull * n_cols) && w->alloc((void**)&w->d_lift, sizeof(LiftCol) * n_cols);
-    ok = ok && check(hipHostMalloc((void**)&w->h_src_ptrs, 8ull * n_cols), "hipHostMalloc");
+    ok = ok && check(hipHostMalloc((void**)&w->h_src_ptrs, 8ull * n_cols), "hipHostMalloc") &&
+         check(hipHostMalloc((void**)&w->h_results, 4 * (8 + 8ull * w->J + 4 + 4 * w->layer_size(w->J - 1) + 1)),
+               "hipHostMalloc");
     w->layer.assign(w->J, nullptr);
     for (uint32_t j = 0; ok && j < w->J; j++) ok = w->alloc((void**)&w->layer[j], 16 * w->layer_size(j));
     ok = ok && w->alloc((void**)&w->scratch.a, 32 * scratch_nodes_a(1ull << S)) &&
@@ -495,25 +501,21 @@ int32_t vx_wide_commit_device(vx_wide* w, const uint32_t* const* h_cols) {
 
 int32_t vx_wide_results(vx_wide* w, uint32_t* root8, uint32_t* fri_roots, uint32_t* last, uint32_t* beta4) {
     if (!w) return -1;
-    hipStream_t s = w->stream;
-    bool ok = true;
-    if (root8) ok = ok && check(hipMemcpyAsync(root8, w->roots, 32, hipMemcpyDeviceToHost, s), "D2H");
-    if (fri_roots) ok = ok && check(hipMemcpyAsync(fri_roots, w->roots + 8, 32ull * w->J, hipMemcpyDeviceToHost, s), "D2H");
-    if (beta4) ok = ok && check(hipMemcpyAsync(beta4, w->chal, 16, hipMemcpyDeviceToHost, s), "D2H");
-    std::vector<uint32_t> soa;
     const uint64_t nl = w->layer_size(w->J - 1);
-    if (last) {
-        soa.resize(4 * nl);
-        ok = ok && check(hipMemcpyAsync(soa.data(), w->layer[w->J - 1], 16 * nl, hipMemcpyDeviceToHost, s), "D2H");
-    }
-    DevChannel ch;
-    ok = ok && check(hipMemcpyAsync(&ch, w->ch, sizeof(ch), hipMemcpyDeviceToHost, s), "D2H");
-    ok = ok && check(hipStreamSynchronize(s), "vx_wide_results");
-    if (!ok) return -1;
+    Fetch f;
+    const uint64_t roots = f.add(w->roots, 8 + 8ull * w->J), beta = f.add(w->chal, 4);
+    const uint64_t lw = last ? f.add(w->layer[w->J - 1], 4 * nl) : 0, failed = f.add(&w->ch->failed, 1);
+    std::lock_guard<std::mutex> g(w->fetch_mu);
+    const uint32_t* h = w->h_results;
+    if (!fetch_to_host(f, w->h_results, w->stream) || !check(hipStreamSynchronize(w->stream), "vx_wide_results"))
+        return -1;
+    if (root8) std::memcpy(root8, h + roots, 32);
+    if (fri_roots) std::memcpy(fri_roots, h + roots + 8, 32ull * w->J);
+    if (beta4) std::memcpy(beta4, h + beta, 16);
     if (last)
         for (uint64_t i = 0; i < nl; i++)
-            for (int c = 0; c < 4; c++) last[4 * i + c] = soa[c * nl + i];
-    if (ch.failed) {
+            for (int c = 0; c < 4; c++) last[4 * i + c] = h[lw + c * nl + i];
+    if (h[failed]) {
         set_error(-3, "transcript: draw_felt exhausted its retry budget");
         return -1;
     }
