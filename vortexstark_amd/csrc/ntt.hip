@@ -99,13 +99,15 @@ __device__ __forceinline__ uint2 ldw2(const uint32_t* T, uint32_t h) {
     return *(const uint2*)((const char*)T + (h << 3));
 }
 
-// Threads of a pass over 2^M x 2^C tiles: two radix-8 groups a thread (16 words)
-// from 2^12 words on, so that every tile size keeps eight waves a SIMD within
-// the CU's LDS (8 workgroups of 2^12 words, 2 of 2^14).
+// Threads of a pass over 2^M x 2^C tiles: a radix-8 group each (8 words; two at
+// 2^14 words, the most threads a workgroup has). A small transform is a few tiles
+// and its time the chain of one thread: 32 tiles of 2^12 words take 5.7 us so, 7.7
+// with two groups a thread, 5.7 with 1024 threads of half a group; large ones,
+// with eight waves a SIMD either way, gain 1-3 %.
 template <int M, int C>
 constexpr uint32_t ntt_threads() {
     constexpr uint32_t words = 1u << (M + C);
-    return words >= (1u << 14) ? 1024 : words >= (1u << 13) ? 512 : words >= (1u << 11) ? 256 : words >= (1u << 9) ? words >> 3 : 64;
+    return words >= (1u << 13) ? 1024 : words >= (1u << 9) ? words >> 3 : 64;
 }
 
 // Twiddle h of a layer whose table is T; circle0: the layer is stride bit 0.
