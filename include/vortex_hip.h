@@ -270,9 +270,9 @@ void* vx_get_stream(void);
  * the provers) have a table of their own, tuned by the same call on such
  * inputs: its plans may end in a replicating top pass (r[i] = 1), whose two
  * top layers only copy the quarter into all four, so the pass holds 2^(m-2)
- * rows in LDS and transforms them once per quarter; lde_plan_set with
- * n_passes = 0 falls back to the general table, plan_reset clears both. No
- * reference counterpart (tuning of this library's pass structure). */
+ * rows in LDS and transforms them once per quarter. A size with no plan of
+ * either table takes a default of this form; lde_plan_set with n_passes = 0
+ * asks for the general table, plan_reset clears both. No reference counterpart (tuning of this library's pass structure). */
 int32_t vx_ntt_autotune(uint32_t log_min, uint32_t log_max, float* best_ms);
 /* Measured int32 VALU issue rate of the current device in T lane-ops/s (a
  * grid of v_add3 / v_xor / v_alignbit chains, the instructions of Blake2s). */

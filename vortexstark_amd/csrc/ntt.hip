@@ -611,7 +611,8 @@ __global__ __launch_bounds__((ntt_threads<M, C>())) void ntt_lde_bridge_kernel(N
 namespace {
 std::mutex g_plan_mu;
 std::vector<Pass> g_plan[32];      // tuned or set plans; empty: default split
-std::vector<Pass> g_lde_plan[32];  // the same for blowup-4 evaluations; empty: g_plan's
+std::vector<Pass> g_lde_plan[32];  // the same for blowup-4 evaluations; empty: g_plan's if set or asked for
+bool g_lde_general[32];            // the general table was asked for
 }  // namespace
 
 static std::vector<Pass> plan_passes(uint32_t k) {
@@ -625,6 +626,7 @@ static std::vector<Pass> lde_plan_passes(uint32_t k) {
     {
         std::lock_guard<std::mutex> g(g_plan_mu);
         if (k < 32 && !g_lde_plan[k].empty()) return g_lde_plan[k];
+        if (k < 32 && !g_lde_general[k] && g_plan[k].empty()) return default_lde_plan(k);
     }
     return plan_passes(k);
 }
@@ -1276,6 +1278,7 @@ void vx_ntt_plan_reset(void) {
     std::lock_guard<std::mutex> g(g_plan_mu);
     for (auto& p : g_plan) p.clear();
     for (auto& p : g_lde_plan) p.clear();
+    for (bool& g : g_lde_general) g = false;
 }
 
 void vx_ntt_set_lde_bridge(int32_t enable) {
@@ -1300,7 +1303,8 @@ int32_t vx_ntt_lde_plan_set(uint32_t log_n, uint32_t n_passes, const uint32_t* m
         return -1;
     }
     std::lock_guard<std::mutex> g(g_plan_mu);
-    g_lde_plan[log_n] = ps;  // empty: the general plan of the size
+    g_lde_plan[log_n] = ps;
+    g_lde_general[log_n] = ps.empty();  // the general plan of the size
     return 0;
 }
 

@@ -51,6 +51,22 @@ inline std::vector<Pass> default_plan(uint32_t k) {
     return ps;
 }
 
+// The default split of a blowup-4 evaluation of 2^k points: one pass while a tile
+// holds it; then, and to 2^24 points, two, the upper one replicating (and so the
+// bridge from the interpolation), which beats every three-pass split: the whole
+// LDE takes as many passes as the evaluation. 2^13 rows 21.1 -> 18.7 us, 2^18 30.7
+// -> 27.0, 2^20 48.0 -> 41.0, 2^22 124.7 -> 114.0. Its 2^c-word segments are 256
+// bytes to 2^17 points, where the launch has few tiles anyway, and 64 bytes above,
+// which keeps a tile of up to 2^10 rows in 2^14 words. Larger ones take a third
+// pass of half the rest (2^24 rows: 436 -> 405 us).
+inline std::vector<Pass> default_lde_plan(uint32_t k) {
+    if (k <= NTT_LOW) return default_plan(k);
+    const uint32_t m0 = std::min(NTT_LOW, k - 3), R = k - m0;
+    if (R - 2 <= NTT_HIGH_MAX4) return {{0, m0, 0}, {m0, R, k < 18 ? 6u : 4u, 1}};
+    const uint32_t a = (R - 1) / 2;
+    return {{0, m0, 0}, {m0, a, NTT_COLS}, {m0 + a, R - a, NTT_COLS, 1}};
+}
+
 // A plan is valid when its passes cover layers 0 .. k-1 in order, the first is
 // contiguous, every strided pass starts at a stride of at least its segment
 // and every shape has a compiled kernel. Replicating top passes are valid only
