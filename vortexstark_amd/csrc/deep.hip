@@ -7,17 +7,20 @@
 //  quotients_combine       out[row] = sum_j (numer_j[lift_j(row)] - a_j * y) / den_j(row)
 //  accumulate_lift         col[i] += curr[lift(i)]   (QM31, 4 words per element)
 //
-// accumulate_numerators is bound by HBM (4 bytes of column a term): each thread
-// takes eight rows (two uint4 loads a column, a wave reading 2 KiB of it), the sum of products c_i * f is kept
-// in 64 bits (one v_mad_u64_u32 per coordinate and column, a partial reduction
-// every three columns, the full one at the end), and sum_i b_i is formed once
-// per thread. quotients_combine is bound by the VALU: den_j(row) is the CM31
+// accumulate_numerators is bound by HBM (4 bytes of column a term) once its rows
+// fill the chip, below by a thread's chain of loads: each thread takes eight
+// consecutive-by-four rows of a large batch (two uint4 loads a column, a wave
+// reading 2 KiB of it), four of a small one. The sum of products c_i * f is kept in
+// 64 bits: one v_mad_u64_u32 per coordinate and column and, every four columns,
+// one more that folds it below 2^34 (fold64). quotients_combine is bound by the
+// VALU: den_j(row) is the CM31
 //   (Re(px) - x) * Im(py) - (Re(py) - y) * Im(px)
 //     = (Re(px) Im(py) - Re(py) Im(px)) - x Im(py) + y Im(px),
 // linear in the domain point, so its constant part is formed once per thread;
-// each thread takes COMBINE_ROWS rows (wave-strided, so every load stays
-// coalesced) and inverts their norms |den|^2 with one M31 inversion per
-// accumulation (Montgomery's trick) instead of one per row.
+// each thread takes several rows (wave-strided, so every load stays coalesced)
+// and inverts their norms |den|^2 with one M31 inversion per accumulation
+// (Montgomery's trick) instead of one per row; the quotients stay 64-bit sums of
+// products until all accumulations are in.
 #include <algorithm>
 #include <cstring>
 #include <mutex>
@@ -31,31 +34,41 @@ namespace vx {
 namespace {
 
 constexpr uint32_t DEEP_THREADS = 256;
-constexpr uint32_t COMBINE_ROWS = 8;  // rows per thread of quotients_combine
+// Rows from which a thread takes more of them, having enough threads either way
+// (us below and above the line; the first two with their launch of about 17 and 5):
+// - fused, two points: 2^17 rows 20.8 at one row a thread, 24.2 at four; 2^18 25.9
+//   and 24.3; 2^22 168 and 121
+// - combine, four accumulations: 2^17 rows 8.9 at two, 11.9 at four, 18.5 at eight;
+//   2^19 22.0, 19.7 and 20.6; 2^22 137, 115 and 110
+// - numerators: 2^16 rows of 12 columns 5.5 at four, 6.7 at eight; 2^18 of 64 columns
+//   30.6 and 34.9, 2^20 56.4 and 55.1, 2^22 252 and 243
+constexpr uint32_t FUSED_WIDE_MIN = 1u << 18;
+constexpr uint32_t COMBINE_MID_MIN = 1u << 18, COMBINE_WIDE_MIN = 1u << 20;
+constexpr uint32_t NUMER_WIDE_MIN = 1u << 20;
 
-// ROWS rows per thread (row_of): 8 (uint4 loads and stores; n_rows % 512 == 0
-// and 16-byte aligned outputs, checked on the host; a column whose pointer is
-// not 16-byte aligned is read word by word, a wave-uniform branch) or 1.
-// Rows of a thread: ROWS = 1: row0; ROWS = 8: row0 .. row0 + 3 and row0 + 256 ..
-// row0 + 259, so that a wave reads 2 KiB of a column contiguously (lane l at
-// row0 = 512 * wave + 4 * l). Wider contiguous reads per wave and column stream
-// faster from HBM when a thread reads many columns.
+// Rows of a thread: ROWS = 1: row0; ROWS = 4 or 8: row0 .. row0 + 3 and row0 + 256
+// .. row0 + 259, so that a wave reads 1 or 2 KiB of a column contiguously (lane l
+// at row0 = 64 * ROWS * wave + 4 * l). Wider contiguous reads per wave and column
+// stream faster from HBM when a thread reads many columns. The wide forms need
+// n_rows % (64 * ROWS) == 0 and 16-byte aligned outputs, checked on the host; a
+// column whose pointer is not 16-byte aligned is read word by word, a
+// wave-uniform branch.
 template <uint32_t ROWS>
 __device__ __forceinline__ uint64_t row_of(uint64_t row0, uint32_t r) {
     return ROWS == 1 ? row0 : row0 + (r & 3) + 256 * (r >> 2);
 }
 template <uint32_t ROWS>
-__device__ __forceinline__ void load_rows(const uint32_t* col, uint64_t row0, uint32_t f[ROWS]) {
-    if (ROWS == 8 && ((uintptr_t)col & 15) == 0) {
-        const uint4 v = *(const uint4*)(col + row0), w = *(const uint4*)(col + row0 + 256);
-        f[0] = v.x;
-        f[1] = v.y;
-        f[2] = v.z;
-        f[3] = v.w;
-        f[4] = w.x;
-        f[5] = w.y;
-        f[6] = w.z;
-        f[7] = w.w;
+__device__ __forceinline__ void load_rows(const uint32_t* column, uint64_t row0, uint32_t f[ROWS]) {
+    const gu32* col = as_global(column);
+    if (ROWS >= 4 && ((uintptr_t)column & 15) == 0) {
+#pragma unroll
+        for (uint32_t r = 0; r < ROWS; r += 4) {
+            const u32x4 v = *(const gu32x4*)(col + row_of<ROWS>(row0, r));
+            f[r] = v.x;
+            f[r + 1] = v.y;
+            f[r + 2] = v.z;
+            f[r + 3] = v.w;
+        }
     } else {
 #pragma unroll
         for (uint32_t r = 0; r < ROWS; r++) f[r] = col[row_of<ROWS>(row0, r)];
@@ -77,26 +90,22 @@ __global__ __launch_bounds__(DEEP_THREADS) void accumulate_numerators_kernel(
     for (uint32_t i = 0; i < n_batch; i++)
 #pragma unroll
         for (int k = 0; k < 4; k++) bs[k] = madd(bs[k], b_coeffs[4 * i + k]);
-    // The accumulators stay below 2^62 + 4 between groups: a group adds three
-    // products of at most (p - 1)^2 < 2^62 - 2^32 (three v_mad_u64_u32, the 64-bit
-    // addend chained), which stays below 2^64, and then folds bits 62..63 back
-    // onto bit 0 (2^62 = 1 mod p): a partial reduction of a few 32-bit ops.
-    constexpr uint64_t M62 = (1ull << 62) - 1;
+    // The accumulators stay below 2^34 between groups: a group adds four products of
+    // at most (p - 1)^2 < 2^62 - 2^32, which stays below 2^64, and folds.
     uint64_t acc[ROWS][4] = {};
     uint32_t i = 0;
-    for (; i + 3 <= n_batch; i += 3) {
-        uint32_t f[3][ROWS];
+    for (; i + 4 <= n_batch; i += 4) {
+        uint32_t f[4][ROWS];
 #pragma unroll
-        for (int g = 0; g < 3; g++) load_rows<ROWS>(col_ptrs[col_indices[i + g]], row0, f[g]);
+        for (int g = 0; g < 4; g++) load_rows<ROWS>(col_ptrs[col_indices[i + g]], row0, f[g]);
 #pragma unroll
         for (uint32_t r = 0; r < ROWS; r++)
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 uint64_t a = acc[r][k];
-                a = (uint64_t)c_coeffs[4 * i + k] * f[0][r] + a;
-                a = (uint64_t)c_coeffs[4 * (i + 1) + k] * f[1][r] + a;
-                a = (uint64_t)c_coeffs[4 * (i + 2) + k] * f[2][r] + a;
-                acc[r][k] = (a & M62) + (a >> 62);
+#pragma unroll
+                for (int g = 0; g < 4; g++) a = (uint64_t)c_coeffs[4 * (i + g) + k] * f[g][r] + a;
+                acc[r][k] = fold64(a);
             }
     }
     for (; i < n_batch; i++) {
@@ -105,10 +114,7 @@ __global__ __launch_bounds__(DEEP_THREADS) void accumulate_numerators_kernel(
 #pragma unroll
         for (uint32_t r = 0; r < ROWS; r++)
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const uint64_t a = (uint64_t)c_coeffs[4 * i + k] * f[r] + acc[r][k];
-                acc[r][k] = (a & M62) + (a >> 62);
-            }
+            for (int k = 0; k < 4; k++) acc[r][k] = fold64((uint64_t)c_coeffs[4 * i + k] * f[r] + acc[r][k]);
     }
     uint32_t o[4][ROWS];
 #pragma unroll
@@ -118,12 +124,56 @@ __global__ __launch_bounds__(DEEP_THREADS) void accumulate_numerators_kernel(
     uint32_t* outs[4] = {out0, out1, out2, out3};
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        if (ROWS == 8) {
-            *(uint4*)(outs[k] + row0) = make_uint4(o[k][0], o[k][1], o[k][2], o[k][3]);
-            *(uint4*)(outs[k] + row0 + 256) = make_uint4(o[k][4], o[k][5], o[k][6], o[k][7]);
+        if (ROWS >= 4) {
+#pragma unroll
+            for (uint32_t r = 0; r < ROWS; r += 4)
+                *(uint4*)(outs[k] + row_of<ROWS>(row0, r)) = make_uint4(o[k][r], o[k][r + 1], o[k][r + 2], o[k][r + 3]);
         } else {
             outs[k][row0] = o[k][0];
         }
+    }
+}
+
+// One sample point at R rows: its denominators, their inverses by one M31
+// inversion, and the rows' quotients num / den added to q, kept as 64-bit sums of
+// products below 2^34 (+ 4 * 2^62 on top of `fresh`, a sum no point has been
+// added to). num(r, k) gives the row's numerator coordinate plus (P - A_k) y, any
+// representative below 2^64.
+template <uint32_t R, class Num>
+__device__ __forceinline__ void add_quotients(const uint32_t x[4], const uint32_t y[4], const uint32_t dx[R],
+                                              const uint32_t dy[R], const bool live[R], uint64_t q[R][4], Num&& num) {
+    const CM31 prx = {x[0], x[1]}, pix = {x[2], x[3]}, pry = {y[0], y[1]}, piy = {y[2], y[3]};
+    const CM31 k0 = csub(cmul(prx, piy), cmul(pry, pix));
+    CM31 den[R];
+    uint32_t nrm[R], pre[R];  // norms |den|^2 and their prefix products
+    uint32_t run = 1;
+#pragma unroll
+    for (uint32_t r = 0; r < R; r++) {
+        // den = k0 - x Im(py) + y Im(px); a dead row gets a unit denominator
+        const uint64_t da = (uint64_t)dy[r] * pix.a + (uint64_t)(P - dx[r]) * piy.a + k0.a;
+        const uint64_t db = (uint64_t)dy[r] * pix.b + (uint64_t)(P - dx[r]) * piy.b + k0.b;
+        den[r] = live[r] ? CM31{reduce64(da), reduce64(db)} : CM31{1u, 0u};
+        nrm[r] = reduce64((uint64_t)den[r].a * den[r].a + (uint64_t)den[r].b * den[r].b);
+        pre[r] = run;
+        // a zero denominator (a domain point on the sample line) inverts to 0, as
+        // cm31_inv(0) does; it is kept out of the running product
+        run = mmul(run, nrm[r] ? nrm[r] : 1u);
+    }
+    uint32_t inv = minv(run);
+#pragma unroll
+    for (int r = R - 1; r >= 0; r--) {
+        const uint32_t ninv = nrm[r] ? mmul(inv, pre[r]) : 0u;
+        inv = mmul(inv, nrm[r] ? nrm[r] : 1u);
+        // 1 / den = d0 - d1 i, and one sum of products per coordinate:
+        // (f0 + f1 i)(d0 - d1 i) = (f0 d0 + f1 d1) + (f1 d0 - f0 d1) i, likewise for f2, f3
+        const uint64_t d0 = mmul(den[r].a, ninv), d1 = mmul(den[r].b, ninv);
+        uint64_t f[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) f[k] = reduce64(num(r, k));
+        q[r][0] = f[1] * d1 + (f[0] * d0 + q[r][0]);
+        q[r][1] = (P - f[0]) * d1 + (f[1] * d0 + q[r][1]);
+        q[r][2] = f[3] * d1 + (f[2] * d0 + q[r][2]);
+        q[r][3] = (P - f[2]) * d1 + (f[3] * d0 + q[r][3]);
     }
 }
 
@@ -151,12 +201,10 @@ __global__ __launch_bounds__(DEEP_THREADS) void quotients_combine_kernel(
         dx[r] = live[r] ? dxs[row] : 1u;
         dy[r] = live[r] ? dys[row] : 0u;
     }
-    QM31 q[R];
-#pragma unroll
-    for (uint32_t r = 0; r < R; r++) q[r] = {{0, 0, 0, 0}};
+    uint64_t q[R][4] = {};
     for (uint32_t j = 0; j < n_accs; j++) {
         const uint32_t sh = lifting_log - acc_logs[j] + 1;
-        const uint32_t *p0 = n0[j], *p1 = n1[j], *p2 = n2[j], *p3 = n3[j];
+        const gu32 *p0 = as_global(n0[j]), *p1 = as_global(n1[j]), *p2 = as_global(n2[j]), *p3 = as_global(n3[j]);
         uint32_t nv[R][4];
 #pragma unroll
         for (uint32_t r = 0; r < R; r++) {
@@ -167,51 +215,22 @@ __global__ __launch_bounds__(DEEP_THREADS) void quotients_combine_kernel(
             nv[r][2] = p2[li];
             nv[r][3] = p3[li];
         }
-        const CM31 prx = {spx[4 * j], spx[4 * j + 1]}, pix = {spx[4 * j + 2], spx[4 * j + 3]};
-        const CM31 pry = {spy[4 * j], spy[4 * j + 1]}, piy = {spy[4 * j + 2], spy[4 * j + 3]};
-        const CM31 k0 = csub(cmul(prx, piy), cmul(pry, pix));
-        const QM31 a = {{fla[4 * j], fla[4 * j + 1], fla[4 * j + 2], fla[4 * j + 3]}};  // canonical
-        CM31 den[R];
-        uint32_t nrm[R], pre[R];  // norms |den|^2 and their prefix products
-        uint32_t run = 1;
+        const uint32_t* a = fla + 4 * j;  // canonical
+        add_quotients<R>(spx + 4 * j, spy + 4 * j, dx, dy, live, q,
+                         [&](uint32_t r, int k) { return (uint64_t)(P - a[k]) * dy[r] + nv[r][k]; });
 #pragma unroll
-        for (uint32_t r = 0; r < R; r++) {
-            // den = k0 - x Im(py) + y Im(px); a dead row gets a unit denominator
-            const uint64_t da = (uint64_t)dy[r] * pix.a + (uint64_t)(P - dx[r]) * piy.a + k0.a;
-            const uint64_t db = (uint64_t)dy[r] * pix.b + (uint64_t)(P - dx[r]) * piy.b + k0.b;
-            den[r] = live[r] ? CM31{reduce64(da), reduce64(db)} : CM31{1u, 0u};
-            nrm[r] = reduce64((uint64_t)den[r].a * den[r].a + (uint64_t)den[r].b * den[r].b);
-            pre[r] = run;
-            // a zero denominator (a domain point on the sample line) inverts to 0, as
-            // cm31_inv(0) does; it is kept out of the running product
-            run = mmul(run, nrm[r] ? nrm[r] : 1u);
-        }
-        uint32_t inv = minv(run);
+        for (uint32_t r = 0; r < R; r++)
 #pragma unroll
-        for (int r = R - 1; r >= 0; r--) {
-            const uint32_t ninv = nrm[r] ? mmul(inv, pre[r]) : 0u;
-            inv = mmul(inv, nrm[r] ? nrm[r] : 1u);
-            // 1 / den = d0 - d1 i
-            const uint64_t d0 = mmul(den[r].a, ninv), d1 = mmul(den[r].b, ninv);
-            // full = numer - a y, then full * (d0 - d1 i), one reduction per coordinate:
-            // (f0 + f1 i)(d0 - d1 i) = (f0 d0 + f1 d1) + (f1 d0 - f0 d1) i, likewise for f2, f3
-            const uint64_t y = dy[r];
-            const uint64_t f0 = reduce64(nv[r][0] + (P - a.v[0]) * y), f1 = reduce64(nv[r][1] + (P - a.v[1]) * y);
-            const uint64_t f2 = reduce64(nv[r][2] + (P - a.v[2]) * y), f3 = reduce64(nv[r][3] + (P - a.v[3]) * y);
-            q[r].v[0] = madd(q[r].v[0], reduce64(f0 * d0 + f1 * d1));
-            q[r].v[1] = madd(q[r].v[1], reduce64(f1 * d0 + (P - f0) * d1));
-            q[r].v[2] = madd(q[r].v[2], reduce64(f2 * d0 + f3 * d1));
-            q[r].v[3] = madd(q[r].v[3], reduce64(f3 * d0 + (P - f2) * d1));
-        }
+            for (int k = 0; k < 4; k++) q[r][k] = fold64(q[r][k]);
     }
 #pragma unroll
     for (uint32_t r = 0; r < R; r++) {
         if (!live[r]) continue;
         const uint64_t row = base + 64u * r + lane;
-        out0[row] = q[r].v[0];
-        out1[row] = q[r].v[1];
-        out2[row] = q[r].v[2];
-        out3[row] = q[r].v[3];
+        out0[row] = reduce64(q[r][0]);
+        out1[row] = reduce64(q[r][1]);
+        out2[row] = reduce64(q[r][2]);
+        out3[row] = reduce64(q[r][3]);
     }
 }
 
@@ -250,25 +269,24 @@ __global__ __launch_bounds__(DEEP_THREADS) void accumulate_lift_kernel(uint32_t*
 constexpr uint32_t DEEP_MAX_POINTS = 4;
 
 // Values of columns c .. c + G - 1 at the rows of this thread (lifted indices).
+constexpr uint32_t FUSED_GROUP = 4;
 template <uint32_t G, uint32_t R>
 __device__ __forceinline__ void fused_load(const uint32_t* __restrict__ cm, uint32_t c, const uint32_t row[R],
-                                           uint32_t f[3][R]) {
+                                           uint32_t f[FUSED_GROUP][R]) {
 #pragma unroll
     for (uint32_t g = 0; g < G; g++) {
-        const uint32_t* ptr = (const uint32_t*)(uintptr_t)(cm[4 * (c + g)] | ((uint64_t)cm[4 * (c + g) + 1] << 32));
+        const gu32* ptr = as_global((const uint32_t*)(uintptr_t)(cm[4 * (c + g)] | ((uint64_t)cm[4 * (c + g) + 1] << 32)));
         const uint32_t sh = cm[4 * (c + g) + 2];
 #pragma unroll
         for (uint32_t r = 0; r < R; r++) f[g][r] = ptr[((row[r] >> sh) << 1) | (row[r] & 1)];
     }
 }
 
-// acc += c_pc * f for columns c .. c + G - 1 (G <= 3): three products on top of
-// a partially reduced value (< 2^62 + 4) stay below 2^64, then bits 62..63 fold
-// onto bit 0.
+// acc += c_pc * f for columns c .. c + G - 1 (G <= 4): four products on top of a
+// folded value (< 2^34) stay below 2^64.
 template <uint32_t G, uint32_t NP, uint32_t R>
-__device__ __forceinline__ void fused_accumulate(const uint32_t* __restrict__ cf, uint32_t c, const uint32_t f[3][R],
-                                                 uint64_t acc[NP][R][4]) {
-    constexpr uint64_t M62 = (1ull << 62) - 1;
+__device__ __forceinline__ void fused_accumulate(const uint32_t* __restrict__ cf, uint32_t c,
+                                                 const uint32_t f[FUSED_GROUP][R], uint64_t acc[NP][R][4]) {
 #pragma unroll
     for (uint32_t p = 0; p < NP; p++)
 #pragma unroll
@@ -278,7 +296,7 @@ __device__ __forceinline__ void fused_accumulate(const uint32_t* __restrict__ cf
                 uint64_t a = acc[p][r][k];
 #pragma unroll
                 for (uint32_t g = 0; g < G; g++) a = (uint64_t)cf[((c + g) * NP + p) * 4 + k] * f[g][r] + a;
-                acc[p][r][k] = (a & M62) + (a >> 62);
+                acc[p][r][k] = fold64(a);
             }
 }
 
@@ -306,30 +324,34 @@ __global__ __launch_bounds__(DEEP_THREADS) void deep_fused_kernel(const uint32_t
         row[r] = live[r] ? x : n_rows - 1;
     }
     uint64_t acc[NP][R][4] = {};
-    // The one or two columns past a multiple of three first (while the first
-    // whole group's loads are in flight), then whole groups of three, the next
-    // group's loads in flight while a group is summed.
-    const uint32_t c0 = n_cols % 3;
-    uint32_t fa[3][R], fb[3][R];
-    if (c0 < n_cols) fused_load<3, R>(cm, c0, row, fa);
+    // The columns past a multiple of four first (while the first whole group's
+    // loads are in flight), then whole groups of four, the next group's loads in
+    // flight while a group is summed.
+    constexpr uint32_t G = FUSED_GROUP;
+    const uint32_t c0 = n_cols % G;
+    uint32_t fa[G][R], fb[G][R];
+    if (c0 < n_cols) fused_load<G, R>(cm, c0, row, fa);
     if (c0 == 1) {
         fused_load<1, R>(cm, 0, row, fb);
         fused_accumulate<1, NP, R>(cf, 0, fb, acc);
     } else if (c0 == 2) {
         fused_load<2, R>(cm, 0, row, fb);
         fused_accumulate<2, NP, R>(cf, 0, fb, acc);
+    } else if (c0 == 3) {
+        fused_load<3, R>(cm, 0, row, fb);
+        fused_accumulate<3, NP, R>(cf, 0, fb, acc);
     }
     if (c0 < n_cols) {
         for (uint32_t c = c0;;) {
-            const bool more_b = c + 3 < n_cols;
-            if (more_b) fused_load<3, R>(cm, c + 3, row, fb);
-            fused_accumulate<3, NP, R>(cf, c, fa, acc);
-            c += 3;
+            const bool more_b = c + G < n_cols;
+            if (more_b) fused_load<G, R>(cm, c + G, row, fb);
+            fused_accumulate<G, NP, R>(cf, c, fa, acc);
+            c += G;
             if (!more_b) break;
-            const bool more_a = c + 3 < n_cols;
-            if (more_a) fused_load<3, R>(cm, c + 3, row, fa);
-            fused_accumulate<3, NP, R>(cf, c, fb, acc);
-            c += 3;
+            const bool more_a = c + G < n_cols;
+            if (more_a) fused_load<G, R>(cm, c + G, row, fa);
+            fused_accumulate<G, NP, R>(cf, c, fb, acc);
+            c += G;
             if (!more_a) break;
         }
     }
@@ -339,54 +361,28 @@ __global__ __launch_bounds__(DEEP_THREADS) void deep_fused_kernel(const uint32_t
         dx[r] = live[r] ? dxs[row[r]] : 1u;
         dy[r] = live[r] ? dys[row[r]] : 0u;
     }
-    QM31 q[R];
-#pragma unroll
-    for (uint32_t r = 0; r < R; r++) q[r] = {{0, 0, 0, 0}};
+    uint64_t q[R][4] = {};
 #pragma unroll
     for (uint32_t p = 0; p < NP; p++) {
         const uint32_t* pp = pts + 16 * p;
-        const CM31 prx = {pp[0], pp[1]}, pix = {pp[2], pp[3]};
-        const CM31 pry = {pp[4], pp[5]}, piy = {pp[6], pp[7]};
-        const CM31 k0 = csub(cmul(prx, piy), cmul(pry, pix));
-        CM31 den[R];
-        uint32_t nrm[R], pre[R];
-        uint32_t run = 1;
+        // numerator - B - A y, A and B canonical
+        add_quotients<R>(pp, pp + 4, dx, dy, live, q, [&](uint32_t r, int k) {
+            return (uint64_t)(P - pp[8 + k]) * dy[r] + (acc[p][r][k] + (P - pp[12 + k]));
+        });
+        if ((p & 1) && p + 1 < NP) {  // four products are in
 #pragma unroll
-        for (uint32_t r = 0; r < R; r++) {
-            const uint64_t da = (uint64_t)dy[r] * pix.a + (uint64_t)(P - dx[r]) * piy.a + k0.a;
-            const uint64_t db = (uint64_t)dy[r] * pix.b + (uint64_t)(P - dx[r]) * piy.b + k0.b;
-            den[r] = live[r] ? CM31{reduce64(da), reduce64(db)} : CM31{1u, 0u};
-            nrm[r] = reduce64((uint64_t)den[r].a * den[r].a + (uint64_t)den[r].b * den[r].b);
-            pre[r] = run;
-            run = mmul(run, nrm[r] ? nrm[r] : 1u);  // a zero denominator inverts to 0 (cm31_inv(0))
-        }
-        uint32_t inv = minv(run);
+            for (uint32_t r = 0; r < R; r++)
 #pragma unroll
-        for (int r = R - 1; r >= 0; r--) {
-            const uint32_t ninv = nrm[r] ? mmul(inv, pre[r]) : 0u;
-            inv = mmul(inv, nrm[r] ? nrm[r] : 1u);
-            const uint64_t d0 = mmul(den[r].a, ninv), d1 = mmul(den[r].b, ninv);
-            const uint64_t y = dy[r];
-            uint64_t f[4];
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                // numerator - B - A y, A and B canonical
-                const uint32_t num = msub(reduce64(acc[p][r][k]), pp[12 + k]);
-                f[k] = reduce64(num + (P - pp[8 + k]) * y);
-            }
-            q[r].v[0] = madd(q[r].v[0], reduce64(f[0] * d0 + f[1] * d1));
-            q[r].v[1] = madd(q[r].v[1], reduce64(f[1] * d0 + (P - f[0]) * d1));
-            q[r].v[2] = madd(q[r].v[2], reduce64(f[2] * d0 + f[3] * d1));
-            q[r].v[3] = madd(q[r].v[3], reduce64(f[3] * d0 + (P - f[2]) * d1));
+                for (int k = 0; k < 4; k++) q[r][k] = fold64(q[r][k]);
         }
     }
 #pragma unroll
     for (uint32_t r = 0; r < R; r++) {
         if (!live[r]) continue;
-        out0[row[r]] = q[r].v[0];
-        out1[row[r]] = q[r].v[1];
-        out2[row[r]] = q[r].v[2];
-        out3[row[r]] = q[r].v[3];
+        out0[row[r]] = reduce64(q[r][0]);
+        out1[row[r]] = reduce64(q[r][1]);
+        out2[row[r]] = reduce64(q[r][2]);
+        out3[row[r]] = reduce64(q[r][3]);
     }
 }
 
@@ -486,18 +482,25 @@ static bool launch_deep_fused(const uint32_t* meta, uint32_t NP, uint32_t n_cols
                               const uint32_t* domain_xs, const uint32_t* domain_ys, uint32_t* out0, uint32_t* out1,
                               uint32_t* out2, uint32_t* out3, hipStream_t s) {
     const uint32_t n_rows = 1u << lifting_log_size;
-    switch (NP) {
-#define VX_DEEP_LAUNCH(np, r)                                                                                  \
-    case np:                                                                                                   \
-        deep_fused_kernel<np, r><<<ceil_div(n_rows, (uint64_t)DEEP_THREADS * r), DEEP_THREADS, 0, s>>>(        \
-            meta, n_cols, domain_xs, domain_ys, n_rows, out0, out1, out2, out3);                               \
-        break;
-        VX_DEEP_LAUNCH(1, 4)
-        VX_DEEP_LAUNCH(2, 4)
-        VX_DEEP_LAUNCH(3, 2)
-        VX_DEEP_LAUNCH(4, 2)
-#undef VX_DEEP_LAUNCH
+#define VX_DEEP_LAUNCH(np, r)                                                                           \
+    deep_fused_kernel<np, r><<<ceil_div(n_rows, (uint64_t)DEEP_THREADS * r), DEEP_THREADS, 0, s>>>(     \
+        meta, n_cols, domain_xs, domain_ys, n_rows, out0, out1, out2, out3)
+    if (n_rows >= FUSED_WIDE_MIN) {
+        switch (NP) {
+            case 1: VX_DEEP_LAUNCH(1, 4); break;
+            case 2: VX_DEEP_LAUNCH(2, 4); break;
+            case 3: VX_DEEP_LAUNCH(3, 2); break;
+            case 4: VX_DEEP_LAUNCH(4, 2); break;
+        }
+    } else {
+        switch (NP) {
+            case 1: VX_DEEP_LAUNCH(1, 1); break;
+            case 2: VX_DEEP_LAUNCH(2, 1); break;
+            case 3: VX_DEEP_LAUNCH(3, 1); break;
+            case 4: VX_DEEP_LAUNCH(4, 1); break;
+        }
     }
+#undef VX_DEEP_LAUNCH
     return check_launch("deep_fused_kernel");
 }
 
@@ -562,14 +565,17 @@ void cuda_accumulate_numerators(const uint32_t* const* col_ptrs, const uint32_t*
                                 const uint32_t* b_coeffs, const uint32_t* c_coeffs, uint32_t n_batch_cols,
                                 uint32_t n_rows, uint32_t* out0, uint32_t* out1, uint32_t* out2, uint32_t* out3) {
     if (!n_rows) return;
-    // whole 512-row wave chunks and 16-byte aligned outputs: the wide form
-    const bool vec = n_rows % 512 == 0 && (((uintptr_t)out0 | (uintptr_t)out1 | (uintptr_t)out2 | (uintptr_t)out3) & 15) == 0;
-    if (vec)
-        accumulate_numerators_kernel<8><<<ceil_div(n_rows, 8 * DEEP_THREADS), DEEP_THREADS, 0, current_stream()>>>(
-            col_ptrs, col_indices, b_coeffs, c_coeffs, n_batch_cols, n_rows, out0, out1, out2, out3);
+    const bool aligned = (((uintptr_t)out0 | (uintptr_t)out1 | (uintptr_t)out2 | (uintptr_t)out3) & 15) == 0;
+#define VX_NUMERATORS(rows)                                                                                     \
+    accumulate_numerators_kernel<rows><<<ceil_div(n_rows, rows * DEEP_THREADS), DEEP_THREADS, 0, current_stream()>>>( \
+        col_ptrs, col_indices, b_coeffs, c_coeffs, n_batch_cols, n_rows, out0, out1, out2, out3)
+    if (aligned && n_rows % 512 == 0 && n_rows >= NUMER_WIDE_MIN)
+        VX_NUMERATORS(8);
+    else if (aligned && n_rows % 256 == 0)
+        VX_NUMERATORS(4);
     else
-        accumulate_numerators_kernel<1><<<ceil_div(n_rows, DEEP_THREADS), DEEP_THREADS, 0, current_stream()>>>(
-            col_ptrs, col_indices, b_coeffs, c_coeffs, n_batch_cols, n_rows, out0, out1, out2, out3);
+        VX_NUMERATORS(1);
+#undef VX_NUMERATORS
     check_launch("cuda_accumulate_numerators");
 }
 
@@ -581,10 +587,17 @@ void cuda_compute_quotients_combine(const uint32_t* sample_points_x, const uint3
                                     uint32_t lifting_log_size, uint32_t n_rows, uint32_t* out0, uint32_t* out1,
                                     uint32_t* out2, uint32_t* out3) {
     if (!n_rows) return;
-    const uint64_t rows_per_block = (uint64_t)DEEP_THREADS * COMBINE_ROWS;
-    quotients_combine_kernel<COMBINE_ROWS><<<ceil_div(n_rows, rows_per_block), DEEP_THREADS, 0, current_stream()>>>(
-        sample_points_x, sample_points_y, first_linear_acc, numer_ptrs0, numer_ptrs1, numer_ptrs2, numer_ptrs3,
-        acc_log_sizes, n_accs, domain_xs, domain_ys, lifting_log_size, n_rows, out0, out1, out2, out3);
+#define VX_COMBINE(rows)                                                                                            \
+    quotients_combine_kernel<rows><<<ceil_div(n_rows, rows * DEEP_THREADS), DEEP_THREADS, 0, current_stream()>>>(       \
+        sample_points_x, sample_points_y, first_linear_acc, numer_ptrs0, numer_ptrs1, numer_ptrs2, numer_ptrs3,        \
+        acc_log_sizes, n_accs, domain_xs, domain_ys, lifting_log_size, n_rows, out0, out1, out2, out3)
+    if (n_rows >= COMBINE_WIDE_MIN)
+        VX_COMBINE(8);
+    else if (n_rows >= COMBINE_MID_MIN)
+        VX_COMBINE(4);
+    else
+        VX_COMBINE(2);
+#undef VX_COMBINE
     check_launch("cuda_compute_quotients_combine");
 }
 

@@ -75,50 +75,65 @@ struct LiftAbiCol {
     uint32_t pad;
 };
 
-// The block flattens the schedule into LDS (column pointer + log size per
-// message word), then each thread hashes one leaf block by block.
+// The block flattens the schedule into LDS (column pointer + log size per message
+// word), a thread per schedule entry: three dependent loads, where a thread per
+// chunk made a chain of them for every column (2^19 leaves of 15 columns: 24 ->
+// 20 us). Then each thread hashes one leaf, 16 columns a compression, at
+// eight waves a SIMD. Lane k of a wave holds the block's column k, whose pointer and
+// shift every lane takes from there into scalar registers: sixteen global loads in
+// flight off scalar bases.
 __global__ __launch_bounds__(256) void lifted_leaves_kernel(const uint32_t* const* col_ptrs,
                                                            const LeafHashChunk* schedule, uint32_t n_chunks,
-                                                           uint32_t S, uint32_t* out, uint64_t n_leaves) {
+                                                           uint32_t S, uint32_t* out, uint32_t n_leaves) {
     __shared__ LiftAbiCol tab[16 * LIFT_ABI_MAX_CHUNKS];
-    __shared__ uint32_t total_s;
-    const uint32_t tid = threadIdx.x;
-    if (tid < n_chunks) {
-        uint32_t start = 0;
-        for (uint32_t c = 0; c < tid; c++) start += min(schedule[c].n_cols, 16u);
-        const LeafHashChunk ch = schedule[tid];
-        const uint32_t nc = min(ch.n_cols, 16u);
-        for (uint32_t k = 0; k < nc; k++) tab[start + k] = {col_ptrs[ch.col_indices[k]], ch.log_size, 0};
-        if (tid == n_chunks - 1) total_s = start + nc;
+    __shared__ uint32_t start[LIFT_ABI_MAX_CHUNKS + 1];  // chunk c's first column; the last entry: their number
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    static_assert(LIFT_ABI_MAX_CHUNKS <= 64);
+    if (tid < 64) {
+        uint32_t sum = lane < n_chunks ? min(schedule[lane].n_cols, 16u) : 0u;
+        for (uint32_t d = 1; d < 64; d <<= 1) {
+            const uint32_t below = __shfl_up(sum, d);
+            if (lane >= d) sum += below;
+        }
+        start[lane + 1] = sum;
+        if (lane == 0) start[0] = 0;
     }
-    if (tid == 0 && n_chunks == 0) total_s = 0;
     __syncthreads();
-    const uint32_t total = total_s;
-    const uint64_t leaf = (uint64_t)blockIdx.x * blockDim.x + tid;
-    if (leaf >= n_leaves) return;
+    for (uint32_t e = tid; e < 16 * n_chunks; e += 256) {
+        const uint32_t c = e >> 4, k = e & 15;
+        if (k < start[c + 1] - start[c])
+            tab[start[c] + k] = {col_ptrs[schedule[c].col_indices[k]], schedule[c].log_size, 0};
+    }
+    const uint32_t total_s = start[LIFT_ABI_MAX_CHUNKS];
+    __syncthreads();
+    const uint32_t total = __builtin_amdgcn_readfirstlane(total_s);
+    const uint32_t leaf = blockIdx.x * 256 + tid;  // n_leaves <= 2^31
+    const uint32_t i = min(leaf, n_leaves - 1);    // whole waves stay active for the lane reads
     uint32_t h[8];
     b2s_init(h);
     for (uint32_t c0 = 0;; c0 += 16) {
         const uint32_t nw = total - c0 < 16 ? total - c0 : 16;
+        const LiftAbiCol mine = tab[min(c0 + (lane & 15), max(total, 1u) - 1)];
+        const uint32_t lo = (uint32_t)(uintptr_t)mine.p, hi = (uint32_t)((uintptr_t)mine.p >> 32);
         uint32_t m[16];
 #pragma unroll
         for (uint32_t k = 0; k < 16; k++) {
-            uint32_t v = 0;
+            m[k] = 0;
             if (k < nw) {
-                const LiftAbiCol c = tab[c0 + k];
-                uint64_t row = leaf;
-                if (c.log != S) row = ((leaf >> (S - c.log + 1)) << 1) | (leaf & 1);
+                const uint32_t log = __builtin_amdgcn_readlane(mine.log, k);
+                const uint64_t base = (uint32_t)__builtin_amdgcn_readlane(lo, k) |
+                                      (uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, k) << 32;
+                uint32_t row = log == S ? i : ((i >> ((S - log + 1) & 31)) << 1) | (i & 1);
                 // a 1-row column would be read at row 1 by the formula; stay inside it
-                if (row >> c.log) row = (1ull << c.log) - 1;
-                v = c.p[row];
+                row = min(row, log < 32 ? (1u << log) - 1 : 0xFFFFFFFFu);
+                m[k] = as_global((const uint32_t*)(uintptr_t)base)[row];
             }
-            m[k] = v;
         }
         const bool last = c0 + 16 >= total;
         b2s_compress(h, m, 4 * (c0 + nw), last ? 0xFFFFFFFFu : 0u);
         if (last) break;
     }
-    store8(out + 8 * leaf, h);
+    if (leaf < n_leaves) store8(out + 8ull * leaf, h);
 }
 
 // ---------------------------------------------------------------- pack / bit reverse
