@@ -66,34 +66,35 @@ void commit_tree(const Src& src, uint64_t n_leaves, LevelStore st, TailOut out, 
 
 // Trees of at most LEAF_QUAD_MAX leaves (and more than a tail kernel should
 // hash by itself) of a single proof commit through leaf_quad_stage_kernel, 16
-// leaves a wave up to 2^13 leaves, 32 at 2^14, 64 at 2^15, so the tail starts
-// from at most 512 nodes. Such a tree's chain is latency-bound for one proof;
-// a batch of proofs fills the device with its waves, where the lane-per-pair
-// stage does the same hashing in fewer instructions (about 980 a compression
-// against 4 x 390), so batches keep it.
-constexpr uint64_t LEAF_QUAD_MAX = 1ull << 15;
-inline uint32_t quad_stage_leaves(uint64_t n) { return n <= (1ull << 13) ? 16u : n <= (1ull << 14) ? 32u : 64u; }
+// leaves a wave up to 2^14 leaves, 32 at 2^15, 64 at 2^16, so the tail starts
+// from at most 256 nodes, all of whose levels go by quads. Such a tree's chain is
+// latency-bound for one proof (2^14 rows: 292 us with 512 nodes handed on and the
+// line at 2^15, 274 so; the line at 2^17 is 1 % slower from 2^15 rows on); a batch
+// of proofs fills the device with its waves, where the lane-per-pair stage does
+// the same hashing in fewer instructions (about 980 a compression against 4 x
+// 390), so batches keep it.
+constexpr uint64_t LEAF_QUAD_MAX = 1ull << 16;
+inline uint32_t quad_stage_leaves(uint64_t n) { return n <= (1ull << 14) ? 16u : n <= (1ull << 15) ? 32u : 64u; }
 
 // Commits a tree of n leaves (1024 <= n <= LEAF_QUAD_MAX, a power of two) with
-// the quad leaf stage and the tail kernel. Its stage hands on n / 16 nodes at
-// most, inside the scratch of any tree of n leaves (n / 32 from 2^14 leaves
-// on; scratch_nodes_a covers the smaller ones).
+// the quad leaf stage and the tail kernel. Its stage hands on n / 64 nodes at
+// most (scratch_nodes_a).
 template <class Src, class Mark>
 void commit_tree_quad(const Src& src, uint64_t n, LevelStore st, TailOut out, Scratch sc, hipStream_t s, Mark&& mark,
                       uint32_t batch = 1, uint64_t bs = 0) {
     const uint32_t lpw = quad_stage_leaves(n);
-    const uint64_t waves = n / lpw;
-    const dim3 grid((uint32_t)ceil_div(waves, LEAF_QUAD_WAVES), batch);
+    const uint32_t blocks = (uint32_t)(n / (lpw * LEAF_QUAD_WAVES));
+    const dim3 grid(blocks, batch);
     if (lpw == 16)
-        leaf_quad_stage_kernel<Src, 1><<<grid, 64 * LEAF_QUAD_WAVES, 0, s>>>(src, n, sc.a, st, bs);
+        leaf_quad_stage_kernel<Src, 1><<<grid, 64 * LEAF_QUAD_WAVES, 0, s>>>(src, sc.a, st, bs);
     else if (lpw == 32)
-        leaf_quad_stage_kernel<Src, 2><<<grid, 64 * LEAF_QUAD_WAVES, 0, s>>>(src, n, sc.a, st, bs);
+        leaf_quad_stage_kernel<Src, 2><<<grid, 64 * LEAF_QUAD_WAVES, 0, s>>>(src, sc.a, st, bs);
     else
-        leaf_quad_stage_kernel<Src, 4><<<grid, 64 * LEAF_QUAD_WAVES, 0, s>>>(src, n, sc.a, st, bs);
+        leaf_quad_stage_kernel<Src, 4><<<grid, 64 * LEAF_QUAD_WAVES, 0, s>>>(src, sc.a, st, bs);
     check_launch("leaf_quad_stage_kernel");
     mark("stage_leaf");
-    merkle_tail_kernel<SrcNodes><<<dim3(1, batch), TAIL_THREADS, 0, s>>>(SrcNodes{sc.a}, floor_log2(lpw),
-                                                                         (uint32_t)waves, st, out, bs);
+    merkle_tail_kernel<SrcNodes><<<dim3(1, batch), TAIL_THREADS, 0, s>>>(SrcNodes{sc.a}, floor_log2(lpw * LEAF_QUAD_WAVES),
+                                                                         blocks, st, out, bs);
     check_launch("merkle_tail_kernel<nodes>");
     mark("tail");
 }
@@ -112,7 +113,7 @@ void commit_leaves(const Src& src, uint64_t n, LevelStore st, TailOut out, Scrat
 // Nodes per proof of the two stage scratch buffers of a tree of n_leaves items:
 // a takes the leaf stage's output and every other node stage's, b the rest.
 inline uint64_t scratch_nodes_a(uint64_t n_leaves) {
-    const uint64_t quad = n_leaves <= QUAD_DIRECT_MAX ? 0 : std::min<uint64_t>(n_leaves, LEAF_QUAD_MAX) / 16;
+    const uint64_t quad = n_leaves <= QUAD_DIRECT_MAX ? 0 : std::min<uint64_t>(n_leaves, LEAF_QUAD_MAX) / (16 * LEAF_QUAD_WAVES);
     return std::max<uint64_t>({1, max_leaf_stage_nodes(n_leaves, QUAD_DIRECT_MAX), quad});
 }
 inline uint64_t scratch_nodes_b(uint64_t n_leaves) {

@@ -708,28 +708,29 @@ __global__ __launch_bounds__(64 * MERKLE_STAGE_WAVES) void merkle_stage_kernel(S
 
 // ---------------------------------------------------------------- small leaf stages
 // Leaf stage of a small tree: one leaf per quad, hashed quad-cooperatively,
-// 16 * R leaves a wave reduced to one node. On the few waves such a tree has
-// (at most one per SIMD), a wave's chain is then R quad compressions for the
-// leaves and log2(16 R) node levels, where the lane-per-pair form (128 leaves
-// a wave) takes three lane compressions and seven quad rounds. Every lane of a
-// quad forms its leaf's words.
+// 16 * R leaves a wave reduced to one node, a workgroup's four to one. On the few
+// waves such a tree has (at most one per SIMD), a wave's chain is then R quad
+// compressions for the leaves and log2(64 R) node levels, where the lane-per-pair
+// form (128 leaves a wave) takes three lane compressions and seven quad rounds. The
+// last two levels cost two quad compressions of one wave and save the tail kernel
+// its two widest levels, which are its dearest (three more, of eight waves a
+// workgroup, cost more than they save). Every lane of a quad forms its leaf's words.
 constexpr uint32_t LEAF_QUAD_WAVES = 4;  // waves per workgroup
 template <class Src, uint32_t R>
-__global__ __launch_bounds__(64 * LEAF_QUAD_WAVES) void leaf_quad_stage_kernel(Src src0, uint64_t n_items,
-                                                                             uint32_t* out_nodes, LevelStore st0,
-                                                                             uint64_t bs) {
+__global__ __launch_bounds__(64 * LEAF_QUAD_WAVES) void leaf_quad_stage_kernel(Src src0, uint32_t* out_nodes,
+                                                                             LevelStore st0, uint64_t bs) {
     constexpr uint32_t LPW = 16 * R;  // leaves a wave
     __shared__ __align__(16) uint32_t lds[LEAF_QUAD_WAVES][8 * LPW + 4 * LPW];
+    __shared__ __align__(16) uint32_t tops[8 * LEAF_QUAD_WAVES], tops2[4 * LEAF_QUAD_WAVES];
     const uint64_t boff = (uint64_t)blockIdx.y * bs;
     const Src src = src0.at(boff);
     const LevelStore st = st0.shifted(boff);
     out_nodes += boff;
     const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6, quad = lane >> 2, l = lane & 3;
     const uint64_t wave_id = (uint64_t)blockIdx.x * LEAF_QUAD_WAVES + w;
-    const uint64_t base = wave_id * LPW;
-    if (base >= n_items) return;  // wave-uniform
-    uint32_t* na = lds[w];        // LPW nodes, node-major
-    uint32_t* nb = na + 8 * LPW;  // the next level
+    const uint64_t base = wave_id * LPW;  // n_items is a multiple of the block's leaves
+    uint32_t* na = lds[w];                // LPW nodes, node-major
+    uint32_t* nb = na + 8 * LPW;          // the next level
     for (uint32_t r = 0; r < R; r++) {
         const uint32_t k = 16 * r + quad;
         uint32_t v[Src::WIDTH], hl, hh;
@@ -740,7 +741,12 @@ __global__ __launch_bounds__(64 * LEAF_QUAD_WAVES) void leaf_quad_stage_kernel(S
     }
     VX_WAVE_SYNC();
     const uint32_t* top = narrow_reduce(na, nb, LPW, 0, base, st);
-    if (lane < 8) out_nodes[8 * wave_id + lane] = top[lane];
+    if (lane < 8) tops[8 * w + lane] = top[lane];
+    lds_barrier();
+    if (w) return;
+    constexpr uint32_t LOG = R == 1 ? 4 : R == 2 ? 5 : 6;
+    top = narrow_reduce(tops, tops2, LEAF_QUAD_WAVES, LOG, (uint64_t)blockIdx.x * LEAF_QUAD_WAVES, st);
+    if (lane < 8) out_nodes[8ull * blockIdx.x + lane] = top[lane];
 }
 
 // ---------------------------------------------------------------- tail kernel
