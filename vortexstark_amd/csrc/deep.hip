@@ -37,7 +37,7 @@ constexpr uint32_t DEEP_THREADS = 256;
 // Rows from which a thread takes more of them, having enough threads either way
 // (us below and above the line; the first two with their launch of about 17 and 5):
 // - fused, two points: 2^17 rows 20.8 at one row a thread, 24.2 at four; 2^18 25.9
-//   and 24.3; 2^22 168 and 121
+//   and 23.8; 2^22 168 and 111
 // - combine, four accumulations: 2^17 rows 8.9 at two, 11.9 at four, 18.5 at eight;
 //   2^19 22.0, 19.7 and 20.6; 2^22 137, 115 and 110
 // - numerators: 2^16 rows of 12 columns 5.5 at four, 6.7 at eight; 2^18 of 64 columns
@@ -85,11 +85,13 @@ __global__ __launch_bounds__(DEEP_THREADS) void accumulate_numerators_kernel(
                                     : ((uint64_t)blockIdx.x * (DEEP_THREADS / 64) + (threadIdx.x >> 6)) * 64 * ROWS +
                                           4 * (threadIdx.x & 63);
     if (row0 >= n_rows) return;
+    ConstU64* ptrs = (ConstU64*)col_ptrs;
+    ConstU32 *idx = (ConstU32*)col_indices, *b = (ConstU32*)b_coeffs, *cc = (ConstU32*)c_coeffs;
     // sum_i b_i: the same for every row
     uint32_t bs[4] = {0, 0, 0, 0};
     for (uint32_t i = 0; i < n_batch; i++)
 #pragma unroll
-        for (int k = 0; k < 4; k++) bs[k] = madd(bs[k], b_coeffs[4 * i + k]);
+        for (int k = 0; k < 4; k++) bs[k] = madd(bs[k], b[4 * i + k]);
     // The accumulators stay below 2^34 between groups: a group adds four products of
     // at most (p - 1)^2 < 2^62 - 2^32, which stays below 2^64, and folds.
     uint64_t acc[ROWS][4] = {};
@@ -97,24 +99,24 @@ __global__ __launch_bounds__(DEEP_THREADS) void accumulate_numerators_kernel(
     for (; i + 4 <= n_batch; i += 4) {
         uint32_t f[4][ROWS];
 #pragma unroll
-        for (int g = 0; g < 4; g++) load_rows<ROWS>(col_ptrs[col_indices[i + g]], row0, f[g]);
+        for (int g = 0; g < 4; g++) load_rows<ROWS>((const uint32_t*)ptrs[idx[i + g]], row0, f[g]);
 #pragma unroll
         for (uint32_t r = 0; r < ROWS; r++)
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 uint64_t a = acc[r][k];
 #pragma unroll
-                for (int g = 0; g < 4; g++) a = (uint64_t)c_coeffs[4 * (i + g) + k] * f[g][r] + a;
+                for (int g = 0; g < 4; g++) a = (uint64_t)cc[4 * (i + g) + k] * f[g][r] + a;
                 acc[r][k] = fold64(a);
             }
     }
     for (; i < n_batch; i++) {
         uint32_t f[ROWS];
-        load_rows<ROWS>(col_ptrs[col_indices[i]], row0, f);
+        load_rows<ROWS>((const uint32_t*)ptrs[idx[i]], row0, f);
 #pragma unroll
         for (uint32_t r = 0; r < ROWS; r++)
 #pragma unroll
-            for (int k = 0; k < 4; k++) acc[r][k] = fold64((uint64_t)c_coeffs[4 * i + k] * f[r] + acc[r][k]);
+            for (int k = 0; k < 4; k++) acc[r][k] = fold64((uint64_t)cc[4 * i + k] * f[r] + acc[r][k]);
     }
     uint32_t o[4][ROWS];
 #pragma unroll
@@ -140,7 +142,7 @@ __global__ __launch_bounds__(DEEP_THREADS) void accumulate_numerators_kernel(
 // added to). num(r, k) gives the row's numerator coordinate plus (P - A_k) y, any
 // representative below 2^64.
 template <uint32_t R, class Num>
-__device__ __forceinline__ void add_quotients(const uint32_t x[4], const uint32_t y[4], const uint32_t dx[R],
+__device__ __forceinline__ void add_quotients(ConstU32* x, ConstU32* y, const uint32_t dx[R],
                                               const uint32_t dy[R], const bool live[R], uint64_t q[R][4], Num&& num) {
     const CM31 prx = {x[0], x[1]}, pix = {x[2], x[3]}, pry = {y[0], y[1]}, piy = {y[2], y[3]};
     const CM31 k0 = csub(cmul(prx, piy), cmul(pry, pix));
@@ -203,20 +205,20 @@ __global__ __launch_bounds__(DEEP_THREADS) void quotients_combine_kernel(
     }
     uint64_t q[R][4] = {};
     for (uint32_t j = 0; j < n_accs; j++) {
-        const uint32_t sh = lifting_log - acc_logs[j] + 1;
-        const gu32 *p0 = as_global(n0[j]), *p1 = as_global(n1[j]), *p2 = as_global(n2[j]), *p3 = as_global(n3[j]);
+        const uint32_t sh = lifting_log - ((ConstU32*)acc_logs)[j] + 1;
+        const uint32_t* const* const n[4] = {n0, n1, n2, n3};
+        const gu32* num[4];
+        for (int k = 0; k < 4; k++) num[k] = as_global((const uint32_t*)((ConstU64*)n[k])[j]);
         uint32_t nv[R][4];
 #pragma unroll
         for (uint32_t r = 0; r < R; r++) {
             const uint64_t row = base + 64u * r + lane;
             const uint64_t li = live[r] ? ((row >> sh) << 1) + (row & 1) : 0;
-            nv[r][0] = p0[li];
-            nv[r][1] = p1[li];
-            nv[r][2] = p2[li];
-            nv[r][3] = p3[li];
+#pragma unroll
+            for (int k = 0; k < 4; k++) nv[r][k] = num[k][li];
         }
-        const uint32_t* a = fla + 4 * j;  // canonical
-        add_quotients<R>(spx + 4 * j, spy + 4 * j, dx, dy, live, q,
+        ConstU32* a = (ConstU32*)fla + 4 * j;  // canonical
+        add_quotients<R>((ConstU32*)spx + 4 * j, (ConstU32*)spy + 4 * j, dx, dy, live, q,
                          [&](uint32_t r, int k) { return (uint64_t)(P - a[k]) * dy[r] + nv[r][k]; });
 #pragma unroll
         for (uint32_t r = 0; r < R; r++)
@@ -269,23 +271,36 @@ __global__ __launch_bounds__(DEEP_THREADS) void accumulate_lift_kernel(uint32_t*
 constexpr uint32_t DEEP_MAX_POINTS = 4;
 
 // Values of columns c .. c + G - 1 at the rows of this thread (lifted indices).
+// R > 1: rows row .. row + R - 1, row a multiple of R; a pair of rows comes from two
+// neighbouring words of any column, one load. (One load of four words where the
+// column has the domain's size needs a branch, at whose end the words are waited
+// for: 160 us for the 34 columns, 156 us so.)
 constexpr uint32_t FUSED_GROUP = 4;
 template <uint32_t G, uint32_t R>
-__device__ __forceinline__ void fused_load(const uint32_t* __restrict__ cm, uint32_t c, const uint32_t row[R],
+__device__ __forceinline__ void fused_load(ConstU32* cm, uint32_t c, uint32_t row,
                                            uint32_t f[FUSED_GROUP][R]) {
 #pragma unroll
     for (uint32_t g = 0; g < G; g++) {
         const gu32* ptr = as_global((const uint32_t*)(uintptr_t)(cm[4 * (c + g)] | ((uint64_t)cm[4 * (c + g) + 1] << 32)));
         const uint32_t sh = cm[4 * (c + g) + 2];
+        if constexpr (R == 1) {
+            f[g][0] = ptr[((row >> sh) << 1) | (row & 1)];
+        } else {
 #pragma unroll
-        for (uint32_t r = 0; r < R; r++) f[g][r] = ptr[((row[r] >> sh) << 1) | (row[r] & 1)];
+            for (uint32_t r = 0; r < R; r += 2) {
+                const u32x2_any v =
+                    *(const __attribute__((address_space(1))) u32x2_any*)(ptr + (((row + r) >> sh) << 1));
+                f[g][r] = v.x;
+                f[g][r + 1] = v.y;
+            }
+        }
     }
 }
 
 // acc += c_pc * f for columns c .. c + G - 1 (G <= 4): four products on top of a
 // folded value (< 2^34) stay below 2^64.
 template <uint32_t G, uint32_t NP, uint32_t R>
-__device__ __forceinline__ void fused_accumulate(const uint32_t* __restrict__ cf, uint32_t c,
+__device__ __forceinline__ void fused_accumulate(ConstU32* cf, uint32_t c,
                                                  const uint32_t f[FUSED_GROUP][R], uint64_t acc[NP][R][4]) {
 #pragma unroll
     for (uint32_t p = 0; p < NP; p++)
@@ -308,21 +323,12 @@ __global__ __launch_bounds__(DEEP_THREADS) void deep_fused_kernel(const uint32_t
                                                                   uint32_t* __restrict__ out1,
                                                                   uint32_t* __restrict__ out2,
                                                                   uint32_t* __restrict__ out3) {
-    const uint32_t lane = threadIdx.x & 63u;
-    // n_rows <= 2^30: row indices fit 32 bits
-    const uint32_t base = (blockIdx.x * (DEEP_THREADS / 64) + (threadIdx.x >> 6)) * (64u * R);
-    if (base >= n_rows) return;
-    const uint32_t* pts = meta;
-    const uint32_t* cm = meta + 16 * NP;
-    const uint32_t* cf = cm + 4 * n_cols;
-    uint32_t row[R];  // rows past the end read the last row; their results are dropped
-    bool live[R];
-#pragma unroll
-    for (uint32_t r = 0; r < R; r++) {
-        const uint32_t x = base + 64u * r + lane;
-        live[r] = x < n_rows;
-        row[r] = live[r] ? x : n_rows - 1;
-    }
+    // n_rows <= 2^30: row indices fit 32 bits; R > 1 divides it
+    const uint32_t row = (blockIdx.x * DEEP_THREADS + threadIdx.x) * R;
+    if (row >= n_rows) return;
+    ConstU32* pts = (ConstU32*)meta;
+    ConstU32* cm = pts + 16 * NP;
+    ConstU32* cf = cm + 4 * n_cols;
     uint64_t acc[NP][R][4] = {};
     // The columns past a multiple of four first (while the first whole group's
     // loads are in flight), then whole groups of four, the next group's loads in
@@ -356,15 +362,17 @@ __global__ __launch_bounds__(DEEP_THREADS) void deep_fused_kernel(const uint32_t
         }
     }
     uint32_t dx[R], dy[R];
+    bool live[R];
 #pragma unroll
-    for (uint32_t r = 0; r < R; r++) {
-        dx[r] = live[r] ? dxs[row[r]] : 1u;
-        dy[r] = live[r] ? dys[row[r]] : 0u;
+    for (uint32_t r = 0; r < R; r++) {  // one load of R words each
+        live[r] = true;
+        dx[r] = dxs[row + r];
+        dy[r] = dys[row + r];
     }
     uint64_t q[R][4] = {};
 #pragma unroll
     for (uint32_t p = 0; p < NP; p++) {
-        const uint32_t* pp = pts + 16 * p;
+        ConstU32* pp = pts + 16 * p;
         // numerator - B - A y, A and B canonical
         add_quotients<R>(pp, pp + 4, dx, dy, live, q, [&](uint32_t r, int k) {
             return (uint64_t)(P - pp[8 + k]) * dy[r] + (acc[p][r][k] + (P - pp[12 + k]));
@@ -376,13 +384,18 @@ __global__ __launch_bounds__(DEEP_THREADS) void deep_fused_kernel(const uint32_t
                 for (int k = 0; k < 4; k++) q[r][k] = fold64(q[r][k]);
         }
     }
+    uint32_t* outs[4] = {out0, out1, out2, out3};
 #pragma unroll
-    for (uint32_t r = 0; r < R; r++) {
-        if (!live[r]) continue;
-        out0[row[r]] = reduce64(q[r][0]);
-        out1[row[r]] = reduce64(q[r][1]);
-        out2[row[r]] = reduce64(q[r][2]);
-        out3[row[r]] = reduce64(q[r][3]);
+    for (int k = 0; k < 4; k++) {
+        uint32_t w[R];
+#pragma unroll
+        for (uint32_t r = 0; r < R; r++) w[r] = reduce64(q[r][k]);
+        if constexpr (R == 4)
+            *(u32x4_any*)(outs[k] + row) = u32x4_any{w[0], w[1], w[2], w[3]};
+        else if constexpr (R == 2)
+            *(u32x2_any*)(outs[k] + row) = u32x2_any{w[0], w[1]};
+        else
+            outs[k][row] = w[0];
     }
 }
 

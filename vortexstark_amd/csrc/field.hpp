@@ -194,7 +194,11 @@ __device__ __forceinline__ uint32_t brev_bits(uint32_t x, uint32_t bits) {
     return bits == 0 ? 0u : (__builtin_bitreverse32(x) >> (32 - bits));
 }
 
-typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(4)));  // any word address
+// Words every lane reads alike, constant while the kernel runs: scalar loads.
+typedef const __attribute__((address_space(4))) uint32_t ConstU32;
+typedef const __attribute__((address_space(4))) uint64_t ConstU64;
+typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(4)));  // any word address
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 // words i .. i + RUN - 1 of an array of len words
 template <uint32_t RUN>
 __device__ __forceinline__ void store_run(uint32_t* out, uint64_t i, uint64_t len, const uint32_t (&w)[RUN]) {

@@ -153,7 +153,6 @@ __device__ __forceinline__ QM31 quotient_at(uint32_t t0, uint32_t t1, uint32_t t
 }
 // A challenge, written by an earlier launch: the same four words for every lane,
 // so they come by scalar loads.
-typedef const __attribute__((address_space(4))) uint32_t ConstU32;
 __device__ __forceinline__ QM31 load_alpha(const uint32_t* a) {
     ConstU32* c = (ConstU32*)a;
     return {{c[0], c[1], c[2], c[3]}};

@@ -166,15 +166,18 @@ __global__ void bit_reverse_qm31_kernel(const uint32_t* in, uint32_t* out, uint6
 }
 
 // ---------------------------------------------------------------- wide commitment
-// beta^c for c < n (one thread; n is a column count)
-__global__ void beta_powers_kernel(const uint32_t* beta, uint32_t n, uint32_t* out) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    const QM31 b = load_alpha(beta);
-    QM31 acc = {{1, 0, 0, 0}};
-    for (uint32_t c = 0; c < n; c++) {
-        for (int k = 0; k < 4; k++) out[4 * c + k] = acc.v[k];
-        acc = qmul(acc, b);
+// beta^c for c < n (a column count), one thread a power by its exponent's bits:
+// the commitment waits for the chain, 12 products for 34 columns where one thread
+// making them all took 34 (10.5 -> 4 us).
+__global__ __launch_bounds__(256) void beta_powers_kernel(const uint32_t* beta, uint32_t n, uint32_t* out) {
+    const uint32_t c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= n) return;
+    QM31 sq = load_alpha(beta), acc = {{1, 0, 0, 0}};
+    for (uint32_t b = 0; (n - 1) >> b; b++) {
+        if ((c >> b) & 1) acc = qmul(acc, sq);
+        sq = qmul(sq, sq);
     }
+    for (int k = 0; k < 4; k++) out[4 * c + k] = acc.v[k];
 }
 
 }  // namespace vx
@@ -473,7 +476,7 @@ int32_t vx_wide_commit_device(vx_wide* w, const uint32_t* const* h_cols) {
     TailOut t0 = {w->roots, w->ch, w->chal, 1};
     t0.n_felts = 2;  // beta, then alpha_0
     commit_tree(SrcLifted{w->d_lift, w->n_cols}, 1ull << S, none, t0, w->scratch, s, mk);
-    beta_powers_kernel<<<1, 64, 0, s>>>(w->chal, w->n_cols, w->beta_pows);
+    beta_powers_kernel<<<ceil_div(w->n_cols, 256), 256, 0, s>>>(w->chal, w->n_cols, w->beta_pows);
     check_launch("beta_powers_kernel");
     w->mark("beta_powers");
     phase = "fri0_circle_fold_commit";
