@@ -330,23 +330,34 @@ __device__ __forceinline__ void b2s_quad_rounds(const uint32_t m[16], uint32_t m
 }
 
 // Lane l: in hl = h[l], hh = h[4+l]; out the same words of the new chaining value.
-// msg: the quad's 16 message words. All four lanes of the quad must be active.
-// Every lane reads the whole message into registers before the first round and
-// picks the words of its G functions by selects, so no LDS access waits inside
-// the dependent chain of the rounds.
-__device__ __forceinline__ void b2s_compress_quad(const uint32_t* msg, uint32_t t, uint32_t f, uint32_t& hl,
-                                                  uint32_t& hh) {
+// Every lane of the quad holds all 16 message words and picks those of its G
+// functions by selects, which issue in the shadow of the rounds' dependent chain.
+// All four lanes of the quad must be active.
+__device__ __forceinline__ void b2s_compress_quad_words(const uint32_t m[16], uint32_t t, uint32_t f, uint32_t& hl,
+                                                        uint32_t& hh) {
     const uint32_t l = threadIdx.x & 3;
     const uint32_t m0 = 0u - (l & 1u), m1 = 0u - ((l >> 1) & 1u);
-    uint32_t m[16];
-#pragma unroll
-    for (int i = 0; i < 16; i++) m[i] = msg[i];  // two words a read: 16-byte reads deliver later
     uint32_t a = hl, b = hh, c, d;
     b2s_quad_start(t, f, c, d);
     b2s_quad_rounds<0>(m, m0, m1, a, b, c, d);
     b2s_quad_finish(a, b, c, d, hl, hh);
 }
-
+// The same with the quad's message in memory, read before the first round, so no
+// LDS access waits inside the chain.
+__device__ __forceinline__ void b2s_compress_quad(const uint32_t* msg, uint32_t t, uint32_t f, uint32_t& hl,
+                                                  uint32_t& hh) {
+    uint32_t m[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) m[i] = msg[i];  // two words a read: 16-byte reads deliver later
+    b2s_compress_quad_words(m, t, f, hl, hh);
+}
+// Message words 4 j .. 4 j + 3 of a quad from word 4 j + l in lane l.
+__device__ __forceinline__ void quad_gather(uint32_t x, uint32_t m[4]) {
+    m[0] = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x00, 0xF, 0xF, true);
+    m[1] = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x55, 0xF, 0xF, true);
+    m[2] = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xAA, 0xF, 0xF, true);
+    m[3] = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xFF, 0xF, 0xF, true);
+}
 // Initial chaining words of lane l (IV with the parameter block folded in).
 __device__ __forceinline__ void b2s_quad_init(uint32_t& hl, uint32_t& hh) {
     const uint32_t l = threadIdx.x & 3;

@@ -49,7 +49,6 @@ static __global__ __launch_bounds__(FRI_TAIL_THREADS) void fri_tail_kernel(FriTa
     __shared__ uint32_t nodes[8 * W];  // wide levels, word-major
     __shared__ __align__(16) uint32_t qa[8 * TAIL_QUAD_NODES], qb[4 * TAIL_QUAD_NODES];
     __shared__ __align__(8) uint32_t val[4][W];  // the layer's values
-    __shared__ __align__(16) uint32_t msg[16];
     __shared__ uint32_t al[4];
     const uint32_t tid = threadIdx.x;
     const uint64_t boff = (uint64_t)blockIdx.y * bs;
@@ -57,7 +56,6 @@ static __global__ __launch_bounds__(FRI_TAIL_THREADS) void fri_tail_kernel(FriTa
     QuadTranscript tr = {};
     if (tid < 64) {
         tr.load(ch, false);
-        tr.put_state(msg);
         if (tid < 4) al[tid] = args.alpha0[boff + tid];
     }
     // value index of this thread in a layer of n values: a quad per value in the
@@ -126,11 +124,15 @@ static __global__ __launch_bounds__(FRI_TAIL_THREADS) void fri_tail_kernel(FriTa
             for (int c = 0; c < 4; c++) in[c] = *(const uint2*)(&val[c][2 * k]);
         }
         if (tid < 64) {  // one wave: narrow levels and transcript
-            const uint32_t* root = narrow_reduce(cur, nxt, m, lvl, idx0, st, 1u, msg + 8);
-            if (tid < 8) L.root_dst[boff + tid] = root[tid];
-            tr.mix(msg);
+            uint32_t rl, rh;
+            narrow_root(cur, nxt, m, lvl, idx0, st, rl, rh);
+            if (tid < 4) {
+                L.root_dst[boff + tid] = rl;
+                L.root_dst[boff + 4 + tid] = rh;
+            }
+            tr.mix(rl, rh);
             uint32_t w = 0;
-            if (L.alpha_dst && tr.draw(msg, w) && tid < 4) {
+            if (L.alpha_dst && tr.draw(w) && tid < 4) {
                 al[tid] = w;
                 L.alpha_dst[boff + tid] = w;
             }

@@ -134,8 +134,12 @@ __global__ __launch_bounds__(FEW ? 1024 : 256) void merkle_tile_kernel(Src src, 
     }
     block_quad_reduce(cur, nxt, n, lvl, idx0, none);
     if (tid >= 64) return;
-    const uint32_t* root = narrow_reduce(cur, nxt, n, lvl, idx0, none);
-    if (tid < 8) roots[8ull * blockIdx.x + tid] = root[tid];
+    uint32_t rl, rh;
+    narrow_root(cur, nxt, n, lvl, idx0, none, rl, rh);
+    if (tid < 4) {
+        roots[8ull * blockIdx.x + tid] = rl;
+        roots[8ull * blockIdx.x + 4 + tid] = rh;
+    }
 }
 
 __global__ void hash_nodes_kernel(const uint32_t* ch, uint32_t* par, uint32_t n) {

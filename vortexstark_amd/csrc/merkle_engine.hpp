@@ -455,21 +455,15 @@ struct SrcWideFold {
 
 // ---------------------------------------------------------------- narrow levels
 // Reduces n (a power of two <= 64) nodes stored node-major ([node][8 words]) in
-// the LDS buffer `a` to `stop` nodes (a power of two, default one) with the
-// quads of the calling wave, ping-ponging with `b`; a single last node goes to
-// `root` instead when that is given. The buffers are 16-byte aligned. The nodes
+// the LDS buffer `a` to `stop` nodes (a power of two) with the quads of the
+// calling wave, ping-ponging with `b`. The buffers are 16-byte aligned. The nodes
 // are at tree level `lvl`, node 0 having index idx0 there. Every lane of the
 // wave must call this; returns the buffer holding the remaining nodes.
 // A level is a lone wave's instruction count, so what does not change from
 // level to level (and the level store's addresses) stays out of it.
 __device__ __forceinline__ uint32_t* narrow_reduce(uint32_t* a, uint32_t* b, uint32_t n, uint32_t lvl, uint64_t idx0,
-                                                   const LevelStore& st, uint32_t stop = 1, uint32_t* root = nullptr) {
+                                                   const LevelStore& st, uint32_t stop) {
     const uint32_t lane = threadIdx.x & 63, quad = lane >> 2, l = lane & 3;
-    if (root && n == 1) {
-        if (lane < 8) root[lane] = a[lane];
-        VX_WAVE_SYNC();
-        return root;
-    }
     n = __builtin_amdgcn_readfirstlane(n);
     lvl = __builtin_amdgcn_readfirstlane(lvl);
     uint32_t h0, h1;
@@ -479,7 +473,6 @@ __device__ __forceinline__ uint32_t* narrow_reduce(uint32_t* a, uint32_t* b, uin
     uint32_t* dst = store ? st.at(lvl + 1, idx0 >> 1) + 8 * quad + l : nullptr;
     while (n > stop) {
         const uint32_t half = n / 2;
-        uint32_t* out = root && half == 1 ? root : b;
         const bool want = store && lvl + 1 >= st.from && lvl + 1 <= st.depth;
         for (uint32_t q0 = 0; q0 < half; q0 += 16) {
             const uint32_t q = q0 + quad;
@@ -487,8 +480,8 @@ __device__ __forceinline__ uint32_t* narrow_reduce(uint32_t* a, uint32_t* b, uin
             uint32_t hl = h0, hh = h1;
             b2s_compress_quad(a + 16 * qq, 64u, 0xFFFFFFFFu, hl, hh);
             if (q < half) {
-                out[8 * q + l] = hl;
-                out[8 * q + 4 + l] = hh;
+                b[8 * q + l] = hl;
+                b[8 * q + 4 + l] = hh;
                 if (want) {
                     dst[8 * q0] = hl;
                     dst[8 * q0 + 4] = hh;
@@ -499,11 +492,42 @@ __device__ __forceinline__ uint32_t* narrow_reduce(uint32_t* a, uint32_t* b, uin
         lvl++;
         idx0 >>= 1;
         if (store) dst = st.at(lvl + 1, idx0 >> 1) + 8 * quad + l;
-        b = a;
-        a = out;
+        uint32_t* t = a;
+        a = b;
+        b = t;
         n = half;
     }
     return a;
+}
+
+// The root of n (a power of two <= 64) such nodes: words l and 4 + l in rl, rh of
+// lane l of every quad. The last level stays in registers, where the transcript
+// hashes it. (Handing every level on in registers, a swap of lanes and sixteen
+// DPP moves a level, takes 805 ns a level where this exchange takes 770: the moves
+// stand before the rounds' chain, about 680 by itself, as the LDS trip does.)
+__device__ __forceinline__ void narrow_root(uint32_t* a, uint32_t* b, uint32_t n, uint32_t lvl, uint64_t idx0,
+                                            const LevelStore& st, uint32_t& rl, uint32_t& rh) {
+    const uint32_t lane = threadIdx.x & 63, l = lane & 3;
+    n = __builtin_amdgcn_readfirstlane(n);
+    lvl = __builtin_amdgcn_readfirstlane(lvl);
+    if (n == 1) {
+        rl = a[l];
+        rh = a[4 + l];
+        return;
+    }
+    if (n > 2) {
+        const uint32_t down = 30 - __builtin_clz(n);
+        a = narrow_reduce(a, b, n, lvl, idx0, st, 2);
+        lvl += down;
+        idx0 >>= down;
+    }
+    b2s_quad_init(rl, rh);
+    b2s_compress_quad(a, 64u, 0xFFFFFFFFu, rl, rh);
+    if (st.want(lvl + 1) && lane < 4) {
+        uint32_t* dst = st.at(lvl + 1, idx0 >> 1);
+        dst[l] = rl;
+        dst[4 + l] = rh;
+    }
 }
 
 // One level of a block: the half = n / 2 parents (at most THREADS / 4, and a
@@ -543,9 +567,8 @@ __device__ __forceinline__ void block_quad_reduce(uint32_t*& a, uint32_t*& b, ui
     }
 }
 
-// The transcript while a wave holds it: lane l of every quad has state words l
-// and 4 + l (channel.rs:15-25). msg (16 LDS words) is the hash input: its first
-// half holds the state, its second takes the root to mix.
+// The transcript while a wave holds it, in registers: lane l of every quad has
+// state words l and 4 + l (channel.rs:15-25).
 struct QuadTranscript {
     uint32_t sl, sh, n_draws, failed;
     __device__ __forceinline__ void load(const DevChannel* ch, bool init) {
@@ -555,35 +578,33 @@ struct QuadTranscript {
         failed = init ? 0u : ch->failed;
         n_draws = 0;
     }
-    __device__ __forceinline__ void put_state(uint32_t* msg) const {
-        const uint32_t lane = threadIdx.x & 63, l = lane & 3;
-        if (lane < 4) {
-            msg[l] = sl;
-            msg[4 + l] = sh;
-        }
+    // H(state || second half) with t bytes counted
+    __device__ __forceinline__ void hash(uint32_t xl, uint32_t xh, uint32_t t, uint32_t& hl, uint32_t& hh) const {
+        uint32_t m[16];
+        quad_gather(sl, m);
+        quad_gather(sh, m + 4);
+        quad_gather(xl, m + 8);
+        quad_gather(xh, m + 12);
+        b2s_quad_init(hl, hh);
+        b2s_compress_quad_words(m, t, 0xFFFFFFFFu, hl, hh);
     }
-    // mix_digest (channel.rs:30-39): msg holds state || root
-    __device__ __forceinline__ void mix(uint32_t* msg) {
-        VX_WAVE_SYNC();
-        b2s_quad_init(sl, sh);
-        b2s_compress_quad(msg, 64u, 0xFFFFFFFFu, sl, sh);
-        VX_WAVE_SYNC();
-        put_state(msg);
+    // mix_digest (channel.rs:30-39) of the root words of lane l
+    __device__ __forceinline__ void mix(uint32_t rl, uint32_t rh) {
+        uint32_t nl, nh;
+        hash(rl, rh, 64u, nl, nh);
+        sl = nl;
+        sh = nh;
         n_draws = 0;
     }
-    // draw_felt (channel.rs:67-86); lane l of every quad gets word l. msg holds
-    // the state. False when the retry budget is exhausted.
-    __device__ __forceinline__ bool draw(uint32_t* msg, uint32_t& w) {
-        const uint32_t lane = threadIdx.x & 63;
+    // draw_felt (channel.rs:67-86); lane l gets word l. False when the retry
+    // budget is exhausted.
+    __device__ __forceinline__ bool draw(uint32_t& w) {
+        const uint32_t l = threadIdx.x & 3;
         for (int tries = 0; tries < 64; tries++) {
-            if (lane < 8) msg[8 + lane] = lane == 0 ? n_draws : 0u;
-            VX_WAVE_SYNC();
             uint32_t wl, wh;
-            b2s_quad_init(wl, wh);
-            b2s_compress_quad(msg, 37u, 0xFFFFFFFFu, wl, wh);
+            hash(l == 0 ? n_draws : 0u, 0u, 37u, wl, wh);
             n_draws++;
             const uint64_t ok = __ballot(wl < 2u * P && wh < 2u * P);
-            VX_WAVE_SYNC();
             if ((ok & 0xFull) == 0xFull) {
                 w = canon(wl);
                 return true;
@@ -739,13 +760,20 @@ __global__ __launch_bounds__(64 * LEAF_QUAD_WAVES) void leaf_quad_stage_kernel(S
         na[8 * k + 4 + l] = hh;
     }
     VX_WAVE_SYNC();
-    const uint32_t* top = narrow_reduce(na, nb, LPW, 0, base, st);
-    if (lane < 8) tops[8 * w + lane] = top[lane];
+    uint32_t rl, rh;
+    narrow_root(na, nb, LPW, 0, base, st, rl, rh);
+    if (lane < 4) {
+        tops[8 * w + lane] = rl;
+        tops[8 * w + 4 + lane] = rh;
+    }
     lds_barrier();
     if (w) return;
     constexpr uint32_t LOG = R == 1 ? 4 : R == 2 ? 5 : 6;
-    top = narrow_reduce(tops, tops2, LEAF_QUAD_WAVES, LOG, (uint64_t)blockIdx.x * LEAF_QUAD_WAVES, st);
-    if (lane < 8) out_nodes[8ull * blockIdx.x + lane] = top[lane];
+    narrow_root(tops, tops2, LEAF_QUAD_WAVES, LOG, (uint64_t)blockIdx.x * LEAF_QUAD_WAVES, st, rl, rh);
+    if (lane < 4) {
+        out_nodes[8ull * blockIdx.x + lane] = rl;
+        out_nodes[8ull * blockIdx.x + 4 + lane] = rh;
+    }
 }
 
 // ---------------------------------------------------------------- tail kernel
@@ -829,7 +857,6 @@ __global__ __launch_bounds__(TAIL_THREADS) void merkle_tail_kernel(Src src0, uin
     }
     __shared__ uint32_t nodes[8 * W];
     __shared__ __align__(16) uint32_t qa[8 * TAIL_QUAD_NODES], qb[4 * TAIL_QUAD_NODES];
-    __shared__ __align__(16) uint32_t msg[16];
     const uint32_t tid = threadIdx.x;
     const uint64_t item_base = (uint64_t)blockIdx.x * n_items;
     QuadTranscript tr = {};
@@ -860,14 +887,17 @@ __global__ __launch_bounds__(TAIL_THREADS) void merkle_tail_kernel(Src src0, uin
     uint32_t *cur = qa, *nxt = qb;
     block_quad_reduce(cur, nxt, n, lvl, idx0, st);
     if (tid >= 64) return;  // one wave finishes: narrow levels and transcript
-    if (out.channel) tr.put_state(msg);
-    const uint32_t* root = narrow_reduce(cur, nxt, n, lvl, idx0, st, 1u, msg + 8);
-    if (out.root_dst && tid < 8) out.root_dst[8ull * blockIdx.x + tid] = root[tid];
+    uint32_t rl, rh;
+    narrow_root(cur, nxt, n, lvl, idx0, st, rl, rh);
+    if (out.root_dst && tid < 4) {
+        out.root_dst[8ull * blockIdx.x + tid] = rl;
+        out.root_dst[8ull * blockIdx.x + 4 + tid] = rh;
+    }
     if (!out.channel) return;
-    tr.mix(msg);
+    tr.mix(rl, rh);
     for (uint32_t k = 0; out.alpha_dst && k < out.n_felts; k++) {
         uint32_t w = 0;
-        if (!tr.draw(msg, w)) break;
+        if (!tr.draw(w)) break;
         if (tid < 4) out.alpha_dst[4 * k + tid] = w;
     }
     tr.store(out.channel);
