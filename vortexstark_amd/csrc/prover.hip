@@ -343,15 +343,18 @@ __global__ void proofs_to_host_kernel(const uint32_t* src, uint64_t R, uint64_t 
     __threadfence_system();
 }
 
-// Bound by the link (a 100 KB proof: about 5 us) and its own launch, where a copy
-// into pageable memory took 40 us an array.
+// Bound by the link and its own launch (a proof of 2^10 rows: 10 us; 15 us by words
+// and with a system fence in every thread, which the end of the kernel makes
+// anyway), where a copy into pageable memory took 40 us an array.
 __global__ void fetch_kernel(Fetch f, uint32_t* dst) {
     const uint64_t nth = (uint64_t)gridDim.x * blockDim.x, tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     for (uint32_t k = 0; k < f.n; k++) {
-        for (uint64_t i = tid; i < f.words[k]; i += nth) dst[i] = f.src[k][i];
-        dst += f.words[k];
+        const uint32_t* src = f.src[k];
+        const uint64_t n = f.words[k], v = (((uintptr_t)src | (uintptr_t)dst) & 15) ? 0 : n / 4;
+        for (uint64_t i = tid; i < v; i += nth) ((uint4*)dst)[i] = ((const uint4*)src)[i];
+        for (uint64_t i = 4 * v + tid; i < n; i += nth) dst[i] = src[i];
+        dst += n;
     }
-    __threadfence_system();
 }
 bool fetch_to_host(const Fetch& f, uint32_t* pinned, hipStream_t s) {
     const uint32_t blocks = (uint32_t)std::min<uint64_t>(P2H_BLOCKS, f.total / 1024 + 1);
