@@ -13,20 +13,22 @@
 // other two. About 840 VALU ops a nonce remain, against 968 for a full
 // compression.
 //
-// The grid is persistent: one workgroup of 256 per CU, so one wave per SIMD,
+// The grid is persistent: two workgroups of 256 per CU, so two waves per SIMD,
 // each lane hashing NONCES_PER_LANE nonces a pass. Nonces are dealt
-// wave-contiguously: pass k gives wave w the 256 nonces start + k * stride +
-// 256 * w + [0, 256). Before each pass a wave reads the current best nonce and
+// wave-contiguously: pass k gives wave w the 128 nonces start + k * stride +
+// 128 * w + [0, 128). Before each pass a wave reads the current best nonce and
 // stops once its next nonce is not below it, so the final value is the
 // smallest valid nonce of [start, start + count) (or what result already held,
 // if smaller), whatever order the waves ran in: the reference returns the
 // first nonce any thread found, a valid one but not always the smallest.
-// Why one wave per SIMD: with several, the SIMD issues for its oldest wave
-// first, the waves stop advancing evenly, and once a valid nonce is found the
-// lagging waves still have to cover every nonce below it: a 26-bit search then
-// hashed 1.4x (2 waves per SIMD) to 2.8x (8 waves) the nonces it needed, for a
-// few percent more issue rate; one wave with four nonces per lane hashes within
-// 1 % of the nonces needed at 96 % of the VALU issue rate (measured on MI355X).
+// Why two waves per SIMD: a second one's xors and adds issue beside the first one's
+// rotations, by the compression's priorities, and as both run the same rows in
+// turn they advance together; a SIMD left to its oldest wave first would let
+// laggards cover every nonce below a find long after it (without the priorities two
+// waves hashed 1.4x the nonces needed). 26 bits: 1.75 ms at one wave without
+// priorities, 2.04 with them (a lone wave only waits for its own), 1.30 at two,
+// 1.51 at four. Two nonces a lane: four take as long at 26 bits, but a pass of them
+// is 2^19 nonces (16 bits: 18 us at two, 27 at four); one polls too often (2.4 ms).
 #include <atomic>
 
 #include "blake2s.hpp"
@@ -38,8 +40,8 @@ namespace vx {
 namespace {
 
 constexpr uint32_t GRIND_THREADS = 256;
-constexpr uint32_t GRIND_BLOCKS_PER_CU = 1;
-constexpr uint32_t NONCES_PER_LANE = 4;
+constexpr uint32_t GRIND_BLOCKS_PER_CU = 2;
+constexpr uint32_t NONCES_PER_LANE = 2;
 constexpr uint32_t NONCES_PER_BLOCK = GRIND_THREADS * NONCES_PER_LANE;
 constexpr uint32_t POW_PREFIX = 0x12345678u;  // Blake2sChannel POW_PREFIX (grind_ops.rs:24)
 
