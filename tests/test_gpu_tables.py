@@ -1,4 +1,4 @@
-"""Tile roots on both sides of the two switches of the work per tile, fold-twiddle
+"""Tile roots and node levels on both sides of the switches of the work per tile, fold-twiddle
 sources and traces at run and block edges, batch inverses of every words-per-thread count:
 against the oracle. Runs on the MI355X."""
 
@@ -101,4 +101,17 @@ def test_fibonacci_trace(vx, log_n, a, b):
     got = out.to_host()
     assert got[0] == 7 and got[n + 1] == 7
     assert np.array_equal(got[1: n + 1], O.fibonacci_trace(a, b, log_n))
+    vx.check()
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 63, 65, 1 << 14, (1 << 14) + 1, 1 << 16, (1 << 16) + 5])
+def test_hash_nodes(vx, n):
+    ch = np.random.default_rng(n).integers(0, 1 << 32, 16 * n, dtype=np.uint64).astype(np.uint32)
+    src, dst = vx.DeviceBuffer.from_host(ch), vx.DeviceBuffer.from_host(np.full(8 * n + 1, 7, np.uint32))
+    vx.lib.cuda_merkle_hash_nodes(src.ptr, dst.ptr, n)
+    vx.synchronize()
+    exp = np.zeros(8 * n, np.uint32)
+    O.lib().orc_merkle_node_layer(ch.ctypes.data, n, exp.ctypes.data)
+    got = dst.to_host()
+    assert np.array_equal(got[:-1], exp) and got[-1] == 7
     vx.check()
