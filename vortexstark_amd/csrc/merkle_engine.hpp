@@ -326,7 +326,7 @@ struct SrcLifted {
     }
     // One block's loads at a time: holding the next block's 32 words as well
     // (to have them in flight while this one is hashed) costs 146 VGPRs, three
-    // waves a SIMD; without them seven waves share it and cover each other's
+    // waves a SIMD; without them four waves share it (98) and cover each other's
     // loads, and the hashing itself pairs better (34 columns, 2^22 leaves:
     // 368 -> 306 us).
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {

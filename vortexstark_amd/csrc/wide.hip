@@ -217,7 +217,7 @@ struct vx_wide {
     uint32_t* chal = nullptr;       // [beta, alpha_0, alpha_1, ...], 4 words each
     uint32_t* beta_pows = nullptr;  // 4 words per column
     uint32_t* roots = nullptr;      // lifted root, then J FRI roots
-    uint32_t* h_results = nullptr;  // pinned: the results on their way to the caller
+    uint32_t* h_results = nullptr;  // behind them: the results on their way to the caller
     std::mutex fetch_mu;            // held while they pass through it
     Timeline tl;
     void mark(const std::string& l) { tl.mark(l, stream); }
@@ -237,7 +237,6 @@ struct vx_wide {
         if (fork) (void)hipEventDestroy(fork);
         for (void* p : allocs) (void)hipFree(p);
         if (h_src_ptrs) (void)hipHostFree((void*)h_src_ptrs);
-        if (h_results) (void)hipHostFree(h_results);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
@@ -382,9 +381,11 @@ vx_wide* vx_wide_create(uint32_t n_cols, const uint32_t* log_sizes, uint32_t log
     }
     ok = ok && w->alloc((void**)&w->lde, 4 * total) && w->alloc((void**)&w->d_lde_ptrs, 8ull * n_cols) &&
          w->alloc((void**)&w->d_src_ptrs, 8ull * n_cols) && w->alloc((void**)&w->d_lift, sizeof(LiftCol) * n_cols);
-    ok = ok && check(hipHostMalloc((void**)&w->h_src_ptrs, 8ull * n_cols), "hipHostMalloc") &&
-         check(hipHostMalloc((void**)&w->h_results, 4 * (8 + 8ull * w->J + 4 + 4 * w->layer_size(w->J - 1) + 1)),
-               "hipHostMalloc");
+    // one pinned block: the column pointers, then the results
+    ok = ok && check(hipHostMalloc((void**)&w->h_src_ptrs,
+                                   8ull * n_cols + 4 * (8 + 8ull * w->J + 4 + 4 * w->layer_size(w->J - 1) + 1)),
+                     "hipHostMalloc");
+    if (ok) w->h_results = (uint32_t*)(w->h_src_ptrs + n_cols);
     w->layer.assign(w->J, nullptr);
     for (uint32_t j = 0; ok && j < w->J; j++) ok = w->alloc((void**)&w->layer[j], 16 * w->layer_size(j));
     ok = ok && w->alloc((void**)&w->scratch.a, 32 * scratch_nodes_a(1ull << S)) &&
