@@ -11,7 +11,7 @@
 // stay in LDS for the next fold, the next twiddles are fetched while a layer
 // is hashed, and the transcript's state stays in the registers of one wave
 // (device memory gets all of them, but nothing is read back from it). Leaves
-// of layers of at most 128 values are hashed a quad each (0.68 us for up to
+// of layers of at most 128 values are hashed a quad each (0.7 us for up to
 // 64), larger ones a lane each (1.7 us at one wave a SIMD). A 2048-value layer
 // is left to a stage launch and a tree tail: its 4095 compressions in one
 // workgroup are bound by one CU's issue rate.
