@@ -1,4 +1,4 @@
-// The default split of blowup-4 evaluations: every size is covered by passes that
+// The splits of sizes without a plan, general and blowup-4 evaluations: every size is covered by passes that
 // have a kernel, and only the top one replicates.
 #include <stdio.h>
 #include <stdlib.h>
@@ -20,6 +20,10 @@ int main() {
         for (const Pass& p : ps) CHECK(pass_rows(p) + p.c <= NTT_LOW_MAX);
         CHECK(ps.size() == (k == 0 ? 0 : k <= 12 ? 1 : k <= 24 ? 2 : 3));
         if (k > 12) CHECK(ps[0].m == std::min(12u, k - 3));
+        const std::vector<Pass> us = untuned_plan(k);
+        CHECK(plan_valid(k, us));
+        if (k <= 23) CHECK(us.size() == (k == 0 ? 0 : k <= 12 ? 1 : 2));
+        for (const Pass& p : us) CHECK(p.m + p.c <= NTT_LOW_MAX);
     }
     printf("lde plans: ok\n");
     return 0;

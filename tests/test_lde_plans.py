@@ -1,10 +1,13 @@
-"""Default splits of blowup-4 evaluations: the rule on the CPU; proofs at the sizes
+"""Splits of sizes without a plan: the rules on the CPU; transforms on both sides of
+the general one's line; proofs at the sizes
 where the number of passes or their segments change, with the general table and
 back, against the oracle."""
 
+import ctypes as C
 import os
 import subprocess
 
+import numpy as np
 import pytest
 
 import oracle_lib as O
@@ -17,6 +20,29 @@ def test_rule(tmp_path):
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror",
                     os.path.join(HERE, "host", "lde_plan_test.cpp"), "-o", str(exe)], check=True)
     assert "lde plans: ok" in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k", [19, 20, 21, 22, 23])
+def test_transforms_without_a_plan(vx, k):
+    """A batch of two columns forward against the oracle, and back."""
+    n = 1 << k
+    vx.lib.vx_ntt_plan_reset()
+    line, circle, iline, icircle, offs, sizes = O.ntt_twiddles(1, k)
+    cols = [np.random.default_rng(10 * k + c).integers(0, (1 << 31) - 1, n, dtype=np.uint32) for c in range(2)]
+    tabs = [vx.DeviceBuffer.from_host(a) for a in (line, circle, iline, icircle)]
+    bufs = [vx.DeviceBuffer.from_host(c) for c in cols]
+    ptrs = vx.DeviceBuffer.from_host(np.array([b.addr for b in bufs], np.uint64).view(np.uint32))
+    ho, hs = ((C.c_uint32 * (k - 1))(*[int(v) for v in a[: k - 1]]) for a in (offs, sizes))
+    vx.lib.cuda_circle_ntt_evaluate_batch(ptrs.ptr, tabs[0].ptr, tabs[1].ptr, ho, hs, k - 1, n, 2)
+    for b, c in zip(bufs, cols):
+        exp = c.copy()
+        O.lib().orc_ntt_evaluate(exp.ctypes.data, line.ctypes.data, circle.ctypes.data, k)
+        assert np.array_equal(b.to_host(), exp)
+    vx.lib.cuda_circle_ntt_interpolate_batch(ptrs.ptr, tabs[2].ptr, tabs[3].ptr, ho, hs, k - 1, n, 2)
+    for b, c in zip(bufs, cols):
+        assert np.array_equal(b.to_host(), c)
+    vx.check()
 
 
 @pytest.mark.gpu

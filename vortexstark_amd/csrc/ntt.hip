@@ -620,7 +620,7 @@ static std::vector<Pass> plan_passes(uint32_t k) {
         std::lock_guard<std::mutex> g(g_plan_mu);
         if (k < 32 && !g_plan[k].empty()) return g_plan[k];
     }
-    return default_plan(k);
+    return untuned_plan(k);
 }
 static std::vector<Pass> lde_plan_passes(uint32_t k) {
     {

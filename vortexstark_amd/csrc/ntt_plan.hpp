@@ -51,6 +51,17 @@ inline std::vector<Pass> default_plan(uint32_t k) {
     return ps;
 }
 
+// The split of a transform of 2^k points that no plan was set or tuned for: the
+// default's, except from 2^20 to 2^23 points, where two passes of larger tiles move
+// the array once less than its three (2^21: 34.9 -> 31.2 us, 2^22 45.6 -> 40.4, 2^23
+// 61.0 -> 57.6, launch and synchronisation included; nine columns of 2^20 80.3 ->
+// 64.5; at 2^24 the two passes need 2^10 rows of 64 bytes and lose, 97.9 -> 104).
+inline std::vector<Pass> untuned_plan(uint32_t k) {
+    if (k < 20 || k > 23) return default_plan(k);
+    const uint32_t m0 = std::min(NTT_LOW_MAX, k - 8);
+    return {{0, m0, 0}, {m0, k - m0, NTT_COLS}};
+}
+
 // The default split of a blowup-4 evaluation of 2^k points: one pass while a tile
 // holds it; then, and to 2^24 points, two, the upper one replicating (and so the
 // bridge from the interpolation), which beats every three-pass split: the whole
