@@ -24,6 +24,7 @@
 #include "common.hpp"
 #include "kernels.hpp"
 #include "ntt_plan.hpp"
+#include "table_plan.hpp"
 
 namespace vx {
 
@@ -888,9 +889,6 @@ __global__ void coset_points_kernel(CPt initial, CPt step, uint32_t* ox, uint32_
 // one inversion, in registers, where they took two more passes. 2^19 sources: 18
 // -> 6 us; the 14 layers of a 2^18-point domain with their inverses: 6.6 us, where
 // each layer took two launches of 4 to 17.
-constexpr uint32_t TABLE_THREADS = 256;
-constexpr uint32_t TABLE_RUN_LOG = 4;   // with inverses, and in the NTT tables
-constexpr uint32_t SOURCE_RUN_LOG = 2;  // sources alone: a shorter chain
 
 // w[r] -> 1 / w[r]; a zero stays zero
 template <uint32_t RUN>
@@ -914,8 +912,7 @@ __device__ __forceinline__ void invert_run(uint32_t (&w)[RUN]) {
 template <uint32_t RUN_LOG>
 __device__ __forceinline__ CPt run_start(CPt start, const CPt* pts, uint32_t blk) {
     CPt p = start;
-    constexpr uint32_t TB = 8;
-    static_assert(TABLE_THREADS == 1u << TB);
+    constexpr uint32_t TB = TABLE_THREADS_LOG;
     for (uint32_t b = RUN_LOG + TB; blk; b++, blk >>= 1)
         if (blk & 1) p = cpmul(p, pts[b]);
 #pragma unroll
@@ -982,7 +979,7 @@ __global__ void squash_kernel(const uint32_t* in, uint32_t* tw_out, uint32_t* sq
 // each thread 16 consecutive words of one, inverted in registers where
 // the transform wants the inverses.
 struct NttTableArgs {
-    CPt sq[64];               // step^(2^b)
+    CPt sq[NTT_TABLE_SQUARES];  // step^(2^b)
     CPt base[32];             // per line layer; the circle layer comes last
     uint32_t offs[32];
     uint32_t first_block[33];
@@ -997,7 +994,7 @@ __global__ __launch_bounds__(TABLE_THREADS) void ntt_tables_kernel(NttTableArgs 
     while (blockIdx.x >= m.first_block[l + 1]) l++;
     const uint32_t blk = blockIdx.x - m.first_block[l];
     const bool circle = l == m.n_line;
-    const uint32_t shift = circle ? 0u : 2 * l + 1;
+    const uint32_t shift = circle ? 0u : line_layer_shift(l);
     const uint64_t len = (1ull << m.log_n) >> (circle ? 1 : l + 1);
     const uint64_t i = ((uint64_t)blk * TABLE_THREADS + threadIdx.x) * RUN;
     // word n - 2 of the n - 1 word layout belongs to no layer; it is zero
@@ -1089,7 +1086,7 @@ void build_ntt_tables(HostPt initial, HostPt step, uint32_t log_n, uint32_t* lin
     if (n < 2) return;
     m.base[m.n_line] = cpt(initial);
     m.first_block[m.n_line + 1] = m.first_block[m.n_line] + table_blocks(n / 2, TABLE_RUN_LOG);
-    for (uint32_t k = 0; k < 64; k++, step = host_pmul(step, step)) m.sq[k] = cpt(step);
+    for (uint32_t k = 0; k < NTT_TABLE_SQUARES; k++, step = host_pmul(step, step)) m.sq[k] = cpt(step);
     if (inverse)
         ntt_tables_kernel<true><<<m.first_block[m.n_line + 1], TABLE_THREADS, 0, s>>>(m);
     else
