@@ -27,6 +27,7 @@
 #include "commit.hpp"
 #include "fri_tail.hpp"
 #include "merkle_engine.hpp"
+#include "trace_plan.hpp"
 
 namespace vx {
 
@@ -38,20 +39,6 @@ namespace vx {
 // number (a block's bits scalar) and then only adds. Latency-bound to 2^18 words:
 // 3-4 us, where a matrix power and 256 words a thread took 14 us at 2^10 and 38 at
 // 2^16; 2^24 words are bound by the stores.
-constexpr uint32_t FIB_RUN_LOG = 4, FIB_THREADS_LOG = 8;
-struct FibSteps {
-    uint32_t f[32][2] = {};  // (F(2^b - 1), F(2^b)) mod p
-    constexpr FibSteps() {
-        uint64_t x = 0, y = 1;
-        for (int b = 0; b < 32; b++) {
-            f[b][0] = (uint32_t)x;
-            f[b][1] = (uint32_t)y;
-            const uint64_t x2 = (x * x % P + y * y % P) % P, y2 = y * ((2 * x + y) % P) % P;
-            x = x2;
-            y = y2;
-        }
-    }
-};
 __device__ __forceinline__ void fib_step(uint32_t& f0, uint32_t& f1, uint32_t x, uint32_t y) {
     const uint32_t z = madd(x, y);
     const uint32_t g0 = reduce64((uint64_t)x * f0 + (uint64_t)y * f1);
@@ -62,14 +49,14 @@ __global__ __launch_bounds__(1 << FIB_THREADS_LOG) void fib_trace_kernel(const u
                                                                         uint64_t n, uint32_t* out, uint64_t bs) {
     static constexpr FibSteps steps;
     constexpr uint32_t RUN = 1u << FIB_RUN_LOG;
-    const uint64_t i = (((uint64_t)blockIdx.x << FIB_THREADS_LOG) + threadIdx.x) << FIB_RUN_LOG;
+    uint64_t blk = ((uint64_t)blockIdx.z << FIB_GRID_LOG) + blockIdx.x;
+    const uint64_t i = ((blk << FIB_THREADS_LOG) + threadIdx.x) << FIB_RUN_LOG;
     if (i >= n) return;
     if (ab) {
         a = ab[2 * blockIdx.y];
         b = ab[2 * blockIdx.y + 1];
     }
     uint32_t f0 = reduce64(a), f1 = reduce64(b);
-    uint32_t blk = blockIdx.x;
     for (uint32_t k = FIB_RUN_LOG + FIB_THREADS_LOG; blk; k++, blk >>= 1)
         if (blk & 1) fib_step(f0, f1, steps.f[k][0], steps.f[k][1]);
 #pragma unroll
@@ -87,7 +74,6 @@ __global__ __launch_bounds__(1 << FIB_THREADS_LOG) void fib_trace_kernel(const u
     }
     store_run(out + blockIdx.y * bs, i, n, w);
 }
-inline uint32_t fib_blocks(uint64_t n) { return (uint32_t)ceil_div(((n - 1) >> FIB_RUN_LOG) + 1, 1u << FIB_THREADS_LOG); }
 
 // ---------------------------------------------------------------- queries
 // Last layer into the proof, mix_felts(last layer), then n_q draw_number(E)
@@ -1036,7 +1022,8 @@ int32_t vx_prove_fibonacci_batch(vx_prover* p, const uint32_t* h_ab, uint32_t co
     std::vector<const uint32_t*> slots(count);
     for (uint32_t i = 0; i < count; i++) slots[i] = p->arena + (uint64_t)i * p->R + p->o_trace;
     if (!upload_call(p, slots.data(), h_ab, count)) return -1;
-    fib_trace_kernel<<<dim3(fib_blocks(p->N), count), 1 << FIB_THREADS_LOG, 0, p->stream>>>(
+    const FibGrid g = fib_grid(p->N);
+    fib_trace_kernel<<<dim3(g.x, count, g.z), 1 << FIB_THREADS_LOG, 0, p->stream>>>(
         p->ab_dev(), 0, 0, p->N, p->arena + p->o_trace, p->R);
     if (!check_launch("fib_trace_kernel")) return -1;
     return run_batch(p, count);
@@ -1195,7 +1182,8 @@ float vx_prover_timeline_ms(vx_prover* p, uint32_t i) { return p ? p->tl.ms(i) :
 
 int32_t vx_fibonacci_trace(uint32_t a, uint32_t b, uint32_t log_n, uint32_t* d_out, void* stream) {
     uint64_t n = 1ull << log_n;
-    fib_trace_kernel<<<fib_blocks(n), 1 << FIB_THREADS_LOG, 0, (hipStream_t)stream>>>(nullptr, a, b, n, d_out, 0);
+    const FibGrid g = fib_grid(n);
+    fib_trace_kernel<<<dim3(g.x, 1, g.z), 1 << FIB_THREADS_LOG, 0, (hipStream_t)stream>>>(nullptr, a, b, n, d_out, 0);
     return check_launch("vx_fibonacci_trace") ? 0 : -1;
 }
 
