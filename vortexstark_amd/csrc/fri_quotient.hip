@@ -121,7 +121,7 @@ __global__ __launch_bounds__(256) void quotient_kernel(const uint32_t* __restric
                                                   mmul(alpha.v[c], d[2]), mmul(alpha.v[c], d[3]));
         return;
     }
-    for (uint32_t l = li; l < chunk_n && l < li + (VEC ? 4 : 1); l++) {
+    for (uint32_t l = li; l < chunk_n && l - li < (VEC ? 4u : 1u); l++) {  // li + 4 may pass 2^32
         const uint32_t i = offset + l;
         // one step at a time, so that every n >= 1 wraps as the reference's remainders do
         const uint32_t i1 = i + 1 == n ? 0u : i + 1, i2 = i1 + 1 == n ? 0u : i1 + 1;
