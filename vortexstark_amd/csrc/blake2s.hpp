@@ -24,7 +24,8 @@
 // priorities 55.8 / 58.0 / 66.1 / 69.9 G/s at 2 / 3 / 4 / 8 waves a SIMD, and
 // with two compressions interleaved 59.7 / 60.1 / 68.9 / 69.6 G/s. A lone wave
 // a SIMD has nothing to pair with and pays for the s_setprio instructions
-// (1.64 -> 2.15 us a compression): PRIO = false.
+// (1.64 -> 2.15 us a compression): PRIO = false, for launches of at most
+// LONE_THREADS threads.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -37,6 +38,8 @@ constexpr uint32_t B2S_IV0 = 0x6A09E667u, B2S_IV1 = 0xBB67AE85u, B2S_IV2 = 0x3C6
 constexpr uint32_t B2S_IV4 = 0x510E527Fu, B2S_IV5 = 0x9B05688Cu, B2S_IV6 = 0x1F83D9ABu, B2S_IV7 = 0x5BE0CD19u;
 // Parameter block word 0: digest length 32, key length 0, fanout 1, depth 1.
 constexpr uint32_t B2S_H0 = B2S_IV0 ^ 0x01010020u;
+
+constexpr uint32_t LONE_THREADS = 1u << 16;  // one wave for each SIMD of 256 CUs
 
 struct Digest {
     uint32_t w[8];
@@ -194,7 +197,7 @@ __device__ __forceinline__ void b2s_node(const uint32_t l[8], const uint32_t r[8
 // Leaves of N words each (N <= 4), K at once: K = 1, or both leaves of a pair
 // with their rounds interleaved (two compressions' rows side by side keep more
 // instructions between dependent ones; see the figures above).
-template <int K, int N>
+template <int K, int N, bool PRIO = true>
 __device__ __forceinline__ void b2s_leaves(const uint32_t w[K][N], uint32_t out[K][8]) {
     uint32_t m[K][16];
 #pragma unroll
@@ -203,7 +206,7 @@ __device__ __forceinline__ void b2s_leaves(const uint32_t w[K][N], uint32_t out[
         for (int i = 0; i < 16; i++) m[k][i] = i < N ? w[k][i < N ? i : 0] : 0u;
         b2s_init(out[k]);
     }
-    b2s_compress_n<K, N>(out, m, 4u * N, 0xFFFFFFFFu);
+    b2s_compress_n<K, N, PRIO>(out, m, 4u * N, 0xFFFFFFFFu);
 }
 
 // Leaf of one M31 word (single-column trace tree, t = 4).
@@ -225,11 +228,23 @@ __device__ __forceinline__ void b2s_leaf4(uint32_t a, uint32_t b, uint32_t c, ui
 }
 
 // Parent of two leaves of N words.
-template <int N>
+template <int N, bool PRIO = true>
 __device__ __forceinline__ void b2s_leaf_pair(const uint32_t w[2][N], uint32_t out[8]) {
     uint32_t h[2][8];
-    b2s_leaves<2, N>(w, h);
-    b2s_node(h[0], h[1], out);
+    if constexpr (PRIO) {
+        b2s_leaves<2, N>(w, h);
+    } else {  // one after the other: interleaved, a lone wave is slower (2^12 pairs 6.74 us, 6.59 so)
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            uint32_t x[1][N], y[1][8];
+#pragma unroll
+            for (int i = 0; i < N; i++) x[0][i] = w[k][i];
+            b2s_leaves<1, N, false>(x, y);
+#pragma unroll
+            for (int i = 0; i < 8; i++) h[k][i] = y[0][i];
+        }
+    }
+    b2s_node<PRIO>(h[0], h[1], out);
 }
 
 // ---------------------------------------------------------------- quad-cooperative form

@@ -16,7 +16,7 @@ struct SrcCols {
     uint32_t n_cols;
     __device__ __forceinline__ SrcCols at(uint64_t) const { return *this; }
     // the words of K consecutive leaves from i on
-    template <uint32_t K>
+    template <uint32_t K, bool PRIO = true>
     __device__ __forceinline__ void hash(uint64_t i, uint32_t h[K][8]) const {
         if constexpr (NC > 0) {
             uint32_t w[K][NC];
@@ -26,7 +26,7 @@ struct SrcCols {
 #pragma unroll
                 for (uint32_t k = 0; k < K; k++) w[k][c] = p[i + k];
             }
-            b2s_leaves<K, NC>(w, h);
+            b2s_leaves<K, NC, PRIO>(w, h);
         } else {
             const uint32_t eff = n_cols > 16 ? 16 : n_cols;
             uint32_t m[K][16];
@@ -37,22 +37,25 @@ struct SrcCols {
             }
 #pragma unroll
             for (uint32_t k = 0; k < K; k++) b2s_init(h[k]);
-            b2s_compress_n<K, 16>(h, m, 4u * eff, 0xFFFFFFFFu);
+            b2s_compress_n<K, 16, PRIO>(h, m, 4u * eff, 0xFFFFFFFFu);
         }
     }
+    template <bool PRIO = true>
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         uint32_t l[2][8];
-        hash<2>(i, l);
-        b2s_node(l[0], l[1], h);
+        hash<2, PRIO>(i, l);
+        b2s_node<PRIO>(l[0], l[1], h);
     }
 };
 
-template <uint32_t NC>
+// A leaf a lane; PRIO = false for launches whose waves have a SIMD each (us at
+// 2^15 leaves of 16 columns: 4.35 with priorities, 4.10 without).
+template <uint32_t NC, bool PRIO>
 __global__ __launch_bounds__(256) void hash_leaves_kernel(SrcCols<NC> src, uint32_t* out, uint32_t n) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
     uint32_t h[1][8];
-    src.template hash<1>(i, h);
+    src.template hash<1, PRIO>(i, h);
     store8(out + 8ull * i, h[0]);
 }
 
@@ -146,7 +149,7 @@ __global__ __launch_bounds__(FEW ? 1024 : 256) void merkle_tile_kernel(Src src, 
 // SIMD the compression goes without priorities, which a lone wave only waits for;
 // up to NODES_QUAD_MAX parents a quad each, a shorter chain (3.4 us a small
 // level with priorities, 1.8 by quads).
-constexpr uint32_t NODES_QUAD_MAX = 1u << 14, NODES_LONE_MAX = 1u << 16;
+constexpr uint32_t NODES_QUAD_MAX = 1u << 14;
 template <bool PRIO>
 __global__ __launch_bounds__(256) void hash_nodes_kernel(const uint32_t* ch, uint32_t* par, uint32_t n) {
     uint32_t i = blockIdx.x * 256 + threadIdx.x;
@@ -166,15 +169,26 @@ __global__ __launch_bounds__(256) void hash_nodes_quad_kernel(const uint32_t* ch
     par[8ull * i + l] = hl;
     par[8ull * i + 4 + l] = hh;
 }
+// A pair of leaves and their parent a lane (2^13 leaves: 7.3 us with priorities, 6.6 without).
+template <bool PRIO>
 __global__ void leaves_merge_soa4_kernel(SrcSoa4 src, uint32_t* par, uint32_t n_pairs) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_pairs) return;
     uint32_t h[8];
-    src.pair(2ull * i, h);
+    src.pair<PRIO>(2ull * i, h);
     store8(par + 8ull * i, h);
 }
 __global__ void copy8_kernel(const uint32_t* s, uint32_t* d) {
     if (threadIdx.x < 8) d[threadIdx.x] = s[threadIdx.x];
+}
+
+template <uint32_t NC>
+static void hash_leaves(SrcCols<NC> src, uint32_t* hashes, uint32_t n) {
+    const uint32_t grid = ceil_div(n, 256);
+    if (n <= LONE_THREADS)
+        hash_leaves_kernel<NC, false><<<grid, 256, 0, current_stream()>>>(src, hashes, n);
+    else
+        hash_leaves_kernel<NC, true><<<grid, 256, 0, current_stream()>>>(src, hashes, n);
 }
 
 template <class Src>
@@ -209,13 +223,12 @@ extern "C" {
 
 void cuda_merkle_hash_leaves(const uint32_t* const* columns, uint32_t* hashes, uint32_t n_cols, uint32_t n_leaves) {
     if (!n_leaves) return;
-    const uint32_t grid = ceil_div(n_leaves, 256);
     if (n_cols == 1)
-        hash_leaves_kernel<<<grid, 256, 0, current_stream()>>>(SrcCols<1>{columns, n_cols}, hashes, n_leaves);
+        hash_leaves(SrcCols<1>{columns, n_cols}, hashes, n_leaves);
     else if (n_cols == 4)
-        hash_leaves_kernel<<<grid, 256, 0, current_stream()>>>(SrcCols<4>{columns, n_cols}, hashes, n_leaves);
+        hash_leaves(SrcCols<4>{columns, n_cols}, hashes, n_leaves);
     else
-        hash_leaves_kernel<<<grid, 256, 0, current_stream()>>>(SrcCols<0>{columns, n_cols}, hashes, n_leaves);
+        hash_leaves(SrcCols<0>{columns, n_cols}, hashes, n_leaves);
     check_launch("cuda_merkle_hash_leaves");
 }
 
@@ -223,7 +236,7 @@ void cuda_merkle_hash_nodes(const uint32_t* children, uint32_t* parents, uint32_
     if (!n_parents) return;
     if (n_parents <= NODES_QUAD_MAX)
         hash_nodes_quad_kernel<<<ceil_div(n_parents, 64), 256, 0, current_stream()>>>(children, parents, n_parents);
-    else if (n_parents <= NODES_LONE_MAX)
+    else if (n_parents <= LONE_THREADS)
         hash_nodes_kernel<false><<<ceil_div(n_parents, 256), 256, 0, current_stream()>>>(children, parents, n_parents);
     else
         hash_nodes_kernel<true><<<ceil_div(n_parents, 256), 256, 0, current_stream()>>>(children, parents, n_parents);
@@ -257,8 +270,12 @@ void cuda_merkle_hash_leaves_merge_soa4(const uint32_t* c0, const uint32_t* c1, 
                                         const uint32_t* c3, uint32_t* parents, uint32_t n_leaves) {
     uint32_t n_pairs = n_leaves / 2;
     if (!n_pairs) return;
-    leaves_merge_soa4_kernel<<<ceil_div(n_pairs, 256), 256, 0, current_stream()>>>(SrcSoa4{c0, c1, c2, c3}, parents,
-                                                                                  n_pairs);
+    const SrcSoa4 src = {c0, c1, c2, c3};
+    const uint32_t grid = ceil_div(n_pairs, 256);
+    if (n_pairs <= LONE_THREADS)
+        leaves_merge_soa4_kernel<false><<<grid, 256, 0, current_stream()>>>(src, parents, n_pairs);
+    else
+        leaves_merge_soa4_kernel<true><<<grid, 256, 0, current_stream()>>>(src, parents, n_pairs);
     check_launch("cuda_merkle_hash_leaves_merge_soa4");
 }
 

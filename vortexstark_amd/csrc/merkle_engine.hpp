@@ -138,11 +138,12 @@ struct SrcSoa4 {
     __device__ __forceinline__ void leaf(uint64_t i, uint32_t h[8]) const {
         b2s_leaf4(c0[i], c1[i], c2[i], c3[i], h);
     }
+    template <bool PRIO = true>
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         uint2 a = *(const uint2*)(c0 + i), b = *(const uint2*)(c1 + i);
         uint2 c = *(const uint2*)(c2 + i), d = *(const uint2*)(c3 + i);
         const uint32_t w[2][4] = {{a.x, b.x, c.x, d.x}, {a.y, b.y, c.y, d.y}};
-        b2s_leaf_pair<4>(w, h);
+        b2s_leaf_pair<4, PRIO>(w, h);
     }
 };
 
