@@ -41,3 +41,25 @@ def test_merge(vx, n):
     leaves, want = O.leaf_hashes(cols), np.zeros(4 * n, np.uint32)
     O.lib().orc_merkle_node_layer(leaves.ctypes.data, n // 2, want.ctypes.data)
     assert np.array_equal(par.to_host(), want)
+
+
+# the tail kernel's first level: nodes copied (16), read in place by quads (256), by lanes
+# (512 items are 256 parents, one wave a SIMD)
+@pytest.mark.parametrize("n", [1, 2, 4, 8, 16, 32, 256, 512, 1024, 2048])
+def test_roots(vx, n):
+    nodes = rnd(5 + n, 8 * n)
+    buf, root = vx.DeviceBuffer.from_host(nodes), vx.DeviceBuffer(8)
+    vx.lib.cuda_merkle_reduce_to_root(buf.addr, root.addr, n)
+    level = nodes
+    while len(level) > 8:
+        up = np.zeros(len(level) // 2, np.uint32)
+        O.lib().orc_merkle_node_layer(level.ctypes.data, len(up) // 8, up.ctypes.data)
+        level = up
+    vx.synchronize()
+    assert np.array_equal(root.to_host(), level)
+    if n > 1:
+        cols = [rnd(9 + c, n) for c in range(4)]
+        bufs, _ = device_columns(vx, cols)
+        vx.lib.cuda_merkle_commit_small_soa4(*[b.addr for b in bufs], root.addr, n)
+        vx.synchronize()
+        assert np.array_equal(root.to_host(), O.merkle_root(cols))

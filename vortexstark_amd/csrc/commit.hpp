@@ -30,7 +30,7 @@ template <class Src, class Mark>
 void commit_tree(const Src& src, uint64_t n_leaves, LevelStore st, TailOut out, Scratch sc, hipStream_t s,
                  Mark&& mark, uint32_t batch = 1, uint64_t bs = 0, uint64_t direct_max = PROVER_TAIL_ITEMS) {
     if (n_leaves <= direct_max) {
-        merkle_tail_kernel<Src><<<dim3(1, batch), TAIL_THREADS, 0, s>>>(src, 0, (uint32_t)n_leaves, st, out, bs);
+        launch_tail(src, 0, (uint32_t)n_leaves, st, out, batch, bs, s);
         check_launch("merkle_tail_kernel");
         mark("tail");
         return;
@@ -59,7 +59,7 @@ void commit_tree(const Src& src, uint64_t n_leaves, LevelStore st, TailOut out, 
         cur = nxt;
         nxt = tmp;
     }
-    merkle_tail_kernel<SrcNodes><<<dim3(1, batch), TAIL_THREADS, 0, s>>>(SrcNodes{cur}, lvl, (uint32_t)n, st, out, bs);
+    launch_tail(SrcNodes{cur}, lvl, (uint32_t)n, st, out, batch, bs, s);
     check_launch("merkle_tail_kernel<nodes>");
     mark("tail");
 }
@@ -93,8 +93,7 @@ void commit_tree_quad(const Src& src, uint64_t n, LevelStore st, TailOut out, Sc
         leaf_quad_stage_kernel<Src, 4><<<grid, 64 * LEAF_QUAD_WAVES, 0, s>>>(src, sc.a, st, bs);
     check_launch("leaf_quad_stage_kernel");
     mark("stage_leaf");
-    merkle_tail_kernel<SrcNodes><<<dim3(1, batch), TAIL_THREADS, 0, s>>>(SrcNodes{sc.a}, floor_log2(lpw * LEAF_QUAD_WAVES),
-                                                                         blocks, st, out, bs);
+    launch_tail(SrcNodes{sc.a}, floor_log2(lpw * LEAF_QUAD_WAVES), blocks, st, out, batch, bs, s);
     check_launch("merkle_tail_kernel<nodes>");
     mark("tail");
 }

@@ -195,7 +195,7 @@ template <class Src>
 static void tail_root(Src src, uint32_t n_items, uint32_t* root, hipStream_t st, const char* what) {
     LevelStore none = {nullptr, 0, 0};
     TailOut out = {root, nullptr, nullptr, 0};
-    merkle_tail_kernel<Src><<<1, TAIL_THREADS, 0, st>>>(src, 0, n_items, none, out, 0);
+    launch_tail(src, 0, n_items, none, out, 1, 0, st);
     check_launch(what);
 }
 

@@ -80,9 +80,10 @@ __device__ __forceinline__ void load8(const uint32_t* src, uint32_t h[8]) {
 }
 
 // Parent of the SoA4 leaves of two QM31 values.
+template <bool PRIO>
 __device__ __forceinline__ void b2s_leaf_pair4(const QM31& x, const QM31& y, uint32_t h[8]) {
     const uint32_t w[2][4] = {{x.v[0], x.v[1], x.v[2], x.v[3]}, {y.v[0], y.v[1], y.v[2], y.v[3]}};
-    b2s_leaf_pair<4>(w, h);
+    b2s_leaf_pair<4, PRIO>(w, h);
 }
 
 // ---------------------------------------------------------------- sources
@@ -98,6 +99,7 @@ __device__ __forceinline__ void b2s_leaf_pair4(const QM31& x, const QM31& y, uin
 struct SrcNodes {
     const uint32_t* nodes;
     __device__ __forceinline__ SrcNodes at(uint64_t off) const { return {nodes + off}; }
+    template <bool PRIO = true>
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         uint32_t l[8], r[8];
         load8(nodes + 8 * i, l);
@@ -114,10 +116,11 @@ struct SrcCol1 {
     __device__ __forceinline__ void values(uint64_t i, uint32_t v[4]) const { v[0] = col[i]; }
     __device__ __forceinline__ void words(uint64_t i, uint32_t, uint32_t v[1]) const { v[0] = col[i]; }
     __device__ __forceinline__ void leaf(uint64_t i, uint32_t h[8]) const { b2s_leaf1(col[i], h); }
+    template <bool PRIO = true>
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         uint2 v = *(const uint2*)(col + i);
         const uint32_t w[2][1] = {{v.x}, {v.y}};
-        b2s_leaf_pair<1>(w, h);
+        b2s_leaf_pair<1, PRIO>(w, h);
     }
 };
 
@@ -177,13 +180,14 @@ struct SrcQuotient {
         QM31 r = q(i, load_alpha(alpha));
         b2s_leaf4(r.v[0], r.v[1], r.v[2], r.v[3], h);
     }
+    template <bool PRIO = true>
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         QM31 al = load_alpha(alpha);
         uint2 a = *(const uint2*)(t + i);
         uint2 b = *(const uint2*)(t + ((i + 2) & mask));
         QM31 q0 = quotient_at(a.x, a.y, b.x, al);
         QM31 q1 = quotient_at(a.y, b.x, b.y, al);
-        b2s_leaf_pair4(q0, q1, h);
+        b2s_leaf_pair4<PRIO>(q0, q1, h);
     }
 };
 
@@ -227,6 +231,7 @@ struct SrcCircleFold {
         uint32_t* o = l == 0 ? o0 : l == 1 ? o1 : l == 2 ? o2 : o3;
         o[i] = l == 0 ? f.v[0] : l == 1 ? f.v[1] : l == 2 ? f.v[2] : f.v[3];
     }
+    template <bool PRIO = true>
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         const QM31 aq = load_alpha(alpha_q), g = qmul(load_alpha(alpha_f), aq);
         uint64_t j = 2 * i;  // quotient index of the first of four inputs
@@ -242,7 +247,7 @@ struct SrcCircleFold {
         *(uint2*)(o1 + i) = make_uint2(f0.v[1], f1.v[1]);
         *(uint2*)(o2 + i) = make_uint2(f0.v[2], f1.v[2]);
         *(uint2*)(o3 + i) = make_uint2(f0.v[3], f1.v[3]);
-        b2s_leaf_pair4(f0, f1, h);
+        b2s_leaf_pair4<PRIO>(f0, f1, h);
     }
 };
 
@@ -270,6 +275,7 @@ struct SrcLineFold {
         uint32_t* o = l == 0 ? o0 : l == 1 ? o1 : l == 2 ? o2 : o3;
         o[i] = l == 0 ? f.v[0] : l == 1 ? f.v[1] : l == 2 ? f.v[2] : f.v[3];
     }
+    template <bool PRIO = true>
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         const QMatrix al(load_alpha(alpha));
         uint64_t j = 2 * i;
@@ -282,7 +288,7 @@ struct SrcLineFold {
         *(uint2*)(o1 + i) = make_uint2(f0.v[1], f1.v[1]);
         *(uint2*)(o2 + i) = make_uint2(f0.v[2], f1.v[2]);
         *(uint2*)(o3 + i) = make_uint2(f0.v[3], f1.v[3]);
-        b2s_leaf_pair4(f0, f1, h);
+        b2s_leaf_pair4<PRIO>(f0, f1, h);
     }
 };
 
@@ -330,6 +336,7 @@ struct SrcLifted {
     // waves a SIMD; without them four waves share it (98) and cover each other's
     // loads, and the hashing itself pairs better (34 columns, 2^22 leaves:
     // 368 -> 306 us).
+    template <bool PRIO = true>
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         ConstLiftCol* tab = const_table(cols);
         uint32_t ha[8], hb[8];
@@ -347,11 +354,11 @@ struct SrcLifted {
             }
             const uint32_t nw = n_cols - c0 < 16 ? n_cols - c0 : 16;
             const uint32_t t = 4 * (c0 + nw), f = last ? 0xFFFFFFFFu : 0u;
-            b2s_compress(ha, ma, t, f);
-            b2s_compress(hb, mb, t, f);
+            b2s_compress<16, PRIO>(ha, ma, t, f);
+            b2s_compress<16, PRIO>(hb, mb, t, f);
             if (last) break;
         }
-        b2s_node(ha, hb, h);
+        b2s_node<PRIO>(ha, hb, h);
     }
 };
 
@@ -378,6 +385,7 @@ struct SrcWideFold {
     // start the four of the full-size columns: 32 fewer registers than keeping
     // both sets, and no prefetched group, leave five waves a SIMD instead of
     // three (34 columns, 2^21 leaves: 219 -> 180 us).
+    template <bool PRIO = true>
     __device__ __forceinline__ void pair(uint64_t i, uint32_t h[8]) const {
         const uint64_t j = 2 * i;  // f index of the first of four inputs (a multiple of 4)
         ConstLiftCol* tab = const_table(cols);
@@ -450,7 +458,7 @@ struct SrcWideFold {
         *(uint2*)(o1 + i) = make_uint2(g0.v[1], g1.v[1]);
         *(uint2*)(o2 + i) = make_uint2(g0.v[2], g1.v[2]);
         *(uint2*)(o3 + i) = make_uint2(g0.v[3], g1.v[3]);
-        b2s_leaf_pair4(g0, g1, h);
+        b2s_leaf_pair4<PRIO>(g0, g1, h);
     }
 };
 
@@ -844,7 +852,8 @@ __device__ __forceinline__ void block_lane_levels(uint32_t* nodes, uint32_t* out
 // while it has more than 128 parents, one quad compression (0.76 us with its exchange) below,
 // then the transcript's two. The transcript's state is fetched before the first
 // level, and the last level writes the root where the transcript hashes it.
-template <class Src>
+// PRIO = false: the first level's waves have a SIMD each (launch_tail).
+template <class Src, bool PRIO>
 __global__ __launch_bounds__(TAIL_THREADS) void merkle_tail_kernel(Src src0, uint32_t item_level, uint32_t n_items,
                                                                   LevelStore st0, TailOut out, uint64_t bs) {
     constexpr uint32_t W = MERKLE_TAIL_MAX / 2;
@@ -863,16 +872,25 @@ __global__ __launch_bounds__(TAIL_THREADS) void merkle_tail_kernel(Src src0, uin
     QuadTranscript tr = {};
     if (out.channel && tid < 64) tr.load(out.channel, out.init_channel != 0);
     uint32_t n = n_items / 2, lvl = item_level + 1;
+    // Nodes that quads can hash from the first level on: up to 16 of them by one
+    // wave, after a copy to LDS, more from where they lie.
     bool narrow = false;
-    if constexpr (IsNodes<Src>::value) narrow = n_items <= TAIL_QUAD_NODES && n_items > 16;
+    if constexpr (IsNodes<Src>::value) {
+        narrow = n_items <= TAIL_QUAD_NODES;
+        if (n_items <= 16) {
+            if (tid < 8 * n_items) qa[tid] = src.nodes[8 * item_base + tid];
+            n = n_items;
+            lvl = item_level;
+        } else if (narrow) {
+            block_quad_level(src.nodes + 8 * item_base, qa, n, item_level, item_base, st);
+        }
+    }
     if (narrow) {
-        // the first level's quads read the nodes in place
-        if constexpr (IsNodes<Src>::value) block_quad_level(src.nodes + 8 * item_base, qa, n, item_level, item_base, st);
         lds_barrier();
     } else {
         for (uint32_t j = tid; j < n; j += TAIL_THREADS) {
             uint32_t h[8];
-            src.pair(item_base + 2ull * j, h);
+            src.template pair<PRIO>(item_base + 2ull * j, h);
             if (st.want(lvl)) store8(st.at(lvl, (item_base >> 1) + j), h);
             if (n > TAIL_QUAD_NODES) {
 #pragma unroll
@@ -902,6 +920,19 @@ __global__ __launch_bounds__(TAIL_THREADS) void merkle_tail_kernel(Src src0, uin
         if (tid < 4) out.alpha_dst[4 * k + tid] = w;
     }
     tr.store(out.channel);
+}
+
+// Tail of `batch` proofs (one block each, all at once on the device up to 256).
+// A first level of at most 256 parents is one wave a SIMD of its block's CU, which
+// hashes without priorities (roots of 2 and 16 leaves: 7.8 and 10.25 us with them, 7.25
+// and 9.85 without).
+template <class Src>
+inline void launch_tail(const Src& src, uint32_t item_level, uint32_t n_items, LevelStore st, TailOut out, uint32_t batch,
+                        uint64_t bs, hipStream_t s) {
+    if (n_items <= 512 && batch <= LONE_THREADS / 256)
+        merkle_tail_kernel<Src, false><<<dim3(1, batch), TAIL_THREADS, 0, s>>>(src, item_level, n_items, st, out, bs);
+    else
+        merkle_tail_kernel<Src, true><<<dim3(1, batch), TAIL_THREADS, 0, s>>>(src, item_level, n_items, st, out, bs);
 }
 
 }  // namespace vx
