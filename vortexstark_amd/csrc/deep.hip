@@ -8,9 +8,9 @@
 //  accumulate_lift         col[i] += curr[lift(i)]   (QM31, 4 words per element)
 //
 // accumulate_numerators is bound by HBM (4 bytes of column a term) once its rows
-// fill the chip, below by a thread's chain of loads: each thread takes eight
-// consecutive-by-four rows of a large batch (two uint4 loads a column, a wave
-// reading 2 KiB of it), four of a small one. The sum of products c_i * f is kept in
+// fill the chip, below by a thread's chain of loads: a thread of a small batch takes
+// one row, of larger ones four or eight, four consecutive rows a uint4 load (a wave
+// reads 1 or 2 KiB of a column). The sum of products c_i * f is kept in
 // 64 bits: one v_mad_u64_u32 per coordinate and column and, every four columns,
 // one more that folds it below 2^34 (fold64). quotients_combine is bound by the
 // VALU: den_j(row) is the CM31
@@ -40,11 +40,17 @@ constexpr uint32_t DEEP_THREADS = 256;
 //   and 23.8; 2^22 168 and 111
 // - combine, four accumulations: 2^17 rows 8.9 at two, 11.9 at four, 18.5 at eight;
 //   2^19 22.0, 19.7 and 20.6; 2^22 137, 115 and 110
-// - numerators: 2^16 rows of 12 columns 5.5 at four, 6.7 at eight; 2^18 of 64 columns
-//   30.6 and 34.9, 2^20 56.4 and 55.1, 2^22 252 and 243
+// - numerators: 2^8 rows of 26 columns 5.7 at one, 8.1 at four; 2^18 of 64 columns 23.9
+//   and 28; 2^19 37.6 and 31; 2^20 56 at four, 53 at eight
 constexpr uint32_t FUSED_WIDE_MIN = 1u << 18;
 constexpr uint32_t COMBINE_MID_MIN = 1u << 18, COMBINE_WIDE_MIN = 1u << 20;
-constexpr uint32_t NUMER_WIDE_MIN = 1u << 20;
+constexpr uint32_t NUMER_MID_MIN = 1u << 19, NUMER_WIDE_MIN = 1u << 20;
+// Batches of at least so many rows and columns are past the caches and load their
+// columns through generic pointers: a flat load takes the LDS path as well, so fewer
+// are in flight, and HBM then streams them faster (2^21 rows of 64 columns 105 us,
+// 120 through global pointers; 2^22 of 26 94 and 106). Below, global loads win (2^20 of 64
+// columns 53 and 59; 2^21 of 4 12.4 and 14.4).
+constexpr uint32_t NUMER_FLAT_MIN = 3u << 19, NUMER_FLAT_COLS = 8;
 
 // Rows of a thread: ROWS = 1: row0; ROWS = 4 or 8: row0 .. row0 + 3 and row0 + 256
 // .. row0 + 259, so that a wave reads 1 or 2 KiB of a column contiguously (lane l
@@ -57,13 +63,14 @@ template <uint32_t ROWS>
 __device__ __forceinline__ uint64_t row_of(uint64_t row0, uint32_t r) {
     return ROWS == 1 ? row0 : row0 + (r & 3) + 256 * (r >> 2);
 }
-template <uint32_t ROWS>
+template <uint32_t ROWS, bool GLOBAL>
 __device__ __forceinline__ void load_rows(const uint32_t* column, uint64_t row0, uint32_t f[ROWS]) {
     const gu32* col = as_global(column);
     if (ROWS >= 4 && ((uintptr_t)column & 15) == 0) {
 #pragma unroll
         for (uint32_t r = 0; r < ROWS; r += 4) {
-            const u32x4 v = *(const gu32x4*)(col + row_of<ROWS>(row0, r));
+            const uint64_t at = row_of<ROWS>(row0, r);
+            const u32x4 v = GLOBAL ? *(const gu32x4*)(col + at) : *(const u32x4*)(column + at);
             f[r] = v.x;
             f[r + 1] = v.y;
             f[r + 2] = v.z;
@@ -75,7 +82,28 @@ __device__ __forceinline__ void load_rows(const uint32_t* column, uint64_t row0,
     }
 }
 
-template <uint32_t ROWS>
+// acc += c_i * f_i for columns i .. i + G - 1 of a batch (G <= 4), whose loads are
+// all in flight before the first is used. The accumulators stay below 2^34 between
+// groups: four products of at most (p - 1)^2 < 2^62 - 2^32 on top of that stay
+// below 2^64, and fold.
+template <uint32_t ROWS, bool GLOBAL, uint32_t G>
+__device__ __forceinline__ void add_columns(ConstU64* ptrs, ConstU32* idx, ConstU32* cc, uint32_t i, uint64_t row0,
+                                            uint64_t acc[ROWS][4]) {
+    uint32_t f[G][ROWS];
+#pragma unroll
+    for (uint32_t g = 0; g < G; g++) load_rows<ROWS, GLOBAL>((const uint32_t*)ptrs[idx[i + g]], row0, f[g]);
+#pragma unroll
+    for (uint32_t r = 0; r < ROWS; r++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            uint64_t a = acc[r][k];
+#pragma unroll
+            for (uint32_t g = 0; g < G; g++) a = (uint64_t)cc[4 * (i + g) + k] * f[g][r] + a;
+            acc[r][k] = fold64(a);
+        }
+}
+
+template <uint32_t ROWS, bool GLOBAL>
 __global__ __launch_bounds__(DEEP_THREADS) void accumulate_numerators_kernel(
     const uint32_t* const* __restrict__ col_ptrs, const uint32_t* __restrict__ col_indices,
     const uint32_t* __restrict__ b_coeffs, const uint32_t* __restrict__ c_coeffs, uint32_t n_batch, uint32_t n_rows,
@@ -92,32 +120,27 @@ __global__ __launch_bounds__(DEEP_THREADS) void accumulate_numerators_kernel(
     for (uint32_t i = 0; i < n_batch; i++)
 #pragma unroll
         for (int k = 0; k < 4; k++) bs[k] = madd(bs[k], b[4 * i + k]);
-    // The accumulators stay below 2^34 between groups: a group adds four products of
-    // at most (p - 1)^2 < 2^62 - 2^32, which stays below 2^64, and folds.
     uint64_t acc[ROWS][4] = {};
+    // The columns past whole groups of four are a group of their own. The eight-row
+    // form takes one or three of them in front of the loop: behind it they cost 45
+    // registers (101 -> 146, three waves a SIMD), while two in front cost 4 % (2^20
+    // rows of 26 columns).
+    const uint32_t rest = n_batch & 3;
     uint32_t i = 0;
-    for (; i + 4 <= n_batch; i += 4) {
-        uint32_t f[4][ROWS];
-#pragma unroll
-        for (int g = 0; g < 4; g++) load_rows<ROWS>((const uint32_t*)ptrs[idx[i + g]], row0, f[g]);
-#pragma unroll
-        for (uint32_t r = 0; r < ROWS; r++)
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                uint64_t a = acc[r][k];
-#pragma unroll
-                for (int g = 0; g < 4; g++) a = (uint64_t)cc[4 * (i + g) + k] * f[g][r] + a;
-                acc[r][k] = fold64(a);
-            }
+    if (ROWS == 8 && rest == 1) {
+        add_columns<ROWS, GLOBAL, 1>(ptrs, idx, cc, 0, row0, acc);
+        i = 1;
+    } else if (ROWS == 8 && rest == 3) {
+        add_columns<ROWS, GLOBAL, 3>(ptrs, idx, cc, 0, row0, acc);
+        i = 3;
     }
-    for (; i < n_batch; i++) {
-        uint32_t f[ROWS];
-        load_rows<ROWS>((const uint32_t*)ptrs[idx[i]], row0, f);
-#pragma unroll
-        for (uint32_t r = 0; r < ROWS; r++)
-#pragma unroll
-            for (int k = 0; k < 4; k++) acc[r][k] = fold64((uint64_t)cc[4 * i + k] * f[r] + acc[r][k]);
-    }
+    for (; i + 4 <= n_batch; i += 4) add_columns<ROWS, GLOBAL, 4>(ptrs, idx, cc, i, row0, acc);
+    if (rest == 2)
+        add_columns<ROWS, GLOBAL, 2>(ptrs, idx, cc, i, row0, acc);
+    else if (ROWS != 8 && rest == 1)
+        add_columns<ROWS, GLOBAL, 1>(ptrs, idx, cc, i, row0, acc);
+    else if (ROWS != 8 && rest == 3)
+        add_columns<ROWS, GLOBAL, 3>(ptrs, idx, cc, i, row0, acc);
     uint32_t o[4][ROWS];
 #pragma unroll
     for (uint32_t r = 0; r < ROWS; r++)
@@ -579,15 +602,17 @@ void cuda_accumulate_numerators(const uint32_t* const* col_ptrs, const uint32_t*
                                 uint32_t n_rows, uint32_t* out0, uint32_t* out1, uint32_t* out2, uint32_t* out3) {
     if (!n_rows) return;
     const bool aligned = (((uintptr_t)out0 | (uintptr_t)out1 | (uintptr_t)out2 | (uintptr_t)out3) & 15) == 0;
-#define VX_NUMERATORS(rows)                                                                                     \
-    accumulate_numerators_kernel<rows><<<ceil_div(n_rows, rows * DEEP_THREADS), DEEP_THREADS, 0, current_stream()>>>( \
+#define VX_NUMERATORS(rows, global)                                                                                     \
+    accumulate_numerators_kernel<rows, global><<<ceil_div(n_rows, rows * DEEP_THREADS), DEEP_THREADS, 0, current_stream()>>>( \
         col_ptrs, col_indices, b_coeffs, c_coeffs, n_batch_cols, n_rows, out0, out1, out2, out3)
-    if (aligned && n_rows % 512 == 0 && n_rows >= NUMER_WIDE_MIN)
-        VX_NUMERATORS(8);
-    else if (aligned && n_rows % 256 == 0)
-        VX_NUMERATORS(4);
+    if (aligned && n_rows % 512 == 0 && n_rows >= NUMER_FLAT_MIN && n_batch_cols >= NUMER_FLAT_COLS)
+        VX_NUMERATORS(8, false);
+    else if (aligned && n_rows % 512 == 0 && n_rows >= NUMER_WIDE_MIN)
+        VX_NUMERATORS(8, true);
+    else if (aligned && n_rows % 256 == 0 && n_rows >= NUMER_MID_MIN)
+        VX_NUMERATORS(4, true);
     else
-        VX_NUMERATORS(1);
+        VX_NUMERATORS(1, true);
 #undef VX_NUMERATORS
     check_launch("cuda_accumulate_numerators");
 }
