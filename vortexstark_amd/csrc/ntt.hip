@@ -261,9 +261,12 @@ template <bool FWD, int M, int C, int R, int J, bool STWO, bool ALT = false>
 __device__ __forceinline__ void load_twiddles(RoundTwiddles<M, C, R, J>& tw, const NttPassArgs& a, uint64_t hi,
                                               uint32_t tid, bool zero_top = false) {
     using S = RoundShape<M, C, R, J>;
+    // Threads past the last group load a live one's twiddles: a branch around the
+    // loads would end by waiting for them, before the tile's are on their way
+    // (interpolation of 2^6 points: 12.86 us with the branch, 12.6 without).
+    if (S::GROUPS < S::NT) tid &= S::GROUPS - 1;
 #pragma unroll
     for (uint32_t it = 0; it < S::ITER; it++) {
-        if (!S::live(tid, it)) break;
         const uint32_t row_hi = S::row_hi(tid, it);
 #pragma unroll
         for (int t = 0; t < R; t++) {
