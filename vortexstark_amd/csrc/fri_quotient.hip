@@ -8,9 +8,11 @@
 namespace vx {
 
 // All four kernels are bound by device memory (52 bytes a folded value, 20 a
-// quotient value), so a thread takes two folded values, or four quotient or
-// padded words, with 16-byte accesses (VEC: the pointers allow it); a ragged
-// end and unaligned pointers go word by word.
+// quotient value). A thread takes one folded value, an 8-byte load of each
+// column (two a thread, with 16-byte loads, are slower at most sizes: half of 2^21 line
+// 17.7 us, 16.7 so, circle 23.7 and 21.0; 2^24 line 153 and 148; 11 values 0.6 slower by their
+// ragged end), or four quotient or padded words with 16-byte accesses (VEC: the
+// pointers allow it); a ragged end and unaligned pointers go word by word.
 struct SoaIn {
     const uint32_t* c[4];
 };
@@ -18,28 +20,11 @@ struct SoaOut {
     uint32_t* c[4];
 };
 
-template <bool VEC>
 __global__ __launch_bounds__(256) void fold_line_soa_kernel(SoaIn in, const uint32_t* __restrict__ tw, SoaOut out,
                                                           QM31 alpha, uint32_t half_n) {
-    const uint32_t i = (blockIdx.x * 256 + threadIdx.x) * (VEC ? 2 : 1);
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i >= half_n) return;
     const QMatrix al(alpha);
-    if (VEC && i + 1 < half_n) {
-        QM31 f[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const uint4 x = *(const uint4*)(in.c[c] + 2ull * i);
-            f[0].v[c] = x.x;
-            f[1].v[c] = x.y;
-            f[2].v[c] = x.z;
-            f[3].v[c] = x.w;
-        }
-        const uint2 w = *(const uint2*)(tw + i);
-        const QM31 r0 = fold_pair(f[0], f[1], al, w.x), r1 = fold_pair(f[2], f[3], al, w.y);
-#pragma unroll
-        for (int c = 0; c < 4; c++) *(uint2*)(out.c[c] + i) = make_uint2(r0.v[c], r1.v[c]);
-        return;
-    }
     QM31 f0, f1;
 #pragma unroll
     for (int c = 0; c < 4; c++) {
@@ -64,31 +49,11 @@ __device__ __forceinline__ QM31 fold_onto(QM31 prev, QM31 f0, QM31 f1, const QMa
     return r;
 }
 
-template <bool VEC>
 __global__ __launch_bounds__(256) void fold_circle_soa_kernel(SoaOut dst, SoaIn src, const uint32_t* __restrict__ tw,
                                                             QM31 alpha, QM31 alpha_sq, uint32_t half_n) {
-    const uint32_t i = (blockIdx.x * 256 + threadIdx.x) * (VEC ? 2 : 1);
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i >= half_n) return;
     const QMatrix al(alpha), sq(alpha_sq);
-    if (VEC && i + 1 < half_n) {
-        QM31 f[4], p[2];
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const uint4 x = *(const uint4*)(src.c[c] + 2ull * i);
-            const uint2 y = *(const uint2*)(dst.c[c] + i);
-            f[0].v[c] = x.x;
-            f[1].v[c] = x.y;
-            f[2].v[c] = x.z;
-            f[3].v[c] = x.w;
-            p[0].v[c] = y.x;
-            p[1].v[c] = y.y;
-        }
-        const uint2 w = *(const uint2*)(tw + i);
-        const QM31 r0 = fold_onto(p[0], f[0], f[1], al, sq, w.x), r1 = fold_onto(p[1], f[2], f[3], al, sq, w.y);
-#pragma unroll
-        for (int c = 0; c < 4; c++) *(uint2*)(dst.c[c] + i) = make_uint2(r0.v[c], r1.v[c]);
-        return;
-    }
     QM31 f0, f1, prev;
 #pragma unroll
     for (int c = 0; c < 4; c++) {
@@ -162,13 +127,7 @@ void cuda_fold_line_soa(const uint32_t* in0, const uint32_t* in1, const uint32_t
     if (!half_n) return;
     const SoaIn in = {{in0, in1, in2, in3}};
     const SoaOut out = {{out0, out1, out2, out3}};
-    const bool vec = aligned(16, in0, in1, in2, in3) && aligned(8, twiddles, out0, out1, out2, out3);
-    if (vec)
-        fold_line_soa_kernel<true>
-            <<<ceil_div(half_n, 512), 256, 0, current_stream()>>>(in, twiddles, out, q_from_host(alpha), half_n);
-    else
-        fold_line_soa_kernel<false>
-            <<<ceil_div(half_n, 256), 256, 0, current_stream()>>>(in, twiddles, out, q_from_host(alpha), half_n);
+    fold_line_soa_kernel<<<ceil_div(half_n, 256), 256, 0, current_stream()>>>(in, twiddles, out, q_from_host(alpha), half_n);
     check_launch("cuda_fold_line_soa");
 }
 
@@ -179,13 +138,8 @@ void cuda_fold_circle_into_line_soa(uint32_t* dst0, uint32_t* dst1, uint32_t* ds
     if (!half_n) return;
     const SoaIn src = {{src0, src1, src2, src3}};
     const SoaOut dst = {{dst0, dst1, dst2, dst3}};
-    const bool vec = aligned(16, src0, src1, src2, src3) && aligned(8, twiddles, dst0, dst1, dst2, dst3);
-    if (vec)
-        fold_circle_soa_kernel<true><<<ceil_div(half_n, 512), 256, 0, current_stream()>>>(
-            dst, src, twiddles, q_from_host(alpha), q_from_host(alpha_sq), half_n);
-    else
-        fold_circle_soa_kernel<false><<<ceil_div(half_n, 256), 256, 0, current_stream()>>>(
-            dst, src, twiddles, q_from_host(alpha), q_from_host(alpha_sq), half_n);
+    fold_circle_soa_kernel<<<ceil_div(half_n, 256), 256, 0, current_stream()>>>(dst, src, twiddles, q_from_host(alpha),
+                                                                               q_from_host(alpha_sq), half_n);
     check_launch("cuda_fold_circle_into_line_soa");
 }
 
