@@ -11,8 +11,8 @@ namespace vx {
 // quotient value). A thread takes one folded value, an 8-byte load of each
 // column (two a thread, with 16-byte loads, are slower at most sizes: half of 2^21 line
 // 17.7 us, 16.7 so, circle 23.7 and 21.0; 2^24 line 153 and 148; 11 values 0.6 slower by their
-// ragged end), or four quotient or padded words with 16-byte accesses (VEC: the
-// pointers allow it); a ragged end and unaligned pointers go word by word.
+// ragged end), or of long arrays four quotient or padded words with 16-byte accesses
+// (VEC); a ragged end goes word by word.
 struct SoaIn {
     const uint32_t* c[4];
 };
@@ -66,8 +66,14 @@ __global__ __launch_bounds__(256) void fold_circle_soa_kernel(SoaOut dst, SoaIn 
     for (int c = 0; c < 4; c++) dst.c[c][i] = r.v[c];
 }
 
+// Words from which a thread takes four. Below, one a thread has the shorter chain and
+// no ragged ends (11 quotients 12.2 us at four, call and wait; 11.65 at one; 2^16 4.05
+// and 3.85 back to back; padding to 44 words 11.45 and 11.2); above, wider accesses
+// stream faster (2^24 quotients 62 and 78, padding to 2^24 words 12.1 and 20).
+constexpr uint32_t QUOTIENT_WIDE_MIN = 1u << 18, PAD_WIDE_MIN = 1u << 19;
+
 // q[i] = alpha * (t[(i+2) mod n] - (t[(i+1) mod n] + t[i]))  (constraint.cu:10-36)
-// VEC: n >= 8, 16-byte aligned outputs and t + offset.
+// VEC (n >= 8): four words a thread by 16-byte accesses at any word address.
 template <bool VEC>
 __global__ __launch_bounds__(256) void quotient_kernel(const uint32_t* __restrict__ t, SoaOut out, QM31 alpha,
                                                      uint32_t offset, uint32_t chunk_n, uint32_t n) {
@@ -75,15 +81,15 @@ __global__ __launch_bounds__(256) void quotient_kernel(const uint32_t* __restric
     if (li >= chunk_n) return;
     if (VEC && chunk_n - li >= 4) {
         const uint32_t i = offset + li;  // i + 3 < n
-        const uint4 a = *(const uint4*)(t + i);
+        const u32x4_any a = *(const u32x4_any*)(t + i);
         const uint32_t e = i + 4 < n ? t[i + 4] : t[0];
         const uint32_t f = n - i > 5 ? t[i + 5] : t[i + 5 - n];
         const uint32_t d[4] = {msub(a.z, madd(a.y, a.x)), msub(a.w, madd(a.z, a.y)), msub(e, madd(a.w, a.z)),
                                msub(f, madd(e, a.w))};
 #pragma unroll
         for (int c = 0; c < 4; c++)
-            *(uint4*)(out.c[c] + li) = make_uint4(mmul(alpha.v[c], d[0]), mmul(alpha.v[c], d[1]),
-                                                  mmul(alpha.v[c], d[2]), mmul(alpha.v[c], d[3]));
+            *(u32x4_any*)(out.c[c] + li) = u32x4_any{mmul(alpha.v[c], d[0]), mmul(alpha.v[c], d[1]),
+                                                     mmul(alpha.v[c], d[2]), mmul(alpha.v[c], d[3])};
         return;
     }
     for (uint32_t l = li; l < chunk_n && l - li < (VEC ? 4u : 1u); l++) {  // li + 4 may pass 2^32
@@ -162,7 +168,7 @@ void cuda_fibonacci_quotient_chunk_stream(const uint32_t* trace, uint32_t* out0,
         return;
     }
     const SoaOut out = {{out0, out1, out2, out3}};
-    if (global_n >= 8 && aligned(16, trace + offset, out0, out1, out2, out3))
+    if (chunk_n >= QUOTIENT_WIDE_MIN && global_n >= 8)
         quotient_kernel<true><<<ceil_div(chunk_n, 1024), 256, 0, (hipStream_t)stream>>>(
             trace, out, q_from_host(alpha), offset, chunk_n, global_n);
     else
@@ -172,7 +178,7 @@ void cuda_fibonacci_quotient_chunk_stream(const uint32_t* trace, uint32_t* out0,
 }
 void cuda_zero_pad(const uint32_t* src, uint32_t* dst, uint32_t src_n, uint32_t dst_n) {
     if (!dst_n) return;
-    if (aligned(16, src, dst))
+    if (dst_n >= PAD_WIDE_MIN && aligned(16, src, dst))
         zero_pad_kernel<true><<<ceil_div(dst_n, 1024), 256, 0, current_stream()>>>(src, dst, src_n, dst_n);
     else
         zero_pad_kernel<false><<<ceil_div(dst_n, 256), 256, 0, current_stream()>>>(src, dst, src_n, dst_n);
