@@ -911,15 +911,16 @@ __device__ __forceinline__ void invert_run(uint32_t (&w)[RUN]) {
     }
 }
 // start * the points of the set bits of run number blk * TABLE_THREADS + tid,
-// bit b being pts[RUN_LOG + b]
+// bit b being pts[RUN_LOG + b]; run numbers have `bits` bits
 template <uint32_t RUN_LOG>
-__device__ __forceinline__ CPt run_start(CPt start, const CPt* pts, uint32_t blk) {
+__device__ __forceinline__ CPt run_start(CPt start, const CPt* pts, uint32_t blk, uint32_t bits = 32) {
     CPt p = start;
     constexpr uint32_t TB = TABLE_THREADS_LOG;
     for (uint32_t b = RUN_LOG + TB; blk; b++, blk >>= 1)
         if (blk & 1) p = cpmul(p, pts[b]);
 #pragma unroll
     for (uint32_t b = 0; b < TB; b++) {
+        if (b >= bits) break;
         const bool on = (threadIdx.x >> b) & 1;
         const CPt q = pts[RUN_LOG + b];
         p = cpmul(p, CPt{on ? q.x : 1u, on ? q.y : 0u});
@@ -934,26 +935,44 @@ struct FoldTables {
     uint32_t first_block[33];
     uint32_t log_len[32];
     uint32_t use_y;           // bit l: layer l takes y
-    uint32_t n_layers;
 };
-template <bool INV>
+// coordinate of p * top[r] for the words r of a run
+template <uint32_t RUN>
+__device__ __forceinline__ void run_words(CPt p, const CPt* top, bool y, uint32_t (&w)[RUN]) {
+#pragma unroll
+    for (uint32_t r = 0; r < RUN; r++) {
+        const uint32_t c0 = y ? top[r].y : top[r].x, c1 = y ? top[r].x : P - top[r].y;
+        w[r] = reduce64((uint64_t)p.x * c0 + (uint64_t)p.y * c1);
+    }
+}
 __global__ __launch_bounds__(TABLE_THREADS) void fold_tables_kernel(FoldTables m) {
-    constexpr uint32_t LOG = INV ? TABLE_RUN_LOG : SOURCE_RUN_LOG, RUN = 1u << LOG;
+    constexpr uint32_t RUN = 1u << TABLE_RUN_LOG;
     uint32_t l = 0;
     while (blockIdx.x >= m.first_block[l + 1]) l++;
     const uint32_t blk = blockIdx.x - m.first_block[l];
     const uint64_t len = 1ull << m.log_len[l], i = ((uint64_t)blk * TABLE_THREADS + threadIdx.x) * RUN;
     if (i >= len) return;
-    const CPt p = run_start<LOG>(m.initial[l], m.u, blk);
-    const bool y = (m.use_y >> l) & 1;
     uint32_t w[RUN];
-#pragma unroll
-    for (uint32_t r = 0; r < RUN; r++) {
-        const uint32_t c0 = y ? m.top[r].y : m.top[r].x, c1 = y ? m.top[r].x : P - m.top[r].y;
-        w[r] = reduce64((uint64_t)p.x * c0 + (uint64_t)p.y * c1);
-    }
-    if constexpr (INV) invert_run(w);
+    run_words(run_start<TABLE_RUN_LOG>(m.initial[l], m.u, blk), m.top, (m.use_y >> l) & 1, w);
+    invert_run(w);
     store_run(m.out[l], i, len, w);
+}
+// Sources of one domain. Small ones are a launch's latency, in which arguments that
+// depend on nothing are fetched once, and the steps of bits an index has not got are
+// left out (2^2 points, call and wait: 12.3 us as a layer of the kernel above, 11.8 so).
+struct FoldSources {
+    CPt u[32], top[1u << SOURCE_RUN_LOG], initial;
+    uint32_t* out;
+    uint32_t log_len, use_y;
+};
+__global__ __launch_bounds__(TABLE_THREADS) void fold_sources_run_kernel(FoldSources m) {
+    constexpr uint32_t RUN = 1u << SOURCE_RUN_LOG;
+    const uint64_t len = 1ull << m.log_len, i = ((uint64_t)blockIdx.x * TABLE_THREADS + threadIdx.x) * RUN;
+    if (i >= len) return;
+    const uint32_t bits = m.log_len > SOURCE_RUN_LOG ? m.log_len - SOURCE_RUN_LOG : 0;
+    uint32_t w[RUN];
+    run_words(run_start<SOURCE_RUN_LOG>(m.initial, m.u, blockIdx.x, bits), m.top, m.use_y != 0, w);
+    store_run(m.out, i, len, w);
 }
 
 // Sources of any n: out[i] = coordinate of initial * step^bitrev_(log_n)(2i).
@@ -1101,18 +1120,22 @@ void build_ntt_tables(HostPt initial, HostPt step, uint32_t log_n, uint32_t* lin
 static void index_points(HostPt step, uint32_t log_len, HostPt u[32]) {
     for (uint32_t b = log_len; b-- > 0; step = host_pmul(step, step)) u[b] = step;
 }
-static void fold_tables(const FoldDomain* d, uint32_t n, bool inverse, hipStream_t s) {
+// the products of u[0 .. run_log - 1], of a domain of log_len bits
+static void top_points(const HostPt* u, uint32_t log_len, uint32_t run_log, CPt* top) {
+    for (uint32_t r = 0; r < 1u << run_log; r++) {
+        HostPt q = {1, 0};
+        for (uint32_t b = 0; b < run_log && b < log_len; b++)
+            if ((r >> b) & 1) q = host_pmul(q, u[b]);
+        top[r] = cpt(q);
+    }
+}
+void build_fold_twiddles(const FoldDomain* d, uint32_t n, hipStream_t s) {
     while (n) {
         FoldTables m = {};
         HostPt u[32] = {}, v[32];
         index_points(d[0].step, d[0].log_len, u);
         for (uint32_t b = 0; b < d[0].log_len; b++) m.u[b] = cpt(u[b]);
-        for (uint32_t r = 0; r < 1u << TABLE_RUN_LOG; r++) {
-            HostPt q = {1, 0};
-            for (uint32_t b = 0; b < TABLE_RUN_LOG; b++)
-                if (((r >> b) & 1) && b < d[0].log_len) q = host_pmul(q, u[b]);
-            m.top[r] = cpt(q);
-        }
+        top_points(u, d[0].log_len, TABLE_RUN_LOG, m.top);
         // the layers that follow with the same points of their (fewer) bits
         uint32_t l = 0;
         for (; l < n && l < 32 && d[l].log_len <= d[0].log_len; l++) {
@@ -1124,19 +1147,27 @@ static void fold_tables(const FoldDomain* d, uint32_t n, bool inverse, hipStream
             m.out[l] = d[l].out;
             m.log_len[l] = d[l].log_len;
             m.use_y |= (d[l].use_y ? 1u : 0u) << l;
-            m.first_block[l + 1] = m.first_block[l] + table_blocks(1ull << d[l].log_len, inverse ? TABLE_RUN_LOG : SOURCE_RUN_LOG);
+            m.first_block[l + 1] = m.first_block[l] + table_blocks(1ull << d[l].log_len, TABLE_RUN_LOG);
         }
-        m.n_layers = l;
-        if (inverse)
-            fold_tables_kernel<true><<<m.first_block[l], TABLE_THREADS, 0, s>>>(m);
-        else
-            fold_tables_kernel<false><<<m.first_block[l], TABLE_THREADS, 0, s>>>(m);
+        fold_tables_kernel<<<m.first_block[l], TABLE_THREADS, 0, s>>>(m);
         check_launch("fold_tables_kernel");
         d += l;
         n -= l;
     }
 }
-void build_fold_twiddles(const FoldDomain* d, uint32_t n, hipStream_t s) { fold_tables(d, n, true, s); }
+static void fold_sources(const FoldDomain& d, hipStream_t s) {
+    FoldSources m = {};
+    HostPt u[32];
+    index_points(d.step, d.log_len, u);
+    for (uint32_t b = 0; b < d.log_len; b++) m.u[b] = cpt(u[b]);
+    top_points(u, d.log_len, SOURCE_RUN_LOG, m.top);
+    m.initial = cpt(d.initial);
+    m.out = d.out;
+    m.log_len = d.log_len;
+    m.use_y = d.use_y ? 1u : 0u;
+    fold_sources_run_kernel<<<table_blocks(1ull << d.log_len, SOURCE_RUN_LOG), TABLE_THREADS, 0, s>>>(m);
+    check_launch("fold_sources_run_kernel");
+}
 
 // The whole group's fold twiddles (log_n = 31), by the two passes of the kernel
 // ABI: its points (1, 0) and (-1, 0) have y = 0, and the batch inverse makes the
@@ -1144,7 +1175,7 @@ void build_fold_twiddles(const FoldDomain* d, uint32_t n, hipStream_t s) { fold_
 void build_fold_twiddles_chunked(const FoldDomain& d, uint32_t* scratch, hipStream_t s) {
     FoldDomain src = d;
     src.out = scratch;
-    fold_tables(&src, 1, false, s);
+    fold_sources(src, s);
     batch_inverse(scratch, d.out, 1ull << d.log_len, s);
 }
 
@@ -1430,7 +1461,7 @@ void cuda_compute_fold_twiddle_sources_stream(uint32_t ix, uint32_t iy, uint32_t
     if (!half) return;
     if (log_n <= 31 && n == 1u << log_n) {
         const FoldDomain d = {{ix, iy}, {sx, sy}, log_n - 1, extract_y != 0, output};
-        fold_tables(&d, 1, false, (hipStream_t)stream);
+        fold_sources(d, (hipStream_t)stream);
         return;
     }
     fold_sources_kernel<<<ceil_div(half, 256), 256, 0, (hipStream_t)stream>>>(CPt{ix, iy}, CPt{sx, sy}, output,
