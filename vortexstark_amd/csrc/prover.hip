@@ -61,6 +61,7 @@ __global__ __launch_bounds__(1 << FIB_THREADS_LOG) void fib_trace_kernel(const u
         if (blk & 1) fib_step(f0, f1, steps.f[k][0], steps.f[k][1]);
 #pragma unroll
     for (uint32_t k = 0; k < FIB_THREADS_LOG; k++) {
+        if (n <= (uint64_t)RUN << k) break;  // no index has the bit (4 words, call and wait: 12.45 us with all steps, 11.9 so)
         const bool on = (threadIdx.x >> k) & 1;
         fib_step(f0, f1, on ? steps.f[FIB_RUN_LOG + k][0] : 1u, on ? steps.f[FIB_RUN_LOG + k][1] : 0u);
     }
