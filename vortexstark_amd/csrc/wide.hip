@@ -88,7 +88,7 @@ __global__ __launch_bounds__(256) void lifted_leaves_kernel(const uint32_t* cons
     __shared__ LiftAbiCol tab[16 * LIFT_ABI_MAX_CHUNKS];
     __shared__ uint32_t start[LIFT_ABI_MAX_CHUNKS + 1];  // chunk c's first column; the last entry: their number
     const uint32_t tid = threadIdx.x, lane = tid & 63;
-    static_assert(LIFT_ABI_MAX_CHUNKS <= 64);
+    static_assert(LIFT_ABI_MAX_CHUNKS == 64, "a chunk a lane of the wave that sums them");
     if (tid < 64) {
         uint32_t sum = lane < n_chunks ? min(schedule[lane].n_cols, 16u) : 0u;
         for (uint32_t d = 1; d < 64; d <<= 1) {
