@@ -41,24 +41,9 @@ constexpr uint32_t B2S_H0 = B2S_IV0 ^ 0x01010020u;
 
 constexpr uint32_t LONE_THREADS = 1u << 16;  // one wave for each SIMD of 256 CUs
 
-struct Digest {
-    uint32_t w[8];
-};
-
 #define VX_ROTR(x, n) __builtin_rotateright32((x), (n))
 // x ^ y ^ z in one gfx950 instruction (v_bitop3_b32, truth table 0x96)
 #define VX_XOR3(x, y, z) __builtin_amdgcn_bitop3_b32((x), (y), (z), 0x96)
-#define VX_G(a, b, c, d, x, y)      \
-    do {                            \
-        a = a + b + (x);            \
-        d = VX_ROTR(d ^ a, 16);     \
-        c = c + d;                  \
-        b = VX_ROTR(b ^ c, 12);     \
-        a = a + b + (y);            \
-        d = VX_ROTR(d ^ a, 8);      \
-        c = c + d;                  \
-        b = VX_ROTR(b ^ c, 7);      \
-    } while (0)
 
 // Message schedule of round r (RFC 7693, section 2.7).
 constexpr uint8_t B2S_SIGMA[10][16] = {
@@ -174,13 +159,6 @@ __device__ __forceinline__ void b2s_init(uint32_t h[8]) {
     h[7] = B2S_IV7;
 }
 
-// Single-block hash of up to 16 words (t = 4 * n_words), the Merkle leaf rule
-// (cuda/blake2s.cu:45-60, merkle.rs:538-556). Words at index >= n_words must be 0.
-__device__ __forceinline__ void b2s_leaf(const uint32_t m[16], uint32_t n_words, uint32_t out[8]) {
-    b2s_init(out);
-    b2s_compress(out, m, 4u * n_words, 0xFFFFFFFFu);
-}
-
 // Merkle node: H(left || right), t = 64 (cuda/blake2s.cu:65-89).
 template <bool PRIO = true>
 __device__ __forceinline__ void b2s_node(const uint32_t l[8], const uint32_t r[8], uint32_t out[8]) {
@@ -194,7 +172,8 @@ __device__ __forceinline__ void b2s_node(const uint32_t l[8], const uint32_t r[8
     b2s_compress<16, PRIO>(out, m, 64u, 0xFFFFFFFFu);
 }
 
-// Leaves of N words each (N <= 4), K at once: K = 1, or both leaves of a pair
+// Leaves of N words each (N <= 4, t = 4 N, the Merkle leaf rule of
+// cuda/blake2s.cu:45-60 and merkle.rs:538-556), K at once: K = 1, or both leaves of a pair
 // with their rounds interleaved (two compressions' rows side by side keep more
 // instructions between dependent ones; see the figures above).
 template <int K, int N, bool PRIO = true>

@@ -78,7 +78,6 @@ struct NttPassArgs {
     const uint32_t* tw2[NTT_LOW_MAX];
     uint64_t src_n;  // words of src that are read; the rest is zero
     uint32_t s;      // lowest global stride bit of this pass
-    uint32_t k;      // log2 of the transform size
     uint32_t scale;  // multiply on store when non-zero
     uint32_t vec;    // every column pointer is 16-byte aligned: move tiles 4 words per lane
     uint32_t zero_top2;  // forward, top pass, src_n = n / 4: the two top layers only copy
@@ -718,7 +717,6 @@ static void run_ntt_plan(bool fwd, uint32_t* dst, const uint32_t* src, uint64_t 
         a.src_n = i == 0 ? src_n : (1ull << k);
         for (uint32_t rb = 0; rb < ps[pi].m && rb < NTT_LOW_MAX; rb++) a.tw[rb] = layer_table(t, ps[pi].s + rb);
         a.s = ps[pi].s;
-        a.k = k;
         a.vec = vec ? 1u : 0u;
         a.scale = (!fwd && last_scale && i + 1 == ps.size()) ? inv_n : 0u;
         // the top pass of an evaluation of n/4 coefficients: its two top layers copy
@@ -815,7 +813,6 @@ static void lde_run(uint32_t* const* cols, uint32_t n_cols, const NttTables& ti,
     }
     a.src_n = 1ull << kt;
     a.s = pt.s;
-    a.k = ke;
     a.vec = 1u;
     a.scale = inverse_scale(kt);
     const uint32_t rows = pt.m - 2;
