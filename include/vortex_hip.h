@@ -272,7 +272,8 @@ void* vx_get_stream(void);
  * top layers only copy the quarter into all four, so the pass holds 2^(m-2)
  * rows in LDS and transforms them once per quarter. A size with no plan of
  * either table takes a default of this form; lde_plan_set with n_passes = 0
- * asks for the general table, plan_reset clears both. No reference counterpart (tuning of this library's pass structure). */
+ * asks for the general table, plan_reset clears both. No reference counterpart
+ * (tuning of this library's pass structure). */
 int32_t vx_ntt_autotune(uint32_t log_min, uint32_t log_max, float* best_ms);
 /* Measured int32 VALU issue rate of the current device in T lane-ops/s (a
  * grid of v_add3 / v_xor / v_alignbit chains, the instructions of Blake2s). */
@@ -296,9 +297,9 @@ uint32_t vx_ntt_lde_plan_get(uint32_t log_n, uint32_t* m, uint32_t* c, uint32_t*
 void vx_ntt_set_lde_bridge(int32_t enable);
 
 /* Chunk depth of the Merkle stage kernels (no reference counterpart): a wave
- * hashes 2^c chunks of 128 items before its 64 -> 1 reduction. The depth is
- * picked per launch by the items it covers (all proofs of a batch): a tuned
- * value when one is set, else the largest c leaving 3072 waves. vx_merkle_autotune
+ * hashes 2^c chunks of 128 items before it reduces its last 64 nodes. The depth
+ * is picked per launch by the items it covers (all proofs of a batch): a tuned
+ * value when one is set, else a default by that number. vx_merkle_autotune
  * times whole tree commitments of 2^log items (12 <= log <= 27) at every
  * depth on the device and keeps the fastest; plan returns the tuned depth of
  * 2^log_items items (-1: default rule); plan_set sets one (-1 clears it). Any
@@ -399,7 +400,8 @@ uint64_t vx_krak_proof_size(uint32_t log_n, uint32_t n_queries, uint32_t log_las
 uint64_t vx_prove_fibonacci(vx_prover* p, uint32_t a, uint32_t b, void* host_out, uint64_t cap);
 
 /* Fibonacci trace t0 = a, t1 = b, t(i+2) = t(i) + t(i+1) mod p generated on the device
- * (chunked by 2x2 matrix powers, air.rs:85-189). */
+ * (a thread's run of words reached by one Fibonacci step per bit of its index; the
+ * reference's chunks take 2x2 matrix powers, air.rs:85-189). */
 int32_t vx_fibonacci_trace(uint32_t a, uint32_t b, uint32_t log_n, uint32_t* d_out, void* stream);
 
 /* Launch timeline: when enabled, the prover records a HIP event on its stream

@@ -160,10 +160,10 @@ __global__ __launch_bounds__(DEEP_THREADS) void accumulate_numerators_kernel(
 }
 
 // One sample point at R rows: its denominators, their inverses by one M31
-// inversion, and the rows' quotients num / den added to q, kept as 64-bit sums of
-// products below 2^34 (+ 4 * 2^62 on top of `fresh`, a sum no point has been
-// added to). num(r, k) gives the row's numerator coordinate plus (P - A_k) y, any
-// representative below 2^64.
+// inversion, and the rows' quotients num / den added to q as products not yet reduced:
+// a point adds two of at most p (p - 1) to each sum, so two points on top of a
+// folded one (below 2^34) stay below 2^64, after which the callers fold. num(r, k)
+// gives the row's numerator coordinate plus (P - A_k) y, any representative below 2^64.
 template <uint32_t R, class Num>
 __device__ __forceinline__ void add_quotients(ConstU32* x, ConstU32* y, const uint32_t dx[R],
                                               const uint32_t dy[R], const bool live[R], uint64_t q[R][4], Num&& num) {

@@ -12,9 +12,11 @@
 //    the 64 lanes compute 64 parents of 128 items (one chunk); chunks merge
 //    pairwise like a binary counter, the left chunk waiting in the wave's LDS
 //    stack, so every compression runs with all 64 lanes busy and no
-//    workgroup barrier is ever needed. The last 64 nodes are reduced to one
-//    with quad-cooperative compressions (4 lanes each), so the wave emits one
-//    node, 7 + logc levels above its items.
+//    workgroup barrier is ever needed. The last 64 nodes are reduced with
+//    quad-cooperative compressions (4 lanes each): to one, 7 + logc levels above
+//    the wave's items, or in large leaf stages to the 4 to 16 nodes where quads
+//    would leave most lanes idle, which the next stage hashes one per lane.
+//  * Small trees of a single proof: a quad per leaf, one node a workgroup.
 //  * Tail kernel: one workgroup reduces the last <= 2048 items to the root,
 //    writes it where the caller asks and advances the Fiat-Shamir transcript
 //    (mix the root, draw the next challenge) in the same launch; its narrow

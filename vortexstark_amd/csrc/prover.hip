@@ -33,9 +33,10 @@ namespace vx {
 
 // ---------------------------------------------------------------- trace generation
 // The trace f(0) = a, f(1) = b, f(i+2) = f(i) + f(i+1) (air.rs:85-131), one per
-// blockIdx.y: the pair (f(i), f(i+1)) moves k words on by
+// blockIdx.y (proof y of a batch takes ab[2y], ab[2y+1] and writes bs words past
+// proof 0): the pair (f(i), f(i+1)) moves k words on by
 // f(i+k) = F(k-1) f(i) + F(k) f(i+1), F the Fibonacci numbers, so a thread
-// reaches its run of FIB_RUN words by one such step for each set bit of the run's
+// reaches its run of words by one such step for each set bit of the run's
 // number (a block's bits scalar) and then only adds. Latency-bound to 2^18 words:
 // 3-4 us, where a matrix power and 256 words a thread took 14 us at 2^10 and 38 at
 // 2^16; 2^24 words are bound by the stores.
@@ -298,9 +299,6 @@ __global__ __launch_bounds__(DECOMMIT_THREADS) void decommit_kernel(const TreeDe
         }
     }
 }
-
-// Fibonacci traces of a batch: proof blockIdx.y gets (a, b) = ab[2y], ab[2y+1]
-// and writes its trace bs words past proof 0's.
 
 // Copies words of src to count - 1 places stride words apart (dst0 = src + stride).
 __global__ void replicate_kernel(const uint32_t* src, uint64_t words, uint64_t stride) {

@@ -1,6 +1,7 @@
 // Chunk depth of the Merkle stage kernels: a wave hashes 2^c chunks of 128
-// items, merging them as it goes, and ends with one 64 -> 1 reduction on
-// narrow levels, so its output is one node 7 + c levels above its items.
+// items, merging them as it goes, and ends with a reduction of its last 64 nodes
+// on narrow levels, to the one node 7 + c levels above its items or, in a large
+// leaf stage, to the several nodes (`keep`) below it.
 // Pure host logic (no device code), shared by the tree driver and its
 // autotuner.
 #pragma once
@@ -11,7 +12,7 @@
 namespace vx {
 
 constexpr uint32_t MERKLE_LOGC_MAX = 5;       // chunks per wave in a stage: up to 32
-constexpr uint32_t STAGE_MIN_WAVES = 3072;    // default rule: three waves per SIMD
+constexpr uint32_t STAGE_MIN_WAVES = 3072;    // pick_logc's own rule: three waves per SIMD
 constexpr uint32_t STAGE_PLAN_LOGS = 40;      // table index: log2 of the items of one launch
 
 // Tuned depth per log2 of the items one stage launch covers (every proof of a
@@ -26,7 +27,9 @@ inline uint32_t floor_log2(uint64_t x) { return x ? 63u - (uint32_t)__builtin_cl
 // Depth of a stage over n items per proof for `batch` proofs: the tuned depth
 // for n * batch items when there is one and use_plan is set, else the largest
 // c that still leaves STAGE_MIN_WAVES waves in the launch; never above
-// logc_max, and always at least two waves per proof.
+// logc_max, and always at least two waves per proof. Launches take their shape
+// from pick_stage below, which comes here for tuned sizes alone and has a
+// measured default of its own.
 inline uint32_t pick_logc(uint64_t n, uint32_t logc_max = MERKLE_LOGC_MAX, uint32_t batch = 1, bool use_plan = true) {
     const uint32_t lt = floor_log2(n * batch);
     int c = use_plan && lt < STAGE_PLAN_LOGS ? (int)stage_plan_table()[lt].load(std::memory_order_relaxed) - 1 : -1;
