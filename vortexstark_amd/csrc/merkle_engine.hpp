@@ -854,8 +854,9 @@ __device__ __forceinline__ void block_lane_levels(uint32_t* nodes, uint32_t* out
 // while it has more than 128 parents, one quad compression (0.76 us with its exchange) below,
 // then the transcript's two. The transcript's state is fetched before the first
 // level, and the last level writes the root where the transcript hashes it.
-// PRIO = false: the first level's waves have a SIMD each (launch_tail).
-template <class Src, bool PRIO>
+// PRIO = false: the first level's waves have a SIMD each; FEW: at most 16 nodes
+// (launch_tail).
+template <class Src, bool PRIO, bool FEW>
 __global__ __launch_bounds__(TAIL_THREADS) void merkle_tail_kernel(Src src0, uint32_t item_level, uint32_t n_items,
                                                                   LevelStore st0, TailOut out, uint64_t bs) {
     constexpr uint32_t W = MERKLE_TAIL_MAX / 2;
@@ -874,20 +875,17 @@ __global__ __launch_bounds__(TAIL_THREADS) void merkle_tail_kernel(Src src0, uin
     QuadTranscript tr = {};
     if (out.channel && tid < 64) tr.load(out.channel, out.init_channel != 0);
     uint32_t n = n_items / 2, lvl = item_level + 1;
-    // Nodes that quads can hash from the first level on: up to 16 of them by one
-    // wave, after a copy to LDS, more from where they lie.
     bool narrow = false;
-    if constexpr (IsNodes<Src>::value) {
-        narrow = n_items <= TAIL_QUAD_NODES;
-        if (n_items <= 16) {
+    if constexpr (IsNodes<Src>::value) narrow = FEW || (n_items <= TAIL_QUAD_NODES && n_items > 16);
+    if (narrow) {
+        if constexpr (IsNodes<Src>::value && FEW) {  // all levels by one wave
             if (tid < 8 * n_items) qa[tid] = src.nodes[8 * item_base + tid];
             n = n_items;
             lvl = item_level;
-        } else if (narrow) {
+        } else if constexpr (IsNodes<Src>::value) {
+            // the first level's quads read the nodes in place
             block_quad_level(src.nodes + 8 * item_base, qa, n, item_level, item_base, st);
         }
-    }
-    if (narrow) {
         lds_barrier();
     } else {
         for (uint32_t j = tid; j < n; j += TAIL_THREADS) {
@@ -931,10 +929,19 @@ __global__ __launch_bounds__(TAIL_THREADS) void merkle_tail_kernel(Src src0, uin
 template <class Src>
 inline void launch_tail(const Src& src, uint32_t item_level, uint32_t n_items, LevelStore st, TailOut out, uint32_t batch,
                         uint64_t bs, hipStream_t s) {
+    const dim3 grid(1, batch);
+    if constexpr (IsNodes<Src>::value) {
+        // nodes that one wave's quads can hash from the first level on; a kernel of its
+        // own, since the choice costs the one for more nodes 0.5 us
+        if (n_items <= 16) {
+            merkle_tail_kernel<Src, false, true><<<grid, TAIL_THREADS, 0, s>>>(src, item_level, n_items, st, out, bs);
+            return;
+        }
+    }
     if (n_items <= 512 && batch <= LONE_THREADS / 256)
-        merkle_tail_kernel<Src, false><<<dim3(1, batch), TAIL_THREADS, 0, s>>>(src, item_level, n_items, st, out, bs);
+        merkle_tail_kernel<Src, false, false><<<grid, TAIL_THREADS, 0, s>>>(src, item_level, n_items, st, out, bs);
     else
-        merkle_tail_kernel<Src, true><<<dim3(1, batch), TAIL_THREADS, 0, s>>>(src, item_level, n_items, st, out, bs);
+        merkle_tail_kernel<Src, true, false><<<grid, TAIL_THREADS, 0, s>>>(src, item_level, n_items, st, out, bs);
 }
 
 }  // namespace vx
