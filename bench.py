@@ -57,7 +57,8 @@ VALU_PEAK_TOPS = 256 * 4 * 16 * 2.4e9 / 1e12
 # The most a SIMD issues: beside one wave's instruction a second wave's plain add,
 # subtract, logic or shift. A compression's 480 v_add3 and v_alignbit take a slot
 # each and its 488 adds and xors can all go beside them, so hashing is priced
-# against twice the rate of one instruction a slot.
+# against twice the rate of one instruction a slot, and so are the transforms: 7 of
+# a butterfly's 12 instructions are plain adds, subtracts and an and.
 VALU_PAIRED_TOPS = 2 * VALU_PEAK_TOPS
 # VALU ops of one Blake2s compression on gfx950: 10 rounds x 8 G x 12 ops (v_add3,
 # v_add, v_xor, v_alignbit) + 8 three-input xors of the feed-forward (v_bitop3)
@@ -112,15 +113,21 @@ def golden_case(label):
     return None
 
 
-def stage_compressions(n_items: int, leaf_blocks: int) -> int:
+def stage_compressions(vx, n_items: int, leaf_blocks: int, depth_max: int = 5) -> int:
     """Blake2s compressions of the first stage kernel of a tree: leaf hashes of
-    n_items leaves (leaf_blocks each) and every node below each wave's output
-    (a wave reduces 128 * 2^logc items to one node; logc as the library picks it)."""
-    logc = 5
-    while logc > 0 and (n_items >> (7 + logc)) < 1024:
-        logc -= 1
-    waves = n_items >> (7 + logc)
-    return n_items * leaf_blocks + (n_items - waves)
+    n_items leaves (leaf_blocks each) and every node below the nodes a wave hands
+    on. A wave covers 128 * 2^c items, c the tuned depth of that size or the
+    library's default, at most depth_max, and from 2^18 items on hands on
+    several nodes."""
+    l = n_items.bit_length() - 1
+    c = vx.merkle_stage_plan(l)
+    if c < 0:
+        c = 4 if l >= 25 else 3 if l >= 22 else 2 if l >= 20 else 1 if l >= 19 else 0
+    c = min(c, depth_max)
+    while c > 0 and (n_items >> (7 + c)) < 2:
+        c -= 1
+    keep = (16 if c >= 2 else 4 << c) if l >= 18 else 1
+    return n_items * leaf_blocks + n_items - (n_items >> (7 + c)) * keep
 
 
 MEASURED = {}  # filled at start-up: measured VALU peak, NTT plans
@@ -278,7 +285,7 @@ def bench_plain(vx, args) -> dict:
     E = 1 << (log_n + 2)
     # dominant kernel: the first commit stage of the quotient tree (Blake2s over E leaves)
     dom_ms = phases.get("quotient_commit:stage_leaf")
-    roofline = valu_roofline("merkle_stage_kernel<SrcQuotient>", stage_compressions(E, 1), dom_ms) if dom_ms else None
+    roofline = valu_roofline("merkle_stage_kernel<SrcQuotient>", stage_compressions(vx, E, 1), dom_ms) if dom_ms else None
     ntt_ms = phases.get("lde:evaluate")
     # the LDE's evaluation plan; when it ends in a replicating pass the library
     # runs the interpolation's layers above the pass's start in that pass too
@@ -309,8 +316,9 @@ def bench_plain(vx, args) -> dict:
         ops = bfly * OPS_PER_BUTTERFLY
         achieved = ops / (ntt_ms * 1e-3) / 1e12
         roofline_ntt = {"bound": "valu", "kernel": "ntt_pass_kernel<true> (%s)" % what,
-                        "achieved": round(achieved, 3), "peak": VALU_PEAK_TOPS, "unit": "Tops/s (int32 lane-ops)",
-                        "frac": round(achieved / VALU_PEAK_TOPS, 4), "butterflies": bfly,
+                        "achieved": round(achieved, 3), "peak": round(VALU_PAIRED_TOPS, 2),
+                        "unit": "Tops/s (int32 lane-ops)",
+                        "frac": round(achieved / VALU_PAIRED_TOPS, 4), "butterflies": bfly,
                         "ops_per_butterfly": OPS_PER_BUTTERFLY, "phase_ms": round(ntt_ms, 4)}
     # pipeline-level bound: 6E Blake2s compressions at the paired issue rate
     t_valu_ms = 6 * E * OPS_PER_COMPRESSION / (VALU_PAIRED_TOPS * 1e12) * 1e3
@@ -405,7 +413,7 @@ def bench_wide(vx, args) -> dict:
     S = w.lifting_log_size
     dom_ms = phases.get("lifted_commit:stage_leaf")
     blocks = (len(logs) + 15) // 16
-    roofline = valu_roofline("merkle_stage_kernel<SrcLifted>", stage_compressions(1 << S, blocks), dom_ms) \
+    roofline = valu_roofline("merkle_stage_kernel<SrcLifted>", stage_compressions(vx, 1 << S, blocks, 2), dom_ms) \
         if dom_ms else None
     log(f"wide: {1e3 * dt:.3f} ms per commitment, {trace_elems / dt / 1e6:.1f} Melem/s, parity {parity}")
     cpu = None
